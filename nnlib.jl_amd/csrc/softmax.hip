@@ -1,209 +1,392 @@
-// softmax over the first (contiguous) dimension of a column-major (rows, cols) matrix.
-// Replaces NNlib's _softmax! for dims = 1 (src/softmax.jl:69-79); arithmetic in fp32.
+// The softmax family over the first (contiguous) dimension of a column-major (len, cols) matrix: softmax, logsoftmax,
+// logsumexp and the two gradients.  Replaces, for dims = 1, NNlib's _softmax! (src/softmax.jl:69-79), _logsoftmax!
+// (:137-147), logsumexp (:200-203), _∇softmax! (:107-110) and _∇logsoftmax! (:175-177).  Arithmetic in fp32.
+//
+// Bound by memory: every element has to be read and written once (the gradients read two arrays).  Columns therefore
+// stay in registers between the reductions and the result, as 16-byte pieces, whatever their length and alignment:
+// * A piece is VEC = 16 / sizeof(T) consecutive elements counted from the column's own start.  Columns of odd length
+//   start at any element, so pieces are loads and stores of element alignment, which the memory pipeline takes at full
+//   width.  The last piece is moved back to end with the column and its lane counts and stores only the elements that the piece
+//   before it does not hold.
+// * Short columns (up to 256 pieces): 4 to 64 lanes of a wavefront per column, up to four pieces a lane, reductions by
+//   shuffles.  Longer ones (up to 8192 pieces): one workgroup of as many wavefronts as the column has work for, 4 or 8
+//   pieces a lane, one barrier per reduction.  Beyond that the column is streamed twice (running maximum and sum, then
+//   the result).
+// Times before are those of the kernels this replaced (at most 4096 elements of a column in registers, one element a lane
+// unless the columns were 16-byte aligned, three passes over longer ones); a large copy moves 4.8 TB/s on this card:
+//   10000 x 4096 Float32          softmax 164 -> 80 us   logsoftmax 174 -> 75    its gradient 196 -> 91 (5.4 TB/s)
+//   10007 x 8192 BFloat16                 269 -> 84                 282 -> 80                 328 -> 104
+//   1001 x 65536 BFloat16                 161 -> 40                 200 -> 40                 357 -> 68
+//   37 x 524288 Float32                    86 -> 30                1077 -> 27                1017 -> 35
+//   131072 x 1024 Float32                 919 -> 293                876 -> 290                625 -> 368
 #include "common.h"
+#include "softmax_columns.h"
 
-// The reference's elementwise rule: with column maximum m,
-//   m == +Inf : e = (x == +Inf) ? 1 : 0          (src/softmax.jl:74-75)
-//   otherwise : e = exp(x - m)                   (src/softmax.jl:72; -Inf - -Inf = NaN stays NaN)
-__device__ static inline float softmax_term(float x, float m) {
+namespace {
+
+typedef u32x4_t piece_any4_t __attribute__((aligned(4)));   // a piece that starts at any 4-byte (2-byte) element
+typedef u32x4_t piece_any2_t __attribute__((aligned(2)));
+
+template <typename T> struct Column {
+    typedef typename T::type t;
+    static constexpr int VEC = 16 / (int)sizeof(t);
+    __device__ static u32x4_t load(const t *p) {
+        if constexpr (VEC == 4) return *(const piece_any4_t *)p;
+        else return *(const piece_any2_t *)p;
+    }
+    __device__ static void store(t *p, const u32x4_t &v) {
+        if constexpr (VEC == 4) *(piece_any4_t *)p = v;
+        else *(piece_any2_t *)p = v;
+    }
+    __device__ static float get(const u32x4_t &v, int e) {
+        if constexpr (VEC == 4) return __builtin_bit_cast(floatx4_t, v)[e];
+        else return T::to_f32(__builtin_bit_cast(typename T::vec8, v)[e]);
+    }
+    __device__ static void set(u32x4_t &v, int e, float x) {
+        if constexpr (VEC == 4) {
+            floatx4_t f = __builtin_bit_cast(floatx4_t, v);
+            f[e] = x;
+            v = __builtin_bit_cast(u32x4_t, f);
+        } else {
+            typename T::vec8 h = __builtin_bit_cast(typename T::vec8, v);
+            h[e] = T::from_f32(x);
+            v = __builtin_bit_cast(u32x4_t, h);
+        }
+    }
+    // e^x: the library function for Float32; 16-bit results are rounded far above the error of the hardware 2^x
+    __device__ static float exp(float x) {
+        if constexpr (VEC == 4) return expf(x);
+        else return mi_exp2(x * MI_LOG2E);
+    }
+};
+
+// the reference's elementwise rules given the column maximum m
+template <typename T> __device__ inline float softmax_term(float x, float m) {   // src/softmax.jl:72-75
     if (m == MI_POS_INF) return x == MI_POS_INF ? 1.0f : 0.0f;
-    return expf(x - m);
+    return Column<T>::exp(x - m);
+}
+__device__ inline float logsoftmax_shift(float x, float m) {   // src/softmax.jl:140-144
+    if (m == MI_POS_INF) return x == MI_POS_INF ? 0.0f : MI_NEG_INF;
+    return x - m;
+}
+template <typename T, int OP> __device__ inline float term(float x, float m) {
+    if (OP == OP_SOFTMAX) return softmax_term<T>(x, m);
+    if (OP == OP_LOGSOFTMAX) return Column<T>::exp(logsoftmax_shift(x, m));
+    return Column<T>::exp(x - m);   // logsumexp: no special cases (src/softmax.jl:202)
+}
+// the result of one element; forward: c0 = maximum, c1 = sum (Float32 softmax), 1 / sum (16-bit softmax) or log(sum);
+// gradients: x = dy, c0 = the sum
+template <typename T, int OP> __device__ inline float result(float x, float y, float c0, float c1) {
+    if (OP == OP_SOFTMAX) return Column<T>::VEC == 4 ? softmax_term<T>(x, c0) / c1 : softmax_term<T>(x, c0) * c1;
+    if (OP == OP_LOGSOFTMAX) return logsoftmax_shift(x, c0) - c1;
+    if (OP == OP_GRAD_SOFTMAX) return y * (x - c0);
+    return x - c0 * Column<T>::exp(y);
 }
 
-__device__ static inline float block_reduce(float v, float *red, bool is_max) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    v = is_max ? mi_wave_max(v) : mi_wave_sum(v);
-    __syncthreads(); // protect `red` from the previous use
-    if (lane == 0) red[wave] = v;
+// The pieces stay in their packed form from pass to pass: without this the compiler keeps what the pass before computed
+// of them (unpacked values, exponentials) as well, twice to three times the registers.
+template <int N> __device__ inline void keep_packed(u32x4_t (&raw)[N]) {
+#pragma unroll
+    for (int u = 0; u < N; u++) asm volatile("" : "+v"(raw[u]));
+}
+
+// Reduction over the lanes of a column: G <= 64 lanes of a wavefront, or (G = 0) the whole workgroup.  `red` is the slot
+// of this reduction; a slot is used again only after another reduction's barrier, so one barrier each is enough.
+template <bool IS_MAX, int G> __device__ inline float reduce(float v, float *red) {
+#pragma unroll
+    for (int o = (G ? G : 64) / 2; o > 0; o >>= 1) {
+        const float u = __shfl_xor(v, o, 64);
+        v = IS_MAX ? fmaxf(v, u) : v + u;
+    }
+    if (G) return v;
+    const int nw = blockDim.x >> 6;
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    float r = red[0];
-    for (int w = 1; w < nw; w++) r = is_max ? fmaxf(r, red[w]) : r + red[w];
-    return r;
+    v = red[0];
+    for (int w = 1; w < nw; w++) v = IS_MAX ? fmaxf(v, red[w]) : v + red[w];
+    return v;
 }
 
-// One workgroup per column.  Columns of up to CACHE*blockDim elements are held in
-// registers between the passes (one HBM read, one write); longer columns are re-read.
-template <typename T, int CACHE>
-__global__ __launch_bounds__(256) void softmax_dim1_kernel(const typename T::type *x,
-                                                            typename T::type *y, int64_t rows,
-                                                            int64_t cols) {
-    __shared__ float red[8];
+// One column held in registers.  G: lanes per column, 0 for a workgroup per column; NP: pieces per lane (the host picks
+// both so that lanes * NP covers the column).
+template <typename T, int OP, int NP, int G>
+__global__ __launch_bounds__(G ? 256 : 1024) void softmax_column_kernel(const typename T::type *x, const typename T::type *x2,
+                                                                         typename T::type *y, int len, int64_t cols) {
+    typedef typename T::type t;
+    typedef Column<T> C;
+    constexpr int VEC = C::VEC;
+    constexpr bool GRAD = OP >= OP_GRAD_SOFTMAX;
+    constexpr bool KEEP_TERMS = OP == OP_SOFTMAX && VEC == 4;   // Float32 softmax: the terms take the place of the elements
+    __shared__ float red[2][16];
+    const int lanes = G ? G : blockDim.x, lane = G ? (int)threadIdx.x & (G - 1) : (int)threadIdx.x;
+    const int per_block = G ? 256 / (G ? G : 1) : 1;
+    const int last = (len - 1) / VEC;   // the column's last piece, which may be a partial one
+    int parity = 0;
+    for (int64_t c = (int64_t)blockIdx.x * per_block + (G ? threadIdx.x / (G ? G : 1) : 0); c < cols; c += (int64_t)gridDim.x * per_block) {
+        const t *xc = x + c * len, *x2c = GRAD ? x2 + c * len : nullptr;
+        t *yc = y + (OP == OP_LOGSUMEXP ? 0 : c * len);
+        u32x4_t raw[NP], raw2[GRAD ? NP : 1];
+        // lanes past the end read the last piece again: loads without branches, all of them in flight together
+#pragma unroll
+        for (int u = 0; u < NP; u++) {
+            const int p = lane + u * lanes, at = p < last ? p * VEC : len - VEC;
+            raw[u] = C::load(xc + at);
+            if (GRAD) raw2[u] = C::load(x2c + at);
+        }
+        // elements of the last piece that another piece holds, and whole pieces past it, count for nothing
+#pragma unroll
+        for (int u = 0; u < NP; u++) {
+            const int p = lane + u * lanes, skip = p * VEC - (len - VEC);
+            if (p >= last && skip > 0) {
+#pragma unroll
+                for (int e = 0; e < VEC; e++)
+                    if (e < skip) {
+                        C::set(raw[u], e, GRAD ? 0.0f : MI_NEG_INF);
+                        if (GRAD) C::set(raw2[u], e, 0.0f);
+                    }
+            }
+        }
+        float c0, c1 = 0.0f;
+        if constexpr (GRAD) {
+            float s = 0.0f;
+#pragma unroll
+            for (int u = 0; u < NP; u++)
+#pragma unroll
+                for (int e = 0; e < VEC; e++) s += OP == OP_GRAD_SOFTMAX ? C::get(raw[u], e) * C::get(raw2[u], e) : C::get(raw[u], e);
+            c0 = reduce<false, G>(s, red[parity]);
+            parity ^= 1;
+            keep_packed(raw);
+            keep_packed(raw2);
+        } else {
+            // fmaxf skips a NaN, but the NaN still reaches every element of its column through the sum
+            float m = MI_NEG_INF, s = 0.0f;
+#pragma unroll
+            for (int u = 0; u < NP; u++)
+#pragma unroll
+                for (int e = 0; e < VEC; e++) m = fmaxf(m, C::get(raw[u], e));
+            c0 = reduce<true, G>(m, red[0]);
+            keep_packed(raw);
+            // one test of the maximum for all elements of the column: a test per element becomes as many live values
+            const auto add_terms = [&](auto rule) {
+#pragma unroll
+                for (int u = 0; u < NP; u++)
+#pragma unroll
+                    for (int e = 0; e < VEC; e++) {
+                        const float v = rule(C::get(raw[u], e));
+                        if (KEEP_TERMS) C::set(raw[u], e, v);
+                        s += v;
+                    }
+            };
+            if (OP != OP_LOGSUMEXP && c0 == MI_POS_INF) add_terms([](float v) { return v == MI_POS_INF ? 1.0f : 0.0f; });
+            else add_terms([&](float v) { return C::exp(v - c0); });
+            s = reduce<false, G>(s, red[1]);
+            keep_packed(raw);
+            c1 = OP != OP_SOFTMAX ? logf(s) : VEC == 4 ? s : 1.0f / s;
+        }
+        if constexpr (OP == OP_LOGSUMEXP) {
+            if (lane == 0) y[c] = T::from_f32(c0 + c1);
+        } else {
+            const auto write = [&](auto rule) {
+#pragma unroll
+                for (int u = 0; u < NP; u++) {
+                    const int p = lane + u * lanes, at = p < last ? p * VEC : len - VEC, skip = p * VEC - at;
+                    if (p > last) continue;
+                    u32x4_t r = raw[u];
+#pragma unroll
+                    for (int e = 0; e < VEC; e++) C::set(r, e, rule(C::get(raw[u], e), GRAD ? C::get(raw2[GRAD ? u : 0], e) : 0.0f));
+                    if (skip == 0) C::store(yc + at, r);
+                    else
+#pragma unroll
+                        for (int e = 0; e < VEC; e++)
+                            if (e >= skip) yc[at + e] = T::from_f32(C::get(r, e));
+                }
+            };
+            if (!GRAD && !KEEP_TERMS && c0 == MI_POS_INF) write([&](float v, float) { return result<T, OP>(v, 0.0f, MI_POS_INF, c1); });
+            else write([&](float v, float v2) {
+                if (KEEP_TERMS) return v / c1;
+                if (OP == OP_SOFTMAX) return C::exp(v - c0) * c1;
+                if (OP == OP_LOGSOFTMAX) return v - c0 - c1;
+                return result<T, OP>(v, v2, c0, c1);
+            });
+        }
+    }
+}
+
+// Columns longer than the registers of a workgroup: one pass for the running maximum and the sum against it, one for the
+// result.  Four pieces in flight per lane; the tail piece is handled element by element.
+template <typename T, int OP>
+__global__ __launch_bounds__(1024) void softmax_column_stream_kernel(const typename T::type *x, const typename T::type *x2,
+                                                                      typename T::type *y, int64_t len, int64_t cols) {
+    typedef typename T::type t;
+    typedef Column<T> C;
+    constexpr int VEC = C::VEC, U = 4;
+    constexpr bool GRAD = OP >= OP_GRAD_SOFTMAX;
+    __shared__ float red[2][16];
+    const int64_t whole = len / VEC, step = (int64_t)blockDim.x * U;
     for (int64_t c = blockIdx.x; c < cols; c += gridDim.x) {
-        const typename T::type *xc = x + c * rows;
-        typename T::type *yc = y + c * rows;
-        const bool cached = rows <= (int64_t)CACHE * blockDim.x;
-        float v[CACHE];
-        float m = MI_NEG_INF;
-        if (cached) {
-#pragma unroll
-            for (int i = 0; i < CACHE; i++) {
-                int64_t r = (int64_t)i * blockDim.x + threadIdx.x;
-                v[i] = r < rows ? T::to_f32(xc[r]) : MI_NEG_INF;
-                m = fmaxf(m, v[i]);
+        const t *xc = x + c * len, *x2c = GRAD ? x2 + c * len : nullptr;
+        t *yc = y + (OP == OP_LOGSUMEXP ? 0 : c * len);
+        float m = MI_NEG_INF, s = 0.0f;
+        const auto add = [&](float v, float v2) {
+            if (GRAD) s += OP == OP_GRAD_SOFTMAX ? v * v2 : v;
+            else s += term<T, OP>(v, m);
+        };
+        // nothing but -Inf so far adds no terms; a column of nothing else is NaN in any case.  A NaN entry stays in the sum.
+        const auto raise = [&](float top) {
+            if (top > m) {
+                s = m == MI_NEG_INF ? (s == s ? 0.0f : s) : s * C::exp(m - top);
+                m = top;
             }
-        } else {
-            for (int64_t r = threadIdx.x; r < rows; r += blockDim.x) m = fmaxf(m, T::to_f32(xc[r]));
-        }
-        m = block_reduce(m, red, true);
-        float s = 0.0f;
-        if (cached) {
+        };
+        for (int64_t p0 = threadIdx.x; p0 < whole; p0 += step) {
+            u32x4_t raw[U], raw2[U];
 #pragma unroll
-            for (int i = 0; i < CACHE; i++) {
-                int64_t r = (int64_t)i * blockDim.x + threadIdx.x;
-                if (r < rows) {
-                    v[i] = softmax_term(v[i], m);
-                    s += v[i];
+            for (int u = 0; u < U; u++) {
+                const int64_t p = p0 + (int64_t)u * blockDim.x, at = (p < whole ? p : p0) * VEC;
+                raw[u] = C::load(xc + at);
+                if (OP == OP_GRAD_SOFTMAX) raw2[u] = C::load(x2c + at);
+            }
+            if constexpr (!GRAD) {
+                float top = MI_NEG_INF;
+#pragma unroll
+                for (int u = 0; u < U; u++)
+#pragma unroll
+                    for (int e = 0; e < VEC; e++) top = fmaxf(top, C::get(raw[u], e));
+                raise(top);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (p0 + (int64_t)u * blockDim.x < whole)
+#pragma unroll
+                    for (int e = 0; e < VEC; e++) {
+                        const float v = C::get(raw[u], e);
+                        if (GRAD || m != MI_NEG_INF || v != v) add(v, OP == OP_GRAD_SOFTMAX ? C::get(raw2[u], e) : 0.0f);
+                    }
+        }
+        for (int64_t j = whole * VEC + threadIdx.x; j < len; j += blockDim.x) {
+            const float v = T::to_f32(xc[j]);
+            if (!GRAD) raise(v);
+            if (GRAD || m != MI_NEG_INF || v != v) add(v, OP == OP_GRAD_SOFTMAX ? T::to_f32(x2c[j]) : 0.0f);
+        }
+        float c0, c1 = 0.0f;
+        if constexpr (GRAD) {
+            c0 = reduce<false, 0>(s, red[0]);
+        } else {
+            c0 = reduce<true, 0>(m, red[0]);
+            // a lane that has seen nothing but -Inf holds no terms (or a NaN)
+            s = m == c0 || s != s ? s : (m == MI_NEG_INF ? 0.0f : s * C::exp(m - c0));
+            s = reduce<false, 0>(s, red[1]);
+            if (c0 == MI_NEG_INF) s = __builtin_nanf("");
+            c1 = OP != OP_SOFTMAX ? logf(s) : VEC == 4 ? s : 1.0f / s;
+        }
+        if constexpr (OP == OP_LOGSUMEXP) {   // the reference's x - max is Inf - Inf for an infinite maximum
+            if (threadIdx.x == 0) y[c] = T::from_f32(c0 == MI_POS_INF ? __builtin_nanf("") : c0 + c1);
+        } else {
+            for (int64_t p0 = threadIdx.x; p0 < whole; p0 += step) {
+                u32x4_t raw[U], raw2[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int64_t p = p0 + (int64_t)u * blockDim.x, at = (p < whole ? p : p0) * VEC;
+                    raw[u] = C::load(xc + at);
+                    if (GRAD) raw2[u] = C::load(x2c + at);
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int64_t p = p0 + (int64_t)u * blockDim.x;
+                    if (p >= whole) break;
+                    u32x4_t r = raw[u];
+#pragma unroll
+                    for (int e = 0; e < VEC; e++) C::set(r, e, result<T, OP>(C::get(raw[u], e), GRAD ? C::get(raw2[u], e) : 0.0f, c0, c1));
+                    C::store(yc + p * VEC, r);
                 }
             }
-        } else {
-            for (int64_t r = threadIdx.x; r < rows; r += blockDim.x) s += softmax_term(T::to_f32(xc[r]), m);
+            for (int64_t j = whole * VEC + threadIdx.x; j < len; j += blockDim.x)
+                yc[j] = T::from_f32(result<T, OP>(T::to_f32(xc[j]), GRAD ? T::to_f32(x2c[j]) : 0.0f, c0, c1));
         }
-        s = block_reduce(s, red, false);
-        if (cached) {
+        __syncthreads();   // red is written again by the next column
+    }
+}
+
+// Columns shorter than one piece: a thread each.
+template <typename T, int OP>
+__global__ __launch_bounds__(256) void softmax_tiny_column_kernel(const typename T::type *x, const typename T::type *x2,
+                                                                   typename T::type *y, int len, int64_t cols) {
+    constexpr int MOST = Column<T>::VEC - 1;
+    constexpr bool GRAD = OP >= OP_GRAD_SOFTMAX;
+    for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < cols; c += (int64_t)gridDim.x * 256) {
+        float v[MOST], v2[MOST], m = MI_NEG_INF, s = 0.0f;
 #pragma unroll
-            for (int i = 0; i < CACHE; i++) {
-                int64_t r = (int64_t)i * blockDim.x + threadIdx.x;
-                if (r < rows) yc[r] = T::from_f32(v[i] / s);
+        for (int j = 0; j < MOST; j++)
+            if (j < len) {
+                v[j] = T::to_f32(x[c * len + j]);
+                v2[j] = GRAD ? T::to_f32(x2[c * len + j]) : 0.0f;
+                m = fmaxf(m, v[j]);
             }
+#pragma unroll
+        for (int j = 0; j < MOST; j++)
+            if (j < len) s += GRAD ? (OP == OP_GRAD_SOFTMAX ? v[j] * v2[j] : v[j]) : term<T, OP>(v[j], m);
+        if constexpr (OP == OP_LOGSUMEXP) {
+            y[c] = T::from_f32(m + logf(s));
         } else {
-            for (int64_t r = threadIdx.x; r < rows; r += blockDim.x)
-                yc[r] = T::from_f32(softmax_term(T::to_f32(xc[r]), m) / s);
+            const float c0 = GRAD ? s : m, c1 = OP == OP_LOGSOFTMAX ? logf(s) : Column<T>::VEC == 4 ? s : 1.0f / s;
+#pragma unroll
+            for (int j = 0; j < MOST; j++)
+                if (j < len) y[c * len + j] = T::from_f32(result<T, OP>(v[j], v2[j], c0, c1));
         }
     }
 }
 
-// Short columns: one wavefront per column, four columns per workgroup.
-template <typename T>
-__global__ __launch_bounds__(256) void softmax_dim1_wave_kernel(const typename T::type *x,
-                                                                 typename T::type *y, int64_t rows,
-                                                                 int64_t cols) {
-    const int lane = threadIdx.x & 63;
-    int64_t c = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int64_t cstride = (int64_t)gridDim.x * 4;
-    for (; c < cols; c += cstride) {
-        const typename T::type *xc = x + c * rows;
-        typename T::type *yc = y + c * rows;
-        float v[4];
-        float m = MI_NEG_INF;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            int64_t r = i * 64 + lane;
-            v[i] = r < rows ? T::to_f32(xc[r]) : MI_NEG_INF;
-            m = fmaxf(m, v[i]);
-        }
-        m = mi_wave_max(m);
-        float s = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            int64_t r = i * 64 + lane;
-            if (r < rows) {
-                v[i] = softmax_term(v[i], m);
-                s += v[i];
-            }
-        }
-        s = mi_wave_sum(s);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            int64_t r = i * 64 + lane;
-            if (r < rows) yc[r] = T::from_f32(v[i] / s);
-        }
-    }
-}
-
-// Columns of up to 64 * NCH * VEC elements whose rows can be moved in 16-byte pieces: one wavefront per
-// column, NCH pieces per lane held in registers, reductions by wavefront shuffles only (no LDS, no
-// barrier): one read and one write per element with four columns in flight per workgroup.
-template <typename T, int NCH>
-__global__ __launch_bounds__(256) void softmax_dim1_wave_vec_kernel(const typename T::type *x, typename T::type *y,
-                                                                     int64_t rows, int64_t cols) {
+template <typename T, int OP>
+void launch(const void *x, const void *x2, void *y, int64_t len, int64_t cols, hipStream_t st) {
     typedef typename T::type t;
-    constexpr int VEC = 16 / (int)sizeof(t);
-    const int lane = threadIdx.x & 63;
-    const int64_t nchunks = rows / VEC;
-    int64_t c = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int64_t cstride = (int64_t)gridDim.x * 4;
-    for (; c < cols; c += cstride) {
-        const t *xc = x + c * rows;
-        t *yc = y + c * rows;
-        float v[NCH][VEC];
-        float m = MI_NEG_INF;
-#pragma unroll
-        for (int i = 0; i < NCH; i++) {
-            const int64_t ch = lane + 64 * i;
-            if (ch < nchunks) {
-                const u32x4_t raw = *(const u32x4_t *)(xc + ch * VEC);
-                if constexpr (VEC == 4) {
-                    const floatx4_t f = __builtin_bit_cast(floatx4_t, raw);
-#pragma unroll
-                    for (int e = 0; e < VEC; e++) v[i][e] = f[e];
-                } else {
-                    const typename T::vec8 h = __builtin_bit_cast(typename T::vec8, raw);
-#pragma unroll
-                    for (int e = 0; e < VEC; e++) v[i][e] = T::to_f32(h[e]);
-                }
-            } else {
-#pragma unroll
-                for (int e = 0; e < VEC; e++) v[i][e] = MI_NEG_INF;
-            }
-#pragma unroll
-            for (int e = 0; e < VEC; e++) m = fmaxf(m, v[i][e]);
-        }
-        m = mi_wave_max(m);
-        float s = 0.0f;
-#pragma unroll
-        for (int i = 0; i < NCH; i++)
-#pragma unroll
-            for (int e = 0; e < VEC; e++) {
-                // padding lanes hold -Inf: their term is 0 unless the whole column is -Inf (then NaN, as for real entries)
-                v[i][e] = (lane + 64 * i < nchunks) ? softmax_term(v[i][e], m) : 0.0f;
-                s += v[i][e];
-            }
-        s = mi_wave_sum(s);
-#pragma unroll
-        for (int i = 0; i < NCH; i++) {
-            const int64_t ch = lane + 64 * i;
-            if (ch < nchunks) {
-                if constexpr (VEC == 4) {
-                    floatx4_t f;
-#pragma unroll
-                    for (int e = 0; e < VEC; e++) f[e] = v[i][e] / s;
-                    *(floatx4_t *)(yc + ch * VEC) = f;
-                } else {
-                    typename T::vec8 h;
-#pragma unroll
-                    for (int e = 0; e < VEC; e++) h[e] = T::from_f32(v[i][e] / s);
-                    *(u32x4_t *)(yc + ch * VEC) = __builtin_bit_cast(u32x4_t, h);
-                }
-            }
-        }
-    }
-}
-
-template <typename T>
-static void launch_softmax(const void *x, void *y, int64_t rows, int64_t cols, hipStream_t st) {
-    typedef typename T::type t;
-    constexpr int VEC = 16 / (int)sizeof(t);
-    const bool vec_ok = rows % VEC == 0 && ((((uintptr_t)x) | ((uintptr_t)y)) & 15) == 0;
-    if (vec_ok && rows > 256 && rows <= 64 * 8 * VEC) {
-        int64_t blocks = (cols + 3) / 4;
-        if (blocks > 262144) blocks = 262144;
-        const dim3 g((unsigned)blocks), b(256);
-        const int64_t nch = (rows / VEC + 63) / 64;
-        if (nch <= 2) hipLaunchKernelGGL((softmax_dim1_wave_vec_kernel<T, 2>), g, b, 0, st, (const t *)x, (t *)y, rows, cols);
-        else if (nch <= 4) hipLaunchKernelGGL((softmax_dim1_wave_vec_kernel<T, 4>), g, b, 0, st, (const t *)x, (t *)y, rows, cols);
-        else hipLaunchKernelGGL((softmax_dim1_wave_vec_kernel<T, 8>), g, b, 0, st, (const t *)x, (t *)y, rows, cols);
-        return;
-    }
-    if (rows <= 256) {
-        int64_t blocks = (cols + 3) / 4;
-        if (blocks > 65536) blocks = 65536;
-        hipLaunchKernelGGL(softmax_dim1_wave_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, st, (const t *)x, (t *)y,
-                           rows, cols);
+    constexpr int VEC = Column<T>::VEC;
+    // A workgroup of 1024 threads (128 registers each) holds 8 pieces a lane.  Streamed instead, columns of 4096 to 8192
+    // pieces are level (softmax, 32000 Float32: 131 / 132 us for 2048 columns) or slower (their gradient: 151 / 193 us);
+    // 16 pieces a lane spill (50257 Float32, 1024 columns: 127 us, streamed 110).
+    constexpr int64_t CACHED = 8192;
+    const int64_t pieces = (len + VEC - 1) / VEC, most_blocks = 1 << 20;
+    const auto blocks = [&](int64_t per_block) {
+        const int64_t n = (cols + per_block - 1) / per_block;
+        return dim3((unsigned)(n < most_blocks ? n : most_blocks));
+    };
+#define MI_COLUMN(NP, G, LANES)                                                                                                 \
+    hipLaunchKernelGGL((softmax_column_kernel<T, OP, NP, G>), blocks(G ? 256 / (G ? G : 1) : 1), dim3(G ? 256 : LANES), 0, st,  \
+                       (const t *)x, (const t *)x2, (t *)y, (int)len, cols)
+    if (len < VEC) {
+        hipLaunchKernelGGL((softmax_tiny_column_kernel<T, OP>), blocks(256), dim3(256), 0, st, (const t *)x, (const t *)x2, (t *)y,
+                           (int)len, cols);
+    } else if (pieces <= 4) MI_COLUMN(1, 4, 256);
+    else if (pieces <= 8) MI_COLUMN(2, 4, 256);
+    else if (pieces <= 16) MI_COLUMN(2, 8, 256);
+    else if (pieces <= 32) MI_COLUMN(2, 16, 256);
+    else if (pieces <= 64) MI_COLUMN(2, 32, 256);
+    else if (pieces <= 128) MI_COLUMN(2, 64, 256);
+    else if (pieces <= 256) MI_COLUMN(4, 64, 256);
+    else if (pieces <= CACHED) {
+        // whole wavefronts, as few as the pieces need
+        const auto lanes = [&](int np) { return (unsigned)((pieces + 64 * np - 1) / (64 * np) * 64); };
+        if (pieces <= 4096) MI_COLUMN(4, 0, lanes(4));
+        else MI_COLUMN(8, 0, lanes(8));
     } else {
-        int64_t blocks = cols > 65536 ? 65536 : cols;
-        hipLaunchKernelGGL((softmax_dim1_kernel<T, 16>), dim3((unsigned)blocks), dim3(256), 0, st, (const t *)x, (t *)y,
-                           rows, cols);
+        hipLaunchKernelGGL((softmax_column_stream_kernel<T, OP>), blocks(1), dim3(1024), 0, st, (const t *)x, (const t *)x2, (t *)y, len, cols);
     }
+#undef MI_COLUMN
+}
+
+template <typename T> void launch_op(int op, const void *x, const void *x2, void *y, int64_t len, int64_t cols, hipStream_t st) {
+    if (op == OP_SOFTMAX) launch<T, OP_SOFTMAX>(x, x2, y, len, cols, st);
+    else if (op == OP_LOGSOFTMAX) launch<T, OP_LOGSOFTMAX>(x, x2, y, len, cols, st);
+    else if (op == OP_LOGSUMEXP) launch<T, OP_LOGSUMEXP>(x, x2, y, len, cols, st);
+    else if (op == OP_GRAD_SOFTMAX) launch<T, OP_GRAD_SOFTMAX>(x, x2, y, len, cols, st);
+    else launch<T, OP_GRAD_LOGSOFTMAX>(x, x2, y, len, cols, st);
+}
+
+}  // namespace
+
+void launch_softmax_columns(int32_t dtype, int op, const void *x, const void *x2, void *y, int64_t len, int64_t cols, hipStream_t st) {
+    if (dtype == MI_F32) launch_op<F32>(op, x, x2, y, len, cols, st);
+    else if (dtype == MI_F16) launch_op<F16>(op, x, x2, y, len, cols, st);
+    else launch_op<BF16>(op, x, x2, y, len, cols, st);
 }
 
 MI_API int32_t mi_softmax_dim1(int32_t dtype, const void *x, void *y, int64_t rows, int64_t cols, mi_stream s) {
@@ -212,10 +395,8 @@ MI_API int32_t mi_softmax_dim1(int32_t dtype, const void *x, void *y, int64_t ro
     if (rows == 0 || cols == 0) return MI_OK;
     if (!x || !y) return mi_set_error(MI_EINVAL, "mi_softmax_dim1: null pointer");
     hipStream_t st = (hipStream_t)s;
-    if (dtype == MI_F64) return launch_softmax_family_f64(0, x, nullptr, y, 1, rows, cols, st);
-    if (dtype == MI_F32) launch_softmax<F32>(x, y, rows, cols, st);
-    else if (dtype == MI_F16) launch_softmax<F16>(x, y, rows, cols, st);
-    else launch_softmax<BF16>(x, y, rows, cols, st);
+    if (dtype == MI_F64) return launch_softmax_family_f64(OP_SOFTMAX, x, nullptr, y, 1, rows, cols, st);
+    launch_softmax_columns(dtype, OP_SOFTMAX, x, nullptr, y, rows, cols, st);
     MI_LAUNCH_CHECK();
     return MI_OK;
 }

@@ -1,0 +1,9 @@
+// The operations of the softmax family and the launcher of its kernels for contiguous columns (softmax.hip).
+#pragma once
+#include "common.h"
+
+enum { OP_SOFTMAX = 0, OP_LOGSOFTMAX = 1, OP_LOGSUMEXP = 2, OP_GRAD_SOFTMAX = 3, OP_GRAD_LOGSOFTMAX = 4 };
+
+// y[:, c] from x[:, c] (gradients: x = dy, x2 = the forward result) for `cols` columns of `len` >= 1 contiguous elements
+// of a Float32 or 16-bit type; logsumexp writes one value per column.  y may be x or x2.
+void launch_softmax_columns(int32_t dtype, int op, const void *x, const void *x2, void *y, int64_t len, int64_t cols, hipStream_t st);

@@ -1,7 +1,8 @@
 // softmax / logsoftmax / logsumexp and the softmax gradients over any run of adjacent dimensions.
 // The array is viewed as (inner, len, outer), element (i, j, o) at i + inner*(j + len*o), and the
-// reduction runs over j.  Replaces, for device arrays, NNlib's
-//   _softmax!      src/softmax.jl:69-79        (dims other than 1; dims = 1 keeps its own kernels in softmax.hip)
+// reduction runs over j; contiguous columns (inner = 1) have kernels of their own in softmax.hip.
+// Replaces, for device arrays, NNlib's
+//   _softmax!      src/softmax.jl:69-79
 //   _logsoftmax!   src/softmax.jl:137-147
 //   logsumexp      src/softmax.jl:200-203
 //   _∇softmax!     src/softmax.jl:107-110      dx = dy*y - y*sum(dy*y)
@@ -10,13 +11,13 @@
 //
 // A workgroup of 256 threads owns TI consecutive `inner` positions of one `outer` slice (TI = a power
 // of two <= 64, chosen by the host from `inner`) and splits j over TJ = 256/TI slices; consecutive
-// lanes touch consecutive addresses whenever inner >= TI or inner == 1.  Columns of up to CACHE*TJ
+// lanes touch consecutive addresses whenever inner >= TI.  Columns of up to CACHE*TJ
 // elements stay in registers between the passes (one HBM read, one write); longer ones are re-read.
 #include "common.h"
+#include "softmax_columns.h"
 
 namespace {
 
-enum { OP_SOFTMAX = 0, OP_LOGSOFTMAX = 1, OP_LOGSUMEXP = 2, OP_GRAD_SOFTMAX = 3, OP_GRAD_LOGSOFTMAX = 4 };
 constexpr int CACHE = 16;
 
 struct Geometry {
@@ -661,7 +662,8 @@ int32_t dispatch(const char *name, int32_t dtype, const void *x, const void *x2,
     if (!x || !y || (OP >= OP_GRAD_SOFTMAX && !x2)) return mi_set_error(MI_EINVAL, "%s: null pointer", name);
     hipStream_t st = (hipStream_t)s;
     if (dtype == MI_F64) return launch_softmax_family_f64(OP, x, x2, y, inner, len, outer, st);
-    if (dtype == MI_F32) launch_nd<F32, OP>(x, x2, y, inner, len, outer, st);
+    if (inner == 1 && len > 0) launch_softmax_columns(dtype, OP, x, x2, y, len, outer, st);
+    else if (dtype == MI_F32) launch_nd<F32, OP>(x, x2, y, inner, len, outer, st);
     else if (dtype == MI_F16) launch_nd<F16, OP>(x, x2, y, inner, len, outer, st);
     else launch_nd<BF16, OP>(x, x2, y, inner, len, outer, st);
     MI_LAUNCH_CHECK();
@@ -714,10 +716,7 @@ MI_API int32_t mi_logsumexp_bwd(int32_t dtype, const void *dy, const void *x, co
 
 MI_API int32_t mi_softmax(int32_t op, int32_t dtype, const void *x, void *y, int64_t inner, int64_t len, int64_t outer,
                           mi_stream s) {
-    if (op == MI_SOFTMAX) {
-        if (inner == 1) return mi_softmax_dim1(dtype, x, y, len, outer, s);
-        return dispatch<OP_SOFTMAX>("mi_softmax", dtype, x, nullptr, y, inner, len, outer, s);
-    }
+    if (op == MI_SOFTMAX) return dispatch<OP_SOFTMAX>("mi_softmax", dtype, x, nullptr, y, inner, len, outer, s);
     if (op == MI_LOGSOFTMAX) return dispatch<OP_LOGSOFTMAX>("mi_softmax", dtype, x, nullptr, y, inner, len, outer, s);
     return mi_set_error(MI_EINVAL, "mi_softmax: op must be MI_SOFTMAX or MI_LOGSOFTMAX, got %d", op);
 }

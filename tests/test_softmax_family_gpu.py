@@ -274,3 +274,40 @@ def test_strided_softmax_at_the_benchmark_shape(nn, oracle, outer):
     for o in (0, outer - 1):
         ref = oracle.grad_softmax(dy[:, :, o:o + 1], y[:, :, o:o + 1], 2)
         assert np.abs(g[:, :, o:o + 1] - ref).max() <= 4 * TOL["bf16"] * max(1.0, np.abs(ref).max())
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("length", [1, 3, 4, 7, 8, 9, 17, 33, 64, 65, 127, 129, 257, 1025, 2047, 4097, 8193, 16385, 32768, 32769, 65537])
+def test_contiguous_columns_of_every_kernel_and_alignment(nn, oracle, dtype, length):
+    """Columns along dimension 1 around every split of the kernels (less than a piece, lanes of a wavefront, a
+    workgroup with 4 and 8 pieces a lane, streamed) at lengths that leave columns at every alignment and the last
+    piece partial; the gradients over the forward results; in place; the +-Inf / NaN rules of src/softmax.jl:72-75."""
+    rng = np.random.default_rng(length)
+    x = round_to(rng.standard_normal((length, 9)) * 2, dtype)
+    dy = round_to(rng.standard_normal((length, 9)), dtype)
+    if length > 3:
+        x[:, 1] = -np.inf                       # NaN column
+        x[length // 2, 2] = np.inf              # one 1, zeros
+        x[length - 1, 3] = np.nan               # NaN column
+        x[:length - 1, 4] = -np.inf             # the only finite entry is the last
+    d, tol = _dev(nn, x, dtype), TOL[dtype]
+    with np.errstate(invalid="ignore", divide="ignore"):
+        for log in (False, True):
+            ref = oracle.softmax(x, 1, log=log)
+            got = (nn.logsoftmax if log else nn.softmax)(d, dims=1).to_numpy()
+            assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isinf(got), np.isinf(ref))
+            fin = np.isfinite(ref)
+            assert np.abs(got[fin] - ref[fin]).max() <= tol * max(1.0, np.abs(ref[fin]).max())
+            same = _dev(nn, x, dtype)
+            (nn.logsoftmax_ if log else nn.softmax_)(same, dims=1)
+            assert np.array_equal(same.to_numpy(), got, equal_nan=True)
+            y = round_to(oracle.softmax(np.where(np.isfinite(x), x, 0), 1, log=log), dtype)
+            ref = oracle.grad_softmax(dy, y, 1, log=log)
+            grad = _dev(nn, dy, dtype)
+            (nn.grad_logsoftmax_ if log else nn.grad_softmax_)(grad, grad, _dev(nn, y, dtype), dims=1)
+            # the sum of `length` terms of size 1 in Float32: sqrt(length) 2^-24 of their size, well below tol
+            assert np.abs(grad.to_numpy() - ref).max() <= 4 * tol * max(1.0, np.abs(ref).max())
+        got, ref = nn.logsumexp(d, dims=1).to_numpy(), oracle.logsumexp(x, 1)
+        assert np.array_equal(np.isnan(got), np.isnan(ref))
+        fin = np.isfinite(ref)
+        assert np.abs(got[fin] - ref[fin]).max() <= tol * 10
