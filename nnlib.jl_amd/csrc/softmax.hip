@@ -24,20 +24,9 @@
 
 namespace {
 
-typedef u32x4_t piece_any4_t __attribute__((aligned(4)));   // a piece that starts at any 4-byte (2-byte) element
-typedef u32x4_t piece_any2_t __attribute__((aligned(2)));
-
-template <typename T> struct Column {
+template <typename T> struct Column : ColumnIO<T> {
     typedef typename T::type t;
     static constexpr int VEC = 16 / (int)sizeof(t);
-    __device__ static u32x4_t load(const t *p) {
-        if constexpr (VEC == 4) return *(const piece_any4_t *)p;
-        else return *(const piece_any2_t *)p;
-    }
-    __device__ static void store(t *p, const u32x4_t &v) {
-        if constexpr (VEC == 4) *(piece_any4_t *)p = v;
-        else *(piece_any2_t *)p = v;
-    }
     __device__ static float get(const u32x4_t &v, int e) {
         if constexpr (VEC == 4) return __builtin_bit_cast(floatx4_t, v)[e];
         else return T::to_f32(__builtin_bit_cast(typename T::vec8, v)[e]);

@@ -4,6 +4,21 @@
 
 enum { OP_SOFTMAX = 0, OP_LOGSOFTMAX = 1, OP_LOGSUMEXP = 2, OP_GRAD_SOFTMAX = 3, OP_GRAD_LOGSOFTMAX = 4 };
 
+// 16-byte pieces that start at any 4-byte (2-byte) element
+typedef u32x4_t piece_any4_t __attribute__((aligned(4)));
+typedef u32x4_t piece_any2_t __attribute__((aligned(2)));
+template <typename T> struct ColumnIO {
+    typedef typename T::type t;
+    __device__ static u32x4_t load(const t *p) {
+        if constexpr (sizeof(t) == 4) return *(const piece_any4_t *)p;
+        else return *(const piece_any2_t *)p;
+    }
+    __device__ static void store(t *p, const u32x4_t &v) {
+        if constexpr (sizeof(t) == 4) *(piece_any4_t *)p = v;
+        else *(piece_any2_t *)p = v;
+    }
+};
+
 // y[:, c] from x[:, c] (gradients: x = dy, x2 = the forward result) for `cols` columns of `len` >= 1 contiguous elements
 // of a Float32 or 16-bit type; logsumexp writes one value per column.  y may be x or x2.
 void launch_softmax_columns(int32_t dtype, int op, const void *x, const void *x2, void *y, int64_t len, int64_t cols, hipStream_t st);

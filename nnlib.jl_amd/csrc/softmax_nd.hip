@@ -9,10 +9,11 @@
 //   _∇logsoftmax!  src/softmax.jl:175-177      dx = dy - sum(dy)*exp(y)
 // Arithmetic in fp32.
 //
-// A workgroup of 256 threads owns TI consecutive `inner` positions of one `outer` slice (TI = a power
-// of two <= 64, chosen by the host from `inner`) and splits j over TJ = 256/TI slices; consecutive
-// lanes touch consecutive addresses whenever inner >= TI.  Columns of up to CACHE*TJ
-// elements stay in registers between the passes (one HBM read, one write); longer ones are re-read.
+// Rows of at least 16 bytes take the kernels further down, which move 16-byte pieces at any alignment.  Narrower ones
+// (inner below 4, 16-bit types below 8) take softmax_nd_kernel: a workgroup of 256 threads owns TI consecutive `inner`
+// positions of one `outer` slice (TI = a power of two, chosen by the host from `inner`) and splits j over TJ = 256/TI
+// slices.  Columns of up to CACHE*TJ elements stay in registers between the passes (one HBM read, one write); longer
+// ones are re-read.
 #include "common.h"
 #include "softmax_columns.h"
 
@@ -164,9 +165,13 @@ __global__ __launch_bounds__(256) void softmax_nd_kernel(const typename T::type 
 }
 
 // ---- reductions over a strided dimension with wide rows ----------------------------------------------
-// inner is a multiple of VEC (16 bytes of elements) and every row starts 16-byte aligned: a thread owns
-// VEC consecutive `inner` positions and walks j in steps of TJ; TI threads side by side cover TI*VEC
-// positions, so a wavefront reads 64/TI rows of TI*16 contiguous bytes per load.  Columns of up to 8192
+// Rows hold at least VEC elements (16 bytes): a thread owns VEC consecutive `inner` positions and walks j in
+// steps of TJ; TI threads side by side cover TI*VEC positions, so a wavefront reads 64/TI rows of TI*16
+// contiguous bytes per load.  Rows may start at any element (the memory pipeline takes 16-byte loads and stores
+// of element alignment), and where `inner` is no multiple of VEC the last thread's positions are moved back to
+// end with the row: it stores only those that the thread before it does not own (`skip`), one by one.
+// (222 x 3664 x 80 Float32 softmax 1242 -> 168 us, its gradient 924 -> 263; 255 x 4096 x 128 bf16 1253 -> 195 and
+// 1014 -> 309; such rows went one element a lane and were read three times.)  Columns of up to 8192
 // elements (4096 for the gradients) are held in registers by a 512-thread workgroup: one read, one
 // write.  Longer ones are streamed: one pass finds the maximum and the sum together (running maximum,
 // sum rescaled when it grows), a second pass writes: two reads and one write per element.
@@ -197,18 +202,14 @@ struct VecIO {
             return __builtin_bit_cast(u32x4_t, h);
         }
     }
-    __device__ static void store(t *p, const float (&v)[VEC]) {
-        if constexpr (VEC == 4) {
-            floatx4_t f;
+    __device__ static u32x4_t load(const t *p) { return ColumnIO<T>::load(p); }
+    // the last VEC - skip positions
+    __device__ static void store(t *p, const float (&v)[VEC], int skip) {
+        if (skip == 0) ColumnIO<T>::store(p, pack(v));
+        else
 #pragma unroll
-            for (int e = 0; e < 4; e++) f[e] = v[e];
-            *(floatx4_t *)p = f;
-        } else {
-            typename T::vec8 h;
-#pragma unroll
-            for (int e = 0; e < 8; e++) h[e] = T::from_f32(v[e]);
-            *(u32x4_t *)p = __builtin_bit_cast(u32x4_t, h);
-        }
+            for (int e = 0; e < VEC; e++)
+                if (e >= skip) p[e] = T::from_f32(v[e]);
     }
 };
 
@@ -291,15 +292,15 @@ template <typename T>
 struct CachedTile {
     __amdgpu_buffer_rsrc_t rx, rx2, ry;   // the slab of the tile's outer index in x, x2 (gradients) and y
     int64_t o;                            // outer index
-    int col;                              // first column of the tile
+    int col, skip;                        // this thread's first column; how many of its columns the thread before it owns
     int voff, nrows;                      // this thread's byte offset in the slab; pieces it holds
     bool ok;                              // the thread's columns exist
 };
 
 // FULL: every thread holds NP pieces of a valid column (len = NP * TJ, inner a multiple of TI * VEC), so
-// the passes are straight-line code.  Columns with infinities take the reference's special cases through
+// the passes are straight-line code.  RAGGED: inner is no multiple of VEC.  Columns with infinities take the reference's special cases through
 // a branch that is uniform over the wavefront.
-template <typename T, int OP, int VEC, int NP, int NT, bool FULL>
+template <typename T, int OP, int VEC, int NP, int NT, bool FULL, bool RAGGED>
 __global__ __launch_bounds__(NT, (NP * (OP >= OP_GRAD_SOFTMAX ? 2 : 1) <= 16 && OP != OP_LOGSUMEXP ? 2 : 1) * NT / 256) void softmax_nd_cached_kernel(
         const typename T::type *x, const typename T::type *x2, typename T::type *y, Geometry g) {
     typedef typename T::type t;
@@ -313,18 +314,19 @@ __global__ __launch_bounds__(NT, (NP * (OP >= OP_GRAD_SOFTMAX ? 2 : 1) <= 16 && 
     const int inner = (int)g.inner, len = (int)g.len;   // a slab is below 2 GiB (host)
     const int slab_bytes = inner * len * SZ;
     const int step_bytes = inner * tj * SZ;   // between consecutive rows of one thread
-    // the thread's offset within a tile whose first column is 0 (threads past the column's end never use it)
-    const int thread_off = js < len ? (il * VEC + inner * js) * SZ : 0;
+    const int row0_off = js < len ? inner * js * SZ : 0;   // the thread's first row (threads past the column's end never use it)
     // scalar offset of a thread's u-th piece; 0 for pieces that lie past the column's end for every thread
     const auto row_off = [&](int u) { return FULL || u * tj < len ? step_bytes * u : 0; };
     const auto locate = [&](int64_t tile0) {
         CachedTile<T> c;
         const int64_t tile = xcd_order(tile0, n_tiles);
         c.o = tile / g.n_itiles;
-        c.col = (int)(tile % g.n_itiles) * ti * VEC;
-        c.ok = FULL || c.col + il * VEC < inner;
+        const int first = ((int)(tile % g.n_itiles) * ti + il) * VEC;
+        c.ok = FULL || first < inner;
+        c.col = !RAGGED || first <= inner - VEC ? first : inner - VEC;
+        c.skip = RAGGED ? first - c.col : 0;
         c.nrows = FULL ? NP : (c.ok && js < len ? (len - js + tj - 1) / tj : 0);   // <= NP (host)
-        c.voff = thread_off + c.col * SZ;
+        c.voff = row0_off + c.col * SZ;
         const int64_t slab = g.inner * g.len * c.o;
         c.rx = __builtin_amdgcn_make_buffer_rsrc((void *)(x + slab), 0, slab_bytes, 0x00020000);
         c.rx2 = __builtin_amdgcn_make_buffer_rsrc((void *)((GRAD ? x2 : x) + slab), 0, slab_bytes, 0x00020000);
@@ -341,9 +343,19 @@ __global__ __launch_bounds__(NT, (NP * (OP >= OP_GRAD_SOFTMAX ? 2 : 1) <= 16 && 
     // data registers of a 16-byte buffer store away from the store only when its scalar offset is not a
     // register, and with one the next piece's arithmetic, which reuses those registers at once, now and
     // then overwrote the first of them before the store had read it (a few elements in ten thousand).
-    const auto put = [&](const CachedTile<T> &c, int u, const u32x4_t &piece) {
-        __builtin_amdgcn_raw_buffer_store_b128(piece, c.ry, c.voff + row_off(u), 0, 0);
+    const auto put_at = [&](const CachedTile<T> &c, int off, const u32x4_t &piece) {
+        if (!RAGGED || c.skip == 0) {
+            __builtin_amdgcn_raw_buffer_store_b128(piece, c.ry, off, 0, 0);
+        } else {   // the last columns of a row that is no multiple of VEC
+            float v[VEC];
+            IO::unpack(piece, v);
+            t *row = y + g.inner * g.len * c.o + off / SZ;
+#pragma unroll
+            for (int e = 0; e < VEC; e++)
+                if (e >= c.skip) row[e] = T::from_f32(v[e]);
+        }
     };
+    const auto put = [&](const CachedTile<T> &c, int u, const u32x4_t &piece) { put_at(c, c.voff + row_off(u), piece); };
     for (int64_t tile0 = blockIdx.x; tile0 < n_tiles; tile0 += gridDim.x) {
         const CachedTile<T> cur = locate(tile0);
 #pragma unroll
@@ -431,7 +443,7 @@ __global__ __launch_bounds__(NT, (NP * (OP >= OP_GRAD_SOFTMAX ? 2 : 1) <= 16 && 
                     float r[VEC];
 #pragma unroll
                     for (int e = 0; e < VEC; e++) r[e] = m[e] + logf(sum[e]);
-                    IO::store(y + cur.col + il * VEC + g.inner * cur.o, r);
+                    IO::store(y + cur.col + g.inner * cur.o, r, cur.skip);
                 }
             } else if (plain) {
                 // m and sum fold into two constants per position
@@ -464,9 +476,112 @@ __global__ __launch_bounds__(NT, (NP * (OP >= OP_GRAD_SOFTMAX ? 2 : 1) <= 16 && 
 #pragma unroll
                     for (int e = 0; e < VEC; e++)
                         r[e] = OP == OP_SOFTMAX ? softmax_term(v[e], m[e]) / sum[e] : logsoftmax_shift(v[e], m[e]) - logf(sum[e]);
-                    __builtin_amdgcn_raw_buffer_store_b128(IO::pack(r), cur.ry, cur.voff + step_bytes * u, 0, 0);
+                    put_at(cur, cur.voff + step_bytes * u, IO::pack(r));
                 }
             }
+        }
+    }
+}
+
+// Short columns (up to NP * 8 elements).  A workgroup per tile of one slab would leave most of its threads without
+// work, so the pieces of all slabs are numbered in one row (piece f = chunk + chunks * o) and a wavefront takes
+// 64 / TJ neighbouring ones, each column held by TJ lanes with up to NP rows a lane: one read, one write, reductions
+// by shuffles, no barrier.  (Before, such columns went one element a lane through softmax_nd_kernel: softmax and its
+// gradient of 1000 x 16 x 2000 bf16 81 -> 31 and 130 -> 32 us, 64 x 64 x 8000 bf16 55 -> 33 and 90 -> 30 us.)
+template <typename T, int OP, int VEC, int NP>
+__global__ __launch_bounds__(256) void softmax_nd_short_kernel(const typename T::type *x, const typename T::type *x2,
+                                                                typename T::type *y, int inner, int len, uint32_t chunks, uint32_t total, int tj_log2) {
+    typedef typename T::type t;
+    typedef VecIO<T, VEC> IO;
+    constexpr bool GRAD = OP >= OP_GRAD_SOFTMAX;
+    const int ti = 64 >> tj_log2, tj = 1 << tj_log2, lane = threadIdx.x & 63;
+    const int js = lane >> (6 - tj_log2);
+    const uint32_t f0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * ti + (lane & (ti - 1));
+    const bool ok = f0 < total;
+    const uint32_t f = ok ? f0 : total - 1, o = f / chunks;
+    const int first = (int)(f - o * chunks) * VEC, col = first <= inner - VEC ? first : inner - VEC, skip = first - col;
+    const int64_t base = (int64_t)o * len * inner + col;
+    const auto row = [&](int u) { return base + (int64_t)(js + (u << tj_log2) < len ? js + (u << tj_log2) : len - 1) * inner; };
+    const auto mine = [&](int u) { return js + (u << tj_log2) < len; };
+    u32x4_t raw[NP], raw2[GRAD ? NP : 1];
+#pragma unroll
+    for (int u = 0; u < NP; u++) {
+        raw[u] = IO::load(x + row(u));
+        if (GRAD) raw2[u] = IO::load(x2 + row(u));
+    }
+    const auto reduce = [&](float (&v)[VEC], bool is_max) {
+        for (int d = 32; d >= ti; d >>= 1)
+#pragma unroll
+            for (int e = 0; e < VEC; e++) {
+                const float w = __shfl_xor(v[e], d, 64);
+                v[e] = is_max ? fmaxf(v[e], w) : v[e] + w;
+            }
+    };
+    float m[VEC], s[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; e++) {
+        m[e] = MI_NEG_INF;
+        s[e] = 0.0f;
+    }
+    if constexpr (GRAD) {
+#pragma unroll
+        for (int u = 0; u < NP; u++) {
+            float v[VEC], v2[VEC];
+            IO::unpack(raw[u], v);
+            IO::unpack(raw2[u], v2);
+#pragma unroll
+            for (int e = 0; e < VEC; e++) s[e] += mine(u) ? (OP == OP_GRAD_SOFTMAX ? v[e] * v2[e] : v[e]) : 0.0f;
+        }
+        reduce(s, false);
+        keep_packed(raw);
+        keep_packed(raw2);
+    } else {
+#pragma unroll
+        for (int u = 0; u < NP; u++) {
+            float v[VEC];
+            IO::unpack(raw[u], v);
+#pragma unroll
+            for (int e = 0; e < VEC; e++) m[e] = fmaxf(m[e], v[e]);   // a repeated last row changes no maximum
+        }
+        reduce(m, true);
+        keep_packed(raw);
+#pragma unroll
+        for (int u = 0; u < NP; u++) {
+            float v[VEC];
+            IO::unpack(raw[u], v);
+#pragma unroll
+            for (int e = 0; e < VEC; e++) {
+                const float w = OP == OP_SOFTMAX ? softmax_term(v[e], m[e]) : OP == OP_LOGSOFTMAX ? fast_exp(logsoftmax_shift(v[e], m[e])) : fast_exp(v[e] - m[e]);
+                s[e] += mine(u) ? w : 0.0f;
+            }
+        }
+        reduce(s, false);
+        keep_packed(raw);
+    }
+    if (!ok) return;
+    if constexpr (OP == OP_LOGSUMEXP) {
+        if (js == 0) {
+#pragma unroll
+            for (int e = 0; e < VEC; e++) s[e] = m[e] + logf(s[e]);
+            IO::store(y + (int64_t)o * inner + col, s, skip);
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < VEC; e++) s[e] = OP == OP_SOFTMAX ? 1.0f / s[e] : OP == OP_LOGSOFTMAX ? logf(s[e]) : s[e];
+#pragma unroll
+        for (int u = 0; u < NP; u++) {
+            if (!mine(u)) break;
+            float v[VEC], v2[VEC], r[VEC];
+            IO::unpack(raw[u], v);
+            if (GRAD) IO::unpack(raw2[u], v2);
+#pragma unroll
+            for (int e = 0; e < VEC; e++) {
+                if (OP == OP_SOFTMAX) r[e] = softmax_term(v[e], m[e]) * s[e];
+                else if (OP == OP_LOGSOFTMAX) r[e] = logsoftmax_shift(v[e], m[e]) - s[e];
+                else if (OP == OP_GRAD_SOFTMAX) r[e] = v2[e] * (v[e] - s[e]);
+                else r[e] = v[e] - s[e] * fast_exp(v2[e]);
+            }
+            IO::store(y + row(u), r, skip);
         }
     }
 }
@@ -485,8 +600,10 @@ __global__ __launch_bounds__(256) void softmax_nd_vec_kernel(const typename T::t
     const int64_t step = g.inner * tj;   // elements between consecutive rows of one thread
     for (int64_t tile0 = blockIdx.x; tile0 < n_tiles; tile0 += gridDim.x) {
         const int64_t tile = xcd_order(tile0, n_tiles);
-        const int64_t o = tile / g.n_itiles, i = ((tile % g.n_itiles) * ti + il) * VEC;
-        const bool ok = i < g.inner;
+        const int64_t o = tile / g.n_itiles, first = ((tile % g.n_itiles) * ti + il) * VEC;
+        const bool ok = first < g.inner;
+        const int64_t i = first <= g.inner - VEC ? first : g.inner - VEC;
+        const int skip = ok ? (int)(first - i) : 0;
         const int64_t base = i + g.inner * g.len * o + g.inner * js;
         const int64_t nrows = ok && js < g.len ? (g.len - js + tj - 1) / tj : 0;   // rows js, js+tj, ... of this thread
         float m[VEC], s[VEC];
@@ -500,8 +617,8 @@ __global__ __launch_bounds__(256) void softmax_nd_vec_kernel(const typename T::t
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 const int64_t at = base + step * (r0 + u < nrows ? r0 + u : nrows - 1);   // the tail repeats the last row (ignored below)
-                raw[u] = *(const u32x4_t *)(x + at);
-                if (OP == OP_GRAD_SOFTMAX) raw2[u] = *(const u32x4_t *)(x2 + at);
+                raw[u] = IO::load(x + at);
+                if (OP == OP_GRAD_SOFTMAX) raw2[u] = IO::load(x2 + at);
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
@@ -544,7 +661,7 @@ __global__ __launch_bounds__(256) void softmax_nd_vec_kernel(const typename T::t
 #pragma unroll
                 for (int e = 0; e < VEC; e++)   // the reference's x - max is Inf - Inf for an infinite maximum
                     r[e] = (m[e] == MI_POS_INF || m[e] == MI_NEG_INF) ? __builtin_nanf("") : m[e] + logf(s[e]);
-                IO::store(y + i + g.inner * o, r);
+                IO::store(y + i + g.inner * o, r, skip);
             }
             continue;
         }
@@ -567,8 +684,8 @@ __global__ __launch_bounds__(256) void softmax_nd_vec_kernel(const typename T::t
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 const int64_t at = base + step * (r0 + u < nrows ? r0 + u : nrows - 1);
-                raw[u] = *(const u32x4_t *)(x + at);
-                if (GRAD) raw2[u] = *(const u32x4_t *)(x2 + at);
+                raw[u] = IO::load(x + at);
+                if (GRAD) raw2[u] = IO::load(x2 + at);
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
@@ -583,7 +700,7 @@ __global__ __launch_bounds__(256) void softmax_nd_vec_kernel(const typename T::t
                     else if (OP == OP_GRAD_SOFTMAX) r[e] = v2[e] * (v[e] - s[e]);
                     else r[e] = v[e] - s[e] * fast_exp(v2[e]);
                 }
-                IO::store(y + base + step * (r0 + u), r);
+                IO::store(y + base + step * (r0 + u), r, skip);
             }
         }
     }
@@ -597,10 +714,24 @@ void launch_nd(const void *x, const void *x2, void *y, int64_t inner, int64_t le
     g.len = len;
     g.outer = outer;
     constexpr int VEC = 16 / (int)sizeof(t);
-    const auto al = [](const void *p) { return (((uintptr_t)p) & 15) == 0; };
-    if (inner % VEC == 0 && inner >= 4 * VEC && len > 64 && al(x) && al(y) && (!x2 || al(x2))) {
-        // wide rows and columns too long for the register cache of the scalar kernel
-        const int64_t chunks = inner / VEC;
+    if (inner >= VEC) {
+        const int64_t chunks = (inner + VEC - 1) / VEC;
+        // Measured where the two cross (us, short / cached): 500 x 128 x 400 softmax bf16 34 / 45, f32 45 / 53, their
+        // gradients 41 / 29 and 76 / 57; at len 64 the short kernel wins everywhere (64 x 64 x 4000 f32 23 / 35, 30 / 31).
+        constexpr int64_t SHORT = OP >= OP_GRAD_SOFTMAX ? 64 : 128;
+        if (len <= SHORT && inner < ((int64_t)1 << 31) && chunks * outer < ((int64_t)1 << 31)) {
+            const int np = len <= 4 ? 4 : 8;
+            int tj = 0;
+            while (((int64_t)np << tj) < len) tj++;
+            const uint32_t total = (uint32_t)(chunks * outer), per_block = (uint32_t)(256 >> tj);
+#define MI_SHORT_LAUNCH(NP_)                                                                                                 \
+    hipLaunchKernelGGL((softmax_nd_short_kernel<T, OP, VEC, NP_>), dim3((total + per_block - 1) / per_block), dim3(256), 0, \
+                       st, (const t *)x, (const t *)x2, (t *)y, (int)inner, (int)len, (uint32_t)chunks, total, tj)
+            if (np == 4) MI_SHORT_LAUNCH(4);
+            else MI_SHORT_LAUNCH(8);
+#undef MI_SHORT_LAUNCH
+            return;
+        }
         // register-cached kernel: a thread holds NP pieces (two workgroups per compute unit) or 2 NP (one);
         // the second is taken when it makes the contiguous pieces of a row wider, which is what the memory
         // system rewards (256 x 4096 x 128 bf16 over dim 2: 0.185 ms with 32-byte pieces, 0.131 with 64)
@@ -619,16 +750,19 @@ void launch_nd(const void *x, const void *x2, void *y, int64_t inner, int64_t le
             g.n_itiles = (chunks + (1 << g.ti_log2) - 1) >> g.ti_log2;
             int64_t blocks = g.n_itiles * outer;
             if (blocks > 262144) blocks = 262144;
-            const bool full = len == (int64_t)(512 >> g.ti_log2) * (wide ? 2 * NP : NP) && chunks % (1 << g.ti_log2) == 0;
-#define MI_CACHED_LAUNCH(NP_, FULL_)                                                                                 \
-    hipLaunchKernelGGL((softmax_nd_cached_kernel<T, OP, VEC, NP_, 512, FULL_>), dim3((unsigned)blocks), dim3(512), 0, \
-                       st, (const t *)x, (const t *)x2, (t *)y, g)
+            const bool full = len == (int64_t)(512 >> g.ti_log2) * (wide ? 2 * NP : NP) && inner % (VEC << g.ti_log2) == 0;
+            const bool ragged = inner % VEC != 0;
+#define MI_CACHED_LAUNCH(NP_, FULL_, RAGGED_)                                                                                \
+    hipLaunchKernelGGL((softmax_nd_cached_kernel<T, OP, VEC, NP_, 512, FULL_, RAGGED_>), dim3((unsigned)blocks), dim3(512), \
+                       0, st, (const t *)x, (const t *)x2, (t *)y, g)
             if (wide) {
-                if (full) MI_CACHED_LAUNCH(2 * NP, true);
-                else MI_CACHED_LAUNCH(2 * NP, false);
+                if (full) MI_CACHED_LAUNCH(2 * NP, true, false);
+                else if (ragged) MI_CACHED_LAUNCH(2 * NP, false, true);
+                else MI_CACHED_LAUNCH(2 * NP, false, false);
             } else {
-                if (full) MI_CACHED_LAUNCH(NP, true);
-                else MI_CACHED_LAUNCH(NP, false);
+                if (full) MI_CACHED_LAUNCH(NP, true, false);
+                else if (ragged) MI_CACHED_LAUNCH(NP, false, true);
+                else MI_CACHED_LAUNCH(NP, false, false);
             }
 #undef MI_CACHED_LAUNCH
             return;

@@ -311,3 +311,38 @@ def test_contiguous_columns_of_every_kernel_and_alignment(nn, oracle, dtype, len
         assert np.array_equal(np.isnan(got), np.isnan(ref))
         fin = np.isfinite(ref)
         assert np.abs(got[fin] - ref[fin]).max() <= tol * 10
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("inner,length,outer", [(4, 64, 3), (9, 65, 2), (8, 128, 2), (15, 129, 2), (33, 7, 40), (100, 1, 3), (222, 700, 2),
+                                                (63, 4097, 1), (17, 16385, 1), (1023, 5, 2)])
+def test_strided_rows_of_any_width(nn, oracle, dtype, inner, length, outer):
+    """Rows that are no multiple of 16 bytes and start at any element, on the three kernels (short columns, columns in
+    registers, streamed), in place and not; an infinite column next to the positions that two threads share."""
+    rng = np.random.default_rng(inner * 7 + length)
+    x = round_to(rng.standard_normal((inner, length, outer)) * 2, dtype)
+    dy = round_to(rng.standard_normal((inner, length, outer)), dtype)
+    x[inner - 2, :, 0] = -np.inf
+    x[inner - 1, length // 2, 0] = np.inf
+    x[0, length - 1, 0] = np.nan
+    d, tol = _dev(nn, x, dtype), TOL[dtype]
+    with np.errstate(invalid="ignore", divide="ignore"):
+        for log in (False, True):
+            ref = oracle.softmax(x, 2, log=log)
+            got = (nn.logsoftmax if log else nn.softmax)(d, dims=2).to_numpy()
+            assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isinf(got), np.isinf(ref))
+            fin = np.isfinite(ref)
+            assert np.abs(got[fin] - ref[fin]).max() <= tol * max(1.0, np.abs(ref[fin]).max())
+            same = _dev(nn, x, dtype)
+            (nn.logsoftmax_ if log else nn.softmax_)(same, dims=2)
+            assert np.array_equal(same.to_numpy(), got, equal_nan=True)
+            y = round_to(oracle.softmax(np.where(np.isfinite(x), x, 0), 2, log=log), dtype)
+            ref = oracle.grad_softmax(dy, y, 2, log=log)
+            grad = _dev(nn, dy, dtype)
+            (nn.grad_logsoftmax_ if log else nn.grad_softmax_)(grad, grad, _dev(nn, y, dtype), dims=2)
+            # the sum of `length` terms of size 1 in Float32: sqrt(length) 2^-24 of their size, well below tol
+            assert np.abs(grad.to_numpy() - ref).max() <= 4 * tol * max(1.0, np.abs(ref).max())
+        got, ref = nn.logsumexp(d, dims=2).to_numpy(), oracle.logsumexp(x, 2)
+        assert np.array_equal(np.isnan(got), np.isnan(ref))
+        fin = np.isfinite(ref)
+        assert np.abs(got[fin] - ref[fin]).max() <= tol * 10
