@@ -1,13 +1,11 @@
-// Tiled strided batched GEMM for bf16 / f16 on MFMA: the fast path of mi_batched_gemm for operands
-// whose rows can be moved in 16-byte pieces (aligned bases, leading dimensions and contiguous extents
-// that are multiples of 8).  Stands where the reference calls BLAS gemm per slice
+// Tiled strided batched GEMM for bf16 / f16 on MFMA: the fast path of mi_batched_gemm, operands moved
+// in 16-byte pieces whatever their alignment.  Stands where the reference calls BLAS gemm per slice
 // (src/gemm.jl:141-149, reached through _batched_gemm!, src/batched/batchedmul.jl:298).
 //
 // Workgroup = 4 wavefronts (2 x 2), output tile 128 (m) x 128 (n), 64 x 64 per wavefront as 2 x 2
 // MFMA blocks of 32 x 32; k advances 64 per stage through double-buffered LDS tiles.
 // Accumulator rows = m, columns = n: a lane holds runs of 4 consecutive m of one C column, lanes l and
-// l + 32 complementary runs; they exchange halves and each lane stores 16 contiguous bytes (C rows that
-// cannot be written in aligned 16-byte pieces take element stores).
+// l + 32 complementary runs; they exchange halves and each lane stores 16 contiguous bytes.
 //
 // An operand tile is kept in the orientation its memory has:
 //   RMAJ  contiguous along its row index (A with 'N', B with 'T'): tile [64 k][128 rows], chunks
@@ -47,8 +45,9 @@ struct Gemm16Args {
     void *C;
     int64_t m, n, k, lda, ldb, ldc, sA, sB, sC;
     float alpha, beta;
-    int32_t c_vec;   // C base, leading dimension, slice stride and m allow aligned 16-byte stores
 };
+
+typedef u32x2_t half_piece_t __attribute__((aligned(2)));   // four elements at any alignment
 
 __device__ inline int rmaj_swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
 // 128-byte rows: two rows share a bank span, the row parity picks the half, so the 8 row pairs of 16
@@ -68,7 +67,12 @@ __device__ inline typename T::vec4 lds_tr4(const char *p) {
 // loads need no branches (a piece outside the matrix gets an offset past the end of the resource and
 // reads as zeros) and the compiler can count outstanding loads exactly: loads run two stages ahead.
 // RM: element (row, kk) at X[row + kk*ld]; else at X[kk + row*ld].
-template <typename T, bool RM, bool LARGE>
+// ANY: bases, leading dimensions and extents are any number of elements (at least 8), so pieces start at any
+// element and the last ones of a row or of k may be partial.  Past the end of a row (RM) a piece holds the next k's
+// elements: they only enter rows of C that are not stored.  Past k (not RM) it holds the next row's: these are
+// zeroed on the way into LDS.  A piece that would end past the slice is moved back to end with it, and shifted
+// into place on the way into LDS.  Both happen in the last stage only.
+template <typename T, bool RM, bool LARGE, bool ANY>
 struct Operand {
     typedef typename T::type t;
     static constexpr int THREADS = Shape<LARGE>::THREADS, RMAJ_ROWB = Shape<LARGE>::RMAJ_ROWB;
@@ -76,6 +80,7 @@ struct Operand {
     __amdgpu_buffer_rsrc_t rsrc;
     int off[4];          // byte offset of this thread's four pieces at k0 = 0, or OOB for rows past the edge
     int kstep;           // bytes per unit of k0
+    int bytes;           // of the slice
     int64_t k;
     u32x4_t regs[2][4];  // two stages in flight
     static constexpr int OOB = 0x7fffffff;
@@ -83,7 +88,8 @@ struct Operand {
     __device__ void init(const t *X, int64_t ld, int64_t rows, int64_t k_, int64_t row0) {
         k = k_;
         const int64_t extent = RM ? (k_ - 1) * ld + rows : (rows - 1) * ld + k_;   // elements the slice spans
-        rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)X, 0, (int)(extent * 2), 0x00020000);
+        bytes = (int)(extent * 2);
+        rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)X, 0, bytes, 0x00020000);
         kstep = RM ? (int)(ld * 2) : 2;
 #pragma unroll
         for (int u = 0; u < 4; u++) {
@@ -97,15 +103,35 @@ struct Operand {
             }
         }
     }
+    __device__ int offset(int u, int64_t k0) const {
+        int o = off[u] == OOB ? OOB : off[u] + (int)k0 * kstep;
+        if (!RM) {   // a piece past k in a row-contiguous-in-k matrix would read the next row
+            const int k8 = ((threadIdx.x + THREADS * u) & 7) * 8;
+            o = k0 + k8 < k ? o : OOB;
+        }
+        return o;
+    }
+    // bytes by which a piece that starts inside the slice ends past it
+    __device__ int overhang(int o) const { return o < bytes && o > bytes - 16 ? o - (bytes - 16) : 0; }
     __device__ void load(int set, int64_t k0) {
+        const bool last = ANY && k0 + KC >= k;
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-            int o = off[u] == OOB ? OOB : off[u] + (int)k0 * kstep;
-            if (!RM) {   // a piece past k in a row-contiguous-in-k matrix would read the next row
-                const int k8 = ((threadIdx.x + THREADS * u) & 7) * 8;
-                o = k0 + k8 < k ? o : OOB;
-            }
+            int o = offset(u, k0);
+            if (last) o -= overhang(o);
             regs[set][u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, o, 0, 0);
+        }
+    }
+    // ANY: the partial pieces of the last stage
+    __device__ void trim(int set, int64_t k0) {
+        if (!ANY || k0 + KC < k) return;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            regs[set][u] = mi_drop_bytes(regs[set][u], overhang(offset(u, k0)));
+            if (!RM) {
+                const int64_t left = k - k0 - ((threadIdx.x + THREADS * u) & 7) * 8;
+                regs[set][u] = mi_keep_bytes(regs[set][u], left < 8 ? (left > 0 ? (int)left * 2 : 0) : 16);
+            }
         }
     }
     __device__ void store(int set, char *tile) const {
@@ -145,8 +171,9 @@ struct Operand {
 };
 
 // Writes a workgroup's accumulators: C = alpha * acc + beta * C.  acc[n block][m block] of the wavefront at (wm, wn) of the
-// workgroup's grid; the tile starts at (m0, n0) of slice bz.
-template <typename T, bool LARGE>
+// workgroup's grid; the tile starts at (m0, n0) of slice bz.  TAIL: m is no multiple of 8, the last piece of a column is
+// stored element by element (the code for it costs the 256 x 256 kernel 5 % at 2048^3 x 16, hence the two variants).
+template <typename T, bool LARGE, bool TAIL>
 __device__ inline void store_tile(const Gemm16Args &g, const floatx16_t (&acc)[Shape<LARGE>::BNB][Shape<LARGE>::BM], int64_t bz, int64_t m0,
                                   int64_t n0, int wm, int wn, int lane) {
     typedef typename T::type t;
@@ -155,7 +182,6 @@ __device__ inline void store_tile(const Gemm16Args &g, const floatx16_t (&acc)[S
     const int r = lane & 31, hh = lane >> 5;
     // accumulator register v of lane (r, hh) of block (i, j): m = 32j + 8*(v/4) + 4*hh + v%4, n = 32i + r
     t *C = (t *)g.C + bz * g.sC;
-    const bool vec_ok = g.c_vec != 0;   // C columns can be written in aligned 16-byte pieces
 #pragma unroll
     for (int i = 0; i < BNB; i++) {
         const int64_t nj = n0 + 32 * BNB * wn + 32 * i + r;
@@ -172,44 +198,50 @@ __device__ inline void store_tile(const Gemm16Args &g, const floatx16_t (&acc)[S
                     xv[e] = g.alpha * acc[i][j][8 * gp + e];
                     yv[e] = g.alpha * acc[i][j][8 * gp + 4 + e];
                 }
-                if (vec_ok) {
-                    if (g.beta != 0.0f && nj < g.n) {
-                        if (mb + 4 * hh < g.m) {
-                            const typename T::vec4 c4 = *(const typename T::vec4 *)(ccol + mb + 4 * hh);
+                if (g.beta != 0.0f && nj < g.n) {
+                    const auto add_old = [&](float (&v)[4], int64_t at) {
+                        if (at + 4 <= g.m || (!TAIL && at < g.m)) {
+                            const typename T::vec4 c4 = __builtin_bit_cast(typename T::vec4, *(const half_piece_t *)(ccol + at));
 #pragma unroll
-                            for (int e = 0; e < 4; e++) xv[e] += g.beta * T::to_f32(c4[e]);
+                            for (int e = 0; e < 4; e++) v[e] += g.beta * T::to_f32(c4[e]);
+                        } else if (TAIL) {
+#pragma unroll
+                            for (int e = 0; e < 4; e++)
+                                if (at + e < g.m) v[e] += g.beta * T::to_f32(ccol[at + e]);
                         }
-                        if (mb + 8 + 4 * hh < g.m) {
-                            const typename T::vec4 c4 = *(const typename T::vec4 *)(ccol + mb + 8 + 4 * hh);
+                    };
+                    add_old(xv, mb + 4 * hh);
+                    add_old(yv, mb + 8 + 4 * hh);
+                }
+                typename T::vec4 xe, yo;
 #pragma unroll
-                            for (int e = 0; e < 4; e++) yv[e] += g.beta * T::to_f32(c4[e]);
-                        }
-                    }
-                    typename T::vec4 xe, yo;
+                for (int e = 0; e < 4; e++) {
+                    xe[e] = T::from_f32(xv[e]);
+                    yo[e] = T::from_f32(yv[e]);
+                }
+                const u32x2_t x = __builtin_bit_cast(u32x2_t, xe), y = __builtin_bit_cast(u32x2_t, yo);
+                uint32_t x0 = x[0], x1 = x[1], y0 = y[0], y1 = y[1];
+                mi_pair_halves(x0, y0);   // every lane takes part; lanes outside C do not store
+                mi_pair_halves(x1, y1);
+                const u32x4_t piece = {x0, x1, y0, y1};
+                if constexpr (!TAIL) {
+                    if (nj < g.n && mb + 8 * hh < g.m) *(mi_piece2_t *)(ccol + mb + 8 * hh) = piece;
+                    continue;
+                }
+                const int64_t left = nj < g.n ? g.m - (mb + 8 * hh) : 0;
+                if (left >= 8) {
+                    *(mi_piece2_t *)(ccol + mb + 8 * hh) = piece;
+                } else if (left > 0) {
+                    const typename T::vec8 h = __builtin_bit_cast(typename T::vec8, piece);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        xe[e] = T::from_f32(xv[e]);
-                        yo[e] = T::from_f32(yv[e]);
-                    }
-                    const u32x2_t x = __builtin_bit_cast(u32x2_t, xe), y = __builtin_bit_cast(u32x2_t, yo);
-                    uint32_t x0 = x[0], x1 = x[1], y0 = y[0], y1 = y[1];
-                    mi_pair_halves(x0, y0);   // every lane takes part; lanes outside C do not store
-                    mi_pair_halves(x1, y1);
-                    const u32x4_t piece = {x0, x1, y0, y1};
-                    if (nj < g.n && mb + 8 * hh < g.m) *(u32x4_t *)(ccol + mb + 8 * hh) = piece;   // m is a multiple of 8 here
-                } else if (nj < g.n) {
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const int64_t mx = mb + 4 * hh + e, my = mx + 8;
-                        if (mx < g.m) ccol[mx] = T::from_f32(g.beta != 0.0f ? xv[e] + g.beta * T::to_f32(ccol[mx]) : xv[e]);
-                        if (my < g.m) ccol[my] = T::from_f32(g.beta != 0.0f ? yv[e] + g.beta * T::to_f32(ccol[my]) : yv[e]);
-                    }
+                    for (int e = 0; e < 8; e++)
+                        if (e < left) ccol[mb + 8 * hh + e] = h[e];
                 }
             }
     }
 }
 
-template <typename T, bool A_RM, bool B_RM, bool LARGE>
+template <typename T, bool A_RM, bool B_RM, bool LARGE, bool ANY>
 __global__ __launch_bounds__(Shape<LARGE>::THREADS, LARGE ? 1 : 2) void gemm16_kernel(Gemm16Args g) {
     typedef typename T::type t;
     typedef Shape<LARGE> S;
@@ -222,8 +254,8 @@ __global__ __launch_bounds__(Shape<LARGE>::THREADS, LARGE ? 1 : 2) void gemm16_k
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave % S::WM, wn = wave / S::WM;
     const int r = lane & 31, hh = lane >> 5;
 
-    Operand<T, A_RM, LARGE> a;
-    Operand<T, B_RM, LARGE> b;
+    Operand<T, A_RM, LARGE, ANY> a;
+    Operand<T, B_RM, LARGE, ANY> b;
     const int64_t m0 = bx * S::TILE, n0 = by * S::TILE;
     a.init((const t *)g.A + bz * g.sA, g.lda, g.m, g.k, m0);
     b.init((const t *)g.B + bz * g.sB, g.ldb, g.n, g.k, n0);
@@ -240,6 +272,8 @@ __global__ __launch_bounds__(Shape<LARGE>::THREADS, LARGE ? 1 : 2) void gemm16_k
     const int nk = (int)((g.k + KC - 1) / KC);
     a.load(0, 0);
     b.load(0, 0);
+    a.trim(0, 0);
+    b.trim(0, 0);
     a.store(0, As);
     b.store(0, Bs);
     a.load(1, KC);
@@ -256,15 +290,17 @@ __global__ __launch_bounds__(Shape<LARGE>::THREADS, LARGE ? 1 : 2) void gemm16_k
         for (int ks = 0; ks < 4; ks++) {
             typename T::vec8 av[BM], bv[BNB];
 #pragma unroll
-            for (int j = 0; j < BM; j++) av[j] = Operand<T, A_RM, LARGE>::fetch(at, BM * wm + j, ks, lane);
+            for (int j = 0; j < BM; j++) av[j] = Operand<T, A_RM, LARGE, ANY>::fetch(at, BM * wm + j, ks, lane);
 #pragma unroll
-            for (int i = 0; i < BNB; i++) bv[i] = Operand<T, B_RM, LARGE>::fetch(bt, BNB * wn + i, ks, lane);
+            for (int i = 0; i < BNB; i++) bv[i] = Operand<T, B_RM, LARGE, ANY>::fetch(bt, BNB * wn + i, ks, lane);
 #pragma unroll
             for (int i = 0; i < BNB; i++)
 #pragma unroll
                 for (int j = 0; j < BM; j++) acc[i][j] = T::mfma32(av[j], bv[i], acc[i][j]);
         }
         if (it + 1 < nk) {
+            a.trim(set_next, (int64_t)(it + 1) * KC);
+            b.trim(set_next, (int64_t)(it + 1) * KC);
             a.store(set_next, As + (buf ^ 1) * TILEB);
             b.store(set_next, Bs + (buf ^ 1) * TILEB);
         }
@@ -277,7 +313,8 @@ __global__ __launch_bounds__(Shape<LARGE>::THREADS, LARGE ? 1 : 2) void gemm16_k
     }
     if (it < nk) stage(it, 1);
 
-    store_tile<T, LARGE>(g, acc, bz, m0, n0, wm, wn, lane);
+    if ((g.m & 7) == 0) store_tile<T, LARGE, false>(g, acc, bz, m0, n0, wm, wn, lane);
+    else store_tile<T, LARGE, true>(g, acc, bz, m0, n0, wm, wn, lane);
 }
 
 // ---- the 256 x 256 tile with the operand tiles copied global -> LDS by the DMA path ---------------------------------
@@ -418,7 +455,8 @@ __global__ __launch_bounds__(Shape<LARGE>::THREADS, LARGE ? 1 : 2) void gemm16_r
                 for (int j = 0; j < BM; j++) acc[i][j] = T::mfma32(av[j], bv[i], acc[i][j]);
         }
     }
-    store_tile<T, LARGE>(g, acc, bz, m0, n0, wm, wn, lane);
+    if ((g.m & 7) == 0) store_tile<T, LARGE, false>(g, acc, bz, m0, n0, wm, wn, lane);
+    else store_tile<T, LARGE, true>(g, acc, bz, m0, n0, wm, wn, lane);
 }
 
 template <typename T, bool A_RM, bool B_RM, bool LARGE>
@@ -444,10 +482,10 @@ int32_t launch_ring_l(const Gemm16Args &g, int transA, int transB, int64_t nb, h
     return b_rm ? launch_ring<T, false, true, LARGE>(g, nb, st) : launch_ring<T, false, false, LARGE>(g, nb, st);
 }
 
-template <typename T, bool A_RM, bool B_RM, bool LARGE>
+template <typename T, bool A_RM, bool B_RM, bool LARGE, bool ANY>
 int32_t launch_one(const Gemm16Args &g, int64_t nb, hipStream_t st) {
     typedef Shape<LARGE> S;
-    auto kern = gemm16_kernel<T, A_RM, B_RM, LARGE>;
+    auto kern = gemm16_kernel<T, A_RM, B_RM, LARGE, ANY>;
     constexpr size_t smem = 4 * S::TILEB;
     static bool attr_set = false;  // per instantiation; the attribute is idempotent, so a race is harmless
     if (!attr_set) {
@@ -460,39 +498,43 @@ int32_t launch_one(const Gemm16Args &g, int64_t nb, hipStream_t st) {
     return MI_OK;
 }
 
-template <typename T, bool LARGE>
+template <typename T, bool LARGE, bool ANY>
 int32_t launch_l(const Gemm16Args &g, int transA, int transB, int64_t nb, hipStream_t st) {
     const bool a_rm = !transA, b_rm = transB != 0;
-    if (a_rm) return b_rm ? launch_one<T, true, true, LARGE>(g, nb, st) : launch_one<T, true, false, LARGE>(g, nb, st);
-    return b_rm ? launch_one<T, false, true, LARGE>(g, nb, st) : launch_one<T, false, false, LARGE>(g, nb, st);
+    if (a_rm) return b_rm ? launch_one<T, true, true, LARGE, ANY>(g, nb, st) : launch_one<T, true, false, LARGE, ANY>(g, nb, st);
+    return b_rm ? launch_one<T, false, true, LARGE, ANY>(g, nb, st) : launch_one<T, false, false, LARGE, ANY>(g, nb, st);
 }
 
 template <typename T>
-int32_t launch_t(const Gemm16Args &g, int transA, int transB, int64_t nb, hipStream_t st) {
-    // the large tile when it still gives every CU a workgroup; the small one otherwise
-    const int64_t big = ((g.m + 255) / 256) * ((g.n + 255) / 256) * nb;
+int32_t launch_t(const Gemm16Args &g, int transA, int transB, int64_t nb, bool aligned, hipStream_t st) {
+    // Operands of any alignment: the small tile (the copies global -> LDS of the ring kernel move whole aligned pieces, and
+    // the large register-staged one spills with them: 513^3 x 64 unaligned 64 us small, 99 large; 2047^3 x 8 237 / 229).
+    if (!aligned) return launch_l<T, false, true>(g, transA, transB, nb, st);
+    // The large tile where the share of its slots that does useful work, counting padded rows and columns and the last round
+    // of workgroups (one per CU; two of the small ones), times its higher rate (1100 against 800 TFLOP/s on whole rounds of
+    // whole tiles) is the larger; the small one otherwise.
+    const auto useful = [&](int64_t tile, int64_t slots) {
+        const int64_t tiles = ((g.m + tile - 1) / tile) * ((g.n + tile - 1) / tile) * nb;
+        return (double)(g.m * g.n * nb) / ((double)((tiles + slots - 1) / slots * slots) * (double)(tile * tile));
+    };
+    const bool large = g.m >= 256 && g.n >= 256 && 1.35 * useful(256, 256) > useful(128, 512);
     static const bool no_ring = getenv("MI355ATTN_GEMM_NO_RING") != nullptr;   // A/B switch: the register-staged kernels
-    const bool large = g.m >= 256 && g.n >= 256 && big >= 256;
     // the ring kernel for the large shape only: at 128 x 128 it was measured level or behind the register-staged kernel
     // (128 x 4096 x 4096 x 64: 593 against 637 TFLOP/s, 64 x 2048 x 2048 x 64: 252 / 290, 1024^3 x 4: 607 / 573)
-    if (large) return no_ring ? launch_l<T, true>(g, transA, transB, nb, st) : launch_ring_l<T, true>(g, transA, transB, nb, st);
-    return launch_l<T, false>(g, transA, transB, nb, st);
+    if (large) return no_ring ? launch_l<T, true, false>(g, transA, transB, nb, st) : launch_ring_l<T, true>(g, transA, transB, nb, st);
+    return launch_l<T, false, false>(g, transA, transB, nb, st);
 }
 
 }  // namespace
 
-// true when every 16-byte piece the kernel moves is aligned and wholly inside or outside its matrix
-bool batched_gemm16_supports(int32_t dtype, int transA, int transB, int64_t m, int64_t n, int64_t k, const void *A, int64_t lda,
-                             int64_t sA, const void *B, int64_t ldb, int64_t sB) {
+// true when the tiled kernels take the product: slices that 32-bit byte offsets address and that hold a 16-byte piece
+bool batched_gemm16_supports(int32_t dtype, int transA, int transB, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb) {
     if (dtype != MI_F16 && dtype != MI_BF16) return false;
     if (k < 1 || m * n < 64 * 64) return false;   // tiny products: the small-tile kernel wastes less
-    auto al = [](const void *p) { return (((uintptr_t)p) & 15) == 0; };
-    if (!al(A) || !al(B) || (lda & 7) || (ldb & 7) || (sA & 7) || (sB & 7)) return false;
-    if ((transA ? k : m) & 7) return false;
-    if ((transB ? n : k) & 7) return false;
-    // slices are addressed with 32-bit byte offsets
     const int64_t extA = transA ? (m - 1) * lda + k : (k - 1) * lda + m, extB = transB ? (k - 1) * ldb + n : (n - 1) * ldb + k;
     if (extA * 2 >= 2147483647LL || extB * 2 >= 2147483647LL) return false;
+    // leading dimensions of at least a piece: only the last k or row of a slice can hold a piece that ends past it
+    if (lda < 8 || ldb < 8 || extA < 8 || extB < 8) return false;
     return (n + 127) / 128 <= 65535;
 }
 
@@ -500,12 +542,14 @@ int32_t launch_batched_gemm16(int32_t dtype, int transA, int transB, int64_t m, 
                               int64_t lda, int64_t sA, const void *B, int64_t ldb, int64_t sB, float beta, void *C, int64_t ldc,
                               int64_t sC, int64_t batch, hipStream_t st) {
     const size_t es = 2;
+    // every 16-byte piece of the operands is aligned and wholly inside or outside its matrix
+    const bool aligned = ((((uintptr_t)A) | ((uintptr_t)B)) & 15) == 0 &&
+                         ((lda | ldb | sA | sB | (transA ? k : m) | (transB ? n : k)) & 7) == 0;
     for (int64_t b0 = 0; b0 < batch; b0 += 65535) {   // gridDim.z is limited to 65535: issue the batch in slabs
         const int64_t nb = batch - b0 < 65535 ? batch - b0 : 65535;
         Gemm16Args g = {(const char *)A + es * b0 * sA, (const char *)B + es * b0 * sB, (char *)C + es * b0 * sC,
-                        m, n, k, lda, ldb, ldc, sA, sB, sC, alpha, beta,
-                        (int32_t)((((uintptr_t)C) & 15) == 0 && (ldc & 7) == 0 && (sC & 7) == 0 && (m & 7) == 0)};
-        const int32_t rc = dtype == MI_F16 ? launch_t<F16>(g, transA, transB, nb, st) : launch_t<BF16>(g, transA, transB, nb, st);
+                        m, n, k, lda, ldb, ldc, sA, sB, sC, alpha, beta};
+        const int32_t rc = dtype == MI_F16 ? launch_t<F16>(g, transA, transB, nb, aligned, st) : launch_t<BF16>(g, transA, transB, nb, aligned, st);
         if (rc != MI_OK) return rc;
     }
     return MI_OK;

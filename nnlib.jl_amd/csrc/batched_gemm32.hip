@@ -1,5 +1,5 @@
-// Tiled strided batched GEMM for Float32 on the fp32 matrix cores (v_mfma_f32_32x32x2_f32): the fast
-// path of mi_batched_gemm for operands whose rows can be moved in 16-byte pieces.  Stands where the
+// Tiled strided batched GEMM for Float32 on the matrix cores: the fast path of mi_batched_gemm, operands
+// moved in 16-byte pieces (of any alignment in the kernels on bf16 planes).  Stands where the
 // reference calls sgemm per slice (src/gemm.jl:141-149, reached through _batched_gemm!,
 // src/batched/batchedmul.jl:298).  Products and sums are true fp32.
 //
@@ -10,6 +10,7 @@
 // the transposed problem so that a half-wave stores 32 consecutive elements of a C column.
 #include "common.h"
 #include <cstdlib>
+#include <type_traits>
 
 namespace {
 
@@ -21,7 +22,6 @@ struct Gemm32Args {
     float *C;
     int64_t m, n, k, lda, ldb, ldc, sA, sB, sC;
     float alpha, beta;
-    int32_t c_vec;   // C base, leading dimension, slice stride and m allow aligned 16-byte stores
 };
 
 // RM: element (row, kk) at X[row + kk*ld] (contiguous along row); else at X[kk + row*ld]
@@ -171,27 +171,69 @@ struct ShapeS {
 
 __device__ inline int rmaj_swz(int kk) { return ((kk & 3) << 2) | ((kk >> 2) & 3); }
 
-template <bool RM, bool LARGE>
+// ANY: bases, leading dimensions and extents are any number of elements (at least 4) and the slice is below 2 GiB: pieces
+// are loads of element alignment through a buffer resource.  Past the end of a row (RM) a piece holds the next k's
+// elements, which only enter rows of C that are not stored; past k (not RM) the next row's, which `trim` zeroes.  A piece
+// that would end past the slice is moved back to end with it and shifted into place by `trim`.  Both happen in the last
+// stage only.
+template <bool RM, bool LARGE, bool ANY>
 struct OperandS {
     typedef ShapeS<LARGE> S;
     static constexpr int ROWB = S::RMAJ_ROWB, PLANEB = S::PLANEB, CPR = S::TILE / 4;   // float4 pieces per k-row
+    static constexpr int OOB = 0x7fffffff;
     const float *X;
     int64_t ld, rows, k, row0;
+    __amdgpu_buffer_rsrc_t rsrc;   // ANY
+    int bytes;                     // ANY: of the slice
     floatx4_t reg[2];   // TILE * KC / 4 pieces per tile: 2 per thread in either shape
 
+    __device__ void init(const float *X_, int64_t ld_, int64_t rows_, int64_t k_, int64_t row0_) {
+        X = X_;
+        ld = ld_;
+        rows = rows_;
+        k = k_;
+        row0 = row0_;
+        bytes = ANY ? (int)((RM ? (k - 1) * ld + rows : (rows - 1) * ld + k) * 4) : 0;
+        if (ANY) rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)X, 0, bytes, 0x00020000);
+    }
+    // ANY: byte offset of this thread's piece u of the stage at k0; OOB: outside the matrix
+    __device__ int offset(int u, int64_t k0) const {
+        const int c = threadIdx.x + S::THREADS * u;
+        const int row = RM ? (c % CPR) * 4 : c >> 2, kk = RM ? c / CPR : (c & 3) * 4;
+        if (row0 + row >= rows || k0 + kk >= k) return OOB;
+        return (int)((RM ? (row0 + row) + (k0 + kk) * ld : (k0 + kk) + (row0 + row) * ld) * 4);
+    }
+    __device__ int overhang(int o) const { return o < bytes && o > bytes - 16 ? o - (bytes - 16) : 0; }
     __device__ void load(int64_t k0) {
         const int tid = threadIdx.x;
+        const bool last = ANY && k0 + KC >= k;
 #pragma unroll
         for (int u = 0; u < 2; u++) {
             const int c = tid + S::THREADS * u;
             const floatx4_t z = {0.f, 0.f, 0.f, 0.f};
-            if (RM) {
+            if (ANY) {
+                int o = offset(u, k0);
+                if (last) o -= overhang(o);
+                reg[u] = __builtin_bit_cast(floatx4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, o, 0, 0));
+            } else if (RM) {
                 const int kk = c / CPR, r4 = (c % CPR) * 4;
                 reg[u] = (k0 + kk < k && row0 + r4 < rows) ? *(const floatx4_t *)(X + (row0 + r4) + (k0 + kk) * ld) : z;
             } else {
                 const int r = c >> 2, k4 = (c & 3) * 4;       // 4 pieces per row
                 reg[u] = (row0 + r < rows && k0 + k4 < k) ? *(const floatx4_t *)(X + (k0 + k4) + (row0 + r) * ld) : z;
             }
+        }
+    }
+    __device__ void trim(int64_t k0) {
+        if (!ANY || k0 + KC < k) return;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            u32x4_t v = mi_drop_bytes(__builtin_bit_cast(u32x4_t, reg[u]), overhang(offset(u, k0)));
+            if (!RM) {
+                const int64_t left = k - k0 - ((threadIdx.x + S::THREADS * u) & 3) * 4;
+                v = mi_keep_bytes(v, left < 4 ? (left > 0 ? (int)left * 4 : 0) : 16);
+            }
+            reg[u] = __builtin_bit_cast(floatx4_t, v);
         }
     }
     // split into planes; `tile` is the LDS byte address of the hi plane
@@ -244,7 +286,7 @@ struct OperandS {
     }
 };
 
-template <bool A_RM, bool B_RM, bool LARGE>
+template <bool A_RM, bool B_RM, bool LARGE, bool ANY>
 __global__ __launch_bounds__(ShapeS<LARGE>::THREADS, LARGE ? 1 : 2) void gemm32s_kernel(Gemm32Args g) {
     typedef ShapeS<LARGE> S;
     constexpr int TILE3B = S::TILE3B, BM = S::BM, BNB = S::BNB;
@@ -258,18 +300,10 @@ __global__ __launch_bounds__(ShapeS<LARGE>::THREADS, LARGE ? 1 : 2) void gemm32s
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave & 1, wn = wave >> 1;
     const int r = lane & 31, hh = lane >> 5;
 
-    OperandS<A_RM, LARGE> a;
-    OperandS<B_RM, LARGE> b;
-    a.X = g.A + bz * g.sA;
-    a.ld = g.lda;
-    a.rows = g.m;
-    a.k = g.k;
-    a.row0 = tile.m * S::TILE;
-    b.X = g.B + bz * g.sB;
-    b.ld = g.ldb;
-    b.rows = g.n;
-    b.k = g.k;
-    b.row0 = tile.n * S::TILE;
+    OperandS<A_RM, LARGE, ANY> a;
+    OperandS<B_RM, LARGE, ANY> b;
+    a.init(g.A + bz * g.sA, g.lda, g.m, g.k, tile.m * S::TILE);
+    b.init(g.B + bz * g.sB, g.ldb, g.n, g.k, tile.n * S::TILE);
 
     floatx16_t acc[BNB][BM];   // [n block][m block]
 #pragma unroll
@@ -282,6 +316,8 @@ __global__ __launch_bounds__(ShapeS<LARGE>::THREADS, LARGE ? 1 : 2) void gemm32s
     const int nk = (int)((g.k + KC - 1) / KC);
     a.load(0);
     b.load(0);
+    a.trim(0);
+    b.trim(0);
     a.store(lds0);
     b.store(lds0 + 2 * TILE3B);
     __syncthreads();
@@ -294,9 +330,9 @@ __global__ __launch_bounds__(ShapeS<LARGE>::THREADS, LARGE ? 1 : 2) void gemm32s
         const unsigned at = lds0 + buf * TILE3B, bt = lds0 + (2 + buf) * TILE3B;
         plane8 av[BM][3], bv[BNB][3];
 #pragma unroll
-        for (int j = 0; j < BM; j++) OperandS<A_RM, LARGE>::fetch(at, BM * wm + j, lane, av[j]);
+        for (int j = 0; j < BM; j++) OperandS<A_RM, LARGE, ANY>::fetch(at, BM * wm + j, lane, av[j]);
 #pragma unroll
-        for (int i = 0; i < BNB; i++) OperandS<B_RM, LARGE>::fetch(bt, BNB * wn + i, lane, bv[i]);
+        for (int i = 0; i < BNB; i++) OperandS<B_RM, LARGE, ANY>::fetch(bt, BNB * wn + i, lane, bv[i]);
         // the transposed problem (rows = n, columns = m), small terms first
         constexpr int ia[6] = {2, 0, 1, 1, 0, 0}, ib[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
@@ -307,6 +343,8 @@ __global__ __launch_bounds__(ShapeS<LARGE>::THREADS, LARGE ? 1 : 2) void gemm32s
                 for (int j = 0; j < BM; j++)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bv[i][ib[t]], av[j][ia[t]], acc[i][j], 0, 0, 0);
         if (it + 1 < nk) {
+            a.trim((int64_t)(it + 1) * KC);
+            b.trim((int64_t)(it + 1) * KC);
             a.store(lds0 + (buf ^ 1) * TILE3B);
             b.store(lds0 + (2 + (buf ^ 1)) * TILE3B);
         }
@@ -314,17 +352,18 @@ __global__ __launch_bounds__(ShapeS<LARGE>::THREADS, LARGE ? 1 : 2) void gemm32s
     }
 
     // accumulator register v of lane (r, hh) of block (i, j): n = 32i + 8*(v/4) + 4*hh + v%4, m = 32j + r
+    // A lane holds single elements of 16 columns of C: stored directly, every instruction moves 4 bytes per lane.
+    // Instead each wavefront passes [32 n][64 m] blocks through a private LDS region (the operand buffers are
+    // free now) and reads them back as rows of m, so that a store instruction writes four columns of 256
+    // contiguous bytes, 16 bytes per lane (C is 512 MiB of the 1024 x 64 x 1024 x 128 product: 0.195 -> 0.178 ms).
     float *C = g.C + bz * g.sC;
-    if (g.c_vec) {
-        // A lane holds single elements of 16 columns of C: stored directly, every instruction moves 4 bytes per lane.
-        // Instead each wavefront passes [32 n][64 m] blocks through a private LDS region (the operand buffers are
-        // free now) and reads them back as rows of m, so that a store instruction writes four columns of 256
-        // contiguous bytes, 16 bytes per lane (C is 512 MiB of the 1024 x 64 x 1024 x 128 product: 0.195 -> 0.178 ms).
-        typedef __attribute__((address_space(3))) float *ldsf_t;
-        typedef __attribute__((address_space(3))) const floatx4_t *ldsf4_t;
-        constexpr int LDW = 64 + 4;   // floats per LDS row
-        const unsigned region = lds0 + (unsigned)wave * (32 * LDW * 4);
-        const int64_t mw = a.row0 + 32 * BM * wm, nw = b.row0 + 32 * BNB * wn;
+    typedef __attribute__((address_space(3))) float *ldsf_t;
+    typedef __attribute__((address_space(3))) const floatx4_t *ldsf4_t;
+    constexpr int LDW = 64 + 4;   // floats per LDS row
+    const unsigned region = lds0 + (unsigned)wave * (32 * LDW * 4);
+    const int64_t mw = a.row0 + 32 * BM * wm, nw = b.row0 + 32 * BNB * wn;
+    const auto write = [&](auto whole_c) {
+        constexpr bool whole = decltype(whole_c)::value;   // columns of C are whole pieces
 #pragma unroll
         for (int i = 0; i < BNB; i++)
 #pragma unroll
@@ -346,42 +385,32 @@ __global__ __launch_bounds__(ShapeS<LARGE>::THREADS, LARGE ? 1 : 2) void gemm32s
                     const int nl = 4 * q + (lane >> 4), ml = (lane & 15) * 4;
                     floatx4_t val = *(ldsf4_t)(uintptr_t)(region + (unsigned)((nl * LDW + ml) * 4));
                     const int64_t nj = nw + 32 * i + nl, mi = mw + 64 * jp + ml;
-                    if (nj < g.n && mi < g.m) {   // m is a multiple of 4 here
-                        floatx4_t *c4 = (floatx4_t *)(C + mi + nj * g.ldc);
+                    if (nj >= g.n || mi >= g.m) continue;
+                    float *c = C + mi + nj * g.ldc;
+                    if (whole || mi + 4 <= g.m) {
                         if (g.beta != 0.0f) {
-                            const floatx4_t old = *c4;
+                            const floatx4_t old = __builtin_bit_cast(floatx4_t, *(const mi_piece4_t *)c);
 #pragma unroll
                             for (int e = 0; e < 4; e++) val[e] += g.beta * old[e];
                         }
-                        *c4 = val;
+                        *(mi_piece4_t *)c = __builtin_bit_cast(u32x4_t, val);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 3; e++)
+                            if (mi + e < g.m) c[e] = g.beta != 0.0f ? val[e] + g.beta * c[e] : val[e];
                     }
                 }
             }
-        return;
-    }
-#pragma unroll
-    for (int j = 0; j < BM; j++) {
-        const int64_t mi = a.row0 + 32 * BM * wm + 32 * j + r;
-        if (mi >= g.m) continue;
-#pragma unroll
-        for (int i = 0; i < BNB; i++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int64_t nj = b.row0 + 32 * BNB * wn + 32 * i + 8 * (v / 4) + 4 * hh + (v % 4);
-                if (nj < g.n) {
-                    float *c = C + mi + nj * g.ldc;
-                    float val = g.alpha * acc[i][j][v];
-                    if (g.beta != 0.0f) val += g.beta * *c;
-                    *c = val;
-                }
-            }
-    }
+    };
+    // two variants: the code for the last piece of columns of odd length costs the others 1.5 %
+    if ((g.m & 3) == 0) write(std::integral_constant<bool, true>());
+    else write(std::integral_constant<bool, false>());
 }
 
-template <bool A_RM, bool B_RM, bool LARGE>
+template <bool A_RM, bool B_RM, bool LARGE, bool ANY>
 int32_t launch_planes(const Gemm32Args &g, int64_t nb, hipStream_t st) {
     typedef ShapeS<LARGE> S;
-    auto kern = gemm32s_kernel<A_RM, B_RM, LARGE>;
+    auto kern = gemm32s_kernel<A_RM, B_RM, LARGE, ANY>;
     constexpr size_t smem = 4 * S::TILE3B;
     static bool attr_set = false;  // per instantiation; the attribute is idempotent, so a race is harmless
     if (!attr_set) {
@@ -394,10 +423,10 @@ int32_t launch_planes(const Gemm32Args &g, int64_t nb, hipStream_t st) {
     return MI_OK;
 }
 
-template <bool LARGE>
+template <bool LARGE, bool ANY>
 int32_t launch_planes_l(const Gemm32Args &g, bool a_rm, bool b_rm, int64_t nb, hipStream_t st) {
-    if (a_rm) return b_rm ? launch_planes<true, true, LARGE>(g, nb, st) : launch_planes<true, false, LARGE>(g, nb, st);
-    return b_rm ? launch_planes<false, true, LARGE>(g, nb, st) : launch_planes<false, false, LARGE>(g, nb, st);
+    if (a_rm) return b_rm ? launch_planes<true, true, LARGE, ANY>(g, nb, st) : launch_planes<true, false, LARGE, ANY>(g, nb, st);
+    return b_rm ? launch_planes<false, true, LARGE, ANY>(g, nb, st) : launch_planes<false, false, LARGE, ANY>(g, nb, st);
 }
 
 // the Float32 matrix instruction instead of the bf16 planes (MI355ATTN_F32_MFMA=1 in the environment, read once)
@@ -411,16 +440,24 @@ bool exact_instruction_wanted() {
 
 }  // namespace
 
-// true when every 16-byte piece the kernel moves is aligned and wholly inside or outside its matrix
+// every 16-byte piece of the operands is aligned and wholly inside or outside its matrix
+static bool aligned_pieces(int transA, int transB, int64_t m, int64_t n, int64_t k, const void *A, int64_t lda, int64_t sA, const void *B,
+                           int64_t ldb, int64_t sB) {
+    return ((((uintptr_t)A) | ((uintptr_t)B)) & 15) == 0 && ((lda | ldb | sA | sB | (transA ? k : m) | (transB ? n : k)) & 3) == 0;
+}
+
+// true when the tiled kernels take the product.  Operands that do not come in aligned pieces need slices that 32-bit byte
+// offsets address and that hold a piece, and the bf16 planes.
 bool batched_gemm32_supports(int32_t dtype, int transA, int transB, int64_t m, int64_t n, int64_t k, const void *A, int64_t lda,
                              int64_t sA, const void *B, int64_t ldb, int64_t sB) {
     if (dtype != MI_F32) return false;
     if (k < 1 || m * n < 64 * 64) return false;   // tiny products: the small-tile kernel wastes less
-    auto al = [](const void *p) { return (((uintptr_t)p) & 15) == 0; };
-    if (!al(A) || !al(B) || (lda & 3) || (ldb & 3) || (sA & 3) || (sB & 3)) return false;
-    if ((transA ? k : m) & 3) return false;
-    if ((transB ? n : k) & 3) return false;
-    return (n + TN - 1) / TN <= 65535;
+    if ((n + TN - 1) / TN > 65535) return false;
+    if (aligned_pieces(transA, transB, m, n, k, A, lda, sA, B, ldb, sB)) return true;
+    if (exact_instruction_wanted()) return false;
+    const int64_t extA = transA ? (m - 1) * lda + k : (k - 1) * lda + m, extB = transB ? (k - 1) * ldb + n : (n - 1) * ldb + k;
+    // leading dimensions of at least a piece: only the last k or row of a slice can hold a piece that ends past it
+    return lda >= 4 && ldb >= 4 && extA >= 4 && extB >= 4 && extA * 4 < 2147483647LL && extB * 4 < 2147483647LL;
 }
 
 int32_t launch_batched_gemm32(int transA, int transB, int64_t m, int64_t n, int64_t k, float alpha, const void *A, int64_t lda,
@@ -430,8 +467,7 @@ int32_t launch_batched_gemm32(int transA, int transB, int64_t m, int64_t n, int6
     for (int64_t b0 = 0; b0 < batch; b0 += 65535) {   // gridDim.z is limited to 65535: issue the batch in slabs
         const int64_t nb = batch - b0 < 65535 ? batch - b0 : 65535;
         Gemm32Args g = {(const float *)A + b0 * sA, (const float *)B + b0 * sB, (float *)C + b0 * sC,
-                        m, n, k, lda, ldb, ldc, sA, sB, sC, alpha, beta,
-                        (int32_t)((((uintptr_t)C) & 15) == 0 && (ldc & 3) == 0 && (sC & 3) == 0 && (m & 3) == 0)};
+                        m, n, k, lda, ldb, ldc, sA, sB, sC, alpha, beta};
         dim3 grid((unsigned)((m + TM - 1) / TM), (unsigned)((n + TN - 1) / TN), (unsigned)nb);
         if (exact_instruction_wanted()) {
             if (a_rm && b_rm) hipLaunchKernelGGL((gemm32_kernel<true, true>), grid, dim3(256), 0, st, g);
@@ -439,10 +475,17 @@ int32_t launch_batched_gemm32(int transA, int transB, int64_t m, int64_t n, int6
             else if (b_rm) hipLaunchKernelGGL((gemm32_kernel<false, true>), grid, dim3(256), 0, st, g);
             else hipLaunchKernelGGL((gemm32_kernel<false, false>), grid, dim3(256), 0, st, g);
         } else {
-            // the large tile when it still gives every CU a workgroup and k is long enough to pay for its longer prologue
-            const int64_t big = ((m + 255) / 256) * ((n + 255) / 256) * nb;
-            const bool large = m >= 256 && n >= 256 && big >= 256 && k >= 128;
-            const int32_t rc = large ? launch_planes_l<true>(g, a_rm, b_rm, nb, st) : launch_planes_l<false>(g, a_rm, b_rm, nb, st);
+            // The large tile where the share of its slots that does useful work, counting padded rows and columns and the
+            // last round of workgroups (one per CU; three of the small ones), times its higher rate once k is long enough
+            // to pay for its prologue (2047^3 x 8: 188 against 163 TFLOP/s; 1000 x 1000 x 130: level) is the larger.
+            const auto useful = [&](int64_t tile, int64_t slots) {
+                const int64_t tiles = ((m + tile - 1) / tile) * ((n + tile - 1) / tile) * nb;
+                return (double)(m * n * nb) / ((double)((tiles + slots - 1) / slots * slots) * (double)(tile * tile));
+            };
+            const bool large = m >= 256 && n >= 256 && k >= 128 && (k >= 512 ? 1.15 : 1.0) * useful(256, 256) > useful(128, 768);
+            const bool aligned = aligned_pieces(transA, transB, m, n, k, g.A, lda, sA, g.B, ldb, sB);
+            const int32_t rc = aligned ? (large ? launch_planes_l<true, false>(g, a_rm, b_rm, nb, st) : launch_planes_l<false, false>(g, a_rm, b_rm, nb, st))
+                                       : (large ? launch_planes_l<true, true>(g, a_rm, b_rm, nb, st) : launch_planes_l<false, true>(g, a_rm, b_rm, nb, st));
             if (rc != MI_OK) return rc;
         }
         MI_LAUNCH_CHECK();

@@ -179,6 +179,27 @@ __device__ static inline V mi_load16_or_zero(const E *p, bool ok) {
     return *src;
 }
 
+// 16-byte pieces that start at any 4-byte (2-byte) element: the memory pipeline takes such loads and stores as they are
+typedef u32x4_t mi_piece4_t __attribute__((aligned(4)));
+typedef u32x4_t mi_piece2_t __attribute__((aligned(2)));
+
+// the 128-bit value without its first `bytes` (0 to 15, even) bytes, zeros coming in at its end
+__device__ static inline u32x4_t mi_drop_bytes(u32x4_t v, int bytes) {
+    if (bytes & 2) v = (u32x4_t){(v[0] >> 16) | (v[1] << 16), (v[1] >> 16) | (v[2] << 16), (v[2] >> 16) | (v[3] << 16), v[3] >> 16};
+    if (bytes & 4) v = (u32x4_t){v[1], v[2], v[3], 0u};
+    if (bytes & 8) v = (u32x4_t){v[2], v[3], 0u, 0u};
+    return v;
+}
+// the first `bytes` (0 to 16, even) bytes of a 128-bit value, zeros after them
+__device__ static inline u32x4_t mi_keep_bytes(u32x4_t v, int bytes) {
+#pragma unroll
+    for (int d = 0; d < 4; d++) {
+        const int left = bytes - 4 * d;
+        v[d] = left >= 4 ? v[d] : left > 0 ? v[d] & 0xffffu : 0u;
+    }
+    return v;
+}
+
 // Workgroup order for kernels whose neighbouring workgroups share operands.  The hardware hands workgroup `id` of a
 // launch to XCD `id % 8` (eight dies, each with its own L2), so neighbours in launch order never share an L2.
 // mi_xcd_order turns the launch id into the id of the work item to take such that every die works through one

@@ -4,18 +4,15 @@
 
 enum { OP_SOFTMAX = 0, OP_LOGSOFTMAX = 1, OP_LOGSUMEXP = 2, OP_GRAD_SOFTMAX = 3, OP_GRAD_LOGSOFTMAX = 4 };
 
-// 16-byte pieces that start at any 4-byte (2-byte) element
-typedef u32x4_t piece_any4_t __attribute__((aligned(4)));
-typedef u32x4_t piece_any2_t __attribute__((aligned(2)));
 template <typename T> struct ColumnIO {
     typedef typename T::type t;
     __device__ static u32x4_t load(const t *p) {
-        if constexpr (sizeof(t) == 4) return *(const piece_any4_t *)p;
-        else return *(const piece_any2_t *)p;
+        if constexpr (sizeof(t) == 4) return *(const mi_piece4_t *)p;
+        else return *(const mi_piece2_t *)p;
     }
     __device__ static void store(t *p, const u32x4_t &v) {
-        if constexpr (sizeof(t) == 4) *(piece_any4_t *)p = v;
-        else *(piece_any2_t *)p = v;
+        if constexpr (sizeof(t) == 4) *(mi_piece4_t *)p = v;
+        else *(mi_piece2_t *)p = v;
     }
 };
 

@@ -423,3 +423,31 @@ def test_float32_products_through_bf16_planes_keep_float32_accuracy(nn, ta, tb):
     dB3 = nn.DeviceArray.from_numpy(B3, "f32")
     C3 = nn.batched_mul(nn.batched_transpose(d3) if ta else d3, nn.batched_transpose(dB3) if tb else dB3).to_numpy()
     assert np.allclose(C3[7, :, 0], np.float64(big) * 2.0 ** -20, rtol=1e-6) and np.all(np.delete(C3[:, :, 0], 7, axis=0) == 0)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("m,n,k,batch", [(65, 64, 1, 2), (129, 127, 7, 2), (67, 130, 65, 3), (131, 257, 129, 1), (257, 259, 515, 1), (300, 270, 131, 130)])
+def test_operands_of_any_alignment(nn, dtype, ta, tb, m, n, k, batch):
+    """Sizes, row strides and starting elements that are no multiple of a 16-byte piece, at the edges of the tiles and
+    of k, alpha and beta, into a C whose columns are strided: against Float64 on the host; nothing outside C changes."""
+    rng = np.random.default_rng(m * 1000 + k)
+
+    def make(rows, cols, pad, off):
+        flat = round_to(rng.standard_normal(off + batch * cols * (rows + pad)).astype(np.float32), dtype)
+        store = nn.DeviceArray.from_numpy(flat, dtype).storage
+        a = nn.DeviceArray(store, (rows, cols, batch), dtype, (1, rows + pad, (rows + pad) * cols), off)
+        return a, flat[off:].reshape(batch, cols, rows + pad)[:, :, :rows].transpose(0, 2, 1).astype(np.float64)
+
+    A, a = make(k, m, 3, 1) if ta else make(m, k, 0, 1)
+    B, b = make(n, k, 1, 0) if tb else make(k, n, 5, 3)
+    C, c = make(m, n, 1, 1)
+    before = C.storage.float().cpu().numpy()
+    A, a = (nn.batched_transpose(A), a.transpose(0, 2, 1)) if ta else (A, a)
+    B, b = (nn.batched_transpose(B), b.transpose(0, 2, 1)) if tb else (B, b)
+    nn.batched_mul_(C, A, B, 1.5, 0.5)
+    after = C.storage.float().cpu().numpy()
+    ref = 1.5 * (a @ b) + 0.5 * c
+    got = after[1:].reshape(batch, n, m + 1)
+    assert np.abs(got[:, :, :m].transpose(0, 2, 1) - ref).max() <= TOL[dtype] * np.abs(ref).max()
+    assert np.array_equal(got[:, :, m], before[1:].reshape(batch, n, m + 1)[:, :, m]) and after[0] == before[0]
