@@ -305,7 +305,7 @@ def test_dense_mask_on_the_lean_paths(nn, oracle, dtype, D, H, Lq, Lkv, batch, m
     ("bf16", 128, 2, 200, 333, 4, False, True, None),
     ("f16", 64, 1, 130, 1101, 3, False, False, None),
     ("f32", 64, 2, 130, 333, 3, False, True, None),
-    ("bf16", 64, 2, 100, 333, 3, False, True, (0.2, 9)),    # with dropout the unaligned case stays on the per-element paths
+    ("bf16", 64, 2, 100, 333, 3, False, True, (0.2, 9)),    # rows that start at any place within a hash group
 ])
 def test_context_lengths_in_the_gradient(nn, oracle, dtype, D, H, Lq, Lkv, B, causal_too, saved, dropout):
     """Key-padding masks with saved statistics: pairs whose mask keeps a prefix of the keys run the unmasked gradient
@@ -615,3 +615,19 @@ def test_different_head_dims_for_qk_and_v(nn, oracle, dtype, D, Dv, mask_kind, s
     Lkv = Lq if mask_kind == "causal" else 210
     _run(nn, oracle, dtype, D * H, Dv * H, Lq, Lkv, (2,), H, mask_kind=mask_kind, saved=saved, scale=0.7, seed=D + Dv,
          expect="flash32" if dtype == "f32" else "flash16")
+
+
+@pytest.mark.parametrize("dtype,D,H,Lq,Lkv,B,mask_kind,saved", [
+    ("bf16", 64, 2, 64, 64, 1, None, True),        # one whole block, rows on hash groups
+    ("bf16", 64, 2, 65, 63, 2, None, True),        # rows at every place within a group, a partial block each way
+    ("f16", 64, 3, 131, 131, 2, "causal", True),   # blocks above the diagonal are not drawn
+    ("bf16", 128, 2, 191, 257, 1, None, False),    # statistics in the workspace too
+    ("f16", 96, 1, 1, 333, 2, None, True),
+    ("bf16", 32, 2, 333, 5, 2, None, True),
+    ("bf16", 128, 2, 130, 131, 2, "keys", True),   # key-padding mask: context lengths and the rest
+])
+def test_dropout_keep_words(nn, oracle, dtype, D, H, Lq, Lkv, B, mask_kind, saved):
+    """Keep decisions drawn once per gradient call as 64 x 64 blocks of bits, rows and columns, at lengths around the
+    blocks and at every alignment of a row within the hash groups of four weights."""
+    _run(nn, oracle, dtype, D * H, D * H, Lq, Lkv, (B,), H, mask_kind=mask_kind, expect="flash16", saved=saved, dropout=(0.3, 31),
+         seed=Lq + Lkv, scale=0.4)
