@@ -73,10 +73,7 @@ __global__ __launch_bounds__(256) void mask_bits_kernel(const uint8_t *mask, int
 size_t attention_bwd_flash16_lengths_bytes(const AttnBwdParams &bp) {
     const AttnParams &p = bp.p;
     if (!flash_is_query_independent_mask(p) || p.H * p.B > 2147483647LL / 4) return 0;
-    // A small call with dropout and rows off the hash groups is bound by its launches: one set of per-element kernels
-    // instead of the classification, the keep words and two sets (16 pairs of 63 x 63, forward and gradient: 71 us, with
-    // the classification 88; 64 pairs of 131 x 131, gradient alone: 63 and 47).
-    if (p.drop_thresh && (p.Lkv & 3) != 0 && p.Lkv <= 64 && p.Lq <= 128 && p.H * p.B <= 256) return 0;
+    if (flash_is_key_mask(p) && p.Lkv <= 128) return 0;   // short sequences: less is saved than the classification costs
     return ((size_t)(bp.p.H * bp.p.B) * sizeof(int32_t) + 15) & ~(size_t)15;
 }
 
@@ -91,7 +88,7 @@ size_t attention_bwd_flash16_lengths_bytes(const AttnBwdParams &bp) {
 static bool takes_drop_words(const AttnBwdParams &bp) {
     const AttnParams &p = bp.p;
     if (p.drop_thresh == 0 || p.bias) return false;
-    return !p.mask || attention_bwd_flash16_lengths_bytes(bp) != 0 || takes_mask_bits(p);   // what the lean kernels take
+    return !p.mask || flash_is_key_mask(p) || attention_bwd_flash16_lengths_bytes(bp) != 0 || takes_mask_bits(p);   // what the lean kernels take
 }
 static int64_t pad128(int64_t n) { return (n + 127) / 128 * 128; }
 static size_t drop_rows_words(const AttnParams &p) { return (size_t)(p.H * p.B * ((p.Lkv + 63) / 64) * pad128(p.Lq)); }

@@ -26,6 +26,8 @@ struct FlashArgs {
     // gradient kernels only: the launch covers batch elements [b0, b0 + nb), and the bias gradient may be summed
     // without atomics (no two workgroups of one launch add to the same element)
     int32_t b0, nb, dbias_plain;
+    // gradient kernels: the mask is a key-padding mask that the key-stationary kernels apply to a lane's own key
+    int32_t key_mask = 0;
     // forward kernels, key-padding masks that are context lengths: per (head, batch) pair [b * H + h] the number of
     // leading keys kept when the mask keeps exactly a prefix (the software-pipelined kernel then treats it as that
     // pair's L_kv and the general kernel leaves the pair alone), 0 otherwise (the general kernel applies the mask)
@@ -94,16 +96,14 @@ enum { EXTRAS_NONE = 0, EXTRAS_DIRECT = 1, EXTRAS_STAGED = 2, EXTRAS_KEYMASK = 3
 constexpr bool flash_uses_staging(int extras) { return extras == EXTRAS_STAGED || extras == EXTRAS_MASKTILE; }
 // true when the accumulators hold the reference's logits in natural units (bias added) rather than raw dot products
 constexpr bool flash_natural_units(int extras) { return extras == EXTRAS_DIRECT || extras == EXTRAS_STAGED; }
-// query-independent mask without bias whose bytes can be read four keys at a time (unit key stride, Lkv a
-// multiple of 4, 4-byte aligned slices): eligible for EXTRAS_KEYMASK
 // any mask without bias that does not depend on the query (a key-padding mask), whatever its strides: what the
 // device-side measurement of context lengths (FlashArgs::kv_len) applies to
 inline bool flash_is_query_independent_mask(const AttnParams &p) {
     return p.mask && !p.bias && (p.mask_strides[1] == 0 || p.Lq == 1);
 }
+// such a mask with unit key stride and room for one group of four bytes: eligible for EXTRAS_KEYMASK
 inline bool flash_is_key_mask(const AttnParams &p) {
-    return p.mask && !p.bias && p.mask_strides[1] == 0 && p.mask_strides[0] == 1 && (p.Lkv & 3) == 0 &&
-           ((p.mask_strides[2] | p.mask_strides[3]) & 3) == 0 && (((uintptr_t)p.mask) & 3) == 0;
+    return flash_is_query_independent_mask(p) && p.mask_strides[0] == 1 && p.Lkv >= 4;
 }
 
 inline void flash_fill_vec_flags(FlashArgs &a) {
@@ -354,17 +354,24 @@ __device__ inline void flash_atomic_add_block(unsigned wlds, const floatx16_t &v
     }
 }
 
+// Four bytes of a key-padding mask, of keys kv .. kv + 3 of the pair whose bytes start at `mk` (any alignment: the memory
+// pipeline takes it).  A group that would end past the last key is moved back to end with it and shifted into place; keys
+// past the end read as dropped.
+typedef uint32_t flash_u32_any __attribute__((aligned(1)));
+__device__ inline uint32_t flash_key_mask4(const uint8_t *mk, int64_t kv, int64_t Lkv) {
+    if (kv >= Lkv) return 0;
+    const int over = kv + 4 > Lkv ? (int)(kv + 4 - Lkv) : 0;
+    return *(const flash_u32_any *)(mk + kv - over) >> (8 * over);
+}
+
 // Key-mask bytes of a 64-key tile in the accumulator layout: word 4*kb + g holds the four bytes of keys
-// j0 + 32kb + 8g + 4hh .. +3 (nonzero = keep; keys past Lkv read as kept, the edge code drops them).  All lanes
-// of a half-wave read the same bytes.  Callers issue this before the QK^T MFMAs so that the loads are hidden.
+// j0 + 32kb + 8g + 4hh .. +3 (nonzero = keep).  All lanes of a half-wave read the same bytes.  Callers issue this
+// before the QK^T MFMAs so that the loads are hidden.
 __device__ inline void flash_load_key_mask(const FlashArgs &a, int64_t b, int64_t h, int64_t j0, int hh, uint32_t (&w)[8]) {
     const AttnParams &p = a.p;
-    const uint8_t *mk = p.mask + h * p.mask_strides[2] + b * p.mask_strides[3] + j0 + 4 * hh;
+    const uint8_t *mk = p.mask + h * p.mask_strides[2] + b * p.mask_strides[3];
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const int off = 32 * (i >> 2) + 8 * (i & 3);
-        w[i] = j0 + 4 * hh + off < p.Lkv ? *(const uint32_t *)(mk + off) : 0x01010101u;   // Lkv is a multiple of 4
-    }
+    for (int i = 0; i < 8; i++) w[i] = flash_key_mask4(mk, j0 + 4 * hh + 32 * (i >> 2) + 8 * (i & 3), p.Lkv);
 }
 
 // Mask bytes applied without lane masks (a compare writes a lane mask to scalar registers, which costs the compare, a
