@@ -136,6 +136,61 @@ __global__ __launch_bounds__(256) void drop_words_kernel(AttnParams p, int64_t n
     keys[(pair * nqt + qt) * lkv_pad + 64 * kt + lane] = (uint64_t)hi << 32 | lo;
 }
 
+// ---- a bias shared by the batch elements, laid out once for the kernels ------------------------------------------
+// Each batch element's workgroups read the same bias.  One small kernel writes two copies in the order the accumulators hold
+// the scores, so that a lane of the dQ (dK, dV) kernel reads its 16 entries of a block as 32 contiguous bytes, whatever the
+// alignment of the bias rows, and the kernels stay lean (two wavefronts per SIMD).
+static bool takes_bias_blocks(const AttnBwdParams &bp) {
+    const AttnParams &p = bp.p;
+    // entries of their own per key, query and head: what the kernel of the bias gradient takes too
+    return p.bias && !p.mask && p.drop_thresh == 0 && bp.have_stats && p.D <= 128 && p.B > 1 && p.bias_strides[3] == 0 &&
+           p.bias_strides[0] == 1 && (p.bias_strides[1] != 0 || p.Lq == 1) && (p.bias_strides[2] != 0 || p.H == 1) &&
+           pad128(p.Lq) / 128 * (pad128(p.Lkv) / 64) * p.H <= 2147483647LL / 16;
+}
+static size_t bias_copy_entries(const AttnParams &p) { return (size_t)(p.H * pad128(p.Lq) * pad128(p.Lkv)); }
+size_t attention_bwd_flash16_bias_bytes(const AttnBwdParams &bp) {
+    return takes_bias_blocks(bp) ? 2 * sizeof(uint16_t) * bias_copy_entries(bp.p) : 0;
+}
+
+// A wavefront copies 64 of the (query, key) rows of one form: grid.y 0 rows (a block of 32 keys per query, read four keys at
+// a time), 1 keys (a block of 32 queries per key, neighbouring lanes reading neighbouring keys).
+typedef uint32_t u32x2_any2_t __attribute__((ext_vector_type(2), aligned(2)));
+__global__ __launch_bounds__(256) void bias_blocks_kernel(AttnParams p, int64_t lq_pad, int64_t lkv_pad, uint16_t *rows, uint16_t *keys) {
+    const bool by_key = blockIdx.y != 0;
+    const int64_t own_len = by_key ? lkv_pad : lq_pad, blocks = (by_key ? lq_pad : lkv_pad) / 32;
+    const int lane = threadIdx.x & 63;
+    for (int64_t item = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); item < p.H * blocks * (own_len / 32); item += 4 * (int64_t)gridDim.x) {
+        // 64 lanes: rows form 32 queries x 2 halves of a block, so that a query's 64 bytes are read and written together; keys
+        // form 64 keys of one half
+        const int64_t per = own_len / 32, part = item % per, blk = item / per % blocks, h = item / (per * blocks);
+        const int hh = by_key ? (int)(part & 1) : lane & 1;
+        const int64_t own = by_key ? 64 * (part >> 1) + lane : 32 * part + (lane >> 1);
+        const uint16_t *src = (const uint16_t *)p.bias + h * p.bias_strides[2];
+        uint32_t out[8];
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const int64_t first = 32 * blk + 8 * g + 4 * hh;
+            uint32_t x[4] = {0, 0, 0, 0};
+            if (!by_key && own < p.Lq && first + 4 <= p.Lkv) {   // four keys at any alignment
+                const u32x2_any2_t v = *(const u32x2_any2_t *)(src + own * p.bias_strides[1] + first);
+                out[2 * g] = v[0];
+                out[2 * g + 1] = v[1];
+                continue;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int64_t q = by_key ? first + e : own, kv = by_key ? own : first + e;
+                if (q < p.Lq && kv < p.Lkv) x[e] = src[q * p.bias_strides[1] + kv];
+            }
+            out[2 * g] = x[0] | x[1] << 16;
+            out[2 * g + 1] = x[2] | x[3] << 16;
+        }
+        u32x4_t *dst = (u32x4_t *)((by_key ? keys : rows) + ((h * blocks + blk) * own_len + own) * 32 + 16 * hh);
+        dst[0] = (u32x4_t){out[0], out[1], out[2], out[3]};
+        dst[1] = (u32x4_t){out[4], out[5], out[6], out[7]};
+    }
+}
+
 // ---- dQ kernel split over the keys ---------------------------------------------------------------------------
 // The dQ kernel has one workgroup per (query tile, head, batch): cross-attention with few queries and many keys
 // leaves most of the chip idle (32 workgroups for 128 queries, 16 heads, 2 batch elements).  With saved statistics
@@ -208,6 +263,14 @@ int32_t launch_attention_bwd_flash16(const AttnBwdParams &bp_in, hipStream_t st)
         MI_LAUNCH_CHECK();
         bp.drop_rows = rows;
         bp.drop_keys = keys;
+    }
+    if (takes_bias_blocks(bp)) {   // saved statistics, no mask, no dropout: behind the partial sums of dQ
+        const int64_t lq_pad = pad128(p.Lq), lkv_pad = pad128(p.Lkv), groups = (int64_t)bias_copy_entries(p) / 4096;   // four wavefronts each
+        uint16_t *rows = (uint16_t *)((char *)bp.workspace + attention_bwd_flash16_dq_partial_bytes(bp)), *keys = rows + bias_copy_entries(p);
+        hipLaunchKernelGGL(bias_blocks_kernel, dim3((unsigned)(groups < 8192 ? groups : 8192), 2), dim3(256), 0, st, p, lq_pad, lkv_pad, rows, keys);
+        MI_LAUNCH_CHECK();
+        bp.bias_rows = rows;
+        bp.bias_keys = keys;
     }
     int32_t rc;
     if (p.dtype == MI_BF16)

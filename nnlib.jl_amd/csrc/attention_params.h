@@ -78,6 +78,10 @@ struct AttnBwdParams {
     // one word per (pair, tile of 64 keys, query), bit = key of the tile; drop_keys one per (pair, tile of 64 queries,
     // key), bit = query of the tile.  [pair][tile][queries / keys rounded up to 128]; null without dropout
     const uint64_t *drop_rows, *drop_keys;
+    // bias shared by the batch elements, copied in the order the gradient kernels' accumulators hold scores (zeros past the
+    // ends, lengths rounded up to 128): bias_rows [h][block of 32 keys][query][hh][16], entry 4g + e = key 8g + 4hh + e of
+    // the block; bias_keys [h][block of 32 queries][key][hh][16], likewise with queries.  null where the call has none
+    const uint16_t *bias_rows, *bias_keys;
     // key-padding mask measured on the device: per (head, batch) pair [b * H + h] the context length, or 0 when the
     // mask of the pair is not a kept prefix; null when the call does not take that path
     const int32_t *kv_len;
@@ -102,6 +106,7 @@ size_t attention_bwd_flash32_lengths_bytes(const AttnBwdParams &bp);
 size_t attention_bwd_flash16_workspace(const AttnParams &p);
 size_t attention_bwd_flash16_mask_bits_bytes(const AttnParams &p);   // 0 when the call does not take the packed-mask path
 size_t attention_bwd_flash16_drop_bytes(const AttnBwdParams &bp);     // 0 when the call does not take the keep words
+size_t attention_bwd_flash16_bias_bytes(const AttnBwdParams &bp);     // 0 when the call does not take the bias copies
 size_t attention_bwd_flash16_lengths_bytes(const AttnBwdParams &bp);  // 0 when the call does not take the context-length path
 int attention_bwd_flash16_dq_nsplit(const AttnBwdParams &bp);         // pieces the dQ kernel's key range is cut into (1: no split)
 size_t attention_bwd_flash16_dq_partial_bytes(const AttnBwdParams &bp);   // the same rule serves the Float32 kernels

@@ -162,6 +162,21 @@ def test_bias_gradient_from_the_mfma_kernels(nn, oracle, dtype, D, H, Lq, Lkv, b
          scale=0.4, expect=expect)
 
 
+@pytest.mark.parametrize("dtype,D,H,Lq,Lkv,B,mask_kind,saved", [
+    ("bf16", 64, 3, 197, 197, 9, None, True),       # odd rows, ragged tiles, the batch in pieces
+    ("bf16", 64, 2, 128, 64, 2, None, False),       # whole tiles
+    ("f16", 40, 2, 129, 65, 5, None, True),         # one row / key past a tile, features past the head dim
+    ("bf16", 128, 2, 161, 161, 4, "causal", True),  # tiles above the diagonal are left out
+    ("bf16", 64, 16, 2040, 70, 3, None, True),      # enough tiles for sums without atomics
+    ("f16", 256, 1, 33, 300, 3, None, True),        # 256-wide tiles
+    ("bf16", 64, 1, 1, 100, 3, None, True),         # one query
+])
+def test_gradient_of_a_bias_shared_by_the_batch(nn, oracle, dtype, D, H, Lq, Lkv, B, mask_kind, saved):
+    """A bias per (key, query, head): its gradient is summed over the batch by a kernel of its own."""
+    _run(nn, oracle, dtype, D * H, D * H, Lq, Lkv, (B,), H, bias_shape=(Lkv, Lq, H, 1), mask_kind=mask_kind, seed=Lq + Lkv + B,
+         scale=0.4, saved=saved, expect="flash16")
+
+
 F32_CASES = [
     # D, H, Lq, Lkv, batch, mask_kind, saved statistics
     (64, 2, 200, 200, (2,), "causal", False),
