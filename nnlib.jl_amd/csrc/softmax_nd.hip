@@ -53,6 +53,8 @@ __device__ inline float softmax_term(float x, float m) {   // src/softmax.jl:72-
     if (m == MI_POS_INF) return x == MI_POS_INF ? 1.0f : 0.0f;
     return fast_exp(x - m);
 }
+// a term over the column's sum: Float32 divides; the 16-bit types, rounded far above the error, take 1 / sum
+template <int VEC> __device__ inline float share(float term, float c) { return VEC == 4 ? term / c : term * c; }
 __device__ inline float logsoftmax_shift(float x, float m) {   // src/softmax.jl:140-144
     if (m == MI_POS_INF) return x == MI_POS_INF ? 0.0f : MI_NEG_INF;
     return x - m;
@@ -411,17 +413,16 @@ __global__ __launch_bounds__(NT, (NP * (OP >= OP_GRAD_SOFTMAX ? 2 : 1) <= 16 && 
             // the same for the whole wavefront; logsumexp has no special cases (src/softmax.jl:202)
             const bool plain = OP == OP_LOGSUMEXP || __builtin_amdgcn_ballot_w64(!finite) == 0;
             keep_packed(raw);
+            // x - m first, exact near the maximum: with m folded into the exponent's constant a column of the type's
+            // lowest value would be Inf - Inf, and maxima of some thousands cost Float32 its last digits
             if (plain) {
-                float cm[VEC];
-#pragma unroll
-                for (int e = 0; e < VEC; e++) cm[e] = -m[e] * MI_LOG2E;
 #pragma unroll
                 for (int u = 0; u < NP; u++) {
                     if (FULL || u < nrows) {
                         float v[VEC];
                         IO::unpack(raw[u], v);
 #pragma unroll
-                        for (int e = 0; e < VEC; e++) sum[e] += mi_exp2(fmaf(v[e], MI_LOG2E, cm[e]));
+                        for (int e = 0; e < VEC; e++) sum[e] += fast_exp(v[e] - m[e]);
                     }
                 }
             } else {
@@ -446,17 +447,9 @@ __global__ __launch_bounds__(NT, (NP * (OP >= OP_GRAD_SOFTMAX ? 2 : 1) <= 16 && 
                     IO::store(y + cur.col + g.inner * cur.o, r, cur.skip);
                 }
             } else if (plain) {
-                // m and sum fold into two constants per position
-                float c0[VEC], c1[VEC];
+                float c1[VEC];
 #pragma unroll
-                for (int e = 0; e < VEC; e++) {
-                    if (OP == OP_SOFTMAX) {
-                        c0[e] = -m[e] * MI_LOG2E;
-                        c1[e] = 1.0f / sum[e];
-                    } else {
-                        c1[e] = -m[e] - logf(sum[e]);
-                    }
-                }
+                for (int e = 0; e < VEC; e++) c1[e] = OP == OP_LOGSOFTMAX ? logf(sum[e]) : VEC == 4 ? sum[e] : 1.0f / sum[e];
 #pragma unroll
                 for (int u = 0; u < NP; u++) {
                     if (FULL || u < nrows) {
@@ -464,7 +457,7 @@ __global__ __launch_bounds__(NT, (NP * (OP >= OP_GRAD_SOFTMAX ? 2 : 1) <= 16 && 
                         IO::unpack(raw[u], v);
 #pragma unroll
                         for (int e = 0; e < VEC; e++)
-                            r[e] = OP == OP_SOFTMAX ? mi_exp2(fmaf(v[e], MI_LOG2E, c0[e])) * c1[e] : v[e] + c1[e];
+                            r[e] = OP == OP_SOFTMAX ? share<VEC>(fast_exp(v[e] - m[e]), c1[e]) : v[e] - m[e] - c1[e];
                         put(cur, u, IO::pack(r));
                     }
                     }
@@ -567,7 +560,7 @@ __global__ __launch_bounds__(256) void softmax_nd_short_kernel(const typename T:
         }
     } else {
 #pragma unroll
-        for (int e = 0; e < VEC; e++) s[e] = OP == OP_SOFTMAX ? 1.0f / s[e] : OP == OP_LOGSOFTMAX ? logf(s[e]) : s[e];
+        for (int e = 0; e < VEC; e++) s[e] = OP == OP_SOFTMAX && VEC != 4 ? 1.0f / s[e] : OP == OP_LOGSOFTMAX ? logf(s[e]) : s[e];
 #pragma unroll
         for (int u = 0; u < NP; u++) {
             if (!mine(u)) break;
@@ -576,7 +569,7 @@ __global__ __launch_bounds__(256) void softmax_nd_short_kernel(const typename T:
             if (GRAD) IO::unpack(raw2[u], v2);
 #pragma unroll
             for (int e = 0; e < VEC; e++) {
-                if (OP == OP_SOFTMAX) r[e] = softmax_term(v[e], m[e]) * s[e];
+                if (OP == OP_SOFTMAX) r[e] = share<VEC>(softmax_term(v[e], m[e]), s[e]);
                 else if (OP == OP_LOGSOFTMAX) r[e] = logsoftmax_shift(v[e], m[e]) - s[e];
                 else if (OP == OP_GRAD_SOFTMAX) r[e] = v2[e] * (v[e] - s[e]);
                 else r[e] = v[e] - s[e] * fast_exp(v2[e]);
@@ -666,18 +659,12 @@ __global__ __launch_bounds__(256) void softmax_nd_vec_kernel(const typename T::t
             continue;
         }
         // per-position constants of the second pass; `plain`: finite maxima, so no special cases
-        float c0[VEC], c1[VEC];
+        float c1[VEC];
         bool plain = true;
 #pragma unroll
         for (int e = 0; e < VEC; e++) {
             plain = plain && m[e] > MI_NEG_INF && m[e] < MI_POS_INF;
-            if (OP == OP_SOFTMAX) {
-                c0[e] = -m[e] * MI_LOG2E;
-                c1[e] = 1.0f / s[e];
-            } else if (OP == OP_LOGSOFTMAX) {
-                c0[e] = logf(s[e]);
-                c1[e] = -m[e] - c0[e];
-            }
+            c1[e] = OP == OP_LOGSOFTMAX ? logf(s[e]) : VEC == 4 ? s[e] : 1.0f / s[e];
         }
         for (int64_t r0 = 0; r0 < nrows; r0 += U) {
             u32x4_t raw[U], raw2[U];
@@ -695,8 +682,8 @@ __global__ __launch_bounds__(256) void softmax_nd_vec_kernel(const typename T::t
                 if (GRAD) IO::unpack(raw2[u], v2);
 #pragma unroll
                 for (int e = 0; e < VEC; e++) {
-                    if (OP == OP_SOFTMAX) r[e] = plain ? mi_exp2(fmaf(v[e], MI_LOG2E, c0[e])) * c1[e] : softmax_term(v[e], m[e]) / s[e];
-                    else if (OP == OP_LOGSOFTMAX) r[e] = plain ? v[e] + c1[e] : logsoftmax_shift(v[e], m[e]) - c0[e];
+                    if (OP == OP_SOFTMAX) r[e] = share<VEC>(plain ? fast_exp(v[e] - m[e]) : softmax_term(v[e], m[e]), c1[e]);
+                    else if (OP == OP_LOGSOFTMAX) r[e] = (plain ? v[e] - m[e] : logsoftmax_shift(v[e], m[e])) - c1[e];
                     else if (OP == OP_GRAD_SOFTMAX) r[e] = v2[e] * (v[e] - s[e]);
                     else r[e] = v[e] - s[e] * fast_exp(v2[e]);
                 }
@@ -714,7 +701,7 @@ void launch_nd(const void *x, const void *x2, void *y, int64_t inner, int64_t le
     g.len = len;
     g.outer = outer;
     constexpr int VEC = 16 / (int)sizeof(t);
-    if (inner >= VEC) {
+    if (inner >= VEC && len > 0) {   // (an empty reduction has no row that the clamped loads below could read)
         const int64_t chunks = (inner + VEC - 1) / VEC;
         // Measured where the two cross (us, short / cached): 500 x 128 x 400 softmax bf16 34 / 45, f32 45 / 53, their
         // gradients 41 / 29 and 76 / 57; at len 64 the short kernel wins everywhere (64 x 64 x 4000 f32 23 / 35, 30 / 31).

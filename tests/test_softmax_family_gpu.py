@@ -346,3 +346,35 @@ def test_strided_rows_of_any_width(nn, oracle, dtype, inner, length, outer):
         assert np.array_equal(np.isnan(got), np.isnan(ref))
         fin = np.isfinite(ref)
         assert np.abs(got[fin] - ref[fin]).max() <= tol * 10
+
+
+@pytest.mark.parametrize("dtype,inner", [("f32", 1), ("f32", 3), ("f32", 4), ("f32", 37), ("f32", 64), ("bf16", 9), ("bf16", 64), ("f16", 12)])
+@pytest.mark.parametrize("length", [1, 5, 200, 9000])
+def test_columns_far_from_zero(nn, oracle, dtype, inner, length):
+    """softmax is invariant under shifts: whole numbers up to 1024 + 15 are exact in every type (bf16 up to 255), so
+    columns shifted by 1024 (240) have the results of the unshifted ones, in the arithmetic's own error; a column of the
+    lowest finite value, as a mask leaves it, is uniform."""
+    rng = np.random.default_rng(inner + length)
+    x = rng.integers(0, 16, (inner, length, 3)).astype(np.float32)
+    shift = 240.0 if dtype == "bf16" else 1024.0
+    low = {"f32": np.finfo(np.float32).min, "f16": np.float32(np.finfo(np.float16).min), "bf16": np.float32(-3.3895313892515355e38)}[dtype]
+    moved = x + np.float32(shift)
+    x[:, :, 1] = 0.0
+    moved[:, :, 1] = low
+    for log, fn in ((False, nn.softmax), (True, nn.logsoftmax)):
+        got = fn(_dev(nn, moved, dtype), dims=2).to_numpy()
+        same = fn(_dev(nn, x, dtype), dims=2).to_numpy()
+        assert np.array_equal(got, same), (log, np.abs(got - same).max())
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("inner", [1, 3, 8, 100])
+def test_empty_logsumexp_reads_nothing(nn, dtype, inner):
+    """logsumexp over no rows is log(0) = -Inf, whatever the width of a row."""
+    import torch
+    _lib = nn._lib
+    tdt, code = (torch.float32, _lib.MI_F32) if dtype == "f32" else (torch.bfloat16, _lib.MI_BF16)
+    y = torch.zeros(inner * 3, dtype=tdt, device="cuda")
+    x = torch.zeros(16, dtype=tdt, device="cuda")
+    _lib.check(_lib.load().mi_logsumexp(code, x.data_ptr(), y.data_ptr(), inner, 0, 3, torch.cuda.current_stream().cuda_stream))
+    assert bool((y == float("-inf")).all())
