@@ -646,3 +646,29 @@ def test_dropout_keep_words(nn, oracle, dtype, D, H, Lq, Lkv, B, mask_kind, save
     blocks and at every alignment of a row within the hash groups of four weights."""
     _run(nn, oracle, dtype, D * H, D * H, Lq, Lkv, (B,), H, mask_kind=mask_kind, expect="flash16", saved=saved, dropout=(0.3, 31),
          seed=Lq + Lkv, scale=0.4)
+
+
+@pytest.mark.parametrize("Lkv", [332, 333])
+def test_weights_of_the_dropout_gradient_keep_float32_accuracy(nn, oracle, Lkv):
+    """The gradient's weights before they are rounded to 16 bits.  dO is the identity, so dV holds the weights themselves,
+    rounded once; q and k are whole numbers whose scores (about 700) are exact in Float32, so that only the exponential, the
+    row sum and the factors err: a few 2^-24, 3e-7 at most.  A relative error e changes the rounding of a share e / 2^-7 to
+    e / 2^-8 of the values: below 8e-5, and 2e-4 is allowed.  With 1 / row sum added to an exponent of 1016 the error is up
+    to 2^-15 ln 2 = 2e-5, and the share about 2e-3.  (Head dim 16: a forward kernel that keeps q as it is.)"""
+    rng = np.random.default_rng(Lkv)
+    D = L = 16
+    H, B, p, seed = 16, 16, 0.5, 11
+    q = rng.integers(-1, 2, (D * H, L, B)).astype(np.float32)
+    k = rng.integers(-1, 2, (D * H, Lkv, B)).astype(np.float32)
+    q[::D], k[::D] = 32.0, 88.0
+    v = round_to(rng.standard_normal((D * H, Lkv, B)), "bf16")
+    dy = np.tile(np.eye(D, dtype=np.float32)[None, :, :, None], (H, 1, 1, B)).reshape(D * H, L, B)
+    d = [nn.DeviceArray.from_numpy(a, "bf16") for a in (q, k, v, dy)]
+    drop = nn.Dropout(p, seed)
+    y, _ = nn.dot_product_attention(*d[:3], nheads=H, return_weights=False, fdrop=drop, save_for_backward=True)
+    dv = nn.dot_product_attention_grad(d[3], *d[:3], y=y, nheads=H, fdrop=drop)[2].to_numpy()
+    s = np.einsum("hdjb,hdib->hjib", k.reshape(H, D, Lkv, B).astype(np.float64), q.reshape(H, D, L, B).astype(np.float64)) / 4
+    w = np.exp(s - s.max(axis=1, keepdims=True))
+    w = w / w.sum(axis=1, keepdims=True) * oracle.dropout_keep_mask((Lkv, L, H, B), p, seed).transpose(2, 0, 1, 3) * 2
+    want = round_to(w.transpose(0, 2, 1, 3).reshape(D * H, Lkv, B), "bf16")
+    assert np.mean(dv != want) <= 2e-4
