@@ -76,13 +76,27 @@ def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
+class _WorkspaceSize(int):
+    """Bytes of the workspace of the most recent call that had one (the memory itself is not held)."""
+
+    def numel(self):
+        return int(self)
+
+
 def _get_workspace(nbytes):
+    """Device scratch for one call: (tensor, bytes), or (None, 0) where none is wanted.  Every call gets its own from
+    torch's caching allocator on the current stream: a kernel that fills it and the kernels that read it may have any
+    other call's launches between them, from another stream or from another thread on the same stream.  The caller keeps
+    the tensor until its launches are issued; memory freed then is handed out again on this stream only, in order."""
     global _workspace
     if nbytes == 0:
         return None, 0
-    if _workspace is None or _workspace.numel() < nbytes:
-        _workspace = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
-    return _workspace, _workspace.numel()
+    _workspace = _WorkspaceSize(nbytes)
+    return torch.empty(nbytes, dtype=torch.uint8, device="cuda"), nbytes
+
+
+def _pointer(tensor):
+    return None if tensor is None else tensor.data_ptr()
 
 
 def _broadcast_strides(x, target, what):
@@ -366,7 +380,7 @@ def _reduction_geometry(dims_of_x, dims):
 
 def _dims_call(x, dims):
     """Arguments of the `*_dims` entry points for a reduction of ``x`` over ``dims`` (a 1-based dimension, a tuple of
-    dimensions, adjacent or not, or ``None`` for Julia's ``:``): (ndim, sizes, mask, workspace pointer, workspace
+    dimensions, adjacent or not, or ``None`` for Julia's ``:``): (ndim, sizes, mask, workspace tensor or None, workspace
     bytes, size of the reduced result).  The library permutes sets that are not runs of adjacent dimensions."""
     size = tuple(x.dims)
     if len(size) > 8:
@@ -383,7 +397,7 @@ def _dims_call(x, dims):
     nb = ctypes.c_size_t(0)
     _lib.check(_lib.load().mi_softmax_dims_workspace(x.code_f64, len(size), sizes, mask, ctypes.byref(nb)))
     wbuf, wsize = _get_workspace(nb.value)
-    return len(size), sizes, mask, (wbuf.data_ptr() if wbuf is not None else None), wsize, kept
+    return len(size), sizes, mask, wbuf, wsize, kept
 
 
 def _assign(out, y):
@@ -419,7 +433,7 @@ def _softmax_like(name, op, out, x, dims):
     if x.dtype == "bool" or out.dtype != x.dtype:
         raise ArgumentError(f"{name} needs floating-point input and output of one element type (integer input: Float64 output)")
     nd, sizes, mask, ws, wsize, _ = _dims_call(x, dims)
-    _lib.check(_lib.load().mi_softmax_dims(op, x.code_f64, x.ptr, out.ptr, nd, sizes, mask, ws, wsize, _stream()))
+    _lib.check(_lib.load().mi_softmax_dims(op, x.code_f64, x.ptr, out.ptr, nd, sizes, mask, _pointer(ws), wsize, _stream()))
     return out
 
 
@@ -461,7 +475,7 @@ def logsumexp(x, *, dims=None):
         raise ArgumentError("logsumexp needs a floating-point array")
     nd, sizes, mask, ws, wsize, kept = _dims_call(x, dims)
     out = DeviceArray.empty(kept, x.dtype)
-    _lib.check(_lib.load().mi_logsumexp_dims(x.code_f64, x.ptr, out.ptr, nd, sizes, mask, ws, wsize, _stream()))
+    _lib.check(_lib.load().mi_logsumexp_dims(x.code_f64, x.ptr, out.ptr, nd, sizes, mask, _pointer(ws), wsize, _stream()))
     return out
 
 
@@ -479,7 +493,7 @@ def grad_logsumexp(dy, x, *, dims=None, lse=None):
     if dy.length != n_out or lse.length != n_out or not (dy.dtype == lse.dtype == x.dtype):
         raise DimensionMismatch(f"dy and lse must have the size {kept} of logsumexp(x; dims) and the element type of x")
     dx = DeviceArray.empty(x.dims, x.dtype)
-    _lib.check(_lib.load().mi_logsumexp_bwd_dims(x.code_f64, dy.ptr, x.ptr, lse.ptr, dx.ptr, nd, sizes, mask, ws, wsize, _stream()))
+    _lib.check(_lib.load().mi_logsumexp_bwd_dims(x.code_f64, dy.ptr, x.ptr, lse.ptr, dx.ptr, nd, sizes, mask, _pointer(ws), wsize, _stream()))
     return dx
 
 
@@ -490,7 +504,7 @@ def _softmax_grad(name, op, dx, dy, y, dims):
     if y.dtype == "bool" or not (dy.dtype == y.dtype == dx.dtype):
         raise ArgumentError(f"{name} needs one floating-point element type for dx, dy and y")
     nd, sizes, mask, ws, wsize, _ = _dims_call(y, dims)
-    _lib.check(_lib.load().mi_softmax_bwd_dims(op, y.code_f64, dy.ptr, y.ptr, dx.ptr, nd, sizes, mask, ws, wsize, _stream()))
+    _lib.check(_lib.load().mi_softmax_bwd_dims(op, y.code_f64, dy.ptr, y.ptr, dx.ptr, nd, sizes, mask, _pointer(ws), wsize, _stream()))
     return dx
 
 
