@@ -215,7 +215,10 @@ int32_t mi_attention_fwd_static(const mi_attn_desc *desc, mi_stream stream);
  *   dbias    : NULL, or FLOAT32 array addressed with fwd.bias_strides; the gradient is ADDED into
  *              it (dims with stride 0 receive the sum over that dim), so the caller zero-fills it.
  *   workspace: at least mi_attention_bwd_plan()'s size, 16-byte aligned (256-byte aligned when q / k and v have
- *              different head dims: the narrower side is zero-padded inside it for the matrix-core kernels).
+ *              different head dims: the narrower side is zero-padded inside it for the matrix-core kernels).  Part of the
+ *              size only saves time in 16-bit calls with fused dropout (keep decisions drawn once) or a bias shared by the
+ *              batch elements (copies of it): they run with less too, and with saved statistics (fwd.stats) and no mask
+ *              with none (unless few queries meet many keys without `causal`: partial sums of dq).
  * A query whose keys are all dropped has NaN weights in the forward pass and NaN gradients here.
  */
 typedef struct mi_attn_bwd_desc {

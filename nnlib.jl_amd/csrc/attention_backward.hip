@@ -22,6 +22,7 @@ static int32_t validate_bwd(const mi_attn_bwd_desc *d, AttnBwdParams *out) {
     bp.dv = d->dv;
     bp.dbias = d->dbias;
     bp.workspace = d->workspace;
+    bp.workspace_bytes = d->workspace ? d->workspace_bytes : 0;
     bp.mask_bits = nullptr;
     bp.drop_rows = bp.drop_keys = nullptr;
     bp.bias_rows = bp.bias_keys = nullptr;
@@ -35,23 +36,23 @@ static int32_t validate_bwd(const mi_attn_bwd_desc *d, AttnBwdParams *out) {
     return MI_OK;
 }
 
-static int32_t choose_bwd(const mi_attn_bwd_desc *d, const AttnBwdParams &bp, size_t *ws) {
+// A workspace: what a call cannot run without, and what it is faster with.
+struct BwdWorkspace {
+    size_t needed = 0, wanted = 0;
+};
+
+static int32_t choose_bwd(const mi_attn_bwd_desc *d, const AttnBwdParams &bp, BwdWorkspace *ws) {
     if (!(d->fwd.flags & MI_ATTN_FORCE_GENERIC) && attention_bwd_flash16_supports(bp)) {
-        *ws = (bp.have_stats ? 0 : attention_bwd_flash16_workspace(bp.p)) + attention_bwd_flash16_mask_bits_bytes(bp.p) +
-              attention_bwd_flash16_lengths_bytes(bp) + attention_bwd_flash16_dq_partial_bytes(bp) + attention_bwd_flash16_drop_bytes(bp) +
-              attention_bwd_flash16_bias_bytes(bp);
+        ws->needed = attention_bwd_flash16_workspace_needed(bp);
+        ws->wanted = attention_bwd_flash16_workspace_wanted(bp);
         return MI_ATTN_KERNEL_FLASH16;
     }
     if (!(d->fwd.flags & MI_ATTN_FORCE_GENERIC) && attention_bwd_flash32_supports(bp)) {
-        *ws = (bp.have_stats ? 0 : attention_stats_bytes(bp.p)) + attention_bwd_flash32_lengths_bytes(bp) +
-              attention_bwd_flash16_dq_partial_bytes(bp);
+        ws->needed = ws->wanted = (bp.have_stats ? 0 : attention_stats_bytes(bp.p)) + attention_bwd_flash32_lengths_bytes(bp) +
+                                  attention_bwd_flash16_dq_partial_bytes(bp);
         return MI_ATTN_KERNEL_FLASH32;
     }
-    if (bp.have_stats) {   // the generic kernels keep their own statistics, in their own layout
-        *ws = attention_bwd_generic_workspace(bp.p);
-        return MI_ATTN_KERNEL_GENERIC;
-    }
-    *ws = attention_bwd_generic_workspace(bp.p);
+    ws->needed = ws->wanted = attention_bwd_generic_workspace(bp.p);   // (saved statistics do not help: its own have another layout)
     return MI_ATTN_KERNEL_GENERIC;
 }
 
@@ -82,7 +83,7 @@ static int32_t resolve_bwd(const mi_attn_bwd_desc *d, mi_attn_bwd_desc *eff, Rec
     probe.fwd.out = (void *)d->dout;   // the right size and alignment class
     st = validate_bwd(&probe, &bp);
     if (st != MI_OK) return st;
-    size_t ws = 0;
+    BwdWorkspace ws;
     if (choose_bwd(&probe, bp, &ws) == MI_ATTN_KERNEL_GENERIC) return MI_OK;
     // what the forward call would be, and whether its kernel saves the row statistics
     mi_attn_desc f = d->fwd;
@@ -110,7 +111,7 @@ static int32_t resolve_bwd(const mi_attn_bwd_desc *d, mi_attn_bwd_desc *eff, Rec
     return MI_OK;
 }
 
-static int32_t bwd_plan_impl(const mi_attn_bwd_desc *d, int32_t *kernel, size_t *workspace_bytes) {
+static int32_t bwd_plan_impl(const mi_attn_bwd_desc *d, int32_t *kernel, BwdWorkspace *workspace) {
     AttnBwdParams bp;
     int32_t rc = validate_bwd(d, &bp);
     if (rc != MI_OK) return rc;
@@ -120,11 +121,12 @@ static int32_t bwd_plan_impl(const mi_attn_bwd_desc *d, int32_t *kernel, size_t 
     if (rc != MI_OK) return rc;
     rc = validate_bwd(&eff, &bp);
     if (rc != MI_OK) return rc;
-    size_t ws = 0;
+    BwdWorkspace ws;
     const int32_t k = choose_bwd(&eff, bp, &ws);
-    if (re.on) ws = re.y_bytes + re.stats_bytes + (ws > re.fwd_ws ? ws : re.fwd_ws);   // the two calls share the tail
+    if (re.on)   // the two calls share the tail
+        for (size_t *n : {&ws.needed, &ws.wanted}) *n = re.y_bytes + re.stats_bytes + (*n > re.fwd_ws ? *n : re.fwd_ws);
     if (kernel) *kernel = k;
-    if (workspace_bytes) *workspace_bytes = ws;
+    *workspace = ws;
     return MI_OK;
 }
 
@@ -137,11 +139,11 @@ static int32_t bwd_impl(const mi_attn_bwd_desc *d, mi_stream s, int64_t scale_D)
     rc = resolve_bwd(d, &eff, &re);
     if (rc != MI_OK) return rc;
     if (re.on) {
-        size_t need = 0;
-        rc = bwd_plan_impl(d, nullptr, &need);
+        BwdWorkspace plan;
+        rc = bwd_plan_impl(d, nullptr, &plan);
         if (rc != MI_OK) return rc;
-        if (!d->workspace || d->workspace_bytes < need)
-            return mi_set_error(MI_EWORKSPACE, "mi_attention_bwd: workspace of %zu bytes required, %zu given", need,
+        if (!d->workspace || d->workspace_bytes < plan.needed)
+            return mi_set_error(MI_EWORKSPACE, "mi_attention_bwd: workspace of %zu bytes required, %zu given", plan.needed,
                                 d->workspace ? d->workspace_bytes : (size_t)0);
         if ((((uintptr_t)d->workspace) & 255) != 0)
             return mi_set_error(MI_EWORKSPACE, "mi_attention_bwd: without the forward result the workspace must be 256-byte aligned");
@@ -176,11 +178,10 @@ static int32_t bwd_impl(const mi_attn_bwd_desc *d, mi_stream s, int64_t scale_D)
         if (bp.dv && (rc = mi_fill_zero(bp.dv, (size_t)(p.Ev * p.Lkv * p.B) * es, s)) != MI_OK) return rc;
         return MI_OK;
     }
-    size_t ws = 0;
+    BwdWorkspace ws;
     const int32_t kernel = choose_bwd(d, bp, &ws);
-    if (ws > 0 && (!d->workspace || d->workspace_bytes < ws))
-        return mi_set_error(MI_EWORKSPACE, "mi_attention_bwd: workspace of %zu bytes required, %zu given", ws,
-                            d->workspace ? d->workspace_bytes : (size_t)0);
+    if (bp.workspace_bytes < ws.needed)
+        return mi_set_error(MI_EWORKSPACE, "mi_attention_bwd: workspace of %zu bytes required, %zu given", ws.needed, bp.workspace_bytes);
     if ((((uintptr_t)d->workspace) & 15) != 0) return mi_set_error(MI_EWORKSPACE, "mi_attention_bwd: workspace must be 16-byte aligned");
     if (kernel == MI_ATTN_KERNEL_FLASH16) return launch_attention_bwd_flash16(bp, st);
     if (kernel == MI_ATTN_KERNEL_FLASH32) return launch_attention_bwd_flash32(bp, st);
@@ -279,30 +280,37 @@ static mi_attn_bwd_desc padded_desc(const mi_attn_bwd_desc *d, const PadPlan &pp
     return e;
 }
 
-MI_API int32_t mi_attention_bwd_plan(const mi_attn_bwd_desc *d, int32_t *kernel, size_t *workspace_bytes) {
-    const PadPlan pp = plan_padding(d);
-    if (!pp.on) return bwd_plan_impl(d, kernel, workspace_bytes);
+static int32_t plan_padded(const mi_attn_bwd_desc *d, const PadPlan &pp, int32_t *kernel, BwdWorkspace *workspace) {
+    if (!pp.on) return bwd_plan_impl(d, kernel, workspace);
     const mi_attn_bwd_desc e = padded_desc(d, pp, nullptr);
-    size_t ws = 0;
+    BwdWorkspace ws;
     int32_t k = 0;
     const int32_t rc = bwd_plan_impl(&e, &k, &ws);
     if (rc != MI_OK) return rc;
-    if (k == MI_ATTN_KERNEL_GENERIC) return bwd_plan_impl(d, kernel, workspace_bytes);   // padding buys nothing there
+    if (k == MI_ATTN_KERNEL_GENERIC) return bwd_plan_impl(d, kernel, workspace);   // padding buys nothing there
     if (kernel) *kernel = k;
-    if (workspace_bytes) *workspace_bytes = pp.total + ws;
+    workspace->needed = pp.total + ws.needed;
+    workspace->wanted = pp.total + ws.wanted;
     return MI_OK;
+}
+
+MI_API int32_t mi_attention_bwd_plan(const mi_attn_bwd_desc *d, int32_t *kernel, size_t *workspace_bytes) {
+    BwdWorkspace ws;
+    const int32_t rc = plan_padded(d, plan_padding(d), kernel, &ws);
+    if (rc == MI_OK && workspace_bytes) *workspace_bytes = ws.wanted;
+    return rc;
 }
 
 MI_API int32_t mi_attention_bwd(const mi_attn_bwd_desc *d, mi_stream s) {
     const PadPlan pp = plan_padding(d);
     if (pp.on) {
-        size_t need = 0;
+        BwdWorkspace plan;
         int32_t k = 0;
-        int32_t rc = mi_attention_bwd_plan(d, &k, &need);
+        int32_t rc = plan_padded(d, pp, &k, &plan);
         if (rc != MI_OK) return rc;
         if (k != MI_ATTN_KERNEL_GENERIC) {
-            if (!d->workspace || d->workspace_bytes < need)
-                return mi_set_error(MI_EWORKSPACE, "mi_attention_bwd: workspace of %zu bytes required, %zu given", need,
+            if (!d->workspace || d->workspace_bytes < plan.needed)
+                return mi_set_error(MI_EWORKSPACE, "mi_attention_bwd: workspace of %zu bytes required, %zu given", plan.needed,
                                     d->workspace ? d->workspace_bytes : (size_t)0);
             if ((((uintptr_t)d->workspace) & 255) != 0)
                 return mi_set_error(MI_EWORKSPACE, "mi_attention_bwd: with different head dims for q / k and v the workspace must be 256-byte aligned");

@@ -28,9 +28,6 @@ bool attention_bwd_flash16_supports(const AttnBwdParams &bp) {
     return tiles * p.H * p.B <= 2147483647LL;
 }
 
-// three float planes [B*H][Lq rounded up to 128]: row maximum (log2 units), 1 / row sum, delta
-size_t attention_bwd_flash16_workspace(const AttnParams &p) { return attention_stats_bytes(p); }
-
 // ---- dense masks packed into bits for the key-stationary kernels ----------------------------------------------
 // A dense mask without bias keeps the lean gradient kernels (raw scores, two wavefronts per SIMD).  The dQ kernel
 // stages the mask tiles through LDS as the forward kernel does; in the dK / dV kernels a lane owns one key and walks
@@ -47,7 +44,7 @@ static bool takes_mask_bits(const AttnParams &p) {
 static int64_t mask_bits_slices(const AttnParams &p) { return (p.mask_strides[2] ? p.H : 1) * (p.mask_strides[3] ? p.B : 1); }
 static int64_t mask_bits_lkv_pad(const AttnParams &p) { return (p.Lkv + 255) / 256 * 256; }
 
-size_t attention_bwd_flash16_mask_bits_bytes(const AttnParams &p) {
+static size_t mask_bits_bytes(const AttnParams &p) {
     if (!takes_mask_bits(p)) return 0;
     return sizeof(uint64_t) * (size_t)(mask_bits_slices(p) * ((p.Lq + 63) / 64) * mask_bits_lkv_pad(p));
 }
@@ -70,11 +67,10 @@ __global__ __launch_bounds__(256) void mask_bits_kernel(const uint8_t *mask, int
 
 // Key-padding masks: the (head, batch) pairs are classified on the device and the pairs whose mask is a context
 // length run the unmasked kernels on that many keys (workgroups past it only write zeros).
-size_t attention_bwd_flash16_lengths_bytes(const AttnBwdParams &bp) {
-    const AttnParams &p = bp.p;
+static size_t lengths_bytes(const AttnParams &p) {
     if (!flash_is_query_independent_mask(p) || p.H * p.B > 2147483647LL / 4) return 0;
     if (flash_is_key_mask(p) && p.Lkv <= 128) return 0;   // short sequences: less is saved than the classification costs
-    return ((size_t)(bp.p.H * bp.p.B) * sizeof(int32_t) + 15) & ~(size_t)15;
+    return ((size_t)(p.H * p.B) * sizeof(int32_t) + 15) & ~(size_t)15;
 }
 
 // ---- fused dropout: the keep decisions drawn once ---------------------------------------------------------------
@@ -85,17 +81,13 @@ size_t attention_bwd_flash16_lengths_bytes(const AttnBwdParams &bp) {
 // pairs of 333 x 333, head dim 64,
 // p = 0.1: 296 -> 114 us, with a key-padding mask 436 -> 114; 332 x 332: 123 -> 112; 64 pairs of 2048 x 2048, head dim
 // 128: 705 -> 659.)
-static bool takes_drop_words(const AttnBwdParams &bp) {
-    const AttnParams &p = bp.p;
+static bool takes_drop_words(const AttnParams &p, bool lengths) {
     if (p.drop_thresh == 0 || p.bias) return false;
-    return !p.mask || flash_is_key_mask(p) || attention_bwd_flash16_lengths_bytes(bp) != 0 || takes_mask_bits(p);   // what the lean kernels take
+    return !p.mask || flash_is_key_mask(p) || lengths || takes_mask_bits(p);   // what the lean kernels take
 }
 static int64_t pad128(int64_t n) { return (n + 127) / 128 * 128; }
 static size_t drop_rows_words(const AttnParams &p) { return (size_t)(p.H * p.B * ((p.Lkv + 63) / 64) * pad128(p.Lq)); }
 static size_t drop_keys_words(const AttnParams &p) { return (size_t)(p.H * p.B * ((p.Lq + 63) / 64) * pad128(p.Lkv)); }
-size_t attention_bwd_flash16_drop_bytes(const AttnBwdParams &bp) {
-    return takes_drop_words(bp) ? sizeof(uint64_t) * (drop_rows_words(bp.p) + drop_keys_words(bp.p)) : 0;
-}
 
 __global__ __launch_bounds__(256) void drop_words_kernel(AttnParams p, int64_t nkt, int64_t nqt, int64_t lq_pad, int64_t lkv_pad, int64_t blocks,
                                                          uint64_t *rows, uint64_t *keys) {
@@ -148,9 +140,6 @@ static bool takes_bias_blocks(const AttnBwdParams &bp) {
            pad128(p.Lq) / 128 * (pad128(p.Lkv) / 64) * p.H <= 2147483647LL / 16;
 }
 static size_t bias_copy_entries(const AttnParams &p) { return (size_t)(p.H * pad128(p.Lq) * pad128(p.Lkv)); }
-size_t attention_bwd_flash16_bias_bytes(const AttnBwdParams &bp) {
-    return takes_bias_blocks(bp) ? 2 * sizeof(uint16_t) * bias_copy_entries(bp.p) : 0;
-}
 
 // A wavefront copies 64 of the (query, key) rows of one form: grid.y 0 rows (a block of 32 keys per query, read four keys at
 // a time), 1 keys (a block of 32 queries per key, neighbouring lanes reading neighbouring keys).
@@ -227,22 +216,51 @@ __global__ __launch_bounds__(256) void dq_merge_kernel(const float *ws, typename
     *(typename T::vec4 *)(dq + i) = r;
 }
 
+// ---- the workspace -------------------------------------------------------------------------------------------------
+// [statistics][packed mask bits | context lengths][partial sums of dQ][keep words | bias copies].  The last part only saves
+// time, as the context lengths do for a mask that also runs without them: a call whose workspace has no room for it (a
+// gradient with saved statistics and dropout or a shared bias may be given none at all) runs without, see
+// DROP_REDRAW and launch_extras in attention_backward_flash16.inc.
+struct BwdScratch {
+    size_t stats = 0, bits = 0, lengths = 0, partial = 0, words = 0, bias = 0;   // bytes of each part, 0: not taken
+    size_t total() const { return stats + bits + lengths + partial + words + bias; }
+};
+static BwdScratch plan_scratch(const AttnBwdParams &bp, size_t room) {
+    const AttnParams &p = bp.p;
+    BwdScratch s;
+    s.stats = bp.have_stats ? 0 : attention_stats_bytes(p);
+    s.bits = mask_bits_bytes(p);
+    s.partial = attention_bwd_flash16_dq_partial_bytes(bp);
+    s.lengths = lengths_bytes(p);
+    const auto fits = [&](size_t more) { return s.total() <= room && more <= room - s.total(); };
+    if (p.drop_thresh && (p.Lkv & 3) != 0) {   // the one kind of call that does without lengths
+        const size_t n = s.lengths;
+        s.lengths = 0;
+        if (fits(n)) s.lengths = n;
+    }
+    if (takes_drop_words(p, s.lengths != 0)) {
+        const size_t n = sizeof(uint64_t) * (drop_rows_words(p) + drop_keys_words(p));
+        if (fits(n)) s.words = n;
+    }
+    if (takes_bias_blocks(bp)) {
+        const size_t n = 2 * sizeof(uint16_t) * bias_copy_entries(p);
+        if (fits(n)) s.bias = n;
+    }
+    return s;
+}
+size_t attention_bwd_flash16_workspace_needed(const AttnBwdParams &bp) { return plan_scratch(bp, 0).total(); }
+size_t attention_bwd_flash16_workspace_wanted(const AttnBwdParams &bp) { return plan_scratch(bp, SIZE_MAX).total(); }
+
 int32_t launch_attention_bwd_flash16(const AttnBwdParams &bp_in, hipStream_t st) {
     AttnBwdParams bp = bp_in;
     const AttnParams &p = bp.p;
+    const BwdScratch scratch = plan_scratch(bp, bp.workspace_bytes);
+    char *at = (char *)bp.workspace + scratch.stats;   // statistics that are not the caller's come first (validate_bwd)
     bp.dq_nsplit = attention_bwd_flash16_dq_nsplit(bp);
-    if (bp.dq_nsplit > 1)   // implies saved statistics: the workspace holds [packed mask bits][lengths][these partial sums]
-        bp.dq_partial = (float *)((char *)bp.workspace + attention_bwd_flash16_mask_bits_bytes(p) + attention_bwd_flash16_lengths_bytes(bp));
-    if (attention_bwd_flash16_lengths_bytes(bp) != 0) {   // after the statistics planes when those live in the workspace (no packed mask bits here)
-        int32_t *lens = (int32_t *)((char *)bp.workspace + (bp.have_stats ? 0 : attention_bwd_flash16_workspace(p)));
-        const int32_t rc = launch_key_mask_lengths(p, lens, st);
-        if (rc != MI_OK) return rc;
-        bp.kv_len = lens;
-    }
-    if (takes_mask_bits(p)) {
+    if (scratch.bits) {
         const int64_t nqt = (p.Lq + 63) / 64, pad = mask_bits_lkv_pad(p), slices = mask_bits_slices(p);
         if (nqt > 65535 || slices > 65535) return mi_set_error(MI_ESHAPE, "attention gradient: mask packing supports at most 65535 query tiles and mask planes");
-        uint64_t *bits = (uint64_t *)((char *)bp.workspace + (bp.have_stats ? 0 : attention_bwd_flash16_workspace(p)));
+        uint64_t *bits = (uint64_t *)at;
         const int64_t heads = p.mask_strides[2] ? p.H : 1;
         hipLaunchKernelGGL(mask_bits_kernel, dim3((unsigned)(pad / 256), (unsigned)nqt, (unsigned)slices), dim3(256), 0, st, p.mask,
                            p.mask_strides[0], p.mask_strides[1], p.mask_strides[2], p.mask_strides[3], p.Lq, p.Lkv, pad, heads, bits);
@@ -252,11 +270,20 @@ int32_t launch_attention_bwd_flash16(const AttnBwdParams &bp_in, hipStream_t st)
         bp.mb_b = p.mask_strides[3] ? heads : 0;
         bp.mb_lkv_pad = pad;
         bp.mb_nqt = nqt;
+        at += scratch.bits;
     }
-    if (takes_drop_words(bp)) {   // behind everything else in the workspace
-        const size_t before = (bp.have_stats ? 0 : attention_bwd_flash16_workspace(p)) + attention_bwd_flash16_mask_bits_bytes(p) +
-                              attention_bwd_flash16_lengths_bytes(bp) + attention_bwd_flash16_dq_partial_bytes(bp);
-        uint64_t *rows = (uint64_t *)((char *)bp.workspace + before), *keys = rows + drop_rows_words(p);
+    if (scratch.lengths) {
+        const int32_t rc = launch_key_mask_lengths(p, (int32_t *)at, st);
+        if (rc != MI_OK) return rc;
+        bp.kv_len = (int32_t *)at;
+        at += scratch.lengths;
+    }
+    if (scratch.partial) {
+        bp.dq_partial = (float *)at;
+        at += scratch.partial;
+    }
+    if (scratch.words) {
+        uint64_t *rows = (uint64_t *)at, *keys = rows + drop_rows_words(p);
         const int64_t nkt = (p.Lkv + 63) / 64, nqt = (p.Lq + 63) / 64, blocks = nkt * nqt * p.H * p.B;
         hipLaunchKernelGGL(drop_words_kernel, dim3((unsigned)((blocks + 3) / 4)), dim3(256), 0, st, p, nkt, nqt, pad128(p.Lq), pad128(p.Lkv), blocks,
                            rows, keys);
@@ -264,9 +291,9 @@ int32_t launch_attention_bwd_flash16(const AttnBwdParams &bp_in, hipStream_t st)
         bp.drop_rows = rows;
         bp.drop_keys = keys;
     }
-    if (takes_bias_blocks(bp)) {   // saved statistics, no mask, no dropout: behind the partial sums of dQ
+    if (scratch.bias) {
         const int64_t lq_pad = pad128(p.Lq), lkv_pad = pad128(p.Lkv), groups = (int64_t)bias_copy_entries(p) / 4096;   // four wavefronts each
-        uint16_t *rows = (uint16_t *)((char *)bp.workspace + attention_bwd_flash16_dq_partial_bytes(bp)), *keys = rows + bias_copy_entries(p);
+        uint16_t *rows = (uint16_t *)at, *keys = rows + bias_copy_entries(p);
         hipLaunchKernelGGL(bias_blocks_kernel, dim3((unsigned)(groups < 8192 ? groups : 8192), 2), dim3(256), 0, st, p, lq_pad, lkv_pad, rows, keys);
         MI_LAUNCH_CHECK();
         bp.bias_rows = rows;

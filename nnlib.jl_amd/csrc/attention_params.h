@@ -70,17 +70,20 @@ struct AttnBwdParams {
     float *stats;      // per (query, head, batch) softmax statistics: the workspace, or the buffer a forward call saved
     int32_t have_stats; // the forward call already filled the first two planes of `stats`
     void *workspace;
+    size_t workspace_bytes;
     // dense mask packed for the key-stationary gradient kernels: word [slice][query tile of 64][key] holds the mask
     // bits of the tile's queries for that key; slice = h * mb_h + b * mb_b (0 where the mask is shared)
     const uint64_t *mask_bits;
     int64_t mb_h, mb_b, mb_lkv_pad, mb_nqt;
     // fused dropout: the keep decisions of the call as 64-bit words, drawn once for all gradient kernels.  drop_rows holds
     // one word per (pair, tile of 64 keys, query), bit = key of the tile; drop_keys one per (pair, tile of 64 queries,
-    // key), bit = query of the tile.  [pair][tile][queries / keys rounded up to 128]; null without dropout
+    // key), bit = query of the tile.  [pair][tile][queries / keys rounded up to 128]; null without dropout, and where the
+    // workspace has no room for them (the kernels then redraw the decisions)
     const uint64_t *drop_rows, *drop_keys;
     // bias shared by the batch elements, copied in the order the gradient kernels' accumulators hold scores (zeros past the
     // ends, lengths rounded up to 128): bias_rows [h][block of 32 keys][query][hh][16], entry 4g + e = key 8g + 4hh + e of
-    // the block; bias_keys [h][block of 32 queries][key][hh][16], likewise with queries.  null where the call has none
+    // the block; bias_keys [h][block of 32 queries][key][hh][16], likewise with queries.  null where the call has none or
+    // the workspace no room for them
     const uint16_t *bias_rows, *bias_keys;
     // key-padding mask measured on the device: per (head, batch) pair [b * H + h] the context length, or 0 when the
     // mask of the pair is not a kept prefix; null when the call does not take that path
@@ -103,11 +106,9 @@ bool attention_bwd_flash16_supports(const AttnBwdParams &bp);
 int32_t launch_attention_bwd_flash32(const AttnBwdParams &bp, hipStream_t st);
 bool attention_bwd_flash32_supports(const AttnBwdParams &bp);
 size_t attention_bwd_flash32_lengths_bytes(const AttnBwdParams &bp);
-size_t attention_bwd_flash16_workspace(const AttnParams &p);
-size_t attention_bwd_flash16_mask_bits_bytes(const AttnParams &p);   // 0 when the call does not take the packed-mask path
-size_t attention_bwd_flash16_drop_bytes(const AttnBwdParams &bp);     // 0 when the call does not take the keep words
-size_t attention_bwd_flash16_bias_bytes(const AttnBwdParams &bp);     // 0 when the call does not take the bias copies
-size_t attention_bwd_flash16_lengths_bytes(const AttnBwdParams &bp);  // 0 when the call does not take the context-length path
+// what the 16-bit gradient cannot do without, and what it takes where it is given more
+size_t attention_bwd_flash16_workspace_needed(const AttnBwdParams &bp);
+size_t attention_bwd_flash16_workspace_wanted(const AttnBwdParams &bp);
 int attention_bwd_flash16_dq_nsplit(const AttnBwdParams &bp);         // pieces the dQ kernel's key range is cut into (1: no split)
 size_t attention_bwd_flash16_dq_partial_bytes(const AttnBwdParams &bp);   // the same rule serves the Float32 kernels
 // dq[i] = sum over the pieces of partial[piece][i], i < n (a multiple of 4), converted to `dtype`

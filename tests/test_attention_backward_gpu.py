@@ -672,3 +672,56 @@ def test_weights_of_the_dropout_gradient_keep_float32_accuracy(nn, oracle, Lkv):
     w = w / w.sum(axis=1, keepdims=True) * oracle.dropout_keep_mask((Lkv, L, H, B), p, seed).transpose(2, 0, 1, 3) * 2
     want = round_to(w.transpose(0, 2, 1, 3).reshape(D * H, Lkv, B), "bf16")
     assert np.mean(dv != want) <= 2e-4
+
+
+@pytest.mark.parametrize("kind,D,Lq,Lkv", [
+    ("dropout", 64, 130, 132),       # rows on hash groups: one hash per four weights, exchanged by the quads of lanes
+    ("dropout", 64, 131, 133),       # rows at any place within a group
+    ("dropout causal", 128, 200, 200),
+    ("dropout keys", 64, 150, 260),  # the context lengths find room in the workspace, the keep words do not
+    ("dropout keys", 64, 150, 261),  # neither does
+    ("dropout dense", 64, 100, 128),
+    ("bias", 64, 197, 197),
+    ("bias", 128, 64, 96),
+])
+def test_gradient_without_the_workspace_it_is_faster_with(nn, monkeypatch, kind, D, Lq, Lkv):
+    """Keep words and copies of a shared bias are there to save time: a caller with saved statistics that gives no workspace
+    for them (no more than the masks need) gets the same gradients.  The keep decisions are the same bits and the arithmetic
+    is the same, so with dropout they are equal; with a bias the kernels differ, and so do the roundings of P and dS to 16
+    bits (2^-9 relative each, two of them and the result's own: 2^-7 of the 2-norm)."""
+    rng = np.random.default_rng(Lq + Lkv)
+    H, B = 3, 3
+    D_ = nn.DeviceArray.from_numpy
+    q, dy = (D_(rng.standard_normal((H * D, Lq, B)).astype(np.float32), "bf16") for _ in range(2))
+    k, v = (D_(rng.standard_normal((H * D, Lkv, B)).astype(np.float32), "bf16") for _ in range(2))
+    bias = D_(rng.standard_normal((Lkv, Lq, H)).astype(np.float32), "bf16") if kind == "bias" else None
+    mask, needed = None, 0
+    if kind.endswith("causal"):
+        mask = nn.make_causal_mask(q)
+    elif kind.endswith("keys"):   # sequence 0: no prefix, 1: a prefix, 2: one key
+        keep = np.ones((Lkv, 1, 1, B), bool)
+        keep[Lkv // 2, 0, 0, 0] = keep[Lkv - 3:, 0, 0, 1] = keep[1:, 0, 0, 2] = False
+        mask, needed = nn.DeviceArray.from_numpy(keep, "bool"), 0 if Lkv % 4 else (4 * H * B + 15) // 16 * 16
+    elif kind.endswith("dense"):
+        mask, needed = nn.DeviceArray.from_numpy(rng.random((Lkv, Lq)) < 0.8, "bool"), 8 * ((Lq + 63) // 64) * ((Lkv + 255) // 256 * 256)
+    fdrop = nn.Dropout(0.3, 5) if kind.startswith("dropout") else nn.identity
+    y, _ = nn.dot_product_attention(q, k, v, bias, nheads=H, mask=mask, return_weights=False, fdrop=fdrop, save_for_backward=True)
+    assert y.saved_stats is not None
+
+    def grads():
+        return [g.to_numpy() for g in nn.dot_product_attention_grad(dy, q, k, v, bias, y=y, mask=mask, nheads=H, fdrop=fdrop) if g is not None]
+
+    want, asked, real = grads(), [], nn.ops._get_workspace
+
+    def least(n):
+        asked.append(n)
+        buf, _ = real(needed)
+        return buf, needed
+    monkeypatch.setattr(nn.ops, "_get_workspace", least)
+    got = grads()
+    assert len(asked) == 1 and asked[0] > needed and nn.ops.last_attention_bwd_kernel() == "flash16"
+    for g, w in zip(got, want):
+        if kind == "bias":
+            assert np.linalg.norm(g - w) <= 2.0 ** -7 * np.linalg.norm(w)
+        else:
+            assert np.array_equal(g, w)
