@@ -81,23 +81,28 @@ static size_t lengths_bytes(const AttnParams &p) {
 // pairs of 333 x 333, head dim 64,
 // p = 0.1: 296 -> 114 us, with a key-padding mask 436 -> 114; 332 x 332: 123 -> 112; 64 pairs of 2048 x 2048, head dim
 // 128: 705 -> 659.)
+// Two bits a weight are O(L^2) bytes where the rest of the call is O(L): the words of as many (head, batch) pairs as
+// DROP_WORDS_MOST bytes hold are drawn at a time, and the gradient kernels run on those pairs before the next are drawn.  A
+// pair whose own words are more than that (65536 x 65536 is 1 GiB) has them redrawn by the kernels.
 static bool takes_drop_words(const AttnParams &p, bool lengths) {
     if (p.drop_thresh == 0 || p.bias) return false;
     return !p.mask || flash_is_key_mask(p) || lengths || takes_mask_bits(p);   // what the lean kernels take
 }
 static int64_t pad128(int64_t n) { return (n + 127) / 128 * 128; }
-static size_t drop_rows_words(const AttnParams &p) { return (size_t)(p.H * p.B * ((p.Lkv + 63) / 64) * pad128(p.Lq)); }
-static size_t drop_keys_words(const AttnParams &p) { return (size_t)(p.H * p.B * ((p.Lq + 63) / 64) * pad128(p.Lkv)); }
+constexpr size_t DROP_WORDS_MOST = (size_t)1 << 30;
+// per pair
+static size_t drop_rows_words(const AttnParams &p) { return (size_t)((p.Lkv + 63) / 64 * pad128(p.Lq)); }
+static size_t drop_keys_words(const AttnParams &p) { return (size_t)((p.Lq + 63) / 64 * pad128(p.Lkv)); }
 
-__global__ __launch_bounds__(256) void drop_words_kernel(AttnParams p, int64_t nkt, int64_t nqt, int64_t lq_pad, int64_t lkv_pad, int64_t blocks,
-                                                         uint64_t *rows, uint64_t *keys) {
+__global__ __launch_bounds__(256) void drop_words_kernel(AttnParams p, int64_t pair0, int64_t nkt, int64_t nqt, int64_t lq_pad, int64_t lkv_pad,
+                                                         int64_t blocks, uint64_t *rows, uint64_t *keys) {
     const int64_t id = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);   // wave-uniform
     if (id >= blocks) return;
     const int lane = threadIdx.x & 63;
-    const int64_t kt = id % nkt, qt = id / nkt % nqt, pair = id / (nkt * nqt);   // pair = b * H + h
+    const int64_t kt = id % nkt, qt = id / nkt % nqt, pair = id / (nkt * nqt);   // of this piece: b * H + h - pair0
     if (p.causal && 64 * kt > 64 * qt + 63) return;   // no kernel visits a tile above the diagonal
     const int64_t qi = 64 * qt + lane;
-    const uint64_t first = (uint64_t)(p.Lkv * (qi + p.Lq * pair) + 64 * kt);   // linear index of the row's first weight
+    const uint64_t first = (uint64_t)(p.Lkv * (qi + p.Lq * (pair0 + pair)) + 64 * kt);   // linear index of the row's first weight
     const int off = (int)(first & 3);
     uint64_t word = 0, z = p.drop_key + (first >> 2) * 0x9E3779B97F4A7C15ull;
     const auto group = [&](int shift) {   // the next group's four decisions from bit `shift` on
@@ -223,6 +228,7 @@ __global__ __launch_bounds__(256) void dq_merge_kernel(const float *ws, typename
 // DROP_REDRAW and launch_extras in attention_backward_flash16.inc.
 struct BwdScratch {
     size_t stats = 0, bits = 0, lengths = 0, partial = 0, words = 0, bias = 0;   // bytes of each part, 0: not taken
+    int64_t word_pairs = 0;                                                      // pairs that `words` holds
     size_t total() const { return stats + bits + lengths + partial + words + bias; }
 };
 static BwdScratch plan_scratch(const AttnBwdParams &bp, size_t room) {
@@ -239,8 +245,10 @@ static BwdScratch plan_scratch(const AttnBwdParams &bp, size_t room) {
         if (fits(n)) s.lengths = n;
     }
     if (takes_drop_words(p, s.lengths != 0)) {
-        const size_t n = sizeof(uint64_t) * (drop_rows_words(p) + drop_keys_words(p));
-        if (fits(n)) s.words = n;
+        const size_t pair = sizeof(uint64_t) * (drop_rows_words(p) + drop_keys_words(p)), left = s.total() < room ? room - s.total() : 0;
+        const size_t pairs = (left < DROP_WORDS_MOST ? left : DROP_WORDS_MOST) / pair;
+        s.word_pairs = pairs < (size_t)(p.H * p.B) ? (int64_t)pairs : p.H * p.B;
+        s.words = pair * (size_t)s.word_pairs;
     }
     if (takes_bias_blocks(bp)) {
         const size_t n = 2 * sizeof(uint16_t) * bias_copy_entries(p);
@@ -282,15 +290,6 @@ int32_t launch_attention_bwd_flash16(const AttnBwdParams &bp_in, hipStream_t st)
         bp.dq_partial = (float *)at;
         at += scratch.partial;
     }
-    if (scratch.words) {
-        uint64_t *rows = (uint64_t *)at, *keys = rows + drop_rows_words(p);
-        const int64_t nkt = (p.Lkv + 63) / 64, nqt = (p.Lq + 63) / 64, blocks = nkt * nqt * p.H * p.B;
-        hipLaunchKernelGGL(drop_words_kernel, dim3((unsigned)((blocks + 3) / 4)), dim3(256), 0, st, p, nkt, nqt, pad128(p.Lq), pad128(p.Lkv), blocks,
-                           rows, keys);
-        MI_LAUNCH_CHECK();
-        bp.drop_rows = rows;
-        bp.drop_keys = keys;
-    }
     if (scratch.bias) {
         const int64_t lq_pad = pad128(p.Lq), lkv_pad = pad128(p.Lkv), groups = (int64_t)bias_copy_entries(p) / 4096;   // four wavefronts each
         uint16_t *rows = (uint16_t *)at, *keys = rows + bias_copy_entries(p);
@@ -299,12 +298,27 @@ int32_t launch_attention_bwd_flash16(const AttnBwdParams &bp_in, hipStream_t st)
         bp.bias_rows = rows;
         bp.bias_keys = keys;
     }
-    int32_t rc;
-    if (p.dtype == MI_BF16)
-        rc = p.D <= 64 ? launch_bwd_flash16_bf16_d64(bp, st) : p.D <= 128 ? launch_bwd_flash16_bf16_d128(bp, st) : launch_bwd_flash16_bf16_d256(bp, st);
-    else
-        rc = p.D <= 64 ? launch_bwd_flash16_f16_d64(bp, st) : p.D <= 128 ? launch_bwd_flash16_f16_d128(bp, st) : launch_bwd_flash16_f16_d256(bp, st);
-    if (rc != MI_OK || bp.dq_nsplit <= 1) return rc;
+    const int64_t pairs = p.H * p.B, step = scratch.words ? scratch.word_pairs : pairs;
+    for (int64_t pair0 = 0; pair0 < pairs; pair0 += step) {   // one piece, unless the keep words of all pairs do not fit
+        bp.pair0 = (int32_t)pair0;
+        bp.npairs = (int32_t)(pairs - pair0 < step ? pairs - pair0 : step);
+        if (scratch.words) {
+            uint64_t *rows = (uint64_t *)at, *keys = rows + drop_rows_words(p) * (size_t)step;
+            const int64_t nkt = (p.Lkv + 63) / 64, nqt = (p.Lq + 63) / 64, blocks = nkt * nqt * bp.npairs;   // at most 2^20 (DROP_WORDS_MOST)
+            hipLaunchKernelGGL(drop_words_kernel, dim3((unsigned)((blocks + 3) / 4)), dim3(256), 0, st, p, pair0, nkt, nqt, pad128(p.Lq),
+                               pad128(p.Lkv), blocks, rows, keys);
+            MI_LAUNCH_CHECK();
+            bp.drop_rows = rows;
+            bp.drop_keys = keys;
+        }
+        int32_t rc;
+        if (p.dtype == MI_BF16)
+            rc = p.D <= 64 ? launch_bwd_flash16_bf16_d64(bp, st) : p.D <= 128 ? launch_bwd_flash16_bf16_d128(bp, st) : launch_bwd_flash16_bf16_d256(bp, st);
+        else
+            rc = p.D <= 64 ? launch_bwd_flash16_f16_d64(bp, st) : p.D <= 128 ? launch_bwd_flash16_f16_d128(bp, st) : launch_bwd_flash16_f16_d256(bp, st);
+        if (rc != MI_OK) return rc;
+    }
+    if (bp.dq_nsplit <= 1) return MI_OK;
     return launch_dq_merge(p.dtype, bp.dq_partial, bp.dq, bp.dq_nsplit, p.B * p.Lq * p.E, st);
 }
 

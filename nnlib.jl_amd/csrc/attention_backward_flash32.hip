@@ -119,11 +119,11 @@ __global__ __launch_bounds__(256, (D == 64 && EXTRAS == EXTRAS_NONE) ? 2 : 1) vo
     extern __shared__ __attribute__((aligned(16))) unsigned char bwd_smem[];
     float *Ks = (float *)bwd_smem, *Vs = Ks + 2 * TILEF;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, hh = lane >> 5;
-    const int64_t HB = p.H * a.nb;   // this launch's batch elements: [a.b0, a.b0 + a.nb)
+    const int64_t HB = a.npairs;   // this launch's (head, batch) pairs: [a.pair0, a.pair0 + a.npairs)
     const int split = (int)(blockIdx.x % a.nsplit);   // piece of the key range (a.nsplit > 1: calls with saved statistics only)
     const int64_t bid = blockIdx.x / a.nsplit;
     const int64_t hb = bid % HB, qt = a.n_qtiles - 1 - bid / HB;
-    const int64_t h = hb % p.H, b = a.b0 + hb / p.H;
+    const int64_t h = (a.pair0 + hb) % p.H, b = (a.pair0 + hb) / p.H;
     const int64_t i0 = qt * 128, iw = i0 + 32 * wave, qi = iw + r;
     const bool qok = qi < p.Lq;
 
@@ -678,11 +678,11 @@ __global__ __launch_bounds__(64 * NW, 1) void bwd32s_dq_kernel(FlashArgs a, Attn
     extern __shared__ __attribute__((aligned(16))) unsigned char bwd_smem[];
     const unsigned Ks = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)bwd_smem, Vs = Ks + C::TILEB;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, hh = lane >> 5;
-    const int64_t HB = p.H * a.nb;
+    const int64_t HB = a.npairs;
     const int split = (int)(blockIdx.x % a.nsplit);   // piece of the key range (a.nsplit > 1: calls with saved statistics only)
     const int64_t bid = blockIdx.x / a.nsplit;
     const int64_t hb = bid % HB, qt = a.n_qtiles - 1 - bid / HB;
-    const int64_t h = hb % p.H, b = a.b0 + hb / p.H;
+    const int64_t h = (a.pair0 + hb) % p.H, b = (a.pair0 + hb) / p.H;
     const int64_t i0 = qt * (32 * NW), iw = i0 + 32 * wave, qi = iw + r;
     const bool qok = qi < p.Lq;
 
@@ -1447,9 +1447,9 @@ int32_t launch_set(const FlashArgs &a, const AttnBwdParams &bp, hipStream_t st) 
     const bool per_batch = own_rows && p.bias_strides[3] == 0 && p.B > 1;
     if (own_rows && (!per_batch || (int64_t)a.n_qtiles * p.H >= 256)) a1.dbias_plain = 1;
     if (a1.dbias_plain && per_batch) {
-        a1.nb = 1;
+        a1.npairs = (int32_t)p.H;
         for (int64_t b = 0; b < p.B; b++) {
-            a1.b0 = (int32_t)b;
+            a1.pair0 = (int32_t)(b * p.H);
             hipLaunchKernelGGL(k1, dim3((unsigned)((int64_t)a.n_qtiles * p.H * a1.nsplit)), dim3(256), SMEM_Q, st, a1, bp);
         }
     } else {
@@ -1562,8 +1562,8 @@ int32_t launch_attention_bwd_flash32(const AttnBwdParams &bp_in, hipStream_t st)
     a.n_qtiles = (int32_t)((bp.p.Lq + 127) / 128);
     a.nsplit = 1;
     a.tiles_per_split = 0;
-    a.b0 = 0;
-    a.nb = (int32_t)bp.p.B;
+    a.pair0 = 0;
+    a.npairs = (int32_t)(bp.p.H * bp.p.B);
     a.dbias_plain = 0;
     flash_fill_vec_flags(a);
     a.bias_lds = a.mask_lds = 0;

@@ -77,9 +77,11 @@ struct AttnBwdParams {
     int64_t mb_h, mb_b, mb_lkv_pad, mb_nqt;
     // fused dropout: the keep decisions of the call as 64-bit words, drawn once for all gradient kernels.  drop_rows holds
     // one word per (pair, tile of 64 keys, query), bit = key of the tile; drop_keys one per (pair, tile of 64 queries,
-    // key), bit = query of the tile.  [pair][tile][queries / keys rounded up to 128]; null without dropout, and where the
-    // workspace has no room for them (the kernels then redraw the decisions)
+    // key), bit = query of the tile.  [pair of the launch][tile][queries / keys rounded up to 128]; null without dropout, and
+    // where the workspace has no room for them (the kernels then redraw the decisions)
     const uint64_t *drop_rows, *drop_keys;
+    // the (head, batch) pairs of the launch, [pair0, pair0 + npairs): all, or a piece whose keep words fit the workspace
+    int32_t pair0, npairs;
     // bias shared by the batch elements, copied in the order the gradient kernels' accumulators hold scores (zeros past the
     // ends, lengths rounded up to 128): bias_rows [h][block of 32 keys][query][hh][16], entry 4g + e = key 8g + 4hh + e of
     // the block; bias_keys [h][block of 32 queries][key][hh][16], likewise with queries.  null where the call has none or

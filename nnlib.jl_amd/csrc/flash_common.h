@@ -23,9 +23,9 @@ struct FlashArgs {
     int32_t bias_lds;  // 16-bit kernels: bias / mask tiles may be staged through LDS with 16-byte DMA pieces
     int32_t mask_lds;
     int32_t w_lds;     // weight rows start 16-byte aligned: tiles may be transposed through LDS and written as full lines
-    // gradient kernels only: the launch covers batch elements [b0, b0 + nb), and the bias gradient may be summed
-    // without atomics (no two workgroups of one launch add to the same element)
-    int32_t b0, nb, dbias_plain;
+    // gradient kernels only: the launch covers the (head, batch) pairs [pair0, pair0 + npairs), pair = b * H + h, and the
+    // bias gradient may be summed without atomics (no two workgroups of one launch add to the same element)
+    int32_t pair0, npairs, dbias_plain;
     // gradient kernels: the mask is a key-padding mask that the key-stationary kernels apply to a lane's own key
     int32_t key_mask = 0;
     // forward kernels, key-padding masks that are context lengths: per (head, batch) pair [b * H + h] the number of

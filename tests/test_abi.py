@@ -120,6 +120,29 @@ def test_plan_workspace_for_key_padding_masks(L):
         assert ws.value == stats_bytes + lens_bytes, (dt, ws.value)   # statistics planes (none saved here), then the lengths
 
 
+def test_plan_workspace_of_dropout_gradients_is_bounded(L):
+    """The keep decisions drawn once take two bits a weight: for all (head, batch) pairs while that is at most 1 GiB, for as
+    many pairs at a time as 1 GiB holds beyond, and none where one pair needs more."""
+    def words(Lq, Lkv, B, D=64, H=8):
+        d = _desc(L, dtype=L.MI_BF16, weights_dtype=L.MI_BF16, E=D * H, Ev=D * H, H=H, Lq=Lq, Lkv=Lkv, B=B, dropout_p=0.1, dropout_seed=1)
+        d.stats = 0x4000
+        b = L.mi_attn_bwd_desc()
+        b.struct_size = ctypes.sizeof(L.mi_attn_bwd_desc)
+        b.fwd = d
+        b.dout = b.dq = b.dk = b.dv = 0x3000
+        kern, ws = ctypes.c_int32(-1), ctypes.c_size_t(0)
+        assert L.load().mi_attention_bwd_plan(ctypes.byref(b), ctypes.byref(kern), ctypes.byref(ws)) == L.MI_OK
+        assert L.KERNEL_NAMES[kern.value] == "flash16"
+        return ws.value
+
+    assert words(1024, 1024, 2) == 16 * 1024 * 1024 // 4
+    assert words(333, 333, 24) == 8 * 24 * 2 * 6 * 384 * 8
+    assert words(16384, 16384, 8) == 1 << 30                       # 16 of the 64 pairs
+    assert words(20000, 20000, 8) == 10 * 8 * 2 * 313 * 20096      # 10 pairs of 100.7 MB
+    assert words(65536, 65536, 1) == 1 << 30
+    assert words(65537, 65537, 1) == 0 and words(131072, 131072, 4) == 0
+
+
 def test_host_side_argument_checks_of_other_entry_points(L):
     lib = L.load()
     assert lib.mi_softmax_dim1(9, None, None, 4, 4, None) == L.MI_EDTYPE

@@ -725,3 +725,44 @@ def test_gradient_without_the_workspace_it_is_faster_with(nn, monkeypatch, kind,
             assert np.linalg.norm(g - w) <= 2.0 ** -7 * np.linalg.norm(w)
         else:
             assert np.array_equal(g, w)
+
+
+@pytest.mark.parametrize("pairs", [1, 2, 4])
+@pytest.mark.parametrize("mask_kind,Lq,Lkv", [(None, 130, 133), ("causal", 191, 191), ("lengths", 70, 261), ("random", 100, 128)])
+def test_dropout_gradient_in_pieces_of_its_pairs(nn, monkeypatch, mask_kind, Lq, Lkv, pairs):
+    """A workspace that holds the keep words of some (head, batch) pairs at a time: the pieces give the bits that all pairs
+    at once give."""
+    rng = np.random.default_rng(Lq + pairs)
+    H, B, D = 3, 3, 64
+    D_ = nn.DeviceArray.from_numpy
+    q, dy = (D_(rng.standard_normal((H * D, Lq, B)).astype(np.float32), "f16") for _ in range(2))
+    k, v = (D_(rng.standard_normal((H * D, Lkv, B)).astype(np.float32), "f16") for _ in range(2))
+    mask = None
+    if mask_kind == "causal":
+        mask = nn.make_causal_mask(q)
+    elif mask_kind == "lengths":
+        keep = rng.random((Lkv, 1, 1, B)) < 0.7
+        keep[0] = True
+        keep[:, 0, 0, 1] = np.arange(Lkv) < 100
+        mask = D_(keep, "bool")
+    elif mask_kind == "random":
+        keep = rng.random((Lkv, Lq)) < 0.8
+        keep[0] = True
+        mask = D_(keep, "bool")
+    fdrop = nn.Dropout(0.2, 9)
+    y, _ = nn.dot_product_attention(q, k, v, nheads=H, mask=mask, return_weights=False, fdrop=fdrop, save_for_backward=True)
+
+    def grads():
+        return [g.to_numpy() for g in nn.dot_product_attention_grad(dy, q, k, v, y=y, mask=mask, nheads=H, fdrop=fdrop) if g is not None]
+
+    want, real = grads(), nn.ops._get_workspace
+    pad = lambda n: (n + 127) // 128 * 128
+    words = 8 * ((Lkv + 63) // 64 * pad(Lq) + (Lq + 63) // 64 * pad(Lkv))
+
+    def less(n):
+        m = n - (H * B - pairs) * words
+        assert m > 0
+        return real(m)
+    monkeypatch.setattr(nn.ops, "_get_workspace", less)
+    assert all(np.array_equal(g, w) for g, w in zip(grads(), want))
+    assert nn.ops._workspace.numel() >= pairs * words
