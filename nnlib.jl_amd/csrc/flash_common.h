@@ -26,8 +26,6 @@ struct FlashArgs {
     // gradient kernels only: the launch covers the (head, batch) pairs [pair0, pair0 + npairs), pair = b * H + h, and the
     // bias gradient may be summed without atomics (no two workgroups of one launch add to the same element)
     int32_t pair0, npairs, dbias_plain;
-    // gradient kernels: the mask is a key-padding mask that the key-stationary kernels apply to a lane's own key
-    int32_t key_mask = 0;
     // forward kernels, key-padding masks that are context lengths: per (head, batch) pair [b * H + h] the number of
     // leading keys kept when the mask keeps exactly a prefix (the software-pipelined kernel then treats it as that
     // pair's L_kv and the general kernel leaves the pair alone), 0 otherwise (the general kernel applies the mask)

@@ -766,3 +766,52 @@ def test_dropout_gradient_in_pieces_of_its_pairs(nn, monkeypatch, mask_kind, Lq,
     monkeypatch.setattr(nn.ops, "_get_workspace", less)
     assert all(np.array_equal(g, w) for g, w in zip(grads(), want))
     assert nn.ops._workspace.numel() >= pairs * words
+
+
+@pytest.mark.parametrize("dtype,D,Lq,Lkv,causal,p,nan_query", [
+    ("bf16", 64, 100, 72, False, 0.0, False),      # up to 128 keys: no context lengths
+    ("f16", 64, 130, 133, False, 0.0, False),
+    ("bf16", 128, 70, 260, False, 0.0, True),
+    ("bf16", 128, 200, 200, True, 0.0, False),
+    ("bf16", 136, 70, 73, False, 0.0, False),      # 256-wide tiles
+    ("bf16", 64, 100, 72, False, 0.2, False),
+    ("f16", 64, 130, 133, False, 0.2, True),
+    ("bf16", 136, 70, 73, False, 0.2, False),
+    ("bf16", 64, 133, 133, True, 0.2, False),
+])
+def test_every_key_of_a_sequence_dropped(nn, dtype, D, Lq, Lkv, causal, p, nan_query):
+    """Key-padding masks: where no key of a sequence is kept, every weight is NaN (src/softmax.jl:73-75), those of the dropped
+    keys among them, and so is the gradient of each query, key and value of the sequence.  Elsewhere a dropped key's
+    gradients are exact zeros whatever its rows hold, and a query that is NaN reaches the key gradients of its own
+    sequence only: those of the dropped keys too."""
+    rng = np.random.default_rng(D + Lkv)
+    H, B = 2, 3
+    D_ = nn.DeviceArray.from_numpy
+    q, dy = (rng.standard_normal((H * D, Lq, B)).astype(np.float32) for _ in range(2))
+    k, v = (rng.standard_normal((H * D, Lkv, B)).astype(np.float32) for _ in range(2))
+    keep = np.ones((Lkv, 1, 1, B), bool)
+    gone = np.arange(3, Lkv, 5)
+    keep[gone, 0, 0, 0] = False
+    keep[:, 0, 0, 1] = False
+    k[:, gone, 0], v[:, gone, 0] = 2e4, -2e4          # scores that would overflow the exponential
+    if nan_query:
+        q[:, 5, 2] = np.nan
+        keep[gone, 0, 0, 2] = False
+    dq_, dk_, dv_, ddy = D_(q, dtype), D_(k, dtype), D_(v, dtype), D_(dy, dtype)
+    mask = D_(keep, "bool")
+    if causal:
+        mask = nn.make_causal_mask(dq_) & mask
+    fdrop = nn.Dropout(p, 3) if p else nn.identity
+    y, _ = nn.dot_product_attention(dq_, dk_, dv_, nheads=H, mask=mask, return_weights=False, fdrop=fdrop, save_for_backward=True)
+    grads = nn.dot_product_attention_grad(ddy, dq_, dk_, dv_, y=y, mask=mask, nheads=H, fdrop=fdrop)[:3]
+    assert nn.last_attention_bwd_kernel() == "flash16"
+    dq, dk, dv = (g.to_numpy() for g in grads)
+    assert np.isnan(dq[:, :, 1]).all() and np.isnan(dk[:, :, 1]).all() and np.isnan(dv[:, :, 1]).all()
+    for g in (dq, dk, dv):
+        assert np.isfinite(g[:, :, 0]).all()
+    assert not dk[:, gone, 0].any() and not dv[:, gone, 0].any()
+    assert np.abs(dk[:, ~np.isin(np.arange(Lkv), gone), 0]).max() > 0
+    if nan_query:
+        assert np.isnan(dk[:, :, 2]).all() and np.isnan(dv[:, :, 2]).all() and np.isnan(dq[:, 5, 2]).all()
+    else:
+        assert np.isfinite(dk[:, :, 2]).all() and np.isfinite(dv[:, :, 2]).all() and np.isfinite(dq[:, :, 2]).all()
