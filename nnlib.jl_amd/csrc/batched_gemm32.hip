@@ -176,6 +176,10 @@ __device__ inline int rmaj_swz(int kk) { return ((kk & 3) << 2) | ((kk >> 2) & 3
 // elements, which only enter rows of C that are not stored; past k (not RM) the next row's, which `trim` zeroes.  A piece
 // that would end past the slice is moved back to end with it and shifted into place by `trim`.  Both happen in the last
 // stage only.
+// Planes do not hold values beyond bf16's largest (an Inf among them: Inf times Inf would be NaN) and lose the low bits of
+// values whose last plane leaves bf16's range (below 2^-110).  ANY products keep what the Float32 instruction gives there:
+// `store` notes the extremes of the tile's operands, and the kernel computes a tile that has such values again on that
+// instruction.  (A NaN is a NaN in the first plane already.)
 template <bool RM, bool LARGE, bool ANY>
 struct OperandS {
     typedef ShapeS<LARGE> S;
@@ -185,6 +189,10 @@ struct OperandS {
     int64_t ld, rows, k, row0;
     __amdgpu_buffer_rsrc_t rsrc;   // ANY
     int bytes;                     // ANY: of the slice
+    float most = 0.0f;             // ANY: largest |x| so far (NaNs do not count)
+    uint32_t least = ~0u;          // ANY: smallest 2 |x| - 1 so far, in bits (a zero counts as the largest)
+    __device__ bool fit() const { return most <= 0x1.fep127f && least >= (27u << 24) - 1; }   // bf16's largest; 2^-100
+    static constexpr int LDR = S::TILE + 4;             // floats per k-row of a tile kept as it is
     floatx4_t reg[2];   // TILE * KC / 4 pieces per tile: 2 per thread in either shape
 
     __device__ void init(const float *X_, int64_t ld_, int64_t rows_, int64_t k_, int64_t row0_) {
@@ -237,7 +245,7 @@ struct OperandS {
         }
     }
     // split into planes; `tile` is the LDS byte address of the hi plane
-    __device__ void store(unsigned tile) const {
+    __device__ void store(unsigned tile) {
         typedef __attribute__((address_space(3))) u32x2_t *lds8_t;
         const int tid = threadIdx.x;
 #pragma unroll
@@ -247,7 +255,15 @@ struct OperandS {
             uint32_t pl[3][2];
             split3_pair(x[0], x[1], pl[0][0], pl[1][0], pl[2][0]);
             split3_pair(x[2], x[3], pl[0][1], pl[1][1], pl[2][1]);
-            if (mi_plane_word_special(pl[0][0]) || mi_plane_word_special(pl[0][1])) {   // an Inf, a NaN or a value beyond the bf16 range among the four (rare)
+            if constexpr (ANY) {
+                const u32x4_t bits = __builtin_bit_cast(u32x4_t, x);
+#pragma unroll
+                for (int e = 0; e < 4; e += 2) {
+                    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(most) : "v"(x[e]), "v"(x[e + 1]));
+                    const uint32_t s0 = (bits[e] << 1) - 1, s1 = (bits[e + 1] << 1) - 1;
+                    least = min(min(s0, s1), least);
+                }
+            } else if (mi_plane_word_special(pl[0][0]) || mi_plane_word_special(pl[0][1])) {   // an Inf, a NaN or a value beyond the bf16 range among the four (rare)
                 split3_pair_wide(x[0], x[1], pl[0][0], pl[1][0], pl[2][0]);
                 split3_pair_wide(x[2], x[3], pl[0][1], pl[1][1], pl[2][1]);
             }
@@ -261,6 +277,21 @@ struct OperandS {
             }
 #pragma unroll
             for (int q = 0; q < 3; q++) *(lds8_t)(uintptr_t)(tile + at + q * PLANEB) = (u32x2_t){pl[q][0], pl[q][1]};
+        }
+    }
+    // ANY: the stage as it is, [16 k][TILE rows + 4], for the Float32 instruction
+    __device__ void store_whole(unsigned tile) const {
+        typedef __attribute__((address_space(3))) float *ldsf_t;
+        typedef __attribute__((address_space(3))) floatx4_t *ldsf4_t;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int c = threadIdx.x + S::THREADS * u;
+            if (RM) {
+                *(ldsf4_t)(uintptr_t)(tile + (unsigned)(((c / CPR) * LDR + (c % CPR) * 4) * 4)) = reg[u];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++) *(ldsf_t)(uintptr_t)(tile + (unsigned)((((c & 3) * 4 + e) * LDR + (c >> 2)) * 4)) = reg[u][e];
+            }
         }
     }
     // the three planes of the MFMA operand of the 32-row block `blk`
@@ -305,6 +336,9 @@ __global__ __launch_bounds__(ShapeS<LARGE>::THREADS, LARGE ? 1 : 2) void gemm32s
     a.init(g.A + bz * g.sA, g.lda, g.m, g.k, tile.m * S::TILE);
     b.init(g.B + bz * g.sB, g.ldb, g.n, g.k, tile.n * S::TILE);
 
+    typedef __attribute__((address_space(3))) uint32_t *lds_word_t;
+    const lds_word_t unfit = (lds_word_t)(uintptr_t)(lds0 + 4 * TILE3B);   // ANY: the planes do not hold the tile's operands
+    if (ANY && threadIdx.x == 0) *unfit = 0;
     floatx16_t acc[BNB][BM];   // [n block][m block]
 #pragma unroll
     for (int i = 0; i < BNB; i++)
@@ -347,8 +381,40 @@ __global__ __launch_bounds__(ShapeS<LARGE>::THREADS, LARGE ? 1 : 2) void gemm32s
             b.trim((int64_t)(it + 1) * KC);
             a.store(lds0 + (buf ^ 1) * TILE3B);
             b.store(lds0 + (2 + (buf ^ 1)) * TILE3B);
+        } else if (ANY && !(a.fit() && b.fit())) {
+            *unfit = 1;
         }
         __syncthreads();
+    }
+    if (ANY && *unfit) {   // the same word for the whole workgroup
+#pragma unroll
+        for (int i = 0; i < BNB; i++)
+#pragma unroll
+            for (int j = 0; j < BM; j++) acc[i][j] = (floatx16_t){0};
+        typedef __attribute__((address_space(3))) const float *ldsf_t;
+        for (int it = 0; it < nk; it++) {
+            a.load((int64_t)it * KC);
+            b.load((int64_t)it * KC);
+            a.trim((int64_t)it * KC);
+            b.trim((int64_t)it * KC);
+            a.store_whole(lds0);
+            b.store_whole(lds0 + 2 * TILE3B);
+            __syncthreads();
+#pragma unroll
+            for (int ks = 0; ks < KC / 2; ks++) {
+                float av[BM], bv[BNB];
+                const unsigned row = (unsigned)((2 * ks + hh) * a.LDR + r);
+#pragma unroll
+                for (int j = 0; j < BM; j++) av[j] = *(ldsf_t)(uintptr_t)(lds0 + (row + 32 * (BM * wm + j)) * 4);
+#pragma unroll
+                for (int i = 0; i < BNB; i++) bv[i] = *(ldsf_t)(uintptr_t)(lds0 + 2 * TILE3B + (row + 32 * (BNB * wn + i)) * 4);
+#pragma unroll
+                for (int i = 0; i < BNB; i++)
+#pragma unroll
+                    for (int j = 0; j < BM; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[i], av[j], acc[i][j], 0, 0, 0);
+            }
+            __syncthreads();
+        }
     }
 
     // accumulator register v of lane (r, hh) of block (i, j): n = 32i + 8*(v/4) + 4*hh + v%4, m = 32j + r
@@ -411,7 +477,7 @@ template <bool A_RM, bool B_RM, bool LARGE, bool ANY>
 int32_t launch_planes(const Gemm32Args &g, int64_t nb, hipStream_t st) {
     typedef ShapeS<LARGE> S;
     auto kern = gemm32s_kernel<A_RM, B_RM, LARGE, ANY>;
-    constexpr size_t smem = 4 * S::TILE3B;
+    constexpr size_t smem = 4 * S::TILE3B + (ANY ? 16 : 0);
     static bool attr_set = false;  // per instantiation; the attribute is idempotent, so a race is harmless
     if (!attr_set) {
         MI_HIP_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));

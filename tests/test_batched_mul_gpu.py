@@ -451,3 +451,54 @@ def test_operands_of_any_alignment(nn, dtype, ta, tb, m, n, k, batch):
     got = after[1:].reshape(batch, n, m + 1)
     assert np.abs(got[:, :, :m].transpose(0, 2, 1) - ref).max() <= TOL[dtype] * np.abs(ref).max()
     assert np.array_equal(got[:, :, m], before[1:].reshape(batch, n, m + 1)[:, :, m]) and after[0] == before[0]
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("m,n,k,batch", [(131, 129, 77, 3), (67, 190, 5, 2), (511, 509, 131, 64)])
+def test_unaligned_float32_products_at_the_ends_of_the_range(nn, ta, tb, m, n, k, batch):
+    """Float32 products of sizes that are no multiple of 16 bytes, where three bf16 planes do not hold the operands: values
+    whose low planes leave bf16's range, alone and next to ordinary ones, and Inf times Inf.  Sums of k Float32 products err
+    by a few 2^-24 sqrt(k) of sum |a||b|, whatever the scale (128 x 128 tiles, and 256 x 256 at 511 x 509 x 64)."""
+    rng = np.random.default_rng(m + 2 * ta + tb)
+    A, B = np.abs(rng.standard_normal((batch, m, k))) + 0.1, np.abs(rng.standard_normal((batch, k, n))) + 0.1
+
+    def run(a, b):
+        dev = lambda x, t: nn.DeviceArray.from_numpy(np.ascontiguousarray(x.transpose(2, 1, 0) if t else x.transpose(1, 2, 0)), "f32")
+        da, db = dev(a, ta), dev(b, tb)
+        C = nn.batched_mul(nn.batched_transpose(da) if ta else da, nn.batched_transpose(db) if tb else db)
+        return C.to_numpy().transpose(2, 0, 1)
+
+    def check(a, b):
+        a, b = a.astype(np.float32), b.astype(np.float32)
+        ref = a.astype(np.float64) @ b.astype(np.float64)   # all terms positive: also sum |a||b|
+        assert (np.abs(run(a, b) - ref) / ref).max() < 4 * 2.0 ** -24 * np.sqrt(k)
+
+    for ea, eb in ((-116, 0), (0, -120), (-122, 100), (-60, -60)):
+        check(np.ldexp(A, ea), np.ldexp(B, eb))
+    mixed = A.copy()
+    mixed[-1, 5] = np.ldexp(mixed[-1, 5], -118)      # one row of one tile
+    check(mixed, B)
+    zeros = A.copy()
+    zeros[:, ::2] = 0.0
+    zeros[:, ::2, 0] = np.ldexp(1.0, -119)           # rows whose only value is tiny, between ordinary ones
+    check(zeros, B)
+    a, b = A.astype(np.float32), B.astype(np.float32)
+    a[0, 7, 3], b[0, 3, 5], a[-1, 2, 1], b[-1, 1, 4] = np.inf, np.inf, -np.inf, np.inf
+    with np.errstate(invalid="ignore"):
+        ref = a.astype(np.float64) @ b.astype(np.float64)
+    got = run(a, b)
+    assert not np.isnan(ref).any() and np.array_equal(np.isinf(got), np.isinf(ref)) and not np.isnan(got).any()
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    fin = np.isfinite(ref)
+    assert (np.abs(got[fin] - ref[fin]) / ref[fin]).max() < 4 * 2.0 ** -24 * np.sqrt(k)
+    big = A.copy()
+    big[0, 3, :] *= 1e-3
+    big[0, 3, 2] = 3.4e38 / 4                        # with B below 4: finite, and not far from the largest Float32
+    big[-1, 4, 1] = np.nan
+    a, b = big.astype(np.float32), np.minimum(B, 3.9).astype(np.float32)
+    a[0, 1, 0] = 3.4e38
+    b[0, 0, :] = 0.5
+    got, ref = run(a, b), a.astype(np.float64) @ b.astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.isnan(ref).any()
+    fin = ~np.isnan(ref)
+    assert (np.abs(got[fin] - ref[fin]) / ref[fin]).max() < 4 * 2.0 ** -24 * np.sqrt(k)
