@@ -904,3 +904,40 @@ def test_float32_products_with_infinite_inputs(nn, oracle):
     v2[5, 90, 0] = np.nan
     y2, _ = _run(nn, q, k, v2, "f32", nheads=1, weights_dtype="f32")
     assert np.isnan(y2[5]).all() and np.isfinite(np.delete(y2, 5, axis=0)).all()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("kind", ["peak", "dense mask"])
+def test_pipelined_forward_where_half_of_a_block_dominates(nn, oracle, dtype, D, kind):
+    """A block of 32 keys lies in two halves of a wavefront (keys with bit 2 clear, and set).  The running maximum is that of
+    both: where the second half holds a score far above all others (f16 weights against the first half's maximum alone
+    would overflow) and where a dense mask keeps keys of the second half only."""
+    rng = np.random.default_rng(D)
+    H, L, B = 8, 512, 8   # 128 workgroups of 256 queries: the pipelined kernel
+    q, k, v = (round_to(rng.standard_normal((D * H, L, B)).astype(np.float32), dtype) for _ in range(3))
+    mask = None
+    if kind == "peak":
+        for j in (5, 100, 300, 511):   # (j & 4) != 0: every head's key j along query j - 1's row
+            for h in range(H):
+                row = q[h * D:(h + 1) * D, j - 1]
+                k[h * D:(h + 1) * D, j] = round_to(row * (25.0 * np.sqrt(D) / (row ** 2).sum(axis=0)), dtype)   # score 25
+    else:
+        mask = rng.random((L, L)) < 0.5
+        mask[:256][(np.arange(256) & 4) == 0] = False
+        mask[5] = True
+        q[::D], k[::D] = 8.0, 0.0
+        k[::D, 256:] = -20.0 * np.sqrt(D) / 8           # 20 below: next to nothing, and their first block must not replace the sums
+    D_ = nn.DeviceArray.from_numpy
+    y, _ = nn.dot_product_attention(D_(q, dtype), D_(k, dtype), D_(v, dtype), nheads=H, return_weights=False,
+                                    mask=None if mask is None else D_(mask))
+    assert nn.last_attention_kernel() == "flash16"
+    s = np.einsum("hdjb,hdib->hjib", k.reshape(H, D, L, B).astype(np.float64), q.reshape(H, D, L, B).astype(np.float64)) / np.sqrt(D)
+    if mask is not None:
+        s = np.where(mask[None, :, :, None], s, -np.inf)
+    w = np.exp(s - s.max(axis=1, keepdims=True))
+    w /= w.sum(axis=1, keepdims=True)
+    ref = np.einsum("hjib,hdjb->hdib", w, v.reshape(H, D, L, B).astype(np.float64)).reshape(D * H, L, B)
+    # no row has keys that compete near the large scores, so the error is that of ordinary inputs (2-norm): rounding of q, the
+    # weights and y to the type, 3.0e-3 and 3.6e-4 measured over many shapes, four times that allowed
+    assert np.linalg.norm(y.to_numpy() - ref) <= (1.2e-2 if dtype == "bf16" else 1.5e-3) * np.linalg.norm(ref)
