@@ -259,7 +259,8 @@ int32_t mi_dropout_dims(int32_t dtype, const void *x, void *y, int32_t ndim, con
 /* y[:, c] = softmax(x[:, c]) for a (rows, cols) column-major matrix; y may alias x
  * (softmax!(x), src/softmax.jl:64).  Arithmetic in fp32 (Float64 arrays: in double); +-Inf / NaN rules of
  * src/softmax.jl:69-79 (a +Inf maximum turns the column into an indicator of its
- * +Inf entries, normalised; NaN poisons its column; an all -Inf column is NaN). */
+ * +Inf entries, normalised, NaN entries among the zeros: the maximum skips a NaN; in any
+ * other column a NaN poisons all of it; an all -Inf column is NaN). */
 int32_t mi_softmax_dim1(int32_t dtype, const void *x, void *y, int64_t rows, int64_t cols,
                         mi_stream stream);
 

@@ -220,10 +220,13 @@ __global__ __launch_bounds__(1024) void softmax_column_stream_kernel(const typen
             if (GRAD) s += OP == OP_GRAD_SOFTMAX ? v * v2 : v;
             else s += term<T, OP>(v, m);
         };
-        // nothing but -Inf so far adds no terms; a column of nothing else is NaN in any case.  A NaN entry stays in the sum.
+        // nothing but -Inf so far adds no terms; a column of nothing else is NaN in any case.  A NaN entry stays in the sum,
+        // unless the maximum is +Inf: the sum then counts the +Inf entries (of logsumexp it is NaN), in any order.
+        constexpr bool INDICATOR = OP == OP_SOFTMAX || OP == OP_LOGSOFTMAX;
         const auto raise = [&](float top) {
             if (top > m) {
-                s = m == MI_NEG_INF ? (s == s ? 0.0f : s) : s * C::exp(m - top);
+                if (INDICATOR && top == MI_POS_INF) s = 0.0f;
+                else s = m == MI_NEG_INF ? (s == s ? 0.0f : s) : s * C::exp(m - top);
                 m = top;
             }
         };
@@ -263,7 +266,8 @@ __global__ __launch_bounds__(1024) void softmax_column_stream_kernel(const typen
         } else {
             c0 = reduce<true, 0>(m, red[0]);
             // a lane that has seen nothing but -Inf holds no terms (or a NaN)
-            s = m == c0 || s != s ? s : (m == MI_NEG_INF ? 0.0f : s * C::exp(m - c0));
+            if (INDICATOR && c0 == MI_POS_INF) s = m == c0 ? s : 0.0f;
+            else s = m == c0 || s != s ? s : (m == MI_NEG_INF ? 0.0f : s * C::exp(m - c0));
             s = reduce<false, 0>(s, red[1]);
             if (c0 == MI_NEG_INF) s = __builtin_nanf("");
             c1 = OP != OP_SOFTMAX ? logf(s) : VEC == 4 ? s : 1.0f / s;

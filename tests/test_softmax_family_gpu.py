@@ -378,3 +378,22 @@ def test_empty_logsumexp_reads_nothing(nn, dtype, inner):
     x = torch.zeros(16, dtype=tdt, device="cuda")
     _lib.check(_lib.load().mi_logsumexp(code, x.data_ptr(), y.data_ptr(), inner, 0, 3, torch.cuda.current_stream().cuda_stream))
     assert bool((y == float("-inf")).all())
+
+
+@pytest.mark.parametrize("dtype,length", [("f32", 70001), ("bf16", 140003), ("f16", 140000), ("f32", 3), ("f32", 700), ("bf16", 30001)])
+def test_columns_with_an_infinity_and_a_nan(nn, oracle, dtype, length):
+    """A +Inf maximum makes a column the indicator of its +Inf entries, NaN entries or not (src/softmax.jl:72-75; the maximum
+    skips a NaN), whichever a lane of the streaming kernel meets first: the two lie on one lane, 4 x 1024 pieces of 16 bytes
+    apart, in either order, on two lanes, and next to each other."""
+    rng = np.random.default_rng(length)
+    x = round_to(rng.standard_normal((length, 5)), dtype)
+    far = 4096 * (4 if dtype == "f32" else 8) if length > 65536 else length // 2
+    first = 8 if length > 16 else 0
+    for c, (nan_at, inf_at) in enumerate([(first, first + far), (first + far, first), (first, length - 1), (length - 1, first), (first, first + 1)]):
+        x[nan_at, c], x[inf_at, c] = np.nan, np.inf
+    with np.errstate(invalid="ignore", divide="ignore"):
+        for log, fn in ((False, nn.softmax), (True, nn.logsoftmax)):
+            ref = oracle.softmax(x, 1, log=log)
+            assert not np.isnan(ref).any()
+            assert np.array_equal(fn(_dev(nn, x, dtype), dims=1).to_numpy(), ref)
+    assert np.isnan(nn.logsumexp(_dev(nn, x, dtype), dims=1).to_numpy()).all()
