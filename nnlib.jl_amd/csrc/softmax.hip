@@ -15,8 +15,8 @@
 // Times before are those of the kernels this replaced (at most 4096 elements of a column in registers, one element a lane
 // unless the columns were 16-byte aligned, three passes over longer ones); a large copy moves 4.8 TB/s on this card:
 //   10000 x 4096 Float32          softmax 164 -> 80 us   logsoftmax 174 -> 75    its gradient 196 -> 91 (5.4 TB/s)
-//   10007 x 8192 BFloat16                 269 -> 84                 282 -> 80                 328 -> 104
-//   1001 x 65536 BFloat16                 161 -> 40                 200 -> 40                 357 -> 68
+//   10007 x 8192 BFloat16                 269 -> 98                 282 -> 80                 328 -> 104
+//   1001 x 65536 BFloat16                 161 -> 64                 200 -> 40                 357 -> 68
 //   37 x 524288 Float32                    86 -> 30                1077 -> 27                1017 -> 35
 //   131072 x 1024 Float32                 919 -> 293                876 -> 290                625 -> 368
 #include "common.h"
@@ -42,17 +42,33 @@ template <typename T> struct Column : ColumnIO<T> {
             v = __builtin_bit_cast(u32x4_t, h);
         }
     }
-    // e^x: the library function for Float32; 16-bit results are rounded far above the error of the hardware 2^x
-    __device__ static float exp(float x) {
+    // e^x: the library function for Float32, the hardware 2^x of x log2(e) for the 16-bit operations but softmax.  16-bit
+    // softmax corrects that for what the product lost (4e-6 of the term at x = -80, a 24-bit x times 2^-24): 2^t e^r with
+    // t = x log2(e) rounded and r = x - t ln 2, so small that e^r = 1 + r; at -Inf r is NaN and the minimum takes 1.  x <= 0.
+    // (10007 x 8192 bf16: uncorrected 79 us, so 98, with the library function 109.)
+    template <int OP> __device__ static float exp(float x) {
         if constexpr (VEC == 4) return expf(x);
-        else return mi_exp2(x * MI_LOG2E);
+        const float t = x * MI_LOG2E, e = mi_exp2(t);
+        if constexpr (OP != OP_SOFTMAX) return e;
+        constexpr float LN2 = 0x1.62e43p-1f, LN2_LOW = -0x1.05c610p-29f;   // ln 2 = LN2 + LN2_LOW
+        return fmaf(e, fminf(fmaf(-t, LN2_LOW, fmaf(-t, LN2, x)), 1.0f), e);
     }
+    // A BFloat16 result may be a subnormal number, which the hardware 2^x flushes to zero: pieces with one (elements 87 or
+    // more below the maximum m) take the library function.
+    static constexpr bool SUBNORMAL = __is_same(T, BF16);
+    __device__ static bool subnormal(const u32x4_t &v, float m) {
+        float low = get(v, 0);
+#pragma unroll
+        for (int e = 1; e < VEC; e++) low = fminf(low, get(v, e));
+        return SUBNORMAL && low - m < -87.0f;
+    }
+    __device__ static float share(float term, float sum, float inv) { return VEC == 4 ? term / sum : quotient(term, sum, inv); }
 };
 
 // the reference's elementwise rules given the column maximum m
 template <typename T> __device__ inline float softmax_term(float x, float m) {   // src/softmax.jl:72-75
     if (m == MI_POS_INF) return x == MI_POS_INF ? 1.0f : 0.0f;
-    return Column<T>::exp(x - m);
+    return Column<T>::template exp<OP_SOFTMAX>(x - m);
 }
 __device__ inline float logsoftmax_shift(float x, float m) {   // src/softmax.jl:140-144
     if (m == MI_POS_INF) return x == MI_POS_INF ? 0.0f : MI_NEG_INF;
@@ -60,16 +76,15 @@ __device__ inline float logsoftmax_shift(float x, float m) {   // src/softmax.jl
 }
 template <typename T, int OP> __device__ inline float term(float x, float m) {
     if (OP == OP_SOFTMAX) return softmax_term<T>(x, m);
-    if (OP == OP_LOGSOFTMAX) return Column<T>::exp(logsoftmax_shift(x, m));
-    return Column<T>::exp(x - m);   // logsumexp: no special cases (src/softmax.jl:202)
+    if (OP == OP_LOGSOFTMAX) return Column<T>::template exp<OP>(logsoftmax_shift(x, m));
+    return Column<T>::template exp<OP>(x - m);   // logsumexp: no special cases (src/softmax.jl:202)
 }
-// the result of one element; forward: c0 = maximum, c1 = sum (Float32 softmax), 1 / sum (16-bit softmax) or log(sum);
-// gradients: x = dy, c0 = the sum
-template <typename T, int OP> __device__ inline float result(float x, float y, float c0, float c1) {
-    if (OP == OP_SOFTMAX) return Column<T>::VEC == 4 ? softmax_term<T>(x, c0) / c1 : softmax_term<T>(x, c0) * c1;
+// the result of one element; forward: c0 = maximum, c1 = sum (softmax; c2 = 1 / sum) or log(sum); gradients: x = dy, c0 = the sum
+template <typename T, int OP> __device__ inline float result(float x, float y, float c0, float c1, float c2, bool subnormal) {
+    if (OP == OP_SOFTMAX) return Column<T>::share(subnormal && c0 < MI_POS_INF ? expf(x - c0) : softmax_term<T>(x, c0), c1, c2);
     if (OP == OP_LOGSOFTMAX) return logsoftmax_shift(x, c0) - c1;
     if (OP == OP_GRAD_SOFTMAX) return y * (x - c0);
-    return x - c0 * Column<T>::exp(y);
+    return x - c0 * Column<T>::template exp<OP>(y);
 }
 
 // The pieces stay in their packed form from pass to pass: without this the compiler keeps what the pass before computed
@@ -135,7 +150,7 @@ __global__ __launch_bounds__(G ? 256 : 1024) void softmax_column_kernel(const ty
                     }
             }
         }
-        float c0, c1 = 0.0f;
+        float c0, c1 = 0.0f, c2 = 0.0f;
         if constexpr (GRAD) {
             float s = 0.0f;
 #pragma unroll
@@ -167,10 +182,11 @@ __global__ __launch_bounds__(G ? 256 : 1024) void softmax_column_kernel(const ty
                     }
             };
             if (OP != OP_LOGSUMEXP && c0 == MI_POS_INF) add_terms([](float v) { return v == MI_POS_INF ? 1.0f : 0.0f; });
-            else add_terms([&](float v) { return C::exp(v - c0); });
+            else add_terms([&](float v) { return C::template exp<OP>(v - c0); });
             s = reduce<false, G>(s, red[1]);
             keep_packed(raw);
-            c1 = OP != OP_SOFTMAX ? logf(s) : VEC == 4 ? s : 1.0f / s;
+            c1 = OP != OP_SOFTMAX ? logf(s) : s;
+            c2 = 1.0f / s;
         }
         if constexpr (OP == OP_LOGSUMEXP) {
             if (lane == 0) y[c] = T::from_f32(c0 + c1);
@@ -181,8 +197,13 @@ __global__ __launch_bounds__(G ? 256 : 1024) void softmax_column_kernel(const ty
                     const int p = lane + u * lanes, at = p < last ? p * VEC : len - VEC, skip = p * VEC - at;
                     if (p > last) continue;
                     u32x4_t r = raw[u];
+                    if (OP == OP_SOFTMAX && C::SUBNORMAL && C::subnormal(r, c0)) {
 #pragma unroll
-                    for (int e = 0; e < VEC; e++) C::set(r, e, rule(C::get(raw[u], e), GRAD ? C::get(raw2[GRAD ? u : 0], e) : 0.0f));
+                        for (int e = 0; e < VEC; e++) C::set(r, e, result<T, OP>(C::get(raw[u], e), 0.0f, c0, c1, c2, true));
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < VEC; e++) C::set(r, e, rule(C::get(raw[u], e), GRAD ? C::get(raw2[GRAD ? u : 0], e) : 0.0f));
+                    }
                     if (skip == 0) C::store(yc + at, r);
                     else
 #pragma unroll
@@ -190,12 +211,12 @@ __global__ __launch_bounds__(G ? 256 : 1024) void softmax_column_kernel(const ty
                             if (e >= skip) yc[at + e] = T::from_f32(C::get(r, e));
                 }
             };
-            if (!GRAD && !KEEP_TERMS && c0 == MI_POS_INF) write([&](float v, float) { return result<T, OP>(v, 0.0f, MI_POS_INF, c1); });
+            if (!GRAD && !KEEP_TERMS && c0 == MI_POS_INF) write([&](float v, float) { return result<T, OP>(v, 0.0f, MI_POS_INF, c1, c2, false); });
             else write([&](float v, float v2) {
                 if (KEEP_TERMS) return v / c1;
-                if (OP == OP_SOFTMAX) return C::exp(v - c0) * c1;
+                if (OP == OP_SOFTMAX) return C::share(C::template exp<OP>(v - c0), c1, c2);
                 if (OP == OP_LOGSOFTMAX) return v - c0 - c1;
-                return result<T, OP>(v, v2, c0, c1);
+                return result<T, OP>(v, v2, c0, c1, c2, false);
             });
         }
     }
@@ -226,7 +247,7 @@ __global__ __launch_bounds__(1024) void softmax_column_stream_kernel(const typen
         const auto raise = [&](float top) {
             if (top > m) {
                 if (INDICATOR && top == MI_POS_INF) s = 0.0f;
-                else s = m == MI_NEG_INF ? (s == s ? 0.0f : s) : s * C::exp(m - top);
+                else s = m == MI_NEG_INF ? (s == s ? 0.0f : s) : s * C::template exp<OP>(m - top);
                 m = top;
             }
         };
@@ -260,17 +281,18 @@ __global__ __launch_bounds__(1024) void softmax_column_stream_kernel(const typen
             if (!GRAD) raise(v);
             if (GRAD || m != MI_NEG_INF || v != v) add(v, OP == OP_GRAD_SOFTMAX ? T::to_f32(x2c[j]) : 0.0f);
         }
-        float c0, c1 = 0.0f;
+        float c0, c1 = 0.0f, c2 = 0.0f;
         if constexpr (GRAD) {
             c0 = reduce<false, 0>(s, red[0]);
         } else {
             c0 = reduce<true, 0>(m, red[0]);
             // a lane that has seen nothing but -Inf holds no terms (or a NaN)
             if (INDICATOR && c0 == MI_POS_INF) s = m == c0 ? s : 0.0f;
-            else s = m == c0 || s != s ? s : (m == MI_NEG_INF ? 0.0f : s * C::exp(m - c0));
+            else s = m == c0 || s != s ? s : (m == MI_NEG_INF ? 0.0f : s * C::template exp<OP>(m - c0));
             s = reduce<false, 0>(s, red[1]);
             if (c0 == MI_NEG_INF) s = __builtin_nanf("");
-            c1 = OP != OP_SOFTMAX ? logf(s) : VEC == 4 ? s : 1.0f / s;
+            c1 = OP != OP_SOFTMAX ? logf(s) : s;
+            c2 = 1.0f / s;
         }
         if constexpr (OP == OP_LOGSUMEXP) {   // the reference's x - max is Inf - Inf for an infinite maximum
             if (threadIdx.x == 0) y[c] = T::from_f32(c0 == MI_POS_INF ? __builtin_nanf("") : c0 + c1);
@@ -288,13 +310,18 @@ __global__ __launch_bounds__(1024) void softmax_column_stream_kernel(const typen
                     const int64_t p = p0 + (int64_t)u * blockDim.x;
                     if (p >= whole) break;
                     u32x4_t r = raw[u];
+                    if (OP == OP_SOFTMAX && C::SUBNORMAL && C::subnormal(r, c0)) {
 #pragma unroll
-                    for (int e = 0; e < VEC; e++) C::set(r, e, result<T, OP>(C::get(raw[u], e), GRAD ? C::get(raw2[u], e) : 0.0f, c0, c1));
+                        for (int e = 0; e < VEC; e++) C::set(r, e, result<T, OP>(C::get(raw[u], e), 0.0f, c0, c1, c2, true));
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < VEC; e++) C::set(r, e, result<T, OP>(C::get(raw[u], e), GRAD ? C::get(raw2[u], e) : 0.0f, c0, c1, c2, false));
+                    }
                     C::store(yc + p * VEC, r);
                 }
             }
             for (int64_t j = whole * VEC + threadIdx.x; j < len; j += blockDim.x)
-                yc[j] = T::from_f32(result<T, OP>(T::to_f32(xc[j]), GRAD ? T::to_f32(x2c[j]) : 0.0f, c0, c1));
+                yc[j] = T::from_f32(result<T, OP>(T::to_f32(xc[j]), GRAD ? T::to_f32(x2c[j]) : 0.0f, c0, c1, c2, Column<T>::SUBNORMAL));
         }
         __syncthreads();   // red is written again by the next column
     }
@@ -321,10 +348,10 @@ __global__ __launch_bounds__(256) void softmax_tiny_column_kernel(const typename
         if constexpr (OP == OP_LOGSUMEXP) {
             y[c] = T::from_f32(m + logf(s));
         } else {
-            const float c0 = GRAD ? s : m, c1 = OP == OP_LOGSOFTMAX ? logf(s) : Column<T>::VEC == 4 ? s : 1.0f / s;
+            const float c0 = GRAD ? s : m, c1 = OP == OP_LOGSOFTMAX ? logf(s) : s, c2 = 1.0f / s;
 #pragma unroll
             for (int j = 0; j < MOST; j++)
-                if (j < len) y[c * len + j] = T::from_f32(result<T, OP>(v[j], v2[j], c0, c1));
+                if (j < len) y[c * len + j] = T::from_f32(result<T, OP>(v[j], v2[j], c0, c1, c2, Column<T>::SUBNORMAL));
         }
     }
 }

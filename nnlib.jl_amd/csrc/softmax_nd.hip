@@ -53,8 +53,8 @@ __device__ inline float softmax_term(float x, float m) {   // src/softmax.jl:72-
     if (m == MI_POS_INF) return x == MI_POS_INF ? 1.0f : 0.0f;
     return fast_exp(x - m);
 }
-// a term over the column's sum: Float32 divides; the 16-bit types, rounded far above the error, take 1 / sum
-template <int VEC> __device__ inline float share(float term, float c) { return VEC == 4 ? term / c : term * c; }
+// a term over the column's sum, inv = 1 / sum
+template <int VEC> __device__ inline float share(float term, float sum, float inv) { return VEC == 4 ? term / sum : quotient(term, sum, inv); }
 __device__ inline float logsoftmax_shift(float x, float m) {   // src/softmax.jl:140-144
     if (m == MI_POS_INF) return x == MI_POS_INF ? 0.0f : MI_NEG_INF;
     return x - m;
@@ -449,7 +449,7 @@ __global__ __launch_bounds__(NT, (NP * (OP >= OP_GRAD_SOFTMAX ? 2 : 1) <= 16 && 
             } else if (plain) {
                 float c1[VEC];
 #pragma unroll
-                for (int e = 0; e < VEC; e++) c1[e] = OP == OP_LOGSOFTMAX ? logf(sum[e]) : VEC == 4 ? sum[e] : 1.0f / sum[e];
+                for (int e = 0; e < VEC; e++) c1[e] = OP == OP_LOGSOFTMAX ? logf(sum[e]) : 1.0f / sum[e];
 #pragma unroll
                 for (int u = 0; u < NP; u++) {
                     if (FULL || u < nrows) {
@@ -457,7 +457,7 @@ __global__ __launch_bounds__(NT, (NP * (OP >= OP_GRAD_SOFTMAX ? 2 : 1) <= 16 && 
                         IO::unpack(raw[u], v);
 #pragma unroll
                         for (int e = 0; e < VEC; e++)
-                            r[e] = OP == OP_SOFTMAX ? share<VEC>(fast_exp(v[e] - m[e]), c1[e]) : v[e] - m[e] - c1[e];
+                            r[e] = OP == OP_SOFTMAX ? share<VEC>(fast_exp(v[e] - m[e]), sum[e], c1[e]) : v[e] - m[e] - c1[e];
                         put(cur, u, IO::pack(r));
                     }
                     }
@@ -559,8 +559,12 @@ __global__ __launch_bounds__(256) void softmax_nd_short_kernel(const typename T:
             IO::store(y + (int64_t)o * inner + col, s, skip);
         }
     } else {
+        float inv[VEC];
 #pragma unroll
-        for (int e = 0; e < VEC; e++) s[e] = OP == OP_SOFTMAX && VEC != 4 ? 1.0f / s[e] : OP == OP_LOGSOFTMAX ? logf(s[e]) : s[e];
+        for (int e = 0; e < VEC; e++) {
+            inv[e] = 1.0f / s[e];
+            if (OP == OP_LOGSOFTMAX) s[e] = logf(s[e]);
+        }
 #pragma unroll
         for (int u = 0; u < NP; u++) {
             if (!mine(u)) break;
@@ -569,7 +573,7 @@ __global__ __launch_bounds__(256) void softmax_nd_short_kernel(const typename T:
             if (GRAD) IO::unpack(raw2[u], v2);
 #pragma unroll
             for (int e = 0; e < VEC; e++) {
-                if (OP == OP_SOFTMAX) r[e] = share<VEC>(softmax_term(v[e], m[e]), s[e]);
+                if (OP == OP_SOFTMAX) r[e] = share<VEC>(softmax_term(v[e], m[e]), s[e], inv[e]);
                 else if (OP == OP_LOGSOFTMAX) r[e] = logsoftmax_shift(v[e], m[e]) - s[e];
                 else if (OP == OP_GRAD_SOFTMAX) r[e] = v2[e] * (v[e] - s[e]);
                 else r[e] = v[e] - s[e] * fast_exp(v2[e]);
@@ -664,7 +668,7 @@ __global__ __launch_bounds__(256) void softmax_nd_vec_kernel(const typename T::t
 #pragma unroll
         for (int e = 0; e < VEC; e++) {
             plain = plain && m[e] > MI_NEG_INF && m[e] < MI_POS_INF;
-            c1[e] = OP == OP_LOGSOFTMAX ? logf(s[e]) : VEC == 4 ? s[e] : 1.0f / s[e];
+            c1[e] = OP == OP_LOGSOFTMAX ? logf(s[e]) : 1.0f / s[e];
         }
         for (int64_t r0 = 0; r0 < nrows; r0 += U) {
             u32x4_t raw[U], raw2[U];
@@ -682,7 +686,7 @@ __global__ __launch_bounds__(256) void softmax_nd_vec_kernel(const typename T::t
                 if (GRAD) IO::unpack(raw2[u], v2);
 #pragma unroll
                 for (int e = 0; e < VEC; e++) {
-                    if (OP == OP_SOFTMAX) r[e] = share<VEC>(plain ? fast_exp(v[e] - m[e]) : softmax_term(v[e], m[e]), c1[e]);
+                    if (OP == OP_SOFTMAX) r[e] = share<VEC>(plain ? fast_exp(v[e] - m[e]) : softmax_term(v[e], m[e]), s[e], c1[e]);
                     else if (OP == OP_LOGSOFTMAX) r[e] = (plain ? v[e] - m[e] : logsoftmax_shift(v[e], m[e])) - c1[e];
                     else if (OP == OP_GRAD_SOFTMAX) r[e] = v2[e] * (v[e] - s[e]);
                     else r[e] = v[e] - s[e] * fast_exp(v2[e]);

@@ -397,3 +397,34 @@ def test_columns_with_an_infinity_and_a_nan(nn, oracle, dtype, length):
             assert not np.isnan(ref).any()
             assert np.array_equal(fn(_dev(nn, x, dtype), dims=1).to_numpy(), ref)
     assert np.isnan(nn.logsumexp(_dev(nn, x, dtype), dims=1).to_numpy()).all()
+
+
+@pytest.mark.parametrize("length", [5, 300, 3001, 20000, 70001])
+def test_bfloat16_softmax_is_rounded_once(nn, length):
+    """Softmax along dimension 1 computes in Float32 and rounds its result: e^x, the sum and the quotient err by about 1e-7
+    together, which changes the rounding of a share 1e-7 / 2^-8 ... 2^-7 of the results, 2e-5; 1e-4 are allowed.  (e^x as the
+    hardware 2^x of x log2(e) errs by 2^-24 |x|: 2e-4 of them at arguments down to -80.)"""
+    rng = np.random.default_rng(length)
+    x = round_to(rng.uniform(-80.0, 0.0, (length, max(4, 600000 // length))), "bf16")
+    x[0] = 0.0
+    w = np.exp(x.astype(np.float64))
+    want = round_to(w / w.sum(axis=0), "bf16")
+    got = nn.softmax(_dev(nn, x, "bf16"), dims=1).to_numpy()
+    assert np.mean(got != want) <= 1e-4
+
+
+@pytest.mark.parametrize("length", [3, 300, 3001, 70001])
+def test_bfloat16_softmax_keeps_subnormal_results(nn, length):
+    """Elements 88 to 92 below the maximum have weights that are subnormal numbers of the type (2^-133 the smallest): held to
+    half a unit of that and the 1e-6 of ordinary ones.  -Inf entries are exact zeros next to them."""
+    x = np.zeros((length, 4), np.float32)
+    x[1::7] = -88.5
+    x[2::5] = -92.0
+    x[4::9] = -np.inf
+    w = np.exp(x.astype(np.float64))
+    want = w / w.sum(axis=0)
+    got = nn.softmax(_dev(nn, x, "bf16"), dims=1).to_numpy().astype(np.float64)
+    assert np.abs(got - want).max() <= np.abs(want).max() * 2.0 ** -8
+    deep = (x < -80) & np.isfinite(x)
+    small = np.abs(got[deep] - want[deep]) <= 2.0 ** -134 + 1e-6 * want[deep]
+    assert small.all() and not got[np.isinf(x)].any()
