@@ -95,7 +95,7 @@ struct Operand {
         for (int u = 0; u < 4; u++) {
             const int c = threadIdx.x + THREADS * u;
             if (RM) {
-                const int kk = c / CPR, r8 = (c % CPR) * 8;     // kk >= k falls past the extent by itself
+                const int kk = c / CPR, r8 = (c % CPR) * 8;     // kk >= k: past the extent by itself, or see `offset`
                 off[u] = row0 + r8 < rows ? (int)(((row0 + r8) + kk * ld) * 2) : OOB;
             } else {
                 const int r = c >> 3, k8 = (c & 7) * 8;         // 8 pieces per row
@@ -105,9 +105,11 @@ struct Operand {
     }
     __device__ int offset(int u, int64_t k0) const {
         int o = off[u] == OOB ? OOB : off[u] + (int)k0 * kstep;
-        if (!RM) {   // a piece past k in a row-contiguous-in-k matrix would read the next row
-            const int k8 = ((threadIdx.x + THREADS * u) & 7) * 8;
-            o = k0 + k8 < k ? o : OOB;
+        // a piece past k would read the next row of a matrix contiguous along k; in one contiguous along its rows its byte
+        // offset may pass 2^32 and come round into the slice (`far` calls, which take ANY)
+        if (!RM || ANY) {
+            const int c = threadIdx.x + THREADS * u, kk = RM ? c / CPR : (c & 7) * 8;
+            o = k0 + kk < k ? o : OOB;
         }
         return o;
     }
@@ -506,7 +508,7 @@ int32_t launch_l(const Gemm16Args &g, int transA, int transB, int64_t nb, hipStr
 }
 
 template <typename T>
-int32_t launch_t(const Gemm16Args &g, int transA, int transB, int64_t nb, bool aligned, hipStream_t st) {
+int32_t launch_t(const Gemm16Args &g, int transA, int transB, int64_t nb, bool aligned, bool far, hipStream_t st) {
     // Operands of any alignment: the small tile (the copies global -> LDS of the ring kernel move whole aligned pieces, and
     // the large register-staged one spills with them: 513^3 x 64 unaligned 64 us small, 99 large; 2047^3 x 8 237 / 229).
     if (!aligned) return launch_l<T, false, true>(g, transA, transB, nb, st);
@@ -521,8 +523,9 @@ int32_t launch_t(const Gemm16Args &g, int transA, int transB, int64_t nb, bool a
     static const bool no_ring = getenv("MI355ATTN_GEMM_NO_RING") != nullptr;   // A/B switch: the register-staged kernels
     // the ring kernel for the large shape only: at 128 x 128 it was measured level or behind the register-staged kernel
     // (128 x 4096 x 4096 x 64: 593 against 637 TFLOP/s, 64 x 2048 x 2048 x 64: 252 / 290, 1024^3 x 4: 607 / 573)
-    if (large) return no_ring ? launch_l<T, true, false>(g, transA, transB, nb, st) : launch_ring_l<T, true>(g, transA, transB, nb, st);
-    return launch_l<T, false, false>(g, transA, transB, nb, st);
+    if (large && !no_ring) return launch_ring_l<T, true>(g, transA, transB, nb, st);
+    if (far) return launch_l<T, false, true>(g, transA, transB, nb, st);
+    return large ? launch_l<T, true, false>(g, transA, transB, nb, st) : launch_l<T, false, false>(g, transA, transB, nb, st);
 }
 
 }  // namespace
@@ -545,11 +548,16 @@ int32_t launch_batched_gemm16(int32_t dtype, int transA, int transB, int64_t m, 
     // every 16-byte piece of the operands is aligned and wholly inside or outside its matrix
     const bool aligned = ((((uintptr_t)A) | ((uintptr_t)B)) & 15) == 0 &&
                          ((lda | ldb | sA | sB | (transA ? k : m) | (transB ? n : k)) & 7) == 0;
+    // an operand contiguous along its rows whose k, rounded up to whole stages and with the two that are fetched ahead, spans
+    // 2^32 bytes (few k, huge leading dimension)
+    const auto spans = [&](bool rm, int64_t ld) { return rm && ((k + KC - 1) / KC + 2) * KC * ld * 2 >= (1LL << 32); };
+    const bool far = spans(!transA, lda) || spans(transB != 0, ldb);
     for (int64_t b0 = 0; b0 < batch; b0 += 65535) {   // gridDim.z is limited to 65535: issue the batch in slabs
         const int64_t nb = batch - b0 < 65535 ? batch - b0 : 65535;
         Gemm16Args g = {(const char *)A + es * b0 * sA, (const char *)B + es * b0 * sB, (char *)C + es * b0 * sC,
                         m, n, k, lda, ldb, ldc, sA, sB, sC, alpha, beta};
-        const int32_t rc = dtype == MI_F16 ? launch_t<F16>(g, transA, transB, nb, aligned, st) : launch_t<BF16>(g, transA, transB, nb, aligned, st);
+        const int32_t rc = dtype == MI_F16 ? launch_t<F16>(g, transA, transB, nb, aligned, far, st)
+                                            : launch_t<BF16>(g, transA, transB, nb, aligned, far, st);
         if (rc != MI_OK) return rc;
     }
     return MI_OK;

@@ -502,3 +502,25 @@ def test_unaligned_float32_products_at_the_ends_of_the_range(nn, ta, tb, m, n, k
     assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.isnan(ref).any()
     fin = ~np.isnan(ref)
     assert (np.abs(got[fin] - ref[fin]) / ref[fin]).max() < 4 * 2.0 ** -24 * np.sqrt(k)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("m,n,k,ld", [(64, 128, 8, 1 << 26), (65, 71, 7, (1 << 26) + 1), (256, 256, 8, 1 << 26), (72, 64, 20, 44739240)])
+def test_few_k_far_apart(nn, dtype, m, n, k, ld):
+    """Both operands contiguous along their rows with k-rows 2^27 bytes and more apart: the padded k of a stage lies past the
+    32-bit offsets, and nothing of it may come round into the product (each k would count twice)."""
+    import torch
+    if dtype == "f32":
+        ld = ld // 2 | (ld & 1)   # the same bytes
+    rng = np.random.default_rng(k)
+    a, b = (round_to(rng.standard_normal((k, x)), dtype) for x in (m, n))
+    off = 512
+    store = torch.empty((k - 1) * ld + off + 512, dtype=torch.bfloat16 if dtype == "bf16" else torch.float32, device="cuda")
+    for j in range(k):
+        store[j * ld:j * ld + m] = torch.from_numpy(a[j].astype(np.float32)).to(store)
+        store[j * ld + off:j * ld + off + n] = torch.from_numpy(b[j].astype(np.float32)).to(store)
+    A = nn.DeviceArray(store, (m, k, 1), dtype, (1, ld, 1), 0)
+    B = nn.DeviceArray(store, (n, k, 1), dtype, (1, ld, 1), off)
+    C = nn.batched_mul(A, nn.batched_transpose(B)).to_numpy()[:, :, 0]
+    ref = a.T.astype(np.float64) @ b.astype(np.float64)
+    assert np.abs(C - ref).max() <= TOL[dtype] * np.abs(ref).max()
