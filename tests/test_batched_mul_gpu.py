@@ -207,8 +207,8 @@ def test_tiled_kernel_all_layouts(nn, dtype, ta, tb, m, n, k, nb):
 @pytest.mark.parametrize("dtype", ["bf16", "f16", "f32"])
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
 def test_large_tile_kernel(nn, dtype, ta, tb):
-    """Enough 256 x 256 tiles to fill the chip: the eight-wavefront shape of the 16-bit kernel and of the Float32
-    kernel on bf16 planes, ragged in m, n and k, with alpha and beta."""
+    """Many ragged tiles of the four-wavefront shape, with alpha and beta: m and n leave the 256 x 256 tiles half empty (the
+    shapes that take those are in test_large_tiles)."""
     rng = np.random.default_rng(17)
     m, n, k, nb = 264, 520, 136, 48
     A = round_to(rng.standard_normal((k, m, nb) if ta else (m, k, nb)), dtype)
@@ -225,7 +225,7 @@ def test_large_tile_kernel(nn, dtype, ta, tb):
 def test_tile_order_covers_every_tile(nn, dtype, m, n, k, nb):
     """The tiled kernels hand their tiles to the workgroups in a permuted order (runs per die, bands of eight tile
     rows): tile counts that are not multiples of eight in m, in total, or both, so that a tile the permutation
-    skipped or visited twice shows as a wrong block of the product."""
+    skipped or visited twice shows as a wrong block of the product.  (128 x 128 tiles; test_large_tiles has the others.)"""
     rng = np.random.default_rng(m + n + nb)
     A = round_to(rng.standard_normal((m, k, nb)), dtype)
     B = round_to(rng.standard_normal((k, n, nb)), dtype)
@@ -524,3 +524,38 @@ def test_few_k_far_apart(nn, dtype, m, n, k, ld):
     C = nn.batched_mul(A, nn.batched_transpose(B)).to_numpy()[:, :, 0]
     ref = a.T.astype(np.float64) @ b.astype(np.float64)
     assert np.abs(C - ref).max() <= TOL[dtype] * np.abs(ref).max()
+
+
+def _takes_large_tiles(dtype, ta, tb, m, n, k, nb):
+    """The rule of batched_gemm16.hip / batched_gemm32.hip for the 256 x 256 tiles."""
+    def useful(tile, slots):
+        tiles = -(-m // tile) * -(-n // tile) * nb
+        return m * n * nb / (-(-tiles // slots) * slots * tile * tile)
+    if m < 256 or n < 256:
+        return False
+    if dtype == "f32":
+        return k >= 128 and (1.15 if k >= 512 else 1.0) * useful(256, 256) > useful(128, 768)
+    aligned = all(x % 8 == 0 for x in (k if ta else m, n if tb else k, m * k, k * n))
+    return aligned and 1.35 * useful(256, 256) > useful(128, 512)
+
+
+@pytest.mark.parametrize("dtype,ta,tb,m,n,k,nb",
+                         [(d, ta, tb, 504, 512, 136, 64) for d in ("bf16", "f16", "f32") for ta in (0, 1) for tb in (0, 1)] +   # 16-byte pieces all over
+                         [(d, 1, 0, 505, 511, 136, 64) for d in ("bf16", "f16", "f32")] +          # aligned operands, C columns of odd length
+                         [("f32", ta, tb, 505, 511, 133, 64) for ta in (0, 1) for tb in (0, 1)] +  # operands of any alignment
+                         [(d, 0, 0, 2312, 600, 136, 17) for d in ("bf16", "f32")] +                # tile order: 10 x 3 tiles
+                         [(d, 0, 0, 1160, 456, 136, 25) for d in ("bf16", "f32")] +                # 250 tiles, 5 x 2
+                         [(d, 0, 0, 504, 2104, 136, 14) for d in ("bf16", "f32")])                 # 2 x 9
+def test_large_tiles(nn, dtype, ta, tb, m, n, k, nb):
+    """Products that fill the chip with 256 x 256 tiles, by the rule the library chooses them by: the ring kernel of the 16-bit
+    types and the eight-wavefront Float32 kernel on bf16 planes (aligned, and of any alignment), ragged in m, n and k,
+    at C columns of odd length, with alpha and beta, and at tile counts that are no multiple of eight."""
+    assert _takes_large_tiles(dtype, ta, tb, m, n, k, nb)
+    rng = np.random.default_rng(m + n + k + 2 * ta + tb)
+    A = round_to(rng.standard_normal((k, m, nb) if ta else (m, k, nb)), dtype)
+    B = round_to(rng.standard_normal((n, k, nb) if tb else (k, n, nb)), dtype)
+    C0 = round_to(rng.standard_normal((m, n, nb)), dtype)
+    dA, dB, dC = (nn.DeviceArray.from_numpy(x, dtype) for x in (A, B, C0))
+    T = nn.batched_transpose
+    nn.batched_mul_(dC, T(dA) if ta else dA, T(dB) if tb else dB, 0.5, 2.0)
+    assert close(dC.to_numpy(), 0.5 * bmm(A, B, ta, tb) + 2.0 * C0, dtype)
