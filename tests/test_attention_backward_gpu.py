@@ -815,3 +815,45 @@ def test_every_key_of_a_sequence_dropped(nn, dtype, D, Lq, Lkv, causal, p, nan_q
         assert np.isnan(dk[:, :, 2]).all() and np.isnan(dv[:, :, 2]).all() and np.isnan(dq[:, 5, 2]).all()
     else:
         assert np.isfinite(dk[:, :, 2]).all() and np.isfinite(dv[:, :, 2]).all() and np.isfinite(dq[:, :, 2]).all()
+
+
+def test_shared_bias_with_the_key_range_in_pieces(nn, oracle):
+    """Few queries, many keys: dQ comes from pieces of the key range, whose partial sums lie in the workspace in front of the
+    copies of the bias."""
+    for dtype, Lkv in (("bf16", 2100), ("f16", 4097)):
+        _run(nn, oracle, dtype, 128, 128, 64, Lkv, (3,), 2, bias_shape=(Lkv, 64, 2, 1), seed=Lkv, scale=0.4, saved=True, expect="flash16")
+
+
+@pytest.mark.parametrize("dtype,D,L,B,saved", [("bf16", 64, 197, 3, True), ("f16", 128, 130, 2, True), ("bf16", 64, 140, 3, False), ("bf16", 136, 70, 2, True)])
+def test_infinite_entries_of_a_shared_bias(nn, oracle, dtype, D, L, B, saved):
+    """A bias shared by the batch with -Inf entries (as a mask folded into it has) in head 0, +Inf entries in one row of head 1
+    (the weights are their indicator, src/softmax.jl:74-75) and a row of nothing but -Inf in head 2 (NaN weights for every
+    key): gradients of q, k, v and the bias, from the kernels on copies of the bias and the one that walks the batch."""
+    rng = np.random.default_rng(L)
+    H = 4
+    q, k, v, dy = (round_to(rng.standard_normal((D * H, L, B)) * (0.4 if i < 2 else 1.0), dtype) for i in range(4))
+    bias = round_to(rng.standard_normal((L, L, H)) * 0.5, dtype)
+    bias[:, :, 0][rng.random((L, L)) < 0.3] = -np.inf
+    bias[0, :, 0] = 0.0
+    bias[[3, 60], 7, 1] = np.inf
+    bias[:, 9, 2] = -np.inf
+    D_ = lambda a: nn.DeviceArray.from_numpy(a, dtype)
+    args = [D_(a) for a in (q, k, v, bias)]
+    y, _ = nn.dot_product_attention(*args, nheads=H, return_weights=False, save_for_backward=saved)
+    got = [g.to_numpy() for g in nn.dot_product_attention_grad(D_(dy), *args, y=y, nheads=H)]
+    assert nn.last_attention_bwd_kernel() == "flash16"
+    x = np.einsum("hdjb,hdib->jihb", k.reshape(H, D, L, B).astype(np.float64), q.reshape(H, D, L, B).astype(np.float64)) / np.sqrt(D) + bias[..., None]
+    with np.errstate(invalid="ignore"):
+        m = x.max(axis=0, keepdims=True)
+        w = np.where(m == np.inf, (x == np.inf) * 1.0, np.exp(x - m))
+        w /= w.sum(axis=0, keepdims=True)
+    rows = lambda a: a.reshape(H, D, L, B).astype(np.float64)
+    dw = np.einsum("hdib,hdjb->jihb", rows(dy), rows(v))
+    ds = w * (dw - (w * dw).sum(axis=0, keepdims=True))
+    back = lambda s, e, a: np.einsum(s, e, rows(a)).reshape(D * H, L, B)
+    want = [back("jihb,hdjb->hdib", ds, k) / np.sqrt(D), back("jihb,hdib->hdjb", ds, q) / np.sqrt(D), back("jihb,hdib->hdjb", w, dy), ds.sum(axis=3)]
+    for g, r in zip(got, want):
+        g = g.reshape(r.shape)
+        assert np.array_equal(np.isnan(g), np.isnan(r)) and np.isnan(r).any()
+        fin = ~np.isnan(r)
+        assert np.abs(g[fin] - r[fin]).max() <= TOL[dtype] * np.abs(r[fin]).max()
