@@ -26,6 +26,7 @@ static int32_t validate_bwd(const mi_attn_bwd_desc *d, AttnBwdParams *out) {
     bp.mask_bits = nullptr;
     bp.drop_rows = bp.drop_keys = nullptr;
     bp.bias_rows = bp.bias_keys = nullptr;
+    bp.pair0 = bp.npairs = bp.dbias_in_dq = 0;
     bp.kv_len = nullptr;
     bp.dq_partial = nullptr;
     bp.dq_nsplit = 1;

@@ -81,11 +81,15 @@ static size_t lengths_bytes(const AttnParams &p) {
 // pairs of 333 x 333, head dim 64,
 // p = 0.1: 296 -> 114 us, with a key-padding mask 436 -> 114; 332 x 332: 123 -> 112; 64 pairs of 2048 x 2048, head dim
 // 128: 705 -> 659.)
+// Redrawn (DROP_REDRAW) where that is faster, rows on hash groups given: causal calls, whose kernels visit half the blocks
+// (16 x 4 pairs of 4096 x 4096, head dim 128: 1518 us with words, 1458 redrawn; 64 pairs of 2048 x 2048: 436 / 413), and
+// calls of less than 2^24 weights, bound by their launches (8 x 4 pairs of 512 x 512, head dim 64: 48 / 42; 128 x 128: 40 / 34).
 // Two bits a weight are O(L^2) bytes where the rest of the call is O(L): the words of as many (head, batch) pairs as
 // DROP_WORDS_MOST bytes hold are drawn at a time, and the gradient kernels run on those pairs before the next are drawn.  A
 // pair whose own words are more than that (65536 x 65536 is 1 GiB) has them redrawn by the kernels.
 static bool takes_drop_words(const AttnParams &p, bool lengths) {
     if (p.drop_thresh == 0 || p.bias) return false;
+    if ((p.Lkv & 3) == 0 && (p.causal || p.H * p.B * p.Lq * p.Lkv < (1 << 24))) return false;
     return !p.mask || flash_is_key_mask(p) || lengths || takes_mask_bits(p);   // what the lean kernels take
 }
 static int64_t pad128(int64_t n) { return (n + 127) / 128 * 128; }
@@ -137,8 +141,22 @@ __global__ __launch_bounds__(256) void drop_words_kernel(AttnParams p, int64_t p
 // Each batch element's workgroups read the same bias.  One small kernel writes two copies in the order the accumulators hold
 // the scores, so that a lane of the dQ (dK, dV) kernel reads its 16 entries of a block as 32 contiguous bytes, whatever the
 // alignment of the bias rows, and the kernels stay lean (two wavefronts per SIMD).
+// Calls of few scores: the dQ kernel's atomics cost less than the two launches more that the copies and the kernel of the
+// bias gradient are (measured, us, dQ kernel / apart; bias rows staged through LDS: 8 x 4 pairs of 128 x 128 47 / 52, 8 x 16
+// 56 / 66, 32 x 8 86 / 99, 8 x 2 of 512 x 512 108 / 111; the other way 8 x 4 of 384 x 384 119 / 90, and sooner where tiles
+// are ragged: 12 x 8 of 192 x 192 92 / 78, 8 x 128 of 64 x 64 105 / 88; unaligned rows: 8 x 4 of 99 x 99 50 / 57, of
+// 131 x 131 68 / 56).
+static bool bias_gradient_in_dq(const AttnParams &p) {
+    FlashArgs a;
+    a.p = p;
+    a.p.weights = nullptr;
+    flash_fill_vec_flags(a);
+    const bool whole = p.Lq % 128 == 0 && p.Lkv % 64 == 0;
+    return p.H * p.B * p.Lq * p.Lkv <= (!a.bias_lds || p.D > 128 ? 3 << 17 : whole ? 1 << 22 : 1 << 21);
+}
 static bool takes_bias_blocks(const AttnBwdParams &bp) {
     const AttnParams &p = bp.p;
+    if (p.bias && bias_gradient_in_dq(p)) return false;
     // entries of their own per key, query and head: what the kernel of the bias gradient takes too
     return p.bias && !p.mask && p.drop_thresh == 0 && bp.have_stats && p.D <= 128 && p.B > 1 && p.bias_strides[3] == 0 &&
            p.bias_strides[0] == 1 && (p.bias_strides[1] != 0 || p.Lq == 1) && (p.bias_strides[2] != 0 || p.H == 1) &&
@@ -238,21 +256,18 @@ static BwdScratch plan_scratch(const AttnBwdParams &bp, size_t room) {
     s.bits = mask_bits_bytes(p);
     s.partial = attention_bwd_flash16_dq_partial_bytes(bp);
     s.lengths = lengths_bytes(p);
-    const auto fits = [&](size_t more) { return s.total() <= room && more <= room - s.total(); };
-    if (p.drop_thresh && (p.Lkv & 3) != 0) {   // the one kind of call that does without lengths
-        const size_t n = s.lengths;
-        s.lengths = 0;
-        if (fits(n)) s.lengths = n;
-    }
+    const auto left = [&] { return s.total() < room ? room - s.total() : (size_t)0; };
     if (takes_drop_words(p, s.lengths != 0)) {
-        const size_t pair = sizeof(uint64_t) * (drop_rows_words(p) + drop_keys_words(p)), left = s.total() < room ? room - s.total() : 0;
-        const size_t pairs = (left < DROP_WORDS_MOST ? left : DROP_WORDS_MOST) / pair;
+        const size_t pair = sizeof(uint64_t) * (drop_rows_words(p) + drop_keys_words(p));
+        const size_t pairs = (left() < DROP_WORDS_MOST ? left() : DROP_WORDS_MOST) / pair;
         s.word_pairs = pairs < (size_t)(p.H * p.B) ? (int64_t)pairs : p.H * p.B;
         s.words = pair * (size_t)s.word_pairs;
     }
+    // the one kind of call that has lengths only along with words: its kernels without mask code cannot redraw
+    if (p.drop_thresh && (p.Lkv & 3) != 0 && !s.words) s.lengths = 0;
     if (takes_bias_blocks(bp)) {
         const size_t n = 2 * sizeof(uint16_t) * bias_copy_entries(p);
-        if (fits(n)) s.bias = n;
+        if (n <= left()) s.bias = n;
     }
     return s;
 }
@@ -265,6 +280,7 @@ int32_t launch_attention_bwd_flash16(const AttnBwdParams &bp_in, hipStream_t st)
     const BwdScratch scratch = plan_scratch(bp, bp.workspace_bytes);
     char *at = (char *)bp.workspace + scratch.stats;   // statistics that are not the caller's come first (validate_bwd)
     bp.dq_nsplit = attention_bwd_flash16_dq_nsplit(bp);
+    bp.dbias_in_dq = p.bias && bias_gradient_in_dq(p);
     if (scratch.bits) {
         const int64_t nqt = (p.Lq + 63) / 64, pad = mask_bits_lkv_pad(p), slices = mask_bits_slices(p);
         if (nqt > 65535 || slices > 65535) return mi_set_error(MI_ESHAPE, "attention gradient: mask packing supports at most 65535 query tiles and mask planes");

@@ -59,6 +59,29 @@ __device__ inline void attention_drop_factors_run4(const AttnParams &p, uint64_t
         for (int e = 0; e < 4; e++) f[e] = mi_dropout_keep(p.drop_key, i0 + 8 * g + e, p.drop_thresh) ? p.drop_scale : 0.0f;
     }
 }
+
+
+// The transposed case: a lane holds ONE key (kv; the four lanes of a quad hold kv = 4t .. 4t+3) and, in register
+// e of a run, query q0 + e.  Each lane hashes the group of query q0 + (lane & 3) and the quad exchanges the words,
+// so a quad still computes one hash per four weights.  f[e]: the factor of weight (kv, q0 + e).  Needs Lkv % 4 == 0.
+__device__ inline void attention_drop_factors_quad(const AttnParams &p, int64_t kv, int64_t q0, int64_t h, int64_t b, float (&f)[4]) {
+    const uint64_t col0 = (uint64_t)(kv + p.Lkv * (q0 + p.Lq * (h + p.H * b)));
+    {
+        const int sub = (int)(kv & 3);                         // == lane & 3 for the 32-aligned key blocks of the kernels
+        const uint64_t mine = mi_dropout_group_bits(p.drop_key, (col0 + (uint64_t)p.Lkv * (uint64_t)sub) >> 2);
+        const int lo = (int)(uint32_t)mine, hi = (int)(uint32_t)(mine >> 32);
+        // the word of quad lane E (quad_perm broadcast), of which a lane keeps its own 16-bit field
+#define MI_QUAD_FIELD(E)                                                                             \
+        {                                                                                            \
+            const int blo = __builtin_amdgcn_mov_dpp(lo, (E) * 0x55, 0xF, 0xF, true);                \
+            const int bhi = __builtin_amdgcn_mov_dpp(hi, (E) * 0x55, 0xF, 0xF, true);                \
+            const uint32_t word = (uint32_t)(sub < 2 ? blo : bhi);                                   \
+            f[E] = ((word >> (16 * (sub & 1))) & 0xFFFFu) >= p.drop_thresh ? p.drop_scale : 0.0f;    \
+        }
+        MI_QUAD_FIELD(0) MI_QUAD_FIELD(1) MI_QUAD_FIELD(2) MI_QUAD_FIELD(3)
+#undef MI_QUAD_FIELD
+    }
+}
 #endif
 
 // One backward call: the forward call it differentiates plus cotangents and gradient buffers.
@@ -87,6 +110,7 @@ struct AttnBwdParams {
     // the block; bias_keys [h][block of 32 queries][key][hh][16], likewise with queries.  null where the call has none or
     // the workspace no room for them
     const uint16_t *bias_rows, *bias_keys;
+    int32_t dbias_in_dq;   // few scores: the gradient of a bias shared by the batch stays with the dQ kernel
     // key-padding mask measured on the device: per (head, batch) pair [b * H + h] the context length, or 0 when the
     // mask of the pair is not a kept prefix; null when the call does not take that path
     const int32_t *kv_len;

@@ -172,7 +172,23 @@ def test_bias_gradient_from_the_mfma_kernels(nn, oracle, dtype, D, H, Lq, Lkv, b
     ("bf16", 64, 1, 1, 100, 3, None, True),         # one query
 ])
 def test_gradient_of_a_bias_shared_by_the_batch(nn, oracle, dtype, D, H, Lq, Lkv, B, mask_kind, saved):
-    """A bias per (key, query, head): its gradient is summed over the batch by a kernel of its own."""
+    """A bias per (key, query, head): its gradient is summed over the batch, by a kernel of its own or, in small calls, by the
+    dQ kernel."""
+    _run(nn, oracle, dtype, D * H, D * H, Lq, Lkv, (B,), H, bias_shape=(Lkv, Lq, H, 1), mask_kind=mask_kind, seed=Lq + Lkv + B,
+         scale=0.4, saved=saved, expect="flash16")
+
+
+@pytest.mark.parametrize("dtype,D,H,Lq,Lkv,B,mask_kind,saved", [
+    ("bf16", 64, 2, 128, 64, 260, None, True),      # whole tiles, rows that go through LDS
+    ("f16", 40, 2, 129, 65, 24, None, True),        # one row / key past a tile, features past the head dim
+    ("bf16", 128, 2, 161, 161, 8, "causal", True),  # tiles above the diagonal are left out
+    ("f16", 256, 1, 33, 300, 40, None, True),       # 256-wide tiles
+    ("bf16", 64, 8, 1, 100, 500, None, True),       # one query
+    ("bf16", 64, 3, 190, 210, 4, None, False),      # statistics in the workspace: no copies
+])
+def test_gradient_of_a_shared_bias_apart_from_dq(nn, oracle, dtype, D, H, Lq, Lkv, B, mask_kind, saved):
+    """The same at more scores than the dQ kernel keeps to itself (3 * 2^17, 2^21 or 2^22, by the bias rows' alignment)."""
+    assert Lq * Lkv * H * B > (4 << 20 if Lq % 128 == 0 else 3 << 17)
     _run(nn, oracle, dtype, D * H, D * H, Lq, Lkv, (B,), H, bias_shape=(Lkv, Lq, H, 1), mask_kind=mask_kind, seed=Lq + Lkv + B,
          scale=0.4, saved=saved, expect="flash16")
 
@@ -675,14 +691,14 @@ def test_weights_of_the_dropout_gradient_keep_float32_accuracy(nn, oracle, Lkv):
 
 
 @pytest.mark.parametrize("kind,D,Lq,Lkv", [
-    ("dropout", 64, 130, 132),       # rows on hash groups: one hash per four weights, exchanged by the quads of lanes
-    ("dropout", 64, 131, 133),       # rows at any place within a group
-    ("dropout causal", 128, 200, 200),
-    ("dropout keys", 64, 150, 260),  # the context lengths find room in the workspace, the keep words do not
-    ("dropout keys", 64, 150, 261),  # neither does
-    ("dropout dense", 64, 100, 128),
-    ("bias", 64, 197, 197),
-    ("bias", 128, 64, 96),
+    ("dropout", 64, 1370, 1372),       # rows on hash groups: one hash per four weights, exchanged by the quads of lanes
+    ("dropout", 64, 131, 133),         # rows at any place within a group
+    ("dropout causal", 128, 201, 201),
+    ("dropout keys", 64, 1500, 1260),  # the context lengths find room in the workspace, the keep words do not
+    ("dropout keys", 64, 150, 261),    # neither does
+    ("dropout dense", 64, 1000, 1904),
+    ("bias", 64, 211, 211),
+    ("bias", 128, 704, 704),
 ])
 def test_gradient_without_the_workspace_it_is_faster_with(nn, monkeypatch, kind, D, Lq, Lkv):
     """Keep words and copies of a shared bias are there to save time: a caller with saved statistics that gives no workspace
@@ -728,7 +744,7 @@ def test_gradient_without_the_workspace_it_is_faster_with(nn, monkeypatch, kind,
 
 
 @pytest.mark.parametrize("pairs", [1, 2, 4])
-@pytest.mark.parametrize("mask_kind,Lq,Lkv", [(None, 130, 133), ("causal", 191, 191), ("lengths", 70, 261), ("random", 100, 128)])
+@pytest.mark.parametrize("mask_kind,Lq,Lkv", [(None, 130, 133), ("causal", 191, 191), ("lengths", 70, 261), ("random", 1024, 2048)])
 def test_dropout_gradient_in_pieces_of_its_pairs(nn, monkeypatch, mask_kind, Lq, Lkv, pairs):
     """A workspace that holds the keep words of some (head, batch) pairs at a time: the pieces give the bits that all pairs
     at once give."""
@@ -824,7 +840,8 @@ def test_shared_bias_with_the_key_range_in_pieces(nn, oracle):
         _run(nn, oracle, dtype, 128, 128, 64, Lkv, (3,), 2, bias_shape=(Lkv, 64, 2, 1), seed=Lkv, scale=0.4, saved=True, expect="flash16")
 
 
-@pytest.mark.parametrize("dtype,D,L,B,saved", [("bf16", 64, 197, 3, True), ("f16", 128, 130, 2, True), ("bf16", 64, 140, 3, False), ("bf16", 136, 70, 2, True)])
+@pytest.mark.parametrize("dtype,D,L,B,saved", [("bf16", 64, 197, 3, True), ("f16", 128, 130, 6, True), ("bf16", 64, 187, 3, False), ("bf16", 136, 150, 5, True),
+                                                ("bf16", 64, 70, 3, True)])
 def test_infinite_entries_of_a_shared_bias(nn, oracle, dtype, D, L, B, saved):
     """A bias shared by the batch with -Inf entries (as a mask folded into it has) in head 0, +Inf entries in one row of head 1
     (the weights are their indicator, src/softmax.jl:74-75) and a row of nothing but -Inf in head 2 (NaN weights for every
