@@ -1,9 +1,10 @@
 // Tiled strided batched GEMM for Float32 on the matrix cores: the fast path of mi_batched_gemm, operands
 // moved in 16-byte pieces (of any alignment in the kernels on bf16 planes).  Stands where the
 // reference calls sgemm per slice (src/gemm.jl:141-149, reached through _batched_gemm!,
-// src/batched/batchedmul.jl:298).  Products and sums are true fp32.
+// src/batched/batchedmul.jl:298).  Sums are Float32; products run on three bf16 planes per operand (gemm32s_kernel
+// below), or, where MI355ATTN_F32_MFMA asks for it, on the Float32 matrix instruction (gemm32_kernel, aligned operands).
 //
-// Workgroup = 4 wavefronts (2 x 2), output tile 128 (m) x 128 (n), 64 x 64 per wavefront as 2 x 2 MFMA
+// gemm32_kernel: workgroup = 4 wavefronts (2 x 2), output tile 128 (m) x 128 (n), 64 x 64 per wavefront as 2 x 2 MFMA
 // blocks; k advances 16 per stage through double-buffered LDS tiles kept as [k][row] (row contiguous),
 // so an MFMA operand (one float per lane: row = lane % 32, k = 2*step + lane / 32) is a conflict-free
 // 4-byte read whatever the memory layout of the matrix.  As in the other GEMM kernels the MFMA runs on
