@@ -322,6 +322,14 @@ int32_t mi_batched_gemm(int32_t dtype, char transA, char transB, int64_t m, int6
                         int64_t ldb, int64_t strideB, float beta, void *C, int64_t ldc,
                         int64_t strideC, int64_t batch, mi_stream stream);
 
+/* C = alpha * sum over b of op(A[:,:,b]) * op(B[:,:,b]) + beta * C: the gradient of an operand that every slice of a
+ * batched product shared (the sum in the pullback at src/batched/batchedmul.jl:96-110).  Float32 (MI_F32) only; arguments
+ * as above, without a batch stride for C. */
+int32_t mi_batched_gemm_sum(int32_t dtype, char transA, char transB, int64_t m, int64_t n, int64_t k,
+                            float alpha, const void *A, int64_t lda, int64_t strideA, const void *B,
+                            int64_t ldb, int64_t strideB, float beta, void *C, int64_t ldc,
+                            int64_t batch, mi_stream stream);
+
 /* ComplexF32 batched_mul: C = alpha * op(A) * op(B) + beta * C per batch slice, complex alpha and beta.
  * Arrays hold interleaved (re, im) Float32 pairs, as Julia stores ComplexF32.  Every operand is given
  * by the ELEMENT strides of its (row, column, batch) indices AFTER op: op(A) is m x k, op(B) is k x n;

@@ -2,8 +2,8 @@
 // Device replacement for the reference's batched_gemm! (src/gemm.jl:89-188), reached
 // through the _batched_gemm! hook (src/batched/batchedmul.jl:298).  Column-major.
 //
-// The kernels of batched_gemm16.hip and batched_gemm32.hip take nearly every product; the one here keeps products of
-// less than 64 x 64 elements, leading dimensions below 16 bytes and slices beyond 2 GiB.
+// The kernels of batched_gemm16.hip, batched_gemm32.hip and batched_gemm32_waves.hip take nearly every product; the one here
+// keeps 16-bit products of less than 64 x 64 elements or with leading dimensions below 16 bytes, and slices beyond 2 GiB.
 //
 // Workgroup = 4 wavefronts, output tile 64 (m) x 64 (n), each wavefront one 32x32 block.
 // The MFMA is issued on the transposed problem (rows = n, columns = m) so that a lane's
@@ -19,7 +19,10 @@ int32_t launch_batched_gemm16(int32_t dtype, int transA, int transB, int64_t m, 
 
 // tiled Float32 fast path (batched_gemm32.hip)
 bool batched_gemm32_supports(int32_t dtype, int transA, int transB, int64_t m, int64_t n, int64_t k, const void *A, int64_t lda,
-                             int64_t sA, const void *B, int64_t ldb, int64_t sB);
+                             int64_t sA, const void *B, int64_t ldb, int64_t sB, int64_t batch);
+int32_t launch_batched_gemm32_sum(int transA, int transB, int64_t m, int64_t n, int64_t k, float alpha, const void *A, int64_t lda,
+                                  int64_t sA, const void *B, int64_t ldb, int64_t sB, float beta, void *C, int64_t ldc, int64_t batch,
+                                  hipStream_t st);
 int32_t launch_batched_gemm32(int transA, int transB, int64_t m, int64_t n, int64_t k, float alpha, const void *A, int64_t lda,
                               int64_t sA, const void *B, int64_t ldb, int64_t sB, float beta, void *C, int64_t ldc, int64_t sC,
                               int64_t batch, hipStream_t st);
@@ -230,9 +233,32 @@ MI_API int32_t mi_batched_gemm(int32_t dtype, char transA, char transB, int64_t 
     hipStream_t st = (hipStream_t)s;
     if (batched_gemm16_supports(dtype, ta, tb, m, n, k, lda, ldb))
         return launch_batched_gemm16(dtype, ta, tb, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, strideC, batch, st);
-    if (batched_gemm32_supports(dtype, ta, tb, m, n, k, A, lda, strideA, B, ldb, strideB))
+    if (batched_gemm32_supports(dtype, ta, tb, m, n, k, A, lda, strideA, B, ldb, strideB, batch))
         return launch_batched_gemm32(ta, tb, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, strideC, batch, st);
     if (dtype == MI_F32) return launch<F32>(g, batch, st);
     if (dtype == MI_F16) return launch<F16>(g, batch, st);
     return launch<BF16>(g, batch, st);
+}
+
+MI_API int32_t mi_batched_gemm_sum(int32_t dtype, char transA, char transB, int64_t m, int64_t n, int64_t k, float alpha,
+                                   const void *A, int64_t lda, int64_t strideA, const void *B, int64_t ldb, int64_t strideB,
+                                   float beta, void *C, int64_t ldc, int64_t batch, mi_stream s) {
+    if (dtype != MI_F32) return mi_set_error(MI_EDTYPE, "mi_batched_gemm_sum: Float32 only (dtype %d)", dtype);
+    const int ta = trans_flag(transA), tb = trans_flag(transB);
+    // the argument rules of mi_batched_gemm, on an empty product
+    const int32_t rc = mi_batched_gemm(dtype, transA, transB, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, 0, 0, s);
+    if (rc != MI_OK) return rc;
+    if (batch < 0) return mi_set_error(MI_ESHAPE, "mi_batched_gemm_sum: negative dimension");
+    if (m == 0 || n == 0) return MI_OK;
+    if (k == 0 || batch == 0)
+        return mi_batched_gemm(dtype, transA, transB, m, n, 0, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, 0, 1, s);
+    if (!C || !A || !B) return mi_set_error(MI_EINVAL, "mi_batched_gemm_sum: null pointer");
+    if (batched_gemm32_supports(dtype, ta, tb, m, n, k, A, lda, strideA, B, ldb, strideB, 1))
+        return launch_batched_gemm32_sum(ta, tb, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, batch, (hipStream_t)s);
+    for (int64_t b = 0; b < batch; b++) {
+        const int32_t rb = mi_batched_gemm(dtype, transA, transB, m, n, k, alpha, (const float *)A + b * strideA, lda, 0, (const float *)B + b * strideB,
+                                           ldb, 0, b == 0 ? beta : 1.0f, C, ldc, 0, 1, s);
+        if (rb != MI_OK) return rb;
+    }
+    return MI_OK;
 }

@@ -1,5 +1,6 @@
-// Tiled strided batched GEMM for Float32 on the matrix cores: the fast path of mi_batched_gemm, operands
-// moved in 16-byte pieces (of any alignment in the kernels on bf16 planes).  Stands where the
+// Strided batched GEMM for Float32 on the matrix cores: the fast path of mi_batched_gemm, operands
+// moved in 16-byte pieces (of any alignment in the kernels on bf16 planes).  Products that would leave these tiles empty or
+// too few run in batched_gemm32_waves.hip.  Stands where the
 // reference calls sgemm per slice (src/gemm.jl:141-149, reached through _batched_gemm!,
 // src/batched/batchedmul.jl:298).  Sums are Float32; products run on three bf16 planes per operand (gemm32s_kernel
 // below), or, where MI355ATTN_F32_MFMA asks for it, on the Float32 matrix instruction (gemm32_kernel, aligned operands).
@@ -12,6 +13,13 @@
 #include "common.h"
 #include <cstdlib>
 #include <type_traits>
+
+// a wavefront per tile, no LDS between operands and products (batched_gemm32_waves.hip)
+bool gemm32_waves_supports(int transA, int transB, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, int64_t batch);
+double gemm32_waves_estimate(int64_t m, int64_t n, int64_t k, int64_t slices, int64_t batch);
+int32_t launch_gemm32_waves(int transA, int transB, int64_t m, int64_t n, int64_t k, float alpha, const void *A, int64_t lda,
+                            int64_t sA, const void *B, int64_t ldb, int64_t sB, float beta, void *C, int64_t ldc, int64_t sC,
+                            int64_t slices, int64_t batch, hipStream_t st);
 
 namespace {
 
@@ -324,10 +332,10 @@ __global__ __launch_bounds__(ShapeS<LARGE>::THREADS, LARGE ? 1 : 2) void gemm32s
     constexpr int TILE3B = S::TILE3B, BM = S::BM, BNB = S::BNB;
     extern __shared__ __attribute__((aligned(16))) unsigned char gemm_smem[];   // A and B tiles, two buffers each
     const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)gemm_smem;
-    // which tile: with the large tiles, an order in which the tiles in flight on one die share operands (a few per cent
-    // on k >= 1024; the small tiles' calls are bound by their output and lose 1 % to it)
+    // tiles in an order in which those in flight on one die share operands and cut cache lines of C: a few per cent on
+    // k >= 1024 with the large tiles; 333 x 517 x 77, 96 slices, with the small ones 45.3 -> 40.8 us, 384 x 512 x 80 36.4 -> 33.0
     const int64_t id = blockIdx.x + (int64_t)gridDim.x * (blockIdx.y + (int64_t)gridDim.y * blockIdx.z);
-    const MiTile tile = LARGE ? mi_gemm_tile_order(id, gridDim.x, gridDim.y, gridDim.z) : MiTile{blockIdx.x, blockIdx.y, blockIdx.z};
+    const MiTile tile = mi_gemm_tile_order(id, gridDim.x, gridDim.y, gridDim.z);
     const int64_t bz = tile.batch;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave & 1, wn = wave >> 1;
     const int r = lane & 31, hh = lane >> 5;
@@ -513,11 +521,10 @@ static bool aligned_pieces(int transA, int transB, int64_t m, int64_t n, int64_t
     return ((((uintptr_t)A) | ((uintptr_t)B)) & 15) == 0 && ((lda | ldb | sA | sB | (transA ? k : m) | (transB ? n : k)) & 3) == 0;
 }
 
-// true when the tiled kernels take the product.  Operands that do not come in aligned pieces need slices that 32-bit byte
-// offsets address and that hold a piece, and the bf16 planes.
-bool batched_gemm32_supports(int32_t dtype, int transA, int transB, int64_t m, int64_t n, int64_t k, const void *A, int64_t lda,
-                             int64_t sA, const void *B, int64_t ldb, int64_t sB) {
-    if (dtype != MI_F32) return false;
+// true when the tiles of this file take the product.  Operands that do not come in aligned pieces need slices that 32-bit
+// byte offsets address and that hold a piece, and the bf16 planes.
+static bool tiles_support(int transA, int transB, int64_t m, int64_t n, int64_t k, const void *A, int64_t lda, int64_t sA, const void *B,
+                          int64_t ldb, int64_t sB) {
     if (k < 1 || m * n < 64 * 64) return false;   // tiny products: the small-tile kernel wastes less
     if ((n + TN - 1) / TN > 65535) return false;
     if (aligned_pieces(transA, transB, m, n, k, A, lda, sA, B, ldb, sB)) return true;
@@ -526,11 +533,41 @@ bool batched_gemm32_supports(int32_t dtype, int transA, int transB, int64_t m, i
     // leading dimensions of at least a piece: only the last k or row of a slice can hold a piece that ends past it
     return lda >= 4 && ldb >= 4 && extA >= 4 && extB >= 4 && extA * 4 < 2147483647LL && extB * 4 < 2147483647LL;
 }
+static bool waves_support(int transA, int transB, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, int64_t batch) {
+    return k >= 1 && !exact_instruction_wanted() && gemm32_waves_supports(transA, transB, m, n, k, lda, ldb, batch);
+}
+
+bool batched_gemm32_supports(int32_t dtype, int transA, int transB, int64_t m, int64_t n, int64_t k, const void *A, int64_t lda,
+                             int64_t sA, const void *B, int64_t ldb, int64_t sB, int64_t batch) {
+    if (dtype != MI_F32) return false;
+    return waves_support(transA, transB, m, n, k, lda, ldb, batch) || tiles_support(transA, transB, m, n, k, A, lda, sA, B, ldb, sB);
+}
+
+// The large tile where the share of its slots that does useful work, counting padded rows and columns and the last round of
+// workgroups (one per CU; three of the small ones), times its higher rate once k is long enough to pay for its prologue
+// (2047^3 x 8: 188 against 163 TFLOP/s; 1000 x 1000 x 130: level) is the larger.
+static bool large_tiles(int64_t m, int64_t n, int64_t k, int64_t nb) {
+    const auto useful = [&](int64_t tile, int64_t slots) {
+        const int64_t tiles = ((m + tile - 1) / tile) * ((n + tile - 1) / tile) * nb;
+        return (double)(m * n * nb) / ((double)((tiles + slots - 1) / slots * slots) * (double)(tile * tile));
+    };
+    return m >= 256 && n >= 256 && k >= 128 && (k >= 512 ? 1.15 : 1.0) * useful(256, 256) > useful(128, 768);
+}
+// Microseconds on the tiles of this file, fitted like those of batched_gemm32_waves.hip (mean deviation 10 %): the chain of
+// a workgroup's steps, or the steps of the fullest CU.
+static double tiles_estimate(int64_t m, int64_t n, int64_t k, int64_t nb) {
+    const double steps = (double)((k + KC - 1) / KC);
+    const double per_cu = ceil((double)((m + TM - 1) / TM) * (double)((n + TN - 1) / TN) * (double)nb / 256.0);
+    return 4.0 + fmax(1.18 * steps + 1.6, per_cu * (0.72 * steps + 2.4)) * (large_tiles(m, n, k, nb) ? 0.87 : 1.0);
+}
 
 int32_t launch_batched_gemm32(int transA, int transB, int64_t m, int64_t n, int64_t k, float alpha, const void *A, int64_t lda,
                               int64_t sA, const void *B, int64_t ldb, int64_t sB, float beta, void *C, int64_t ldc, int64_t sC,
                               int64_t batch, hipStream_t st) {
     const bool a_rm = !transA, b_rm = transB != 0;
+    if (waves_support(transA, transB, m, n, k, lda, ldb, batch) &&
+        (!tiles_support(transA, transB, m, n, k, A, lda, sA, B, ldb, sB) || gemm32_waves_estimate(m, n, k, 1, batch) < tiles_estimate(m, n, k, batch)))
+        return launch_gemm32_waves(transA, transB, m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, 1, batch, st);
     for (int64_t b0 = 0; b0 < batch; b0 += 65535) {   // gridDim.z is limited to 65535: issue the batch in slabs
         const int64_t nb = batch - b0 < 65535 ? batch - b0 : 65535;
         Gemm32Args g = {(const float *)A + b0 * sA, (const float *)B + b0 * sB, (float *)C + b0 * sC,
@@ -542,20 +579,30 @@ int32_t launch_batched_gemm32(int transA, int transB, int64_t m, int64_t n, int6
             else if (b_rm) hipLaunchKernelGGL((gemm32_kernel<false, true>), grid, dim3(256), 0, st, g);
             else hipLaunchKernelGGL((gemm32_kernel<false, false>), grid, dim3(256), 0, st, g);
         } else {
-            // The large tile where the share of its slots that does useful work, counting padded rows and columns and the
-            // last round of workgroups (one per CU; three of the small ones), times its higher rate once k is long enough
-            // to pay for its prologue (2047^3 x 8: 188 against 163 TFLOP/s; 1000 x 1000 x 130: level) is the larger.
-            const auto useful = [&](int64_t tile, int64_t slots) {
-                const int64_t tiles = ((m + tile - 1) / tile) * ((n + tile - 1) / tile) * nb;
-                return (double)(m * n * nb) / ((double)((tiles + slots - 1) / slots * slots) * (double)(tile * tile));
-            };
-            const bool large = m >= 256 && n >= 256 && k >= 128 && (k >= 512 ? 1.15 : 1.0) * useful(256, 256) > useful(128, 768);
+            const bool large = large_tiles(m, n, k, nb);
             const bool aligned = aligned_pieces(transA, transB, m, n, k, g.A, lda, sA, g.B, ldb, sB);
             const int32_t rc = aligned ? (large ? launch_planes_l<true, false>(g, a_rm, b_rm, nb, st) : launch_planes_l<false, false>(g, a_rm, b_rm, nb, st))
                                        : (large ? launch_planes_l<true, true>(g, a_rm, b_rm, nb, st) : launch_planes_l<false, true>(g, a_rm, b_rm, nb, st));
             if (rc != MI_OK) return rc;
         }
         MI_LAUNCH_CHECK();
+    }
+    return MI_OK;
+}
+
+// C = alpha * sum over the batch of op(A) op(B) + beta*C: one launch that walks the slices, or a product per slice where
+// these fill the chip by themselves
+int32_t launch_batched_gemm32_sum(int transA, int transB, int64_t m, int64_t n, int64_t k, float alpha, const void *A, int64_t lda,
+                                  int64_t sA, const void *B, int64_t ldb, int64_t sB, float beta, void *C, int64_t ldc, int64_t batch,
+                                  hipStream_t st) {
+    const bool tiles = tiles_support(transA, transB, m, n, k, A, lda, sA, B, ldb, sB);
+    const double apart = (double)batch * fmin(gemm32_waves_estimate(m, n, k, 1, 1), tiles ? tiles_estimate(m, n, k, 1) : 1e30);
+    if (batch <= 2147483647LL / ((k + 15) / 16) && waves_support(transA, transB, m, n, k, lda, ldb, 1) && gemm32_waves_estimate(m, n, k, batch, 1) < apart)
+        return launch_gemm32_waves(transA, transB, m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, 0, batch, 1, st);
+    for (int64_t b = 0; b < batch; b++) {
+        const int32_t rc = launch_batched_gemm32(transA, transB, m, n, k, alpha, (const float *)A + b * sA, lda, sA, (const float *)B + b * sB, ldb, sB,
+                                                 b == 0 ? beta : 1.0f, C, ldc, 0, 1, st);
+        if (rc != MI_OK) return rc;
     }
     return MI_OK;
 }

@@ -87,6 +87,8 @@ SIGNATURES = {
                                 c_vp, c_i64, c_i64, c_f32, c_vp, c_i64, c_i64, c_i64, c_vp]),
     "mi_dropout_dims": (c_i32, [c_i32, c_vp, c_vp, c_i32, ctypes.POINTER(c_i64), ctypes.c_uint32, c_f32, c_u64, c_vp]),
     "mi_logsumexp_bwd": (c_i32, [c_i32, c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_i64, c_vp]),
+    "mi_batched_gemm_sum": (c_i32, [c_i32, ctypes.c_char, ctypes.c_char, c_i64, c_i64, c_i64, c_f32, c_vp, c_i64, c_i64,
+                                    c_vp, c_i64, c_i64, c_f32, c_vp, c_i64, c_i64, c_vp]),
     "mi_batched_gemm_f64": (c_i32, [ctypes.c_char, ctypes.c_char, c_i64, c_i64, c_i64, ctypes.c_double, c_vp, c_i64, c_i64,
                                     c_vp, c_i64, c_i64, ctypes.c_double, c_vp, c_i64, c_i64, c_i64, c_vp]),
     "mi_batched_mul_generic": (c_i32, [c_i32, c_i32, c_i32, c_i64, c_i64, c_i64, ctypes.c_double, ctypes.c_double, c_vp, c_i64, c_i64, c_i64,

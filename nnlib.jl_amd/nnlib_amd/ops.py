@@ -760,10 +760,24 @@ def batched_mul_pullback(A, B, dC):
     def summed(X, make):
         if X.dims[2] != 1 or nb == 1:
             return make(None)
-        # sum over slices: accumulate slice by slice into one (m, n, 1) result with beta = 1
+        # sum over slices: one call for Float32, else slice by slice into one (m, n, 1) result with beta = 1
+        out = make("sum")
+        if out is not None:
+            return out
         out = DeviceArray.zeros(X.dims, X.dtype)
         for b in range(nb):
             make((out, b))
+        return out
+
+    def sum_of(X, P, Q):
+        if not (P.dtype == Q.dtype == X.dtype == "f32" and _is_blas_layout(P) and _is_blas_layout(Q)) or X.dims[:2] != (P.dims[0], Q.dims[1]) or P.dims[1] != Q.dims[0]:
+            return None
+        tP, ldp, sP = _blas_layout(P, "A")
+        tQ, ldq, sQ = _blas_layout(Q, "B")
+        out = DeviceArray.empty(X.dims, X.dtype)
+        _lib.check(_lib.load().mi_batched_gemm_sum(out.code, tP, tQ, P.dims[0], Q.dims[1], P.dims[1], 1.0, P.ptr, ldp, sP if P.dims[2] > 1 else 0,
+                                                   Q.ptr, ldq, sQ if Q.dims[2] > 1 else 0, 0.0, out.ptr, max(out.dims[0], 1), nb, _stream()),
+                   DimensionMismatch)
         return out
 
     def slice3(X, b):
@@ -772,12 +786,16 @@ def batched_mul_pullback(A, B, dC):
     def dA_of(acc):
         if acc is None:
             return batched_mul(dC, batched_adjoint(B))
+        if acc == "sum":
+            return sum_of(A, dC, batched_adjoint(B))
         out, b = acc
         return batched_mul_(out, slice3(dC, b), batched_adjoint(slice3(B, b)), 1.0, 1.0)
 
     def dB_of(acc):
         if acc is None:
             return batched_mul(batched_adjoint(A), dC)
+        if acc == "sum":
+            return sum_of(B, batched_adjoint(A), dC)
         out, b = acc
         return batched_mul_(out, batched_adjoint(slice3(A, b)), slice3(dC, b), 1.0, 1.0)
 

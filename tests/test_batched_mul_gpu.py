@@ -559,3 +559,52 @@ def test_large_tiles(nn, dtype, ta, tb, m, n, k, nb):
     T = nn.batched_transpose
     nn.batched_mul_(dC, T(dA) if ta else dA, T(dB) if tb else dB, 0.5, 2.0)
     assert close(dC.to_numpy(), 0.5 * bmm(A, B, ta, tb) + 2.0 * C0, dtype)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("m,n,k,batch", [(1, 1, 1, 1), (1, 33, 17, 3), (33, 31, 16, 2), (32, 32, 15, 2), (31, 97, 160, 5), (65, 63, 47, 4), (64, 96, 129, 2),
+                                         (20, 40, 840, 2), (16, 17, 1024, 1), (130, 70, 333, 41), (101, 650, 20, 64), (64, 64, 512, 200)])
+def test_float32_products_of_few_or_narrow_tiles(nn, ta, tb, m, n, k, batch):
+    """Every variant of the kernel that gives a wavefront its own tile: one block of 32 x 32 and four, k in one piece and in
+    four and eight, remainders of rows, columns and k, strided columns, a value beyond the planes' range in the last k.
+    Sums of k Float32 products err by a few 2^-24 sqrt(k) of sum |a||b|."""
+    rng = np.random.default_rng(m + 31 * n + k)
+    A, B = rng.standard_normal((batch, m, k)).astype(np.float32), rng.standard_normal((batch, k, n)).astype(np.float32)
+    A[-1, -1, -1] = 1e-36
+    A[0, 0, -1] = 3.4e38                  # products and their sums stay finite
+    B[0, -1] *= 1e-3
+    dev = lambda x, t: nn.DeviceArray.from_numpy(np.ascontiguousarray(x.transpose(2, 1, 0) if t else x.transpose(1, 2, 0)), "f32")
+    da, db = dev(A, ta), dev(B, tb)
+    c = rng.standard_normal((batch, n, m + 3)).astype(np.float32)
+    C = nn.DeviceArray(nn.DeviceArray.from_numpy(c.reshape(-1)).storage, (m, n, batch), "f32", (1, m + 3, n * (m + 3)), 1)
+    nn.batched_mul_(C, nn.batched_transpose(da) if ta else da, nn.batched_transpose(db) if tb else db, 0.5, 2.0)
+    got = C.storage.cpu().numpy()
+    ref, scale = 0.5 * (A.astype(np.float64) @ B.astype(np.float64)), 0.5 * (np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64))
+    flat = c.reshape(-1).astype(np.float64).copy()
+    at = np.arange(batch)[:, None, None] * (n * (m + 3)) + np.arange(n)[None, None, :] * (m + 3) + np.arange(m)[None, :, None] + 1
+    bound = np.zeros_like(flat)
+    bound[at] = 4 * 2.0 ** -24 * (np.sqrt(k) * scale + np.abs(2.0 * flat[at]) + np.abs(ref))
+    flat[at] = ref + 2.0 * flat[at]
+    assert (np.abs(got - flat) <= bound).all()      # nothing outside C changes
+    summed = nn.batched_mul(nn.batched_transpose(da) if ta else da, nn.batched_transpose(db) if tb else db).to_numpy().sum(axis=2, dtype=np.float64)
+    lib, out = nn._lib.load(), nn.DeviceArray.from_numpy(np.ones((m, n), np.float32))
+    nn._lib.check(lib.mi_batched_gemm_sum(out.code, b"T" if ta else b"N", b"T" if tb else b"N", m, n, k, 1.0, da.ptr, k if ta else m, m * k, db.ptr,
+                                          n if tb else k, n * k, 3.0, out.ptr, m, batch, 0))
+    total = np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64)
+    assert (np.abs(out.to_numpy() - 3.0 - summed) <= 4 * 2.0 ** -24 * (np.sqrt(k * batch) * total.sum(axis=0) + 3.0)).all()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("m,n,k,nb", [(46, 16, 41, 28), (256, 256, 512, 3), (5, 3, 1, 1000)])
+def test_pullback_of_a_shared_operand(nn, dtype, m, n, k, nb):
+    """The gradient of an operand with batch extent 1 is the sum over the slices: dA = sum dC B', dB = sum A' dC."""
+    rng = np.random.default_rng(m + n)
+    A, B, dC = (round_to(rng.standard_normal(s).astype(np.float32), dtype) for s in ((m, k, nb), (k, n, nb), (m, n, nb)))
+    D = lambda x: nn.DeviceArray.from_numpy(x, dtype)
+    dA, dB = nn.batched_mul_pullback(D(A[:, :, :1]), D(B), D(dC))
+    ref = np.einsum("mnb,knb->mk", dC.astype(np.float64), B.astype(np.float64))
+    tol = TOL[dtype] if dtype == "f32" else TOL[dtype] * np.sqrt(nb)   # 16 bits: rounded once per slice
+    assert dA.dims == (m, k, 1) and np.abs(dA.to_numpy()[:, :, 0] - ref).max() <= tol * np.abs(ref).max()
+    _, dB = nn.batched_mul_pullback(D(A), D(B[:, :, :1]), D(dC))
+    ref = np.einsum("mkb,mnb->kn", A.astype(np.float64), dC.astype(np.float64))
+    assert dB.dims == (k, n, 1) and np.abs(dB.to_numpy()[:, :, 0] - ref).max() <= tol * np.abs(ref).max()
