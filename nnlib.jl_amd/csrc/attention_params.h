@@ -21,7 +21,7 @@ struct AttnParams {
     // none) where the key-split plan would ask for more than the built-in workspace holds
     bool keep_pipelined = false;
     // and the same for the packed dense mask of the pipelined kernel: a caller whose workspace cannot hold it gets the
-    // general kernel, which reads the mask as it is
+    // general kernel, which reads the mask as it is, or one workgroup per query tile for a bias and few keys
     bool lean_workspace = false;
     // gradient kernels: the head dim the logits are scaled by (1 / sqrt) when it is not D, i.e. when q and k arrive
     // zero-padded to the head dim of v (attention_backward.hip pads the narrower of the two); 0: D

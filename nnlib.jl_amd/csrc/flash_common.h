@@ -67,7 +67,14 @@ __device__ inline void flash_zero_stats_padding(const AttnParams &p, int64_t b, 
 inline int flash_pick_nsplit(const AttnParams &p, int bm) {
     if (p.weights || !p.out || p.stats) return 1;           // weights need the global maximum up front; saved statistics are per whole row
     const int64_t wgs = ((p.Lq + bm - 1) / bm) * p.H * p.B;
-    if (wgs >= 512 || p.Lkv < 2048) return 1;
+    if (wgs >= 512) return 1;
+    if (p.Lkv < 2048) {
+        // Calls with a bias stay on the general kernel, where a workgroup that is alone on its CU takes 2.6 us per 64 keys: a
+        // few of them are worth the merge (5 us) from 768 keys on, at least 256 a piece (8 workgroups x 1511 keys: 64 -> 20 us)
+        if (p.dtype == MI_F32 || !p.bias || p.lean_workspace || wgs > 128 || p.Lkv < 768) return 1;
+        const int64_t n = 512 / wgs, most = p.Lkv / 256;
+        return (int)(n < most ? n : most);
+    }
     // aim at one resident round: two workgroups per CU on 256 CUs (measured best on the f16 cross-attention case)
     int64_t n = (512 + wgs - 1) / wgs;
     const int64_t max_by_len = p.Lkv / 512;                 // at least 512 keys per piece
@@ -89,11 +96,13 @@ enum { PHASE_ONLINE = 0, PHASE_STATS = 1, PHASE_FINAL = 2 };
 // EXTRAS_MASKTILE: no bias and a dense mask whose tiles can be staged through LDS: raw dot products as with
 // EXTRAS_NONE, dropped entries set to -Inf from the staged mask bytes; only the mask half of the staging is allocated,
 // which keeps two workgroups per CU.
-enum { EXTRAS_NONE = 0, EXTRAS_DIRECT = 1, EXTRAS_STAGED = 2, EXTRAS_KEYMASK = 3, EXTRAS_MASKTILE = 4 };
+// EXTRAS_ROWS (general 16-bit kernel): bias / mask rows of any alignment with unit key stride, through registers into the
+// LDS tiles of EXTRAS_STAGED (FlashRows).
+enum { EXTRAS_NONE = 0, EXTRAS_DIRECT = 1, EXTRAS_STAGED = 2, EXTRAS_KEYMASK = 3, EXTRAS_MASKTILE = 4, EXTRAS_ROWS = 6 };
 // variants that copy bias / mask tiles through LDS (FlashStaged), and the LDS bytes per wavefront they need
 constexpr bool flash_uses_staging(int extras) { return extras == EXTRAS_STAGED || extras == EXTRAS_MASKTILE; }
 // true when the accumulators hold the reference's logits in natural units (bias added) rather than raw dot products
-constexpr bool flash_natural_units(int extras) { return extras == EXTRAS_DIRECT || extras == EXTRAS_STAGED; }
+constexpr bool flash_natural_units(int extras) { return extras == EXTRAS_DIRECT || extras == EXTRAS_STAGED || extras == EXTRAS_ROWS; }
 // any mask without bias that does not depend on the query (a key-padding mask), whatever its strides: what the
 // device-side measurement of context lengths (FlashArgs::kv_len) applies to
 inline bool flash_is_query_independent_mask(const AttnParams &p) {
@@ -276,11 +285,6 @@ struct FlashStaged {
     }
 };
 
-// On entry s[qb][kb] holds raw dot products k.q of tile rows [j0, j0+64) for the wavefront's query
-// blocks; on exit it holds exp2(x - m) (ONLINE / STATS) or the final normalised weights (FINAL),
-// with m, l (and, ONLINE only, the output accumulators o) updated.
-//   T      element traits of the bias array
-//   NDV    number of 32-row blocks of the output accumulator
 // Orders a wavefront's LDS stores and loads around a cross-lane exchange: a compiler-level barrier (no instruction
 // is emitted; the LDS unit completes the operations of one wavefront in issue order).
 __device__ inline void flash_wave_lds_fence() {
@@ -289,6 +293,91 @@ __device__ inline void flash_wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The same tiles for rows that do not start 16-byte aligned, which the copies to LDS need: a wavefront loads its pieces of
+// the next tile into registers (16 bytes from any element on, as the memory pipeline takes them) while it works on this one,
+// and stores them to LDS once this tile's entries have been read, so one stage of LDS is enough.  Read straight from global
+// memory in the accumulator layout, 2 bytes a load, 64 x 12 pairs of 197 x 197 scores with a shared bias took 92 us (47.7 so;
+// 41 at 200 x 200 through the copies), 64 pairs of 1000 x 1001 with a bias per score 198 us (52; head dim 128: 365 / 117).
+// Pieces that would end past the (head, batch) slice are moved back to end with it and shifted into place.
+__device__ inline u32x4_t flash_drop_bytes(u32x4_t v, int bytes) {   // the value without its first 0 to 16 bytes, zeros at its end
+    if (bytes & 1) v = (u32x4_t){(v[0] >> 8) | (v[1] << 24), (v[1] >> 8) | (v[2] << 24), (v[2] >> 8) | (v[3] << 24), v[3] >> 8};
+    return bytes >= 16 ? (u32x4_t){0u, 0u, 0u, 0u} : mi_drop_bytes(v, bytes & 14);
+}
+inline bool flash_rows_fit(const AttnParams &p, const int64_t *st, int64_t elem) {
+    const int64_t reach = ((p.Lq + 256) * st[1] + p.Lkv + 128) * elem;   // tiles reach up to 127 keys past Lkv
+    return st[0] == 1 && reach < (int64_t)0x7fffffff && ((p.Lq - 1) * st[1] + p.Lkv) * elem >= 16;
+}
+struct FlashRows {
+    typedef u32x4_t piece_any __attribute__((aligned(1)));
+    typedef __attribute__((address_space(3))) u32x4_t *lds16_t;
+    const char *bbase, *mbase;
+    int bytes_b, bytes_m;                // of the slice
+    int boff[4], moff[2];                // byte offsets of this lane's pieces, the tile's first key excluded
+    u32x4_t breg[4], mreg[2];
+
+    // lays `sg` out over one stage of bias and one of mask tiles from lds_wave_base on
+    __device__ void init(const FlashArgs &a, FlashStaged<1> &sg, unsigned lds_wave_base, int lane, int64_t iw, int64_t h, int64_t b) {
+        const AttnParams &p = a.p;
+        sg.bias = p.bias != nullptr;
+        sg.mask = p.mask != nullptr;
+        sg.blds = lds_wave_base;
+        sg.mlds = lds_wave_base + (sg.bias ? FlashStaged<1>::BIAS_STAGE : 0);
+        const int64_t sb = p.bias_strides[1], sm = p.mask_strides[1];
+        bbase = (const char *)p.bias + 2 * (h * p.bias_strides[2] + b * p.bias_strides[3]);
+        mbase = (const char *)p.mask + h * p.mask_strides[2] + b * p.mask_strides[3];
+        bytes_b = (int)(2 * ((p.Lq - 1) * sb + p.Lkv));
+        bytes_m = (int)((p.Lq - 1) * sm + p.Lkv);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int64_t row = iw + 8 * i + (lane >> 3);
+            boff[i] = (int)(2 * (row < p.Lq ? row : p.Lq - 1) * sb) + ((lane & 7) << 4);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int64_t row = iw + 16 * i + (lane >> 2);
+            moff[i] = (int)((row < p.Lq ? row : p.Lq - 1) * sm) + ((lane & 3) << 4);
+        }
+    }
+    __device__ void issue(const FlashStaged<1> &sg, int j0) {
+        if (sg.bias) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) breg[i] = *(const piece_any *)(bbase + min(boff[i] + 2 * j0, bytes_b - 16));
+        }
+        if (sg.mask) {
+#pragma unroll
+            for (int i = 0; i < 2; i++) mreg[i] = *(const piece_any *)(mbase + min(moff[i] + j0, bytes_m - 16));
+        }
+    }
+    // the pieces issued for the tile at j0 into LDS
+    __device__ void commit(const FlashStaged<1> &sg, int j0, int lane) {
+        flash_wave_lds_fence();
+        if (sg.bias) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int row = 8 * i + (lane >> 3), over = boff[i] + 2 * j0 + 16 - bytes_b;
+                u32x4_t v = breg[i];
+                if (__builtin_amdgcn_ballot_w64(over > 0) != 0) v = flash_drop_bytes(v, over < 0 ? 0 : (over > 16 ? 16 : over));
+                *(lds16_t)(uintptr_t)(sg.blds + row * 128 + (((lane & 7) ^ FlashStaged<1>::bias_swz(row)) << 4)) = v;
+            }
+        }
+        if (sg.mask) {
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const int row = 16 * i + (lane >> 2), over = moff[i] + j0 + 16 - bytes_m;
+                u32x4_t v = mreg[i];
+                if (__builtin_amdgcn_ballot_w64(over > 0) != 0) v = flash_drop_bytes(v, over < 0 ? 0 : (over > 16 ? 16 : over));
+                *(lds16_t)(uintptr_t)(sg.mlds + row * 64 + (((lane & 3) ^ FlashStaged<1>::mask_swz(row)) << 4)) = v;
+            }
+        }
+        flash_wave_lds_fence();
+    }
+};
+
+// On entry s[qb][kb] holds raw dot products k.q of tile rows [j0, j0+64) for the wavefront's query
+// blocks; on exit it holds exp2(x - m) (ONLINE / STATS) or the final normalised weights (FINAL),
+// with m, l (and, ONLINE only, the output accumulators o) updated.
+//   T      element traits of the bias array
+//   NDV    number of 32-row blocks of the output accumulator
 // Adds a 32-key x 32-query block of Float32 values held in the MFMA accumulator layout (lane (r, hh): query row r
 // of the wavefront; register 4g + e: key 8g + 4hh + e of the block) to a Float32 array whose keys are contiguous:
 // dst points at (first key of the block, first query row of the wavefront), rows are qstride elements apart (0: every
@@ -419,7 +508,7 @@ __device__ inline void flash_softmax_tile(const FlashArgs &a, floatx16_t (&s)[QB
         // ---- scale, bias, mask.  With bias / mask the accumulators end up holding the reference's
         // logits (natural units); without, they keep the raw dot products and the positive factor c
         // is folded into the exponent below (max commutes with a positive scale).
-        if (EXTRAS == EXTRAS_STAGED) {
+        if (EXTRAS == EXTRAS_STAGED || EXTRAS == EXTRAS_ROWS) {
             const int row = 32 * qb + r;
             if (sg.bias) {
 #pragma unroll

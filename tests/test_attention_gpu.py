@@ -5,6 +5,7 @@ Tolerances: Float32 max error <= 1e-4 of output scale; Float16/BFloat16 <= 1e-2 
 Float32 CPU result on the same (already rounded) inputs; weight columns sum to 1 within 1e-5
 (checked on Float32 weights).
 """
+import ctypes
 import itertools
 import json
 import os
@@ -941,3 +942,62 @@ def test_pipelined_forward_where_half_of_a_block_dominates(nn, oracle, dtype, D,
     # no row has keys that compete near the large scores, so the error is that of ordinary inputs (2-norm): rounding of q, the
     # weights and y to the type, 3.0e-3 and 3.6e-4 measured over many shapes, four times that allowed
     assert np.linalg.norm(y.to_numpy() - ref) <= (1.2e-2 if dtype == "bf16" else 1.5e-3) * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("D,Lq,Lkv,H,B,causal,weights,bias_dims,mask_dims", [
+    (64, 197, 197, 3, 2, False, False, 3, 0), (64, 33, 9, 2, 1, False, True, 3, 2), (40, 131, 131, 2, 2, True, True, 4, 0),
+    (128, 301, 77, 2, 2, False, False, 4, 2), (128, 65, 191, 1, 2, True, False, 3, 0) , (96, 45, 1001, 2, 1, False, False, 3, 4),
+    (64, 7, 803, 2, 2, False, False, 4, 2), (128, 64, 63, 1, 1, False, True, 4, 4), (64, 1, 65, 2, 2, False, True, 3, 0)])
+def test_bias_and_mask_rows_of_any_alignment(nn, oracle, dtype, D, Lq, Lkv, H, B, causal, weights, bias_dims, mask_dims):
+    """Bias and mask rows that do not start on 16 bytes (compact arrays with an odd number of keys) against the same entries
+    in rows padded to 16 bytes, which the LDS copies take, and against the oracle; the last piece of an array included."""
+    if causal:
+        Lkv = Lq
+    rng = np.random.default_rng(D + Lq + Lkv)
+    q, k, v = (round_to(rng.standard_normal((D * H, n, B)), dtype) for n in (Lq, Lkv, Lkv))
+    dims = (Lkv, Lq, H, B)
+    bias = round_to(rng.standard_normal(dims[:bias_dims]), dtype)
+    mask = rng.random(dims[:mask_dims]) < 0.8 if mask_dims else None
+    if mask is not None:
+        mask[0] = True
+    D_ = lambda a, *t: nn.DeviceArray.from_numpy(a, *t)
+
+    def padded(a, t):
+        pad = (a.shape[0] + 15) // 16 * 16
+        wide = np.zeros((pad,) + a.shape[1:], a.dtype)
+        wide[:a.shape[0]] = a
+        w = D_(wide, t)
+        return nn.DeviceArray(w.storage, a.shape, w.dtype, w.strides)
+
+    args = [D_(a, dtype) for a in (q, k, v)]
+    causal_mask = nn.make_causal_mask(args[0]) if causal else None
+
+    def run(b, m):
+        m = causal_mask if m is None else m if causal_mask is None else causal_mask & m
+        y, a = nn.dot_product_attention(*args, b, mask=m, nheads=H, return_weights=weights)
+        return y.to_numpy(), a.to_numpy() if weights else None
+
+    y, a = run(D_(bias, dtype), D_(mask) if mask is not None else None)
+    y2, a2 = run(padded(bias, dtype), padded(mask, "bool") if mask is not None else None)
+    assert nn.last_attention_kernel() in ("flash16", "decode")
+    assert np.array_equal(y, y2) and (not weights or np.array_equal(a, a2))
+    omask = oracle.make_causal_mask(Lq) if causal else mask
+    yr, _ = oracle.nnlib_attention_f32(q, k, v, bias, omask, H)
+    assert rel_err(y, yr) <= TOL[dtype]
+
+
+def test_a_short_key_range_with_a_bias_needs_no_workspace(nn):
+    """Few queries, a bias and 768 to 2047 keys: split over the keys where the workspace has room for the pieces, one
+    workgroup per query tile where it has none; the two agree to the rounding of the output."""
+    rng = np.random.default_rng(3)
+    q, k, v = (nn.DeviceArray.from_numpy(round_to(rng.standard_normal((128, n, 1)), "f16"), "f16") for n in (50, 1001, 1001))
+    bias = nn.DeviceArray.from_numpy(round_to(rng.standard_normal((1001, 50, 2)), "f16"), "f16")
+    y, _ = nn.dot_product_attention(q, k, v, bias, nheads=2, return_weights=False)
+    assert nn.ops.last_attention_workspace() > 0
+    lib, d = nn._lib.load(), nn._lib.mi_attn_desc()
+    out = nn.DeviceArray.empty((128, 50, 1), "f16")
+    nn.ops._fill_desc(d, q, k, v, bias, None, 2, 1, 128, 128, 50, 1001, 0)
+    d.out = out.ptr
+    nn._lib.check(lib.mi_attention_fwd(ctypes.byref(d), None))
+    assert rel_err(out.to_numpy(), y.to_numpy()) <= 2 * 2.0 ** -11
