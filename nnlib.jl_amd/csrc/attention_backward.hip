@@ -25,6 +25,7 @@ static int32_t validate_bwd(const mi_attn_bwd_desc *d, AttnBwdParams *out) {
     bp.workspace_bytes = d->workspace ? d->workspace_bytes : 0;
     bp.mask_bits = nullptr;
     bp.drop_rows = bp.drop_keys = nullptr;
+    bp.dbias_only = 0;
     bp.bias_rows = bp.bias_keys = nullptr;
     bp.pair0 = bp.npairs = bp.dbias_in_dq = 0;
     bp.kv_len = nullptr;

@@ -11,6 +11,10 @@ int32_t launch_bwd_flash16_f16_d128(const AttnBwdParams &, hipStream_t);
 int32_t launch_bwd_flash16_bf16_d256(const AttnBwdParams &, hipStream_t);
 int32_t launch_bwd_flash16_f16_d256(const AttnBwdParams &, hipStream_t);
 
+// dQ, dK and dV of a (head, batch) pair in one workgroup (attention_backward_pair16.inc)
+int32_t launch_bwd_pair16_bf16(const AttnBwdParams &, hipStream_t);
+int32_t launch_bwd_pair16_f16(const AttnBwdParams &, hipStream_t);
+
 static inline bool aligned16(const void *p) { return (((uintptr_t)p) & 15) == 0; }
 
 bool attention_bwd_flash16_supports(const AttnBwdParams &bp) {
@@ -73,6 +77,17 @@ static size_t lengths_bytes(const AttnParams &p) {
     return ((size_t)(p.H * p.B) * sizeof(int32_t) + 15) & ~(size_t)15;
 }
 
+// ---- short sequences: one workgroup per (head, batch) pair --------------------------------------------------------------
+// Up to 256 keys (eight wavefronts) at head dims up to 64, all three gradients wanted, saved statistics, no mask that depends
+// on the query.  The tiles of queries are one chain on a wavefront per 32 keys: not many more queries than keys (16 x 16 pairs of
+// 1000 x 77: 77 us against 68), and more than 256 only where the pairs fill the chip (500 x 200: 41 against 60).
+static bool pair_kernel_fits(const AttnBwdParams &bp) {
+    const AttnParams &p = bp.p;
+    return bp.have_stats && bp.dq && bp.dk && bp.dv && p.D <= 64 && p.Lkv <= 256 && (p.Lq <= 3 * p.Lkv || p.Lq <= 64) &&
+           (p.Lq <= 256 || p.H * p.B >= 256) &&
+           (!p.mask || flash_is_key_mask(p)) && !(p.bias && p.drop_thresh);
+}
+
 // ---- fused dropout: the keep decisions drawn once ---------------------------------------------------------------
 // A keep decision costs a 64-bit hash per four weights (about 175 issue cycles a wavefront instruction), and each of the
 // three gradient kernels needs every decision.  This kernel draws them once, any L_kv: a wavefront takes a block of 64
@@ -87,8 +102,10 @@ static size_t lengths_bytes(const AttnParams &p) {
 // Two bits a weight are O(L^2) bytes where the rest of the call is O(L): the words of as many (head, batch) pairs as
 // DROP_WORDS_MOST bytes hold are drawn at a time, and the gradient kernels run on those pairs before the next are drawn.  A
 // pair whose own words are more than that (65536 x 65536 is 1 GiB) has them redrawn by the kernels.
-static bool takes_drop_words(const AttnParams &p, bool lengths) {
+static bool takes_drop_words(const AttnBwdParams &bp, bool lengths) {
+    const AttnParams &p = bp.p;
     if (p.drop_thresh == 0 || p.bias) return false;
+    if (pair_kernel_fits(bp)) return (p.Lkv & 3) != 0;   // meets every decision once
     if ((p.Lkv & 3) == 0 && (p.causal || p.H * p.B * p.Lq * p.Lkv < (1 << 24))) return false;
     return !p.mask || flash_is_key_mask(p) || lengths || takes_mask_bits(p);   // what the lean kernels take
 }
@@ -122,7 +139,7 @@ __global__ __launch_bounds__(256) void drop_words_kernel(AttnParams p, int64_t p
     if (p.Lkv & 3) {
         if (off) group(64 - off);
     }
-    rows[(pair * nkt + kt) * lq_pad + qi] = word;
+    if (rows) rows[(pair * nkt + kt) * lq_pad + qi] = word;
     // transpose: bit k of lane i becomes bit i of lane k; first the halves, then within 32 x 32
     uint32_t lo = (uint32_t)word, hi = (uint32_t)(word >> 32);
     mi_pair_halves(lo, hi);   // lo of lanes 32-63 <-> hi of lanes 0-31
@@ -257,7 +274,7 @@ static BwdScratch plan_scratch(const AttnBwdParams &bp, size_t room) {
     s.partial = attention_bwd_flash16_dq_partial_bytes(bp);
     s.lengths = lengths_bytes(p);
     const auto left = [&] { return s.total() < room ? room - s.total() : (size_t)0; };
-    if (takes_drop_words(p, s.lengths != 0)) {
+    if (takes_drop_words(bp, s.lengths != 0)) {
         const size_t pair = sizeof(uint64_t) * (drop_rows_words(p) + drop_keys_words(p));
         const size_t pairs = (left() < DROP_WORDS_MOST ? left() : DROP_WORDS_MOST) / pair;
         s.word_pairs = pairs < (size_t)(p.H * p.B) ? (int64_t)pairs : p.H * p.B;
@@ -322,12 +339,21 @@ int32_t launch_attention_bwd_flash16(const AttnBwdParams &bp_in, hipStream_t st)
             uint64_t *rows = (uint64_t *)at, *keys = rows + drop_rows_words(p) * (size_t)step;
             const int64_t nkt = (p.Lkv + 63) / 64, nqt = (p.Lq + 63) / 64, blocks = nkt * nqt * bp.npairs;   // at most 2^20 (DROP_WORDS_MOST)
             hipLaunchKernelGGL(drop_words_kernel, dim3((unsigned)((blocks + 3) / 4)), dim3(256), 0, st, p, pair0, nkt, nqt, pad128(p.Lq),
-                               pad128(p.Lkv), blocks, rows, keys);
+                               pad128(p.Lkv), blocks, pair_kernel_fits(bp) ? nullptr : rows, keys);   // the pair kernel's lanes hold keys
             MI_LAUNCH_CHECK();
             bp.drop_rows = rows;
             bp.drop_keys = keys;
         }
         int32_t rc;
+        // a bias only from its copies, whose calls have a kernel of their own for its gradient; dropout at rows that do not
+        // start on a hash group only from words
+        const bool pair = pair_kernel_fits(bp) && (p.bias ? bp.bias_keys != nullptr : !p.drop_thresh || bp.drop_keys || (p.Lkv & 3) == 0);
+        if (pair) {
+            rc = p.dtype == MI_BF16 ? launch_bwd_pair16_bf16(bp, st) : launch_bwd_pair16_f16(bp, st);
+            if (rc != MI_OK) return rc;
+            if (!bp.dbias) continue;
+            bp.dbias_only = 1;
+        }
         if (p.dtype == MI_BF16)
             rc = p.D <= 64 ? launch_bwd_flash16_bf16_d64(bp, st) : p.D <= 128 ? launch_bwd_flash16_bf16_d128(bp, st) : launch_bwd_flash16_bf16_d256(bp, st);
         else

@@ -111,6 +111,7 @@ struct AttnBwdParams {
     // the workspace no room for them
     const uint16_t *bias_rows, *bias_keys;
     int32_t dbias_in_dq;   // few scores: the gradient of a bias shared by the batch stays with the dQ kernel
+    int32_t dbias_only;    // the other gradients are done (attention_backward_pair16.inc): launch the bias gradient alone
     // key-padding mask measured on the device: per (head, batch) pair [b * H + h] the context length, or 0 when the
     // mask of the pair is not a kept prefix; null when the call does not take that path
     const int32_t *kv_len;

@@ -874,3 +874,30 @@ def test_infinite_entries_of_a_shared_bias(nn, oracle, dtype, D, L, B, saved):
         assert np.array_equal(np.isnan(g), np.isnan(r)) and np.isnan(r).any()
         fin = ~np.isnan(r)
         assert np.abs(g[fin] - r[fin]).max() <= TOL[dtype] * np.abs(r[fin]).max()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("D,H,Lq,Lkv,batch,mask_kind,dropout,bias", [
+    (64, 2, 1, 1, (2,), None, None, False), (8, 3, 33, 31, (2,), None, None, False), (64, 2, 32, 32, (2,), "causal", None, False),
+    (40, 2, 65, 127, (3,), "lengths", None, False), (64, 2, 128, 128, (2,), "causal", (0.2, 7), False), (64, 1, 96, 129, (3,), "keys", None, False),
+    (64, 2, 129, 129, (2,), "causal", None, False), (56, 2, 250, 161, (3,), "lengths", (0.3, 8), False), (64, 2, 191, 224, (2,), None, (0.3, 9), False),
+    (64, 2, 255, 255, (2,), "causal", (0.1, 10), False), (64, 2, 256, 256, (3,), "lengths", None, False), (32, 4, 200, 256, (2,), None, None, False),
+    (64, 2, 300, 130, (130,), None, None, False), (48, 3, 197, 197, (12,), None, None, True), (64, 2, 225, 225, (16,), "causal", None, True)])
+def test_short_sequences_in_one_kernel_per_pair(nn, oracle, dtype, D, H, Lq, Lkv, batch, mask_kind, dropout, bias):
+    """Up to 256 keys at head dims up to 64 with saved statistics: blocks of 32 keys and tiles of 32 and 64 queries with
+    remainders, keys past a sequence's length, masks that are no length, dropout at rows on and off the hash groups, a bias
+    shared by the batch; against the oracle, and against the kernels that calls without saved statistics take."""
+    E = D * H
+    _run(nn, oracle, dtype, E, E, Lq, Lkv, batch, H, mask_kind=mask_kind, dropout=dropout, bias_shape=(Lkv, Lq, H) if bias else None,
+         expect="flash16", saved=True, seed=Lq + Lkv)
+    rng = np.random.default_rng(Lkv)
+    D_ = lambda *s: nn.DeviceArray.from_numpy(round_to(rng.standard_normal(s), dtype), dtype)
+    q, k, v, dy = D_(E, Lq, 3), D_(E, Lkv, 3), D_(E, Lkv, 3), D_(E, Lq, 3)
+    mask = nn.make_causal_mask(q) if mask_kind == "causal" else None
+    fdrop = nn.Dropout(*dropout) if dropout else nn.identity
+    grads = []
+    for saved in (True, False):
+        y, _ = nn.dot_product_attention(q, k, v, mask=mask, nheads=H, return_weights=False, fdrop=fdrop, save_for_backward=saved)
+        grads.append([g.to_numpy() for g in nn.dot_product_attention_grad(dy, q, k, v, y=y, mask=mask, nheads=H, fdrop=fdrop)[:3]])
+    for a, b in zip(*grads):   # P and dS rounded to 16 bits in both, the result too
+        assert np.linalg.norm(a - b) <= (2.0 ** -7 if dtype == "bf16" else 2.0 ** -9) * np.linalg.norm(b) + 1e-6
