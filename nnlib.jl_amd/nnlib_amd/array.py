@@ -4,6 +4,8 @@ A ``DeviceArray`` has a Julia ``size`` tuple and column-major memory, exactly as
 reference operates on; element ``(i1, i2, ...)`` is at ``i1 + i2*size[0] + ...``.  PyTorch is used
 only as the owner of the device allocation (and for host<->device copies).
 """
+import math
+
 import numpy as np
 import torch
 
@@ -25,9 +27,15 @@ _NP2NAME = {np.dtype(np.float32): "f32", np.dtype(np.float16): "f16", np.dtype(n
 COMPLEX = ("c64", "c128")
 
 
+_gpu_seen = False   # a GPU that was there stays; asking again costs a call more than the allocation it guards
+
+
 def _require_gpu():
-    if not torch.cuda.is_available():
-        raise RuntimeError("nnlib_amd needs a GPU (torch.cuda.is_available() is False); there is no CPU path")
+    global _gpu_seen
+    if not _gpu_seen:
+        if not torch.cuda.is_available():
+            raise RuntimeError("nnlib_amd needs a GPU (torch.cuda.is_available() is False); there is no CPU path")
+        _gpu_seen = True
 
 
 class DeviceArray:
@@ -39,7 +47,7 @@ class DeviceArray:
 
     def __init__(self, storage, dims, dtype, strides=None, offset=0):
         self.storage = storage          # 1-D torch tensor that owns the memory
-        self.dims = tuple(int(d) for d in dims)
+        self.dims = tuple(map(int, dims))
         self.dtype = dtype              # "f32" | "f16" | "bf16" | "bool"; batched_mul also takes "f64", "i32", "i64", "c64", "c128"
         self.conj = False               # set by batched_adjoint of a complex array: elements read conjugated
         if strides is None:
@@ -47,15 +55,15 @@ class DeviceArray:
             for d in self.dims:
                 strides.append(acc)
                 acc *= d
-        self.strides = tuple(int(s) for s in strides)
+        self.strides = tuple(map(int, strides))
         self.offset = int(offset)       # in elements
 
     # ---- construction --------------------------------------------------------------------
     @classmethod
     def empty(cls, dims, dtype="f32"):
         _require_gpu()
-        n = int(np.prod(dims, dtype=np.int64)) if len(dims) else 1
-        return cls(torch.empty(max(n, 1), dtype=_TORCH[dtype], device="cuda"), dims, dtype)
+        dims = tuple(map(int, dims))
+        return cls(torch.empty(max(math.prod(dims), 1), dtype=_TORCH[dtype], device="cuda"), dims, dtype)
 
     @classmethod
     def zeros(cls, dims, dtype="f32"):
@@ -101,7 +109,7 @@ class DeviceArray:
 
     @property
     def length(self):
-        return int(np.prod(self.dims, dtype=np.int64)) if self.dims else 1
+        return math.prod(self.dims)
 
     def is_contiguous(self):
         acc = 1
@@ -115,10 +123,10 @@ class DeviceArray:
         if len(dims) == 1 and isinstance(dims[0], (tuple, list)):
             dims = tuple(dims[0])
         if -1 in dims:
-            known = int(np.prod([d for d in dims if d != -1], dtype=np.int64))
+            known = math.prod(d for d in dims if d != -1)
             dims = tuple(self.length // max(known, 1) if d == -1 else d for d in dims)
         assert self.is_contiguous(), "reshape needs a contiguous array"
-        assert int(np.prod(dims, dtype=np.int64)) == self.length, "reshape must keep the element count"
+        assert math.prod(dims) == self.length, "reshape must keep the element count"
         out = DeviceArray(self.storage, dims, self.dtype, None, self.offset)
         out.conj = self.conj
         return out
@@ -163,7 +171,8 @@ class DeviceArray:
 
     @property
     def ptr(self):
-        return self.storage.data_ptr() + self.offset * self.itemsize
+        at = self.storage.data_ptr()
+        return at + self.offset * self.itemsize if self.offset else at
 
     @property
     def code(self):

@@ -5,8 +5,8 @@ NNlib.jl source tree).  Every function marshals arguments and calls the C ABI
 (``include/mi355attn.h``); all arithmetic happens in the HIP kernels.
 """
 import ctypes
+import math
 
-import numpy as np
 import torch
 
 from . import _lib
@@ -73,7 +73,12 @@ def last_attention_workspace():
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current stream's handle: what torch.cuda.current_stream().cuda_stream is, without the Stream object."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+
+
+_Strides = ctypes.c_int64 * 4
+_ATTN_DESC_BYTES = ctypes.sizeof(_lib.mi_attn_desc)
 
 
 class _WorkspaceSize(int):
@@ -120,7 +125,7 @@ def _broadcast_strides(x, target, what):
 
 def _fill_desc(d, q, k, v, bias, mask, H, B, E, Ev, Lq, Lkv, flags, fdrop=None):
     """Forward-call part of a descriptor: element type, sizes, inputs, bias / mask strides."""
-    d.struct_size = ctypes.sizeof(_lib.mi_attn_desc)
+    d.struct_size = _ATTN_DESC_BYTES
     if fdrop is not None:
         d.dropout_p, d.dropout_seed = fdrop.p, fdrop.seed
     d.dtype = d.weights_dtype = q.code_f64
@@ -134,7 +139,7 @@ def _fill_desc(d, q, k, v, bias, mask, H, B, E, Ev, Lq, Lkv, flags, fdrop=None):
             raise ArgumentError(f"bias must have the element type of q ({q.dtype}), got {bias.dtype}")
         st = _broadcast_strides(bias, target, "bias")
         d.bias = bias.ptr
-        d.bias_strides = (ctypes.c_int64 * 4)(*st)
+        d.bias_strides = _Strides(*st)
     d.causal = 0
     if isinstance(mask, (CausalMask, CausalAnd)):
         if mask.length != Lkv or mask.length != Lq:
@@ -147,7 +152,7 @@ def _fill_desc(d, q, k, v, bias, mask, H, B, E, Ev, Lq, Lkv, flags, fdrop=None):
             raise ArgumentError("mask must be a Bool array")
         st = _broadcast_strides(mask, target, "mask")
         d.mask = mask.ptr
-        d.mask_strides = (ctypes.c_int64 * 4)(*st)
+        d.mask_strides = _Strides(*st)
 
 
 def _attention_call(q, k, v, bias, mask, H, B, E, Ev, Lq, Lkv, want_out, want_weights, weights_dtype, flags,
@@ -202,7 +207,7 @@ def _check_qkv(q, k, v, nheads):
     bq, bk, bv = q.dims[2:], k.dims[2:], v.dims[2:]
     if not (bq == bk == bv):                                     # src/attention.jl:42, :63
         raise ArgumentError("Batch dimensions have to be the same.")
-    B = int(np.prod(bq, dtype=np.int64)) if bq else 1
+    B = math.prod(bq)
     E, Lq, Lkv, Ev = q.dims[0], q.dims[1], k.dims[1], v.dims[0]
     if E % nheads or k.dims[0] % nheads or Ev % nheads:          # src/attention.jl:55
         raise ArgumentError("First dimension in query, key and value must be divisible by `nheads`.\n"
@@ -238,12 +243,13 @@ def dot_product_attention(q, k, v, bias=None, *, fdrop=identity, mask=None, nhea
                                    _flags)
         alpha = fdrop(alpha)
         x = _weights_times_values(alpha, v, nheads, B, Ev, Lq, Lkv)
-    stats = getattr(x, "saved_stats", None)
-    x = x.reshape((Ev, Lq) + tuple(bq))
-    if stats is not None:
-        x.saved_stats = stats
-    if alpha is not None:
-        alpha = alpha.reshape((Lkv, Lq, nheads) + tuple(bq))
+    if len(bq) != 1:
+        stats = getattr(x, "saved_stats", None)
+        x = x.reshape((Ev, Lq) + tuple(bq))
+        if stats is not None:
+            x.saved_stats = stats
+        if alpha is not None:
+            alpha = alpha.reshape((Lkv, Lq, nheads) + tuple(bq))
     return x, alpha
 
 
@@ -362,20 +368,19 @@ def _reduction_geometry(dims_of_x, dims):
     size of the reduced result (extent 1 along ``dims``, as Julia's ``sum(x; dims)`` keeps them)."""
     size = tuple(dims_of_x)
     if dims is None:
-        n = int(np.prod(size, dtype=np.int64)) if size else 1
+        n = math.prod(size)
         return 1, n, 1, ()
     ds = sorted({int(d) for d in (dims if isinstance(dims, (tuple, list)) else (dims,))})
     if not ds or ds[0] < 1:
         raise ArgumentError(f"dims must be positive dimension numbers, got {dims}")
     ds = [d for d in ds if d <= len(size)]       # trailing singleton dimensions reduce to themselves
     if not ds:
-        return int(np.prod(size, dtype=np.int64)) if size else 1, 1, 1, size
+        return math.prod(size), 1, 1, size
     if ds != list(range(ds[0], ds[-1] + 1)):   # callers route such sets through _nonadjacent_plan first
         raise ArgumentError(f"dims = {dims}: a single kernel call reduces over a run of adjacent dimensions")
     lo, hi = ds[0] - 1, ds[-1]
-    prod = lambda t: int(np.prod(t, dtype=np.int64)) if t else 1
     kept = size[:lo] + (1,) * (hi - lo) + size[hi:]
-    return prod(size[:lo]), prod(size[lo:hi]), prod(size[hi:]), kept
+    return math.prod(size[:lo]), math.prod(size[lo:hi]), math.prod(size[hi:]), kept
 
 
 def _dims_call(x, dims):
@@ -489,7 +494,7 @@ def grad_logsumexp(dy, x, *, dims=None, lse=None):
         lse = logsumexp(x, dims=dims)
     lse = _contig(lse, "lse")
     nd, sizes, mask, ws, wsize, kept = _dims_call(x, dims)
-    n_out = int(np.prod(kept, dtype=np.int64)) if kept else 1
+    n_out = math.prod(kept)
     if dy.length != n_out or lse.length != n_out or not (dy.dtype == lse.dtype == x.dtype):
         raise DimensionMismatch(f"dy and lse must have the size {kept} of logsumexp(x; dims) and the element type of x")
     dx = DeviceArray.empty(x.dims, x.dtype)
