@@ -61,6 +61,33 @@ __device__ inline void attention_drop_factors_run4(const AttnParams &p, uint64_t
 }
 
 
+// The same for rows that start anywhere within a hash group (Lkv not a multiple of 4), one call a run: the two half-waves of
+// a query hold alternate runs, so the groups a lane's runs start in and those they end in are its own and the other half's.
+// Each lane hashes one group a run and the halves exchange the words (one hash per four weights and one more per tile,
+// where looking each weight up alone took four).  row: linear index of the tile's first key for this lane's query.
+struct AttnDropRow {
+    uint64_t z, own;   // hash input of the next group, bits of this one
+    int shift;         // bits before the first weight in its group
+    __device__ void init(const AttnParams &p, uint64_t row, int hh) {
+        z = p.drop_key + ((row >> 2) + (uint64_t)hh) * 0x9E3779B97F4A7C15ull;
+        shift = 16 * (int)(row & 3);
+        own = mi_mix64(z);
+    }
+    __device__ void next(const AttnParams &p, int hh, float (&f)[4]) {
+        z += 2 * 0x9E3779B97F4A7C15ull;
+        const uint64_t ahead = mi_mix64(z);
+        // lower half: the upper half's group of this run; upper half: the lower half's group of the next
+        const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)own, (uint32_t)ahead, false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(own >> 32), (uint32_t)(ahead >> 32), false, false);
+        const uint32_t lo0 = lo[0], lo1 = lo[1], hi0 = hi[0], hi1 = hi[1];
+        const uint64_t other = (uint64_t)(hh ? hi0 : hi1) << 32 | (hh ? lo0 : lo1);
+        const uint64_t bits = (own >> shift) | ((other << 1) << (63 - shift));
+#pragma unroll
+        for (int e = 0; e < 4; e++) f[e] = mi_dropout_keep_in(bits, e, p.drop_thresh) ? p.drop_scale : 0.0f;
+        own = ahead;
+    }
+};
+
 // The transposed case: a lane holds ONE key (kv; the four lanes of a quad hold kv = 4t .. 4t+3) and, in register
 // e of a run, query q0 + e.  Each lane hashes the group of query q0 + (lane & 3) and the quad exchanges the words,
 // so a quad still computes one hash per four weights.  f[e]: the factor of weight (kv, q0 + e).  Needs Lkv % 4 == 0.

@@ -675,18 +675,30 @@ __device__ inline void flash_softmax_tile(const FlashArgs &a, floatx16_t (&s)[QB
         // fdrop = dropout (src/attention.jl:126): after the softmax, so the row sum above is untouched;
         // before the value product and before the weights are written, which are post-dropout.
         if (PHASE != PHASE_STATS && p.drop_thresh != 0) {
-            const uint64_t row0 = (uint64_t)(p.Lkv * (qi + p.Lq * (h + p.H * b)) + j0 + 4 * hh);
-            const bool aligned = (p.Lkv & 3) == 0;   // every run of four keys of a lane is one hash group
+            const uint64_t row0 = (uint64_t)(p.Lkv * (qi + p.Lq * (h + p.H * b)) + j0);
+            if ((p.Lkv & 3) == 0) {   // every run of four keys of a lane is one hash group
 #pragma unroll
-            for (int kb = 0; kb < KBLK; kb++)
+                for (int kb = 0; kb < KBLK; kb++)
 #pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    float f[4];
-                    if (aligned) attention_drop_factors_run4<true>(p, row0 + 32 * kb, g, f);
-                    else attention_drop_factors_run4<false>(p, row0 + 32 * kb, g, f);
+                    for (int g = 0; g < 4; g++) {
+                        float f[4];
+                        attention_drop_factors_run4<true>(p, row0 + 4 * hh + 32 * kb, g, f);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) s[qb][kb][4 * g + e] *= f[e];
-                }
+                        for (int e = 0; e < 4; e++) s[qb][kb][4 * g + e] *= f[e];
+                    }
+            } else {
+                AttnDropRow row;
+                row.init(p, row0, hh);
+#pragma unroll
+                for (int kb = 0; kb < KBLK; kb++)
+#pragma unroll
+                    for (int g = 0; g < 4; g++) {
+                        float f[4];
+                        row.next(p, hh, f);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) s[qb][kb][4 * g + e] *= f[e];
+                    }
+            }
         }
 
         if (PHASE == PHASE_FINAL && p.weights && wlds != 0 && a.w_lds) {
