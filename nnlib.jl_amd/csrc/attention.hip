@@ -91,8 +91,16 @@ static bool fast_kernel_fits(const AttnParams &p) {   // everything but the mask
     if (p.dtype == MI_F16) return flash16_fast_supports_f16(p) || flash16_fast_supports_f16_d64(p);
     return false;
 }
+// Dropout: the hashes bound both kernels, and the pipelined one is ahead by its tiles of 128 keys a barrier only (4 to 8 % at
+// 1024 and 4096 queries), while it pads the queries to 256 where the general one pads to 128.  24 x 12 pairs of 336 x 336,
+// pipelined / general: head dim 64 56 / 39 us (padding mask 47 / 35), head dim 128 68 / 49.
+static bool dropout_pads_less(const AttnParams &p) {
+    const int64_t fast = (p.Lq + 255) / 256 * 256, general = (p.Lq + 127) / 128 * 128;
+    return p.drop_thresh && 12 * fast > 13 * general;
+}
 static bool takes_fast_path(const AttnParams &p) {
     if (p.mask || !fast_kernel_fits(p)) return false;
+    if (!p.keep_pipelined && dropout_pads_less(p)) return false;
     // The pipelined kernel never splits the keys and has one workgroup per 256 queries of a (head, batch) pair: with
     // few queries and many keys (cross-attention, a short chunk of queries against a long context) it would leave most
     // of the chip idle, where the general kernel cuts the key range into pieces.  Measured, pipelined / general:
@@ -287,9 +295,10 @@ int32_t launch_attention_flash16(const AttnParams &p, hipStream_t st) {
         int32_t *lens = (int32_t *)p.workspace;
         int32_t rc = launch_key_mask_lengths(p, lens, st);
         if (rc != MI_OK) return rc;
-        // pairs with a context length: the software-pipelined kernel where it fits the call, else the general kernel's
-        // variant without mask code (weights, dropout, other head dims); the other pairs: the key-mask variant
-        rc = fast_kernel_fits(p) ? launch_fast16(p, st, lens) : launch_general16(p, st, lens, true);
+        // pairs with a context length: the software-pipelined kernel where it fits the call, and the general kernel's key-mask
+        // variant for the others; else the general kernel for both kinds
+        if (!fast_kernel_fits(p) || dropout_pads_less(p)) return launch_general16(p, st, lens, true);
+        rc = launch_fast16(p, st, lens);
         if (rc != MI_OK) return rc;
         return launch_general16(p, st, lens);
     }
