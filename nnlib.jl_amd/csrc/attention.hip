@@ -91,16 +91,22 @@ static bool fast_kernel_fits(const AttnParams &p) {   // everything but the mask
     if (p.dtype == MI_F16) return flash16_fast_supports_f16(p) || flash16_fast_supports_f16_d64(p);
     return false;
 }
-// Dropout: the hashes bound both kernels, and the pipelined one is ahead by its tiles of 128 keys a barrier only (4 to 8 % at
-// 1024 and 4096 queries), while it pads the queries to 256 where the general one pads to 128.  24 x 12 pairs of 336 x 336,
-// pipelined / general: head dim 64 56 / 39 us (padding mask 47 / 35), head dim 128 68 / 49.
-static bool dropout_pads_less(const AttnParams &p) {
-    const int64_t fast = (p.Lq + 255) / 256 * 256, general = (p.Lq + 127) / 128 * 128;
-    return p.drop_thresh && 12 * fast > 13 * general;
+// The pipelined kernel pads the queries to 256, the general one to 128, on two workgroups per CU.  Its lead at equal padding,
+// 5 to 15 % without a causal mask, less with one, 4 to 8 % with dropout, whose hashes bound both, is what the padding may cost
+// it (measured, us, pipelined / general, 12 heads): head dim 64, 24 sequences of 333 33 / 27, causal 29 / 23, with dropout
+// 56 / 39; 64 of 128 21 / 16; 12 of 640 28 / 31, causal 25 / 23, causal with dropout 42 / 33; 4 of 1152 23 / 34; head dim 128,
+// 24 of 333 49 / 39, causal 42 / 35; 64 of 128 32 / 27; 12 of 640 45 / 47, causal 39 / 35; 512 pairs of 128 x 4096 304 / 256.
+// A workgroup that has its CU to itself through many keys is faster on the pipelined kernel whatever it pads (128 pairs of
+// 300 x 1500: 35 / 41, of 300 x 700 21 / 23, head dim 128 30 / 34; 32 of 77 x 1000 26 / 28; but 16 of 333 x 333 12.2 / 10.9,
+// 128 of 77 x 700 16.8 / 15.6).
+static bool general_pads_less(const AttnParams &p) {
+    const double padding = (double)((p.Lq + 255) / 256 * 256) / (double)((p.Lq + 127) / 128 * 128);
+    if ((p.Lq + 255) / 256 * p.H * p.B <= 256 && p.Lkv > (padding >= 2.0 ? 768 : 512)) return false;
+    return padding > (p.drop_thresh ? 1.08 : p.causal ? 1.16 : 1.25);
 }
 static bool takes_fast_path(const AttnParams &p) {
     if (p.mask || !fast_kernel_fits(p)) return false;
-    if (!p.keep_pipelined && dropout_pads_less(p)) return false;
+    if (!p.keep_pipelined && general_pads_less(p)) return false;
     // The pipelined kernel never splits the keys and has one workgroup per 256 queries of a (head, batch) pair: with
     // few queries and many keys (cross-attention, a short chunk of queries against a long context) it would leave most
     // of the chip idle, where the general kernel cuts the key range into pieces.  Measured, pipelined / general:
@@ -297,7 +303,7 @@ int32_t launch_attention_flash16(const AttnParams &p, hipStream_t st) {
         if (rc != MI_OK) return rc;
         // pairs with a context length: the software-pipelined kernel where it fits the call, and the general kernel's key-mask
         // variant for the others; else the general kernel for both kinds
-        if (!fast_kernel_fits(p) || dropout_pads_less(p)) return launch_general16(p, st, lens, true);
+        if (!fast_kernel_fits(p) || general_pads_less(p)) return launch_general16(p, st, lens, true);
         rc = launch_fast16(p, st, lens);
         if (rc != MI_OK) return rc;
         return launch_general16(p, st, lens);
