@@ -89,10 +89,13 @@ static bool pair_kernel_fits(const AttnBwdParams &bp) {
 }
 
 // ---- fused dropout: the keep decisions drawn once ---------------------------------------------------------------
-// A keep decision costs a 64-bit hash per four weights (about 175 issue cycles a wavefront instruction), and each of the
+// A keep decision costs a 64-bit hash per four weights (about 175 issue cycles a wavefront instruction: 64-bit products at a
+// quarter of the rate), and each of the
 // three gradient kernels needs every decision.  This kernel draws them once, any L_kv: a wavefront takes a block of 64
 // queries x 64 keys, a lane hashes the 16 or (rows that do not start on a group of four) 17 groups of its query's row,
-// and the 64 x 64 bits are transposed between the lanes for the kernels whose lanes hold a key.  (Gradient of 24 x 12
+// and the 64 x 64 bits are transposed between the lanes for the kernels whose lanes hold a key.  Bound by the hashes; the
+// decisions are taken from a hash two at a time, and blocks past a context length are not drawn (24 x 12 pairs of 333 x 333
+// 17.3 -> 15.8 us, with a key-padding mask 19.6 -> 15.1; 32 pairs of 2000 x 2000 44.6 -> 38.7).  (Gradient of 24 x 12
 // pairs of 333 x 333, head dim 64,
 // p = 0.1: 296 -> 114 us, with a key-padding mask 436 -> 114; 332 x 332: 123 -> 112; 64 pairs of 2048 x 2048, head dim
 // 128: 705 -> 659.)
@@ -116,29 +119,36 @@ static size_t drop_rows_words(const AttnParams &p) { return (size_t)((p.Lkv + 63
 static size_t drop_keys_words(const AttnParams &p) { return (size_t)((p.Lq + 63) / 64 * pad128(p.Lkv)); }
 
 __global__ __launch_bounds__(256) void drop_words_kernel(AttnParams p, int64_t pair0, int64_t nkt, int64_t nqt, int64_t lq_pad, int64_t lkv_pad,
-                                                         int64_t blocks, uint64_t *rows, uint64_t *keys) {
-    const int64_t id = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);   // wave-uniform
+                                                         int64_t blocks, uint64_t *rows, uint64_t *keys, const int32_t *lens) {
+    const uint32_t id = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), per = (uint32_t)(nkt * nqt);   // `blocks` is at most 2^20
     if (id >= blocks) return;
     const int lane = threadIdx.x & 63;
-    const int64_t kt = id % nkt, qt = id / nkt % nqt, pair = id / (nkt * nqt);   // of this piece: b * H + h - pair0
+    const int64_t kt = id % (uint32_t)nkt, qt = id / (uint32_t)nkt % (uint32_t)nqt, pair = id / per;   // of this piece: b * H + h - pair0
     if (p.causal && 64 * kt > 64 * qt + 63) return;   // no kernel visits a tile above the diagonal
+    if (lens && lens[pair0 + pair] != 0 && 64 * kt >= lens[pair0 + pair]) return;   // nor one past a context length
     const int64_t qi = 64 * qt + lane;
     const uint64_t first = (uint64_t)(p.Lkv * (qi + p.Lq * (pair0 + pair)) + 64 * kt);   // linear index of the row's first weight
     const int off = (int)(first & 3);
-    uint64_t word = 0, z = p.drop_key + (first >> 2) * 0x9E3779B97F4A7C15ull;
-    const auto group = [&](int shift) {   // the next group's four decisions from bit `shift` on
+    // four decisions of a group as bits 0 to 3: in 16-bit lanes, u -sat (thresh - 1) is not zero iff u >= thresh (thresh >= 1);
+    // in assembly, since the compiler turns the builtins into compares, whose lane masks cost wait states and selects
+    const uint32_t below = (p.drop_thresh - 1) * 0x10001u, ones = 0x10001u;
+    uint64_t z = p.drop_key + (first >> 2) * 0x9E3779B97F4A7C15ull;
+    const auto group = [&]() -> uint32_t {
         const uint64_t bits = mi_mix64(z);
         z += 0x9E3779B97F4A7C15ull;
-        uint64_t nibble = 0;
-#pragma unroll
-        for (int e = 0; e < 4; e++) nibble |= (uint64_t)(mi_dropout_keep_in(bits, e, p.drop_thresh) ? 1u << e : 0u);
-        word |= shift < 0 ? nibble >> -shift : nibble << shift;
+        const auto kept = [&](uint32_t w) {
+            uint32_t d;
+            asm("v_pk_sub_u16 %0, %1, %2 clamp\n\tv_pk_min_u16 %0, %0, %3" : "=&v"(d) : "v"(w), "v"(below), "v"(ones));
+            return d;
+        };
+        const uint32_t t = kept((uint32_t)bits) | kept((uint32_t)(bits >> 32)) << 2;   // bits 0, 16, 2, 18
+        return (t | t >> 15) & 15u;
     };
+    uint32_t half[2] = {0, 0};
 #pragma unroll
-    for (int g = 0; g < 16; g++) group(4 * g - off);
-    if (p.Lkv & 3) {
-        if (off) group(64 - off);
-    }
+    for (int g = 0; g < 16; g++) half[g >> 3] |= group() << (4 * (g & 7));
+    uint64_t word = (uint64_t)half[1] << 32 | half[0];
+    if (p.Lkv & 3) word = word >> off | ((uint64_t)group() << 1) << (63 - off);   // the row starts `off` decisions into its first group
     if (rows) rows[(pair * nkt + kt) * lq_pad + qi] = word;
     // transpose: bit k of lane i becomes bit i of lane k; first the halves, then within 32 x 32
     uint32_t lo = (uint32_t)word, hi = (uint32_t)(word >> 32);
@@ -339,7 +349,7 @@ int32_t launch_attention_bwd_flash16(const AttnBwdParams &bp_in, hipStream_t st)
             uint64_t *rows = (uint64_t *)at, *keys = rows + drop_rows_words(p) * (size_t)step;
             const int64_t nkt = (p.Lkv + 63) / 64, nqt = (p.Lq + 63) / 64, blocks = nkt * nqt * bp.npairs;   // at most 2^20 (DROP_WORDS_MOST)
             hipLaunchKernelGGL(drop_words_kernel, dim3((unsigned)((blocks + 3) / 4)), dim3(256), 0, st, p, pair0, nkt, nqt, pad128(p.Lq),
-                               pad128(p.Lkv), blocks, pair_kernel_fits(bp) ? nullptr : rows, keys);   // the pair kernel's lanes hold keys
+                               pad128(p.Lkv), blocks, pair_kernel_fits(bp) ? nullptr : rows, keys, bp.kv_len);   // the pair kernel's lanes hold keys
             MI_LAUNCH_CHECK();
             bp.drop_rows = rows;
             bp.drop_keys = keys;
