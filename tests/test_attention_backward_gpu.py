@@ -901,3 +901,15 @@ def test_short_sequences_in_one_kernel_per_pair(nn, oracle, dtype, D, H, Lq, Lkv
         grads.append([g.to_numpy() for g in nn.dot_product_attention_grad(dy, q, k, v, y=y, mask=mask, nheads=H, fdrop=fdrop)[:3]])
     for a, b in zip(*grads):   # P and dS rounded to 16 bits in both, the result too
         assert np.linalg.norm(a - b) <= (2.0 ** -7 if dtype == "bf16" else 2.0 ** -9) * np.linalg.norm(b) + 1e-6
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("D,H,Lq,Lkv,batch,mask_kind", [
+    (64, 4, 131, 65, (13,), None), (64, 2, 150, 127, (12,), None), (40, 3, 129, 193, (8,), None), (64, 2, 385, 385, (4,), "causal"),
+    (64, 4, 1, 449, (230,), None), (64, 128, 129, 67, (2,), None), (48, 130, 131, 131, (2,), "causal")])
+def test_shared_bias_gradient_in_tiles_of_128(nn, oracle, dtype, D, H, Lq, Lkv, batch, mask_kind):
+    """The gradient of a bias shared by the batch: tiles of 128 queries x 128 keys with a remainder in each, a last half tile
+    without keys, the batch in pieces and (many heads) in one, 192 keys at most and at least in between."""
+    E = D * H
+    for saved in (True, False):
+        _run(nn, oracle, dtype, E, E, Lq, Lkv, batch, H, mask_kind=mask_kind, bias_shape=(Lkv, Lq, H), expect="flash16", saved=saved, seed=Lq + Lkv)
