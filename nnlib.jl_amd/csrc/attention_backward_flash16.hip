@@ -169,17 +169,21 @@ __global__ __launch_bounds__(256) void drop_words_kernel(AttnParams p, int64_t p
 // the scores, so that a lane of the dQ (dK, dV) kernel reads its 16 entries of a block as 32 contiguous bytes, whatever the
 // alignment of the bias rows, and the kernels stay lean (two wavefronts per SIMD).
 // Calls of few scores: the dQ kernel's atomics cost less than the two launches more that the copies and the kernel of the
-// bias gradient are (measured, us, dQ kernel / apart; bias rows staged through LDS: 8 x 4 pairs of 128 x 128 47 / 52, 8 x 16
-// 56 / 66, 32 x 8 86 / 99, 8 x 2 of 512 x 512 108 / 111; the other way 8 x 4 of 384 x 384 119 / 90, and sooner where tiles
-// are ragged: 12 x 8 of 192 x 192 92 / 78, 8 x 128 of 64 x 64 105 / 88; unaligned rows: 8 x 4 of 99 x 99 50 / 57, of
-// 131 x 131 68 / 56).
+// bias gradient are, as long as its chain of tiles with atomics is short (training steps, bf16, us, dQ kernel / apart; bias rows
+// staged through LDS: 8 x 4 pairs of 128 x 128 43 / 49, 32 x 8 48 / 57, 16 x 8 of 96 x 160 48 / 49; 2 x 4 of 200 x 200 58 / 51,
+// 4 x 4 of 512 x 128 63 / 52, of 128 x 512 70 / 58, 2 x 2 of 512 x 512 95 / 70; unaligned rows: 12 x 4 of 61 x 61 44 / 48,
+// 4 x 8 of 77 x 77 49 / 49, 8 x 4 of 99 x 99 53 / 49, 8 x 2 of 81 x 81 at head dim 128 59 / 52).  Whole tiles of up to 256 once
+// there are enough pairs that the bias gradient's two products count (8 x 8 of 256 x 256 61 / 65, 4 x 8 58 / 56, 2 x 4 58 / 51;
+// head dim 128 78 / 87 and 74 / 66).
 static bool bias_gradient_in_dq(const AttnParams &p) {
     FlashArgs a;
     a.p = p;
     a.p.weights = nullptr;
     flash_fill_vec_flags(a);
     const bool whole = p.Lq % 128 == 0 && p.Lkv % 64 == 0;
-    return p.H * p.B * p.Lq * p.Lkv <= (!a.bias_lds || p.D > 128 ? 3 << 17 : whole ? 1 << 22 : 1 << 21);
+    const int64_t scores = p.H * p.B * p.Lq * p.Lkv, longest = p.Lq > p.Lkv ? p.Lq : p.Lkv;
+    if (!a.bias_lds || p.D > 128) return scores <= 3 << 17 && (longest <= 80 || p.D > 128);
+    return scores <= (whole ? 1 << 22 : 1 << 21) && (longest <= 160 || (whole && longest <= 256 && scores > 1 << 21));
 }
 static bool takes_bias_blocks(const AttnBwdParams &bp) {
     const AttnParams &p = bp.p;
