@@ -25,7 +25,9 @@ static inline bool aligned16(const void *p) { return (((uintptr_t)p) & 15) == 0;
 
 // ---- merge of split-kv partials -------------------------------------------------------------------
 // out[e, q, b] = sum_s o_s * 2^(m_s - m) / sum_s l_s * 2^(m_s - m), m = max_s m_s.  A row whose every
-// piece was fully masked has m = -Inf and comes out NaN, as the unsplit kernel (and the reference) gives.
+// piece was fully masked has m = -Inf and comes out NaN, as the unsplit kernel (and the reference) gives; one with
+// m = +Inf is the normalised indicator of its +Inf logits (src/softmax.jl:74-75), and a piece that has some holds the
+// sums of that indicator.
 template <typename T>
 __global__ __launch_bounds__(256) void flash_merge_kernel(const float *ws, typename T::type *out, int nsplit, int64_t B,
                                                            int64_t Lq, int64_t Ev, int64_t H) {
@@ -45,7 +47,7 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(const float *ws, typen
     for (int s = 0; s < nsplit; s++) {
         const floatx2_t ml = *(const floatx2_t *)(wml + s * ml_step);
         const floatx4_t o4 = *(const floatx4_t *)(wo + s * o_step);
-        const float w = mi_exp2(ml[0] - m);
+        const float w = m == MI_POS_INF && ml[0] == m ? 1.0f : mi_exp2(ml[0] - m);
         l = fmaf(ml[1], w, l);
 #pragma unroll
         for (int i = 0; i < 4; i++) o[i] = fmaf(o4[i], w, o[i]);

@@ -531,6 +531,45 @@ def test_plus_inf_logits(nn, oracle, dtype, E, Lkv, expect, weights):
         assert a[3, 5, 0, 0] == 0.5 and a[Lkv - 2, 5, 1, 1] == 0.5 and a[70, 9, 0, 1] == 1.0 and a[1, 5, 0, 0] == 0.0
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("Lkv", [1500, 1001, 4096])
+def test_plus_inf_logits_in_pieces_of_the_key_range(nn, oracle, dtype, Lkv):
+    """Few queries: the key range is cut into pieces that another kernel merges (16 bits with a bias from 768 keys on,
+    otherwise from 2048).  +Inf logits in one piece, in two, beside a piece whose keys are all dropped, and dropped
+    themselves; and the same calls in one piece, where the workspace has no room for more."""
+    rng = np.random.default_rng(Lkv)
+    Lq, B, H, E = 40, 2, 2, 128
+    q, k, v = (round_to(rng.standard_normal((E, n, B)), dtype) for n in (Lq, Lkv, Lkv))
+    bias = round_to(0.5 * rng.standard_normal((Lkv, Lq, H, B)), dtype)
+    mask = np.ones((Lkv, Lq), bool)
+    bias[3, 5] = bias[Lkv - 2, 5] = np.inf
+    bias[Lkv // 2, 9] = np.inf
+    bias[0, 11, 1, 0] = np.inf
+    bias[Lkv - 9, 13] = np.inf
+    mask[:Lkv // 2, 13] = False
+    bias[7, 15] = np.inf
+    mask[7, 15] = False
+    mask[:, 17] = False
+    yr, _ = oracle.nnlib_attention_f32(q, k, v, bias, mask, H, nthreads=8)
+    assert np.isnan(yr[:, 17]).all() and np.isfinite(np.delete(yr, 17, axis=1)).all()
+    y, _ = _run(nn, q, k, v, dtype, bias, mask, H, return_weights=False)
+    split = nn.ops.last_attention_workspace() > 0
+    assert split == (Lkv >= 2048 or dtype != "f32")
+    results = [y]
+    if split and Lkv < 2048:
+        lib, d = nn._lib.load(), nn._lib.mi_attn_desc()
+        dq, dk, dv, db = (nn.DeviceArray.from_numpy(a, dtype) for a in (q, k, v, bias))
+        dm, out = nn.DeviceArray.from_numpy(mask), nn.DeviceArray.empty((E, Lq, B), dtype)
+        nn.ops._fill_desc(d, dq, dk, dv, db, dm, H, B, E, E, Lq, Lkv, 0)
+        d.out = out.ptr
+        nn._lib.check(lib.mi_attention_fwd(ctypes.byref(d), None))
+        results.append(out.to_numpy())
+    for y in results:
+        assert np.isnan(y[:, 17]).all() and np.isfinite(np.delete(y, 17, axis=1)).all()
+        assert rel_err(np.delete(y, 17, axis=1), np.delete(yr, 17, axis=1)) <= TOL[dtype]
+        assert np.array_equal(y[:, 9], v[:, Lkv // 2]) and np.array_equal(y[:, 13], v[:, Lkv - 9])
+
+
 @pytest.mark.parametrize("dtype,E,H", [("bf16", 256, 2), ("f16", 128, 2)])
 @pytest.mark.parametrize("weights", [False, True], ids=["noweights", "weights"])
 def test_key_padding_masks(nn, oracle, dtype, E, H, weights):
