@@ -3,6 +3,7 @@
 #include "common.h"
 #include "attention_params.h"
 #include "flash_common.h"
+#include "attention_pair_rule.h"
 
 int32_t launch_bwd_flash16_bf16_d64(const AttnBwdParams &, hipStream_t);
 int32_t launch_bwd_flash16_bf16_d128(const AttnBwdParams &, hipStream_t);
@@ -78,14 +79,12 @@ static size_t lengths_bytes(const AttnParams &p) {
 }
 
 // ---- short sequences: one workgroup per (head, batch) pair --------------------------------------------------------------
-// Up to 256 keys (eight wavefronts) at head dims up to 64, all three gradients wanted, saved statistics, no mask that depends
-// on the query.  The tiles of queries are one chain on a wavefront per 32 keys: not many more queries than keys (16 x 16 pairs of
-// 1000 x 77: 77 us against 68), and more than 256 only where the pairs fill the chip (500 x 200: 41 against 60).
+// Head dims up to 64, all three gradients wanted, saved statistics, no mask that depends on the query.  Dropout at rows that do
+// not start on a hash group takes the decisions from words.
 static bool pair_kernel_fits(const AttnBwdParams &bp) {
     const AttnParams &p = bp.p;
-    return bp.have_stats && bp.dq && bp.dk && bp.dv && p.D <= 64 && p.Lkv <= 256 && (p.Lq <= 3 * p.Lkv || p.Lq <= 64) &&
-           (p.Lq <= 256 || p.H * p.B >= 256) &&
-           (!p.mask || flash_is_key_mask(p)) && !(p.bias && p.drop_thresh);
+    return bp.have_stats && bp.dq && bp.dk && bp.dv && p.D <= 64 && (!p.mask || flash_is_key_mask(p)) && !(p.bias && p.drop_thresh) &&
+           pair_kernel_sizes(p.Lq, p.Lkv, p.H * p.B, p.drop_thresh && (p.Lkv & 3) != 0);
 }
 
 // ---- fused dropout: the keep decisions drawn once ---------------------------------------------------------------

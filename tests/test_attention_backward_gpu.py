@@ -882,7 +882,8 @@ def test_infinite_entries_of_a_shared_bias(nn, oracle, dtype, D, L, B, saved):
     (40, 2, 65, 127, (3,), "lengths", None, False), (64, 2, 128, 128, (2,), "causal", (0.2, 7), False), (64, 1, 96, 129, (3,), "keys", None, False),
     (64, 2, 129, 129, (2,), "causal", None, False), (56, 2, 250, 161, (3,), "lengths", (0.3, 8), False), (64, 2, 191, 224, (2,), None, (0.3, 9), False),
     (64, 2, 255, 255, (2,), "causal", (0.1, 10), False), (64, 2, 256, 256, (3,), "lengths", None, False), (32, 4, 200, 256, (2,), None, None, False),
-    (64, 2, 300, 130, (130,), None, None, False), (48, 3, 197, 197, (12,), None, None, True), (64, 2, 225, 225, (16,), "causal", None, True)])
+    (64, 2, 300, 130, (130,), None, None, False), (48, 3, 197, 197, (12,), None, None, True), (64, 2, 225, 225, (16,), "causal", None, True),
+    (16, 4, 400, 255, (64,), None, (0.1, 11), False), (16, 4, 720, 255, (64,), None, (0.1, 12), False)])
 def test_short_sequences_in_one_kernel_per_pair(nn, oracle, dtype, D, H, Lq, Lkv, batch, mask_kind, dropout, bias):
     """Up to 256 keys at head dims up to 64 with saved statistics: blocks of 32 keys and tiles of 32 and 64 queries with
     remainders, keys past a sequence's length, masks that are no length, dropout at rows on and off the hash groups, a bias
