@@ -16,9 +16,24 @@
 #include <cstdlib>
 #include <type_traits>
 
+// Calls with fused dropout have kernels of their own: the hashes' code, behind a run-time test, costs the others registers
+// (flash32_resident_pair_kernel<64, false, true> 160 -> 169, a workgroup less per compute unit).  They are a translation unit
+// of their own too (attention_flash32_drop.hip, which defines this and includes this file), compiled beside this one.
+#ifndef FLASH32_DROP
+#define FLASH32_DROP 0
+#define FLASH32_LAUNCH launch_flash32_plain
+#else
+#define FLASH32_LAUNCH launch_flash32_drop
+#endif
+int32_t launch_flash32_plain(const AttnParams &, hipStream_t);
+int32_t launch_flash32_drop(const AttnParams &, hipStream_t);
+int attention_flash32_nsplit(const AttnParams &);
+size_t attention_flash32_lengths_bytes(const AttnParams &);
+
 namespace {
 
 typedef F32 T;
+constexpr bool DROP = FLASH32_DROP;
 constexpr int BN = FLASH_BN;
 
 template <int D, int QB>
@@ -110,7 +125,7 @@ __device__ inline void run_tiles32(const FlashArgs &a, Frag32<D, QB> &f, float *
                     }
             }
 
-            flash_softmax_tile<T, QB, D / 32, CAUSAL, EXTRAS ? EXTRAS_DIRECT : EXTRAS_NONE, PHASE, float>(a, s, f.o, f.m, f.l, b, h, iw, j0,
+            flash_softmax_tile<T, QB, D / 32, CAUSAL, EXTRAS ? EXTRAS_DIRECT : EXTRAS_NONE, PHASE, float, DROP>(a, s, f.o, f.m, f.l, b, h, iw, j0,
                                                                                                           FlashStaged<QB>(), 0, wlds, nullptr, kv_len);
 
             if (do_pv) {
@@ -327,7 +342,7 @@ __device__ inline void run_tiles32s(const FlashArgs &a, Frag32S<D, QB> &f, unsig
             floatx16_t s[QB][2];
             scores32s<D, QB>(f, Ks, s);
 
-            flash_softmax_tile<T, QB, D / 32, CAUSAL, EXTRAS ? EXTRAS_DIRECT : EXTRAS_NONE, PHASE, float>(a, s, f.o, f.m, f.l, b, h, iw, j0,
+            flash_softmax_tile<T, QB, D / 32, CAUSAL, EXTRAS ? EXTRAS_DIRECT : EXTRAS_NONE, PHASE, float, DROP>(a, s, f.o, f.m, f.l, b, h, iw, j0,
                                                                                                           FlashStaged<QB>(), 0, wlds, nullptr, kv_len);
 
             if (do_pv) weights_times_values32s<D, QB>(f, Vs, s);
@@ -661,7 +676,7 @@ __global__ __launch_bounds__(256, 1) void flash32_resident_kernel(FlashArgs a) {
     for (int t = 0; t < RES_TILES; t++)
         if (active[t]) {
             floatx16_t s[1][2] = {{keep[t][0][0], keep[t][0][1]}};
-            flash_softmax_tile<T, 1, D / 32, CAUSAL, XT, PHASE_STATS, float>(a, s, f.o, f.m, f.l, b, h, iw, (int64_t)t * BN, FlashStaged<1>(), 0, 0u,
+            flash_softmax_tile<T, 1, D / 32, CAUSAL, XT, PHASE_STATS, float, DROP>(a, s, f.o, f.m, f.l, b, h, iw, (int64_t)t * BN, FlashStaged<1>(), 0, 0u,
                                                                              nullptr, p.Lkv);
         }
     f.l[0] = 1.0f / (f.l[0] + mi_swap32(f.l[0]));
@@ -672,7 +687,7 @@ __global__ __launch_bounds__(256, 1) void flash32_resident_kernel(FlashArgs a) {
 #pragma unroll
     for (int t = 0; t < RES_TILES; t++)
         if (active[t]) {
-            flash_softmax_tile<T, 1, D / 32, CAUSAL, XT, PHASE_FINAL, float>(a, keep[t], f.o, f.m, f.l, b, h, iw, (int64_t)t * BN, FlashStaged<1>(), 0, wlds,
+            flash_softmax_tile<T, 1, D / 32, CAUSAL, XT, PHASE_FINAL, float, DROP>(a, keep[t], f.o, f.m, f.l, b, h, iw, (int64_t)t * BN, FlashStaged<1>(), 0, wlds,
                                                                              nullptr, p.Lkv);
             if (do_pv) weights_times_values32s<D, 1>(f, Vp + t * TILEB, keep[t]);
         }
@@ -824,7 +839,7 @@ __global__ __launch_bounds__(512, 1) void flash32_resident_pair_kernel(FlashArgs
     if (tile == 0) split_v();
     if (active) {
         floatx16_t s[1][2] = {{keep[0][0], keep[0][1]}};
-        flash_softmax_tile<T, 1, D / 32, CAUSAL, XT, PHASE_STATS, float>(a, s, f.o, f.m, f.l, b, h, iw, j0, FlashStaged<1>(), 0, 0u, nullptr, p.Lkv);
+        flash_softmax_tile<T, 1, D / 32, CAUSAL, XT, PHASE_STATS, float, DROP>(a, s, f.o, f.m, f.l, b, h, iw, j0, FlashStaged<1>(), 0, 0u, nullptr, p.Lkv);
     }
     // the pair's statistics: (m, l) of both tiles, combined as the online softmax combines tiles (src/softmax.jl:69-79
     // over the whole row): m = max, l = sum of l_i 2^((m_i - m) c); equal maxima (two -Inf or two +Inf included) keep
@@ -847,7 +862,7 @@ __global__ __launch_bounds__(512, 1) void flash32_resident_pair_kernel(FlashArgs
     // ---- weights and the wavefront's share of the output
     const unsigned wlds = lds0 + 4u * TILEB + wave * FLASH_WSTAGE_BYTES;
     if (active) {
-        flash_softmax_tile<T, 1, D / 32, CAUSAL, XT, PHASE_FINAL, float>(a, keep, f.o, f.m, f.l, b, h, iw, j0, FlashStaged<1>(), 0, wlds, nullptr, p.Lkv);
+        flash_softmax_tile<T, 1, D / 32, CAUSAL, XT, PHASE_FINAL, float, DROP>(a, keep, f.o, f.m, f.l, b, h, iw, j0, FlashStaged<1>(), 0, wlds, nullptr, p.Lkv);
         if (do_pv) weights_times_values32s<D, 1>(f, Vp + tile * TILEB, keep);
     }
     if (tile == 0 && p.weights) flash_zero_skipped_weights<1, float>(a, b, h, iw, n_tiles, CAUSAL);
@@ -1014,7 +1029,7 @@ __global__ __launch_bounds__(256, 1) void flash32_resident_quad_kernel(FlashArgs
     }
     if (active) {
         floatx16_t s[1][1] = {{keep[0][0]}};
-        flash_softmax_tile<T, 1, D / 32, CAUSAL, XT, PHASE_STATS, float, 1>(a, s, f.o, f.m, f.l, b, h, iw, j0, FlashStaged<1>(), 0, 0u, nullptr, p.Lkv);
+        flash_softmax_tile<T, 1, D / 32, CAUSAL, XT, PHASE_STATS, float, DROP, 1>(a, s, f.o, f.m, f.l, b, h, iw, j0, FlashStaged<1>(), 0, 0u, nullptr, p.Lkv);
     }
     // the workgroup's statistics: (m, l) of the four blocks, combined as the online softmax combines tiles
     // (src/softmax.jl:69-79 over the whole row): m = max, l = sum of l_i 2^((m_i - m) c); a block whose maximum is the
@@ -1043,7 +1058,7 @@ __global__ __launch_bounds__(256, 1) void flash32_resident_quad_kernel(FlashArgs
     // ---- weights and the wavefront's share of the output
     const unsigned wlds = lds0 + behind + wave * FLASH_WSTAGE_BYTES;
     if (active) {
-        flash_softmax_tile<T, 1, D / 32, CAUSAL, XT, PHASE_FINAL, float, 1>(a, keep, f.o, f.m, f.l, b, h, iw, j0, FlashStaged<1>(), 0, wlds, nullptr, p.Lkv);
+        flash_softmax_tile<T, 1, D / 32, CAUSAL, XT, PHASE_FINAL, float, DROP, 1>(a, keep, f.o, f.m, f.l, b, h, iw, j0, FlashStaged<1>(), 0, wlds, nullptr, p.Lkv);
         if (do_pv) weights_times_values32s<D, 1, 1>(f, Vp + blk, keep);
     }
     if (wave == 0 && p.weights) flash_zero_skipped_weights<1, float>(a, b, h, iw, n_tiles, false);
@@ -1207,7 +1222,7 @@ __global__ __launch_bounds__(256, 1) void flash32_resident_chunks_kernel(FlashAr
             }
             scores32s<D, 1, 1>(f, buf + blk, keep[c]);
             floatx16_t s[1][1] = {{keep[c][0][0]}};
-            flash_softmax_tile<T, 1, D / 32, CAUSAL, XT, PHASE_STATS, float, 1>(a, s, f.o, f.m, f.l, b, h, iw, 128 * (int64_t)c + 32 * wave, FlashStaged<1>(), 0,
+            flash_softmax_tile<T, 1, D / 32, CAUSAL, XT, PHASE_STATS, float, DROP, 1>(a, s, f.o, f.m, f.l, b, h, iw, 128 * (int64_t)c + 32 * wave, FlashStaged<1>(), 0,
                                                                                  0u, nullptr, p.Lkv);
 #pragma unroll
             for (int t = 0; t < 2; t++)
@@ -1249,7 +1264,7 @@ __global__ __launch_bounds__(256, 1) void flash32_resident_chunks_kernel(FlashAr
                 store_chunk(buf, reg);
                 __syncthreads();   // V chunk c in LDS; with two buffers: every wavefront is done with chunk c - 1
             }
-            flash_softmax_tile<T, 1, D / 32, CAUSAL, XT, PHASE_FINAL, float, 1>(a, keep[c], f.o, f.m, f.l, b, h, iw, 128 * (int64_t)c + 32 * wave, FlashStaged<1>(),
+            flash_softmax_tile<T, 1, D / 32, CAUSAL, XT, PHASE_FINAL, float, DROP, 1>(a, keep[c], f.o, f.m, f.l, b, h, iw, 128 * (int64_t)c + 32 * wave, FlashStaged<1>(),
                                                                                  0, wlds, nullptr, p.Lkv);
             if (do_pv) {
                 weights_times_values32s<D, 1, 1>(f, buf + blk, keep[c]);
@@ -1405,6 +1420,7 @@ int32_t launch_d(const FlashArgs &a, hipStream_t st, bool extras) {
 
 }  // namespace
 
+#if !FLASH32_DROP
 int attention_flash32_nsplit(const AttnParams &p) {
     if (flash_is_query_independent_mask(p) || p.Lq > 65535 || p.B > 65535) return 1;   // context lengths instead / merge kernel's grid limits
     return flash_pick_nsplit(p, 128);
@@ -1425,8 +1441,9 @@ bool attention_flash32_supports(const AttnParams &p) {
     const int64_t tiles = (p.Lq + 127) / 128;
     return tiles * p.H * p.B <= 2147483647LL;
 }
+#endif
 
-int32_t launch_attention_flash32(const AttnParams &p, hipStream_t st) {
+int32_t FLASH32_LAUNCH(const AttnParams &p, hipStream_t st) {
     FlashArgs a;
     a.p = p;
     a.nsplit = 1;
@@ -1483,3 +1500,9 @@ int32_t launch_attention_flash32(const AttnParams &p, hipStream_t st) {
     }
     return narrow ? launch_d<64, 1>(a, st, extras) : launch_d<128, 1>(a, st, extras);
 }
+
+#if !FLASH32_DROP
+int32_t launch_attention_flash32(const AttnParams &p, hipStream_t st) {
+    return p.drop_thresh ? launch_flash32_drop(p, st) : launch_flash32_plain(p, st);
+}
+#endif

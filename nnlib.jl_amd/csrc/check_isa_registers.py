@@ -10,6 +10,9 @@ flow-insensitive on purpose: it only asks, per kernel, that every VGPR / AGPR th
 a destination somewhere, which is cheap, has no false positives beyond the registers the hardware initialises (v0 - v2:
 work-item ids), and catches exactly that class of miscompile.
 
+It also holds the kernels of NO_SCRATCH to their registers: those whose 512 registers have spilled, or whose workgroups per
+compute unit have dropped, when code behind a run-time test grew that their calls never reach.
+
 usage: check_isa_registers.py file.s [file.s ...]   (exit status 1 and one line per finding if any)
 """
 import re
@@ -18,6 +21,10 @@ import sys
 REG = re.compile(r'\b([av])(\d+)\b|\b([av])\[(\d+):(\d+)\]')
 # instructions without a register destination: every operand is a source
 STORES = ('scratch_store', 'global_store', 'flat_store', 'buffer_store', 'ds_write', 'ds_store', 's_waitcnt', 's_nop')
+# (source file, mangled kernel name) of kernels without scratch memory: Float32 forward with bias / mask code; 16-bit forward
+# up to head dim 64 without weights or keep decisions, bias by rows or direct loads apart
+NO_SCRATCH = [(re.compile(r'attention_flash32'), re.compile(r'14flash32_kernelILi(64|128)ELi1ELb[01]ELb1E')),
+              (re.compile(r'attention_flash16_b?f16_d64'), re.compile(r'14flash16_kernelILi1ELb[01]ELi[02347]ELb0EfLb0E'))]
 
 
 def regs(text):
@@ -33,6 +40,7 @@ def regs(text):
 def check(path):
     findings = []
     kernel, written, read, first_read = None, set(), set(), {}
+    described = None   # the kernel whose descriptor this is
     for ln, line in enumerate(open(path, errors='replace'), 1):
         code = line.split(';')[0].strip()
         if not code:
@@ -40,6 +48,11 @@ def check(path):
         if code.endswith(':') and not code.startswith('.'):
             kernel, written, read, first_read = code[:-1], set(), set(), {}
             continue
+        if code.startswith('.amdhsa_kernel'):
+            described = code.split()[1]
+        if code.startswith('.amdhsa_private_segment_fixed_size') and int(code.split()[1]) > 0:
+            if any(f.search(path) and k.search(described) for f, k in NO_SCRATCH):
+                findings.append(f"{path}: {described}: {code.split()[1]} bytes of scratch memory, none allowed")
         if code.startswith('.end_amdhsa_kernel') or code.startswith('.section'):
             continue
         if kernel is None or code.startswith('.'):
@@ -70,5 +83,5 @@ if __name__ == '__main__':
         bad += check(f)
     for b in bad:
         print(b)
-    print(f"{len(sys.argv) - 1} files, {len(bad)} registers read and never written")
+    print(f"{len(sys.argv) - 1} files, {len(bad)} findings")
     sys.exit(1 if bad else 0)

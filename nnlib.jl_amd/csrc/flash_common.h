@@ -498,8 +498,9 @@ __device__ inline void flash_mask_apply4(floatx16_t &v, int g, uint32_t m4) {
 // it stay below 2^8, which Float32 sums and 16-bit operands hold without loss.
 constexpr float FLASH_LAZY_MAX_LOG2 = 8.0f;
 
-// KBLK: 32-key blocks per tile (2: the 64-key tile of the tile loops; 1: a wavefront that owns a single block)
-template <typename T, int QB, int NDV, bool CAUSAL, int EXTRAS, int PHASE, typename TW, int KBLK = 2>
+// DROP: the call has fused dropout.  KBLK: 32-key blocks per tile (2: the 64-key tile of the tile loops; 1: a wavefront that
+// owns a single block)
+template <typename T, int QB, int NDV, bool CAUSAL, int EXTRAS, int PHASE, typename TW, bool DROP = false, int KBLK = 2>
 __device__ inline void flash_softmax_tile(const FlashArgs &a, floatx16_t (&s)[QB][KBLK], floatx16_t (&o)[QB][NDV],
                                           float (&fm)[QB], float (&fl)[QB], int64_t b, int64_t h, int64_t iw,
                                           int64_t j0, const FlashStaged<QB> &sg = FlashStaged<QB>(), int stage = 0,
@@ -546,50 +547,59 @@ __device__ inline void flash_softmax_tile(const FlashArgs &a, floatx16_t (&s)[QB
                     }
             }
         } else if (EXTRAS == EXTRAS_DIRECT) {
+            // The offsets of a lane's first entries are opaque, so that every tile computes the others from them: the compiler
+            // otherwise keeps a pointer for every entry of a tile through the loop, 64 a lane (Float32 with a causal mask:
+            // 496 to 592 bytes of scratch at head dims 65 to 128, none so; 199 to 222 AGPRs at 64, 81 so)
             const elem_t *bias = (const elem_t *)p.bias;
-            const int64_t boff = qi * p.bias_strides[1] + h * p.bias_strides[2] + b * p.bias_strides[3];
-            const int64_t moff = qi * p.mask_strides[1] + h * p.mask_strides[2] + b * p.mask_strides[3];
+            const int64_t bstep = p.bias_strides[0], mstep = p.mask_strides[0];
+            int64_t boff = qi * p.bias_strides[1] + h * p.bias_strides[2] + b * p.bias_strides[3] + (j0 + 4 * hh) * bstep;
+            int64_t moff = qi * p.mask_strides[1] + h * p.mask_strides[2] + b * p.mask_strides[3] + (j0 + 4 * hh) * mstep;
+            if (KBLK == 2) asm volatile("" : "+v"(boff), "+v"(moff));   // (single blocks are in no such loop)
+            const int there = (int)(p.Lkv - j0 > BN ? BN : p.Lkv - j0) - 4 * hh;   // keys of the tile from this lane's first one on
+            if (bias && qok) {
 #pragma unroll
-            for (int kb = 0; kb < KBLK; kb++)
+                for (int kb = 0; kb < KBLK; kb++)
 #pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    const int64_t kv = j0 + 32 * kb + 8 * g + 4 * hh;
-                    float bv[4] = {0.f, 0.f, 0.f, 0.f};
-                    bool keep[4];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) keep[e] = kv + e < p.Lkv && (!CAUSAL || kv + e <= qi);
-                    if (bias && qok) {
+                    for (int g = 0; g < 4; g++) {
+                        const int at = 32 * kb + 8 * g;
+                        float bv[4] = {0.f, 0.f, 0.f, 0.f};
                         if (a.bias_vec) {
-                            if (kv < p.Lkv) {
-                                typename T::vec4 t4 = *(const typename T::vec4 *)(bias + boff + kv);
+                            if (at < there) {
+                                typename T::vec4 t4 = *(const typename T::vec4 *)(bias + boff + at);
 #pragma unroll
                                 for (int e = 0; e < 4; e++) bv[e] = T::to_f32(t4[e]);
                             }
                         } else {
 #pragma unroll
                             for (int e = 0; e < 4; e++)
-                                if (kv + e < p.Lkv) bv[e] = T::to_f32(bias[boff + (kv + e) * p.bias_strides[0]]);
+                                if (at + e < there) bv[e] = T::to_f32(bias[boff + (at + e) * bstep]);
                         }
-                    }
-                    if (p.mask && qok) {
-                        if (a.mask_vec) {
-                            if (kv < p.Lkv) {
-                                uint32_t m4 = *(const uint32_t *)(p.mask + moff + kv);
 #pragma unroll
-                                for (int e = 0; e < 4; e++) keep[e] = keep[e] && ((m4 >> (8 * e)) & 0xFF);
-                            }
+                        for (int e = 0; e < 4; e++) s[qb][kb][4 * g + e] = fmaf(s[qb][kb][4 * g + e], a.cn, bv[e]);
+                    }
+            } else {
+#pragma unroll
+                for (int kb = 0; kb < KBLK; kb++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) s[qb][kb][v] *= a.cn;
+            }
+            if (p.mask && qok) {
+#pragma unroll
+                for (int kb = 0; kb < KBLK; kb++)
+#pragma unroll
+                    for (int g = 0; g < 4; g++) {
+                        const int at = 32 * kb + 8 * g;
+                        uint32_t m4 = 0;
+                        if (a.mask_vec) {
+                            if (at < there) m4 = *(const uint32_t *)(p.mask + moff + at);
                         } else {
 #pragma unroll
                             for (int e = 0; e < 4; e++)
-                                if (kv + e < p.Lkv) keep[e] = keep[e] && p.mask[moff + (kv + e) * p.mask_strides[0]];
+                                if (at + e < there) m4 |= (uint32_t)p.mask[moff + (at + e) * mstep] << (8 * e);
                         }
+                        flash_mask_apply4(s[qb][kb], g, m4);
                     }
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        float x = fmaf(s[qb][kb][4 * g + e], a.cn, bv[e]);
-                        s[qb][kb][4 * g + e] = keep[e] ? x : MI_NEG_INF;
-                    }
-                }
+            }
         }
         if (EXTRAS == EXTRAS_MASKTILE) {
             const int row = 32 * qb + r;
@@ -609,7 +619,7 @@ __device__ inline void flash_softmax_tile(const FlashArgs &a, floatx16_t (&s)[QB
                 for (int g = 0; g < 4; g++) flash_mask_apply4(s[qb][kb], g, key_mask ? key_mask[4 * kb + g] : own[4 * kb + g]);
             }
         }
-        if (EXTRAS != EXTRAS_DIRECT && edge) {
+        if (edge) {
             // keys past the end of the sequence or, causal, after the query: tile-local limit per lane
             int64_t lim64 = lkv - j0;
             if (CAUSAL && qi - j0 + 1 < lim64) lim64 = qi - j0 + 1;
@@ -686,7 +696,7 @@ __device__ inline void flash_softmax_tile(const FlashArgs &a, floatx16_t (&s)[QB
 
         // fdrop = dropout (src/attention.jl:126): after the softmax, so the row sum above is untouched;
         // before the value product and before the weights are written, which are post-dropout.
-        if (PHASE != PHASE_STATS && p.drop_thresh != 0) {
+        if constexpr (DROP && PHASE != PHASE_STATS) {
             const uint64_t row0 = (uint64_t)(p.Lkv * (qi + p.Lq * (h + p.H * b)) + j0);
             if ((p.Lkv & 3) == 0) {   // every run of four keys of a lane is one hash group
 #pragma unroll

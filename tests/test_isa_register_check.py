@@ -61,3 +61,21 @@ def test_two_kernels_are_checked_apart(tmp_path):
                  + "\t.globl\tother\nother:\n\tglobal_store_dword v[0:1], v5, off\n\ts_endpgm\n\t.amdhsa_kernel other\n\t.end_amdhsa_kernel\n")
     found = chk.check(str(f))
     assert len(found) == 1 and "other" in found[0] and "v5" in found[0], found
+
+
+def test_scratch_of_kernels_that_have_none(tmp_path):
+    """A Float32 kernel with bias / mask code that spills is found (it took 588 bytes a lane once, for the code of a dropout
+    that its calls did not have); its neighbours without that code may."""
+    def described(name, scratch):
+        return f"\t.amdhsa_kernel {name}\n\t\t.amdhsa_private_segment_fixed_size {scratch}\n\t.end_amdhsa_kernel\n"
+    kern = "_ZN12_GLOBAL__N_114flash32_kernelILi128ELi1ELb1ELb%dELb0ELb1EEEv9FlashArgs"
+    f = tmp_path / "attention_flash32-hip-amdgcn.s"
+    f.write_text(described(kern % 1, 588) + described(kern % 0, 28))
+    found = chk.check(str(f))
+    assert len(found) == 1 and kern % 1 in found[0] and "588" in found[0], found
+    f.write_text(described(kern % 1, 0))
+    assert chk.check(str(f)) == []
+    g = tmp_path / "attention_flash16_bf16_d64-hip-amdgcn.s"
+    g.write_text(described("_ZN12_GLOBAL__N_114flash16_kernelILi1ELb0ELi0ELb0EfLb0EEEv9FlashArgs", 4)
+                 + described("_ZN12_GLOBAL__N_114flash16_kernelILi1ELb0ELi7ELb0EfLb1EEEv9FlashArgs", 12))
+    assert len(chk.check(str(g))) == 1
