@@ -19,7 +19,7 @@ int32_t launch_batched_gemm16(int32_t dtype, int transA, int transB, int64_t m, 
 
 // tiled Float32 fast path (batched_gemm32.hip)
 bool batched_gemm32_supports(int32_t dtype, int transA, int transB, int64_t m, int64_t n, int64_t k, const void *A, int64_t lda,
-                             int64_t sA, const void *B, int64_t ldb, int64_t sB, int64_t batch);
+                             int64_t sA, const void *B, int64_t ldb, int64_t sB);
 int32_t launch_batched_gemm32_sum(int transA, int transB, int64_t m, int64_t n, int64_t k, float alpha, const void *A, int64_t lda,
                                   int64_t sA, const void *B, int64_t ldb, int64_t sB, float beta, void *C, int64_t ldc, int64_t batch,
                                   hipStream_t st);
@@ -233,7 +233,7 @@ MI_API int32_t mi_batched_gemm(int32_t dtype, char transA, char transB, int64_t 
     hipStream_t st = (hipStream_t)s;
     if (batched_gemm16_supports(dtype, ta, tb, m, n, k, lda, ldb))
         return launch_batched_gemm16(dtype, ta, tb, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, strideC, batch, st);
-    if (batched_gemm32_supports(dtype, ta, tb, m, n, k, A, lda, strideA, B, ldb, strideB, batch))
+    if (batched_gemm32_supports(dtype, ta, tb, m, n, k, A, lda, strideA, B, ldb, strideB))
         return launch_batched_gemm32(ta, tb, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, strideC, batch, st);
     if (dtype == MI_F32) return launch<F32>(g, batch, st);
     if (dtype == MI_F16) return launch<F16>(g, batch, st);
@@ -253,7 +253,7 @@ MI_API int32_t mi_batched_gemm_sum(int32_t dtype, char transA, char transB, int6
     if (k == 0 || batch == 0)
         return mi_batched_gemm(dtype, transA, transB, m, n, 0, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, 0, 1, s);
     if (!C || !A || !B) return mi_set_error(MI_EINVAL, "mi_batched_gemm_sum: null pointer");
-    if (batched_gemm32_supports(dtype, ta, tb, m, n, k, A, lda, strideA, B, ldb, strideB, 1))
+    if (batched_gemm32_supports(dtype, ta, tb, m, n, k, A, lda, strideA, B, ldb, strideB))
         return launch_batched_gemm32_sum(ta, tb, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, batch, (hipStream_t)s);
     for (int64_t b = 0; b < batch; b++) {
         const int32_t rb = mi_batched_gemm(dtype, transA, transB, m, n, k, alpha, (const float *)A + b * strideA, lda, 0, (const float *)B + b * strideB,

@@ -15,7 +15,7 @@
 #include <type_traits>
 
 // a wavefront per tile, no LDS between operands and products (batched_gemm32_waves.hip)
-bool gemm32_waves_supports(int transA, int transB, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, int64_t batch);
+bool gemm32_waves_supports(int transA, int transB, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb);
 double gemm32_waves_estimate(int64_t m, int64_t n, int64_t k, int64_t slices, int64_t batch);
 int32_t launch_gemm32_waves(int transA, int transB, int64_t m, int64_t n, int64_t k, float alpha, const void *A, int64_t lda,
                             int64_t sA, const void *B, int64_t ldb, int64_t sB, float beta, void *C, int64_t ldc, int64_t sC,
@@ -533,14 +533,14 @@ static bool tiles_support(int transA, int transB, int64_t m, int64_t n, int64_t 
     // leading dimensions of at least a piece: only the last k or row of a slice can hold a piece that ends past it
     return lda >= 4 && ldb >= 4 && extA >= 4 && extB >= 4 && extA * 4 < 2147483647LL && extB * 4 < 2147483647LL;
 }
-static bool waves_support(int transA, int transB, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, int64_t batch) {
-    return k >= 1 && !exact_instruction_wanted() && gemm32_waves_supports(transA, transB, m, n, k, lda, ldb, batch);
+static bool waves_support(int transA, int transB, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb) {
+    return k >= 1 && !exact_instruction_wanted() && gemm32_waves_supports(transA, transB, m, n, k, lda, ldb);
 }
 
 bool batched_gemm32_supports(int32_t dtype, int transA, int transB, int64_t m, int64_t n, int64_t k, const void *A, int64_t lda,
-                             int64_t sA, const void *B, int64_t ldb, int64_t sB, int64_t batch) {
+                             int64_t sA, const void *B, int64_t ldb, int64_t sB) {
     if (dtype != MI_F32) return false;
-    return waves_support(transA, transB, m, n, k, lda, ldb, batch) || tiles_support(transA, transB, m, n, k, A, lda, sA, B, ldb, sB);
+    return waves_support(transA, transB, m, n, k, lda, ldb) || tiles_support(transA, transB, m, n, k, A, lda, sA, B, ldb, sB);
 }
 
 // The large tile where the share of its slots that does useful work, counting padded rows and columns and the last round of
@@ -565,7 +565,7 @@ int32_t launch_batched_gemm32(int transA, int transB, int64_t m, int64_t n, int6
                               int64_t sA, const void *B, int64_t ldb, int64_t sB, float beta, void *C, int64_t ldc, int64_t sC,
                               int64_t batch, hipStream_t st) {
     const bool a_rm = !transA, b_rm = transB != 0;
-    if (waves_support(transA, transB, m, n, k, lda, ldb, batch) &&
+    if (waves_support(transA, transB, m, n, k, lda, ldb) &&
         (!tiles_support(transA, transB, m, n, k, A, lda, sA, B, ldb, sB) || gemm32_waves_estimate(m, n, k, 1, batch) < tiles_estimate(m, n, k, batch)))
         return launch_gemm32_waves(transA, transB, m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, 1, batch, st);
     for (int64_t b0 = 0; b0 < batch; b0 += 65535) {   // gridDim.z is limited to 65535: issue the batch in slabs
@@ -597,7 +597,7 @@ int32_t launch_batched_gemm32_sum(int transA, int transB, int64_t m, int64_t n, 
                                   hipStream_t st) {
     const bool tiles = tiles_support(transA, transB, m, n, k, A, lda, sA, B, ldb, sB);
     const double apart = (double)batch * fmin(gemm32_waves_estimate(m, n, k, 1, 1), tiles ? tiles_estimate(m, n, k, 1) : 1e30);
-    if (batch <= 2147483647LL / ((k + 15) / 16) && waves_support(transA, transB, m, n, k, lda, ldb, 1) && gemm32_waves_estimate(m, n, k, batch, 1) < apart)
+    if (batch <= 2147483647LL / ((k + 15) / 16) && waves_support(transA, transB, m, n, k, lda, ldb) && gemm32_waves_estimate(m, n, k, batch, 1) < apart)
         return launch_gemm32_waves(transA, transB, m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, 0, batch, 1, st);
     for (int64_t b = 0; b < batch; b++) {
         const int32_t rc = launch_batched_gemm32(transA, transB, m, n, k, alpha, (const float *)A + b * sA, lda, sA, (const float *)B + b * sB, ldb, sB,

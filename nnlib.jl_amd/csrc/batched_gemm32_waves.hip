@@ -257,16 +257,25 @@ __global__ __launch_bounds__(64 * SPLIT, BM * BN == 1 ? 5 : 2) void gemm32_waves
     }
 }
 
+// work items of a launch are counted in 32 bits: larger batches go in slabs of slices
+constexpr int64_t MOST_THREADS = ((int64_t)1 << 32) - 1;
+
 template <int BM, int BN, int SPLIT>
 int32_t launch_waves(WaveArgs g, bool a_rm, bool b_rm, int64_t nb, hipStream_t st) {
     g.tiles_m = (int32_t)((g.m + 32 * BM - 1) / (32 * BM));
     g.tiles_n = (int32_t)((g.n + 32 * BN - 1) / (32 * BN));
-    const dim3 grid((unsigned)((int64_t)g.tiles_m * g.tiles_n * nb)), block(64 * SPLIT);
-    if (a_rm && b_rm) hipLaunchKernelGGL((gemm32_waves_kernel<true, true, BM, BN, SPLIT>), grid, block, 0, st, g);
-    else if (a_rm) hipLaunchKernelGGL((gemm32_waves_kernel<true, false, BM, BN, SPLIT>), grid, block, 0, st, g);
-    else if (b_rm) hipLaunchKernelGGL((gemm32_waves_kernel<false, true, BM, BN, SPLIT>), grid, block, 0, st, g);
-    else hipLaunchKernelGGL((gemm32_waves_kernel<false, false, BM, BN, SPLIT>), grid, block, 0, st, g);
-    MI_LAUNCH_CHECK();
+    const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n, most = MOST_THREADS / (64 * SPLIT) / tiles;   // slices per launch, at least one
+    for (int64_t b0 = 0; b0 < nb; b0 += most) {
+        const dim3 grid((unsigned)(tiles * (nb - b0 < most ? nb - b0 : most))), block(64 * SPLIT);
+        if (a_rm && b_rm) hipLaunchKernelGGL((gemm32_waves_kernel<true, true, BM, BN, SPLIT>), grid, block, 0, st, g);
+        else if (a_rm) hipLaunchKernelGGL((gemm32_waves_kernel<true, false, BM, BN, SPLIT>), grid, block, 0, st, g);
+        else if (b_rm) hipLaunchKernelGGL((gemm32_waves_kernel<false, true, BM, BN, SPLIT>), grid, block, 0, st, g);
+        else hipLaunchKernelGGL((gemm32_waves_kernel<false, false, BM, BN, SPLIT>), grid, block, 0, st, g);
+        MI_LAUNCH_CHECK();
+        g.A += most * g.sA;
+        g.B += most * g.sB;
+        g.C += most * g.sC;
+    }
     return MI_OK;
 }
 
@@ -296,11 +305,12 @@ const Variant &fastest(int64_t m, int64_t n, int64_t steps, int64_t batch) {
 
 }  // namespace
 
-// 32-bit byte offsets reach every element of a slice, and the end of its last step of 16 k
-bool gemm32_waves_supports(int transA, int transB, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, int64_t batch) {
+// 32-bit byte offsets reach every element of a slice, and the end of its last step of 16 k; a slice fits one launch of eight
+// wavefronts a tile
+bool gemm32_waves_supports(int transA, int transB, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb) {
     const int64_t reachA = transA ? m * lda + k : (k + 16) * lda + m, reachB = transB ? (k + 16) * ldb + n : n * ldb + k;
     if (reachA >= (int64_t)1 << 29 || reachB >= (int64_t)1 << 29) return false;
-    return ((m + 31) / 32) * ((n + 31) / 32) <= 2147483647LL / batch;
+    return ((m + 31) / 32) * ((n + 31) / 32) <= MOST_THREADS / 512;
 }
 
 double gemm32_waves_estimate(int64_t m, int64_t n, int64_t k, int64_t slices, int64_t batch) {

@@ -608,3 +608,16 @@ def test_pullback_of_a_shared_operand(nn, dtype, m, n, k, nb):
     _, dB = nn.batched_mul_pullback(D(A), D(B[:, :, :1]), D(dC))
     ref = np.einsum("mkb,mnb->kn", A.astype(np.float64), dC.astype(np.float64))
     assert dB.dims == (k, n, 1) and np.abs(dB.to_numpy()[:, :, 0] - ref).max() <= tol * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("batch", [2 ** 26 - 1, 2 ** 26 + 70000])
+def test_very_many_tiny_float32_products(nn, batch):
+    """More slices than one launch of a wavefront per slice can count (2^32 work items): the batch goes in slabs, the last
+    slices of the first and the first of the second included."""
+    import torch
+    rng = torch.Generator(device="cuda").manual_seed(batch)
+    a, b = (torch.rand(batch, generator=rng, device="cuda") + 0.5 for _ in range(2))
+    A, B = (nn.DeviceArray(x, (1, 1, batch), "f32") for x in (a, b))
+    C = nn.batched_mul(A, B)
+    ref = a.double() * b.double()
+    assert C.dims == (1, 1, batch) and bool(((C.storage.double() - ref).abs() <= 2.0 ** -22 * ref).all())
