@@ -113,8 +113,14 @@ __device__ inline void split_step(const float (&x)[NB][8], plane8 (&pl)[NB][3]) 
     }
 }
 
-template <bool A_RM, bool B_RM, int BM, int BN, int SPLIT>
-__global__ __launch_bounds__(64 * SPLIT, BM * BN == 1 ? 5 : 2) void gemm32_waves_kernel(WaveArgs g) {
+// SUM: one result, the sum over the slices.  Every slice's products have an accumulator of their own, which is added to the
+// sum when the next slice starts, as a product per slice adds to C.  One accumulator over all of them errs with the root of
+// its length (against 64 bits, 2-norm, one accumulator / this / a product per slice: 333 x 77 x 517 over 96 slices 1.5e-6 /
+// 3.0e-7 / 3.0e-7, 32 x 32 x 77 over 96 5.1e-7 / 2.5e-7 / 2.7e-7), and is 3 to 9 % faster: the sums wait for a slice's last
+// matrix instruction and take registers of their own (464 x 16 x 416 over 28 slices 69.4 / 71.6 us, 16 x 16 x 16 over 1000
+// 122 / 132), for which the wavefronts a SIMD go from five to four, with 2 x 2 blocks from two to one.
+template <bool A_RM, bool B_RM, int BM, int BN, int SPLIT, bool SUM>
+__global__ __launch_bounds__(64 * SPLIT, BM * BN == 1 ? (SUM ? 4 : 5) : (SUM ? 1 : 2)) void gemm32_waves_kernel(WaveArgs g) {
     constexpr int LDW = 32 * BM + 4;   // floats per LDS row
     __shared__ __attribute__((aligned(16))) float part[SPLIT][32 * LDW];
     const int lane = threadIdx.x & 63, r = lane & 31, hh = lane >> 5;
@@ -128,7 +134,7 @@ __global__ __launch_bounds__(64 * SPLIT, BM * BN == 1 ? 5 : 2) void gemm32_waves
 
     WaveOperand<A_RM, BM> a;
     WaveOperand<B_RM, BN> b;
-    const int64_t z = g.slices > 1 ? 0 : bz;
+    const int64_t z = SUM ? 0 : bz;
     a.init(g.A + z * g.sA, g.lda, g.sA, g.m, g.k, m0);
     b.init(g.B + z * g.sB, g.ldb, g.sB, g.n, g.k, n0);
 
@@ -137,6 +143,22 @@ __global__ __launch_bounds__(64 * SPLIT, BM * BN == 1 ? 5 : 2) void gemm32_waves
     for (int i = 0; i < BN; i++)
 #pragma unroll
         for (int j = 0; j < BM; j++) acc[i][j] = (floatx16_t){0};
+
+    floatx16_t total[BN][BM];   // SUM: the slices before the present one
+#pragma unroll
+    for (int i = 0; i < BN; i++)
+#pragma unroll
+        for (int j = 0; j < BM; j++) total[i][j] = (floatx16_t){0};
+    const auto next_slice = [&] {
+#pragma unroll
+        for (int i = 0; i < BN; i++)
+#pragma unroll
+            for (int j = 0; j < BM; j++) {
+#pragma unroll
+                for (int v = 0; v < 16; v++) total[i][j][v] += acc[i][j][v];
+                acc[i][j] = (floatx16_t){0};
+            }
+    };
 
     // steps wave, wave + SPLIT, ... of the slices' steps, one after the other; two steps' loads are in flight
     const int per_slice = (int)((g.k + 15) / 16), k = (int)g.k;
@@ -157,13 +179,14 @@ __global__ __launch_bounds__(64 * SPLIT, BM * BN == 1 ? 5 : 2) void gemm32_waves
         a.load(s.sl, 16 * s.st, k - 16 * s.st, xa[at]);
         b.load(s.sl, 16 * s.st, k - 16 * s.st, xb[at]);
     };
-    const auto multiply = [&](Step ahead, int at) {
+    const auto multiply = [&](Step ahead, int at, bool first_of_slice) {
         extremes<BM>(xa[at], lo, hi);
         extremes<BN>(xb[at], lo, hi);
         plane8 av[BM][3], bv[BN][3];
         split_step<BM>(xa[at], av);
         split_step<BN>(xb[at], bv);
         fetch(ahead, at);
+        if (SUM && first_of_slice) next_slice();
         constexpr int ia[6] = {2, 0, 1, 1, 0, 0}, ib[6] = {0, 2, 1, 0, 1, 0};   // small terms first
 #pragma unroll
         for (int t = 0; t < 6; t++)
@@ -176,12 +199,14 @@ __global__ __launch_bounds__(64 * SPLIT, BM * BN == 1 ? 5 : 2) void gemm32_waves
     const Step first = next({0, wave - SPLIT});
     {
         Step s0 = first, s1 = next(first);
+        int slice = first.sl;
         fetch(s0, 0);
         fetch(s1, 1);
         while (s0.sl < g.slices) {
             const Step s2 = next(s1), s3 = next(s2);
-            multiply(s2, 0);
-            if (s1.sl < g.slices) multiply(s3, 1);
+            multiply(s2, 0, s0.sl != slice);
+            if (s1.sl < g.slices) multiply(s3, 1, s1.sl != s0.sl);
+            slice = s1.sl;
             s0 = s2;
             s1 = s3;
         }
@@ -191,9 +216,12 @@ __global__ __launch_bounds__(64 * SPLIT, BM * BN == 1 ? 5 : 2) void gemm32_waves
 #pragma unroll
         for (int i = 0; i < BN; i++)
 #pragma unroll
-            for (int j = 0; j < BM; j++) acc[i][j] = (floatx16_t){0};
+            for (int j = 0; j < BM; j++) acc[i][j] = total[i][j] = (floatx16_t){0};
+        int slice = first.sl;
         for (Step s = first; s.sl < g.slices; s = next(s)) {
             fetch(s, 0);
+            if (SUM && s.sl != slice) next_slice();
+            slice = s.sl;
 #pragma unroll
             for (int e = 0; e < 8; e++)
 #pragma unroll
@@ -202,6 +230,8 @@ __global__ __launch_bounds__(64 * SPLIT, BM * BN == 1 ? 5 : 2) void gemm32_waves
                     for (int j = 0; j < BM; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(xb[0][i][e], xa[0][j][e], acc[i][j], 0, 0, 0);
         }
     }
+
+    if (SUM) next_slice();
 
     // 32 columns of the tile at a time: every wavefront leaves its sums in LDS, the workgroup adds them and stores 16-byte
     // pieces along m.  Register v of lane (r, hh) of block (i, j): n = 32i + 8*(v/4) + 4*hh + v%4, m = 32j + r.
@@ -217,7 +247,7 @@ __global__ __launch_bounds__(64 * SPLIT, BM * BN == 1 ? 5 : 2) void gemm32_waves
 #pragma unroll
         for (int j = 0; j < BM; j++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) part[wave][(8 * (v / 4) + 4 * hh + (v % 4)) * LDW + 32 * j + r] = acc[i][j][v];
+            for (int v = 0; v < 16; v++) part[wave][(8 * (v / 4) + 4 * hh + (v % 4)) * LDW + 32 * j + r] = SUM ? total[i][j][v] : acc[i][j][v];
         if (SPLIT > 1) __syncthreads();
         else {
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -260,17 +290,17 @@ __global__ __launch_bounds__(64 * SPLIT, BM * BN == 1 ? 5 : 2) void gemm32_waves
 // work items of a launch are counted in 32 bits: larger batches go in slabs of slices
 constexpr int64_t MOST_THREADS = ((int64_t)1 << 32) - 1;
 
-template <int BM, int BN, int SPLIT>
+template <int BM, int BN, int SPLIT, bool SUM>
 int32_t launch_waves(WaveArgs g, bool a_rm, bool b_rm, int64_t nb, hipStream_t st) {
     g.tiles_m = (int32_t)((g.m + 32 * BM - 1) / (32 * BM));
     g.tiles_n = (int32_t)((g.n + 32 * BN - 1) / (32 * BN));
     const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n, most = MOST_THREADS / (64 * SPLIT) / tiles;   // slices per launch, at least one
     for (int64_t b0 = 0; b0 < nb; b0 += most) {
         const dim3 grid((unsigned)(tiles * (nb - b0 < most ? nb - b0 : most))), block(64 * SPLIT);
-        if (a_rm && b_rm) hipLaunchKernelGGL((gemm32_waves_kernel<true, true, BM, BN, SPLIT>), grid, block, 0, st, g);
-        else if (a_rm) hipLaunchKernelGGL((gemm32_waves_kernel<true, false, BM, BN, SPLIT>), grid, block, 0, st, g);
-        else if (b_rm) hipLaunchKernelGGL((gemm32_waves_kernel<false, true, BM, BN, SPLIT>), grid, block, 0, st, g);
-        else hipLaunchKernelGGL((gemm32_waves_kernel<false, false, BM, BN, SPLIT>), grid, block, 0, st, g);
+        if (a_rm && b_rm) hipLaunchKernelGGL((gemm32_waves_kernel<true, true, BM, BN, SPLIT, SUM>), grid, block, 0, st, g);
+        else if (a_rm) hipLaunchKernelGGL((gemm32_waves_kernel<true, false, BM, BN, SPLIT, SUM>), grid, block, 0, st, g);
+        else if (b_rm) hipLaunchKernelGGL((gemm32_waves_kernel<false, true, BM, BN, SPLIT, SUM>), grid, block, 0, st, g);
+        else hipLaunchKernelGGL((gemm32_waves_kernel<false, false, BM, BN, SPLIT, SUM>), grid, block, 0, st, g);
         MI_LAUNCH_CHECK();
         g.A += most * g.sA;
         g.B += most * g.sB;
@@ -303,6 +333,13 @@ const Variant &fastest(int64_t m, int64_t n, int64_t steps, int64_t batch) {
     return *best;
 }
 
+template <bool SUM>
+int32_t launch_variant(const WaveArgs &g, const Variant &v, bool a_rm, bool b_rm, int64_t batch, hipStream_t st) {
+    if (v.bm == 2) return v.split == 1 ? launch_waves<2, 2, 1, SUM>(g, a_rm, b_rm, batch, st) : launch_waves<2, 2, 4, SUM>(g, a_rm, b_rm, batch, st);
+    if (v.split == 1) return launch_waves<1, 1, 1, SUM>(g, a_rm, b_rm, batch, st);
+    return v.split == 4 ? launch_waves<1, 1, 4, SUM>(g, a_rm, b_rm, batch, st) : launch_waves<1, 1, 8, SUM>(g, a_rm, b_rm, batch, st);
+}
+
 }  // namespace
 
 // 32-bit byte offsets reach every element of a slice, and the end of its last step of 16 k; a slice fits one launch of eight
@@ -324,8 +361,5 @@ int32_t launch_gemm32_waves(int transA, int transB, int64_t m, int64_t n, int64_
                             int64_t slices, int64_t batch, hipStream_t st) {
     const WaveArgs g = {(const float *)A, (const float *)B, (float *)C, m, n, k, lda, ldb, ldc, sA, sB, sC, alpha, beta, (int32_t)slices, 0, 0};
     const Variant &v = fastest(m, n, slices * ((k + 15) / 16), batch);
-    const bool a_rm = !transA, b_rm = transB != 0;
-    if (v.bm == 2) return v.split == 1 ? launch_waves<2, 2, 1>(g, a_rm, b_rm, batch, st) : launch_waves<2, 2, 4>(g, a_rm, b_rm, batch, st);
-    if (v.split == 1) return launch_waves<1, 1, 1>(g, a_rm, b_rm, batch, st);
-    return v.split == 4 ? launch_waves<1, 1, 4>(g, a_rm, b_rm, batch, st) : launch_waves<1, 1, 8>(g, a_rm, b_rm, batch, st);
+    return slices > 1 ? launch_variant<true>(g, v, !transA, transB != 0, batch, st) : launch_variant<false>(g, v, !transA, transB != 0, batch, st);
 }

@@ -590,8 +590,31 @@ def test_float32_products_of_few_or_narrow_tiles(nn, ta, tb, m, n, k, batch):
     lib, out = nn._lib.load(), nn.DeviceArray.from_numpy(np.ones((m, n), np.float32))
     nn._lib.check(lib.mi_batched_gemm_sum(out.code, b"T" if ta else b"N", b"T" if tb else b"N", m, n, k, 1.0, da.ptr, k if ta else m, m * k, db.ptr,
                                           n if tb else k, n * k, 3.0, out.ptr, m, batch, 0))
+    # each slice errs as a product does, independently of the others, and the sum in one rounding per slice
     total = np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64)
-    assert (np.abs(out.to_numpy() - 3.0 - summed) <= 4 * 2.0 ** -24 * (np.sqrt(k * batch) * total.sum(axis=0) + 3.0)).all()
+    bound = np.sqrt(k * (total ** 2).sum(axis=0)) + np.sqrt(batch) * total.sum(axis=0) + 3.0
+    assert (np.abs(out.to_numpy() - 3.0 - summed) <= 4 * 2.0 ** -24 * bound).all()
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 1)])
+@pytest.mark.parametrize("m,n,k,batch", [(32, 32, 77, 96), (333, 77, 517, 96), (464, 16, 416, 28), (32, 32, 1024, 64), (16, 16, 16, 1000), (5, 3, 1, 1000),
+                                         (64, 96, 300, 40)])
+def test_float32_sum_over_the_batch_errs_no_more_than_a_product_per_slice(nn, ta, tb, m, n, k, batch):
+    """mi_batched_gemm_sum against mi_batched_gemm slice by slice with beta = 1, both measured in 64 bits (2-norm); a tenth
+    more for the order of the roundings."""
+    import torch
+    rng = torch.Generator(device="cuda").manual_seed(m + n + k)
+    A, B = (torch.randn(s, device="cuda", generator=rng) for s in ((batch, k, m), (batch, n, k)))   # columns of m and of k
+    ref = torch.matmul(B.double(), A.double()).sum(0)
+    a, b = A.transpose(1, 2).contiguous() if ta else A, B.transpose(1, 2).contiguous() if tb else B
+    lib, st, code = nn._lib.load(), torch.cuda.current_stream().cuda_stream, nn.DeviceArray(A.reshape(-1), (m, k, batch), "f32").code
+    head, lda, ldb = (code, b"T" if ta else b"N", b"T" if tb else b"N", m, n, k, 1.0), k if ta else m, n if tb else k
+    one, apart = torch.zeros(n, m, device="cuda"), torch.zeros(n, m, device="cuda")
+    nn._lib.check(lib.mi_batched_gemm_sum(*head, a.data_ptr(), lda, m * k, b.data_ptr(), ldb, n * k, 0.0, one.data_ptr(), m, batch, st))
+    for i in range(batch):
+        nn._lib.check(lib.mi_batched_gemm(*head, a[i].data_ptr(), lda, 0, b[i].data_ptr(), ldb, 0, 1.0, apart.data_ptr(), m, 0, 1, st))
+    err = lambda c: float((c.double() - ref).norm() / ref.norm())
+    assert err(one) <= 1.1 * err(apart)
 
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
