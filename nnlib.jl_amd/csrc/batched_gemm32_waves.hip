@@ -197,7 +197,10 @@ __global__ __launch_bounds__(64 * SPLIT, BM * BN == 1 ? (SUM ? 4 : 5) : (SUM ? 1
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bv[i][ib[t]], av[j][ia[t]], acc[i][j], 0, 0, 0);
     };
     const Step first = next({0, wave - SPLIT});
-    {
+    // one or two terms a sum: the planes' own error, up to 2.6 * 2^-24 of a product, would show (2-norm against 64 bits, planes /
+    // Float32 instruction: k = 1 3.5e-8 / 2.5e-8, 2 3.4e-8 / 3.1e-8, 3 3.3e-8 / 3.6e-8)
+    const bool planes = k >= 3;
+    if (planes) {
         Step s0 = first, s1 = next(first);
         int slice = first.sl;
         fetch(s0, 0);
@@ -211,8 +214,8 @@ __global__ __launch_bounds__(64 * SPLIT, BM * BN == 1 ? (SUM ? 4 : 5) : (SUM ? 1
             s1 = s3;
         }
     }
-    if (__builtin_amdgcn_ballot_w64(!(hi <= 0x1.fep127f && lo >= (27u << 24) - 1)) != 0) {
-        // again on the Float32 instruction, which takes one k of each half-wave: the registers as they are, in eight steps
+    if (!planes || __builtin_amdgcn_ballot_w64(!(hi <= 0x1.fep127f && lo >= (27u << 24) - 1)) != 0) {
+        // on the Float32 instruction, which takes one k of each half-wave: the registers as they are, in eight steps
 #pragma unroll
         for (int i = 0; i < BN; i++)
 #pragma unroll
@@ -223,11 +226,13 @@ __global__ __launch_bounds__(64 * SPLIT, BM * BN == 1 ? (SUM ? 4 : 5) : (SUM ? 1
             if (SUM && s.sl != slice) next_slice();
             slice = s.sl;
 #pragma unroll
-            for (int e = 0; e < 8; e++)
+            for (int e = 0; e < 8; e++) {
+                if (e >= 2 && !planes) break;
 #pragma unroll
                 for (int i = 0; i < BN; i++)
 #pragma unroll
                     for (int j = 0; j < BM; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(xb[0][i][e], xa[0][j][e], acc[i][j], 0, 0, 0);
+            }
         }
     }
 

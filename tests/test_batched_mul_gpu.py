@@ -644,3 +644,19 @@ def test_very_many_tiny_float32_products(nn, batch):
     C = nn.batched_mul(A, B)
     ref = a.double() * b.double()
     assert C.dims == (1, 1, batch) and bool(((C.storage.double() - ref).abs() <= 2.0 ** -22 * ref).all())
+
+
+@pytest.mark.parametrize("m,n,k,batch", [(5, 7, 1, 64), (33, 50, 1, 30), (1, 1, 1, 5000), (40, 40, 2, 64), (31, 65, 2, 7), (200, 2, 2, 9), (3, 3, 2, 1)])
+def test_float32_products_of_one_or_two_terms(nn, m, n, k, batch):
+    """k of 1 and 2 runs on the Float32 instruction: one product is rounded once, a sum of two errs by at most a rounding per
+    product and per addition."""
+    rng = np.random.default_rng(m + n + k)
+    A, B = (rng.standard_normal(s).astype(np.float32) for s in ((m, k, batch), (k, n, batch)))
+    dev = lambda x: nn.DeviceArray.from_numpy(np.ascontiguousarray(x), "f32")
+    for ta in (False, True):
+        C = nn.batched_mul(nn.batched_transpose(dev(A.transpose(1, 0, 2))) if ta else dev(A), dev(B)).to_numpy()
+        if k == 1:
+            assert np.array_equal(C, A * B)
+        A64, B64 = A.astype(np.float64).transpose(2, 0, 1), B.astype(np.float64).transpose(2, 0, 1)
+        bound = (2 * k - 1) * 2.0 ** -24 * (np.abs(A64) @ np.abs(B64)) * (1 + 2.0 ** -20)
+        assert (np.abs(C.transpose(2, 0, 1) - A64 @ B64) <= bound).all()
