@@ -373,11 +373,6 @@ struct FlashRows {
     }
 };
 
-// On entry s[qb][kb] holds raw dot products k.q of tile rows [j0, j0+64) for the wavefront's query
-// blocks; on exit it holds exp2(x - m) (ONLINE / STATS) or the final normalised weights (FINAL),
-// with m, l (and, ONLINE only, the output accumulators o) updated.
-//   T      element traits of the bias array
-//   NDV    number of 32-row blocks of the output accumulator
 // Adds a 32-key x 32-query block of Float32 values held in the MFMA accumulator layout (lane (r, hh): query row r
 // of the wavefront; register 4g + e: key 8g + 4hh + e of the block) to a Float32 array whose keys are contiguous:
 // dst points at (first key of the block, first query row of the wavefront), rows are qstride elements apart (0: every
@@ -498,6 +493,11 @@ __device__ inline void flash_mask_apply4(floatx16_t &v, int g, uint32_t m4) {
 // it stay below 2^8, which Float32 sums and 16-bit operands hold without loss.
 constexpr float FLASH_LAZY_MAX_LOG2 = 8.0f;
 
+// On entry s[qb][kb] holds raw dot products k.q of tile rows [j0, j0+64) for the wavefront's query
+// blocks; on exit it holds exp2(x - m) (ONLINE / STATS) or the final normalised weights (FINAL),
+// with m, l (and, ONLINE only, the output accumulators o) updated.
+//   T      element traits of the bias array
+//   NDV    number of 32-row blocks of the output accumulator
 // DROP: the call has fused dropout.  KBLK: 32-key blocks per tile (2: the 64-key tile of the tile loops; 1: a wavefront that
 // owns a single block)
 template <typename T, int QB, int NDV, bool CAUSAL, int EXTRAS, int PHASE, typename TW, bool DROP = false, int KBLK = 2>
