@@ -21,9 +21,9 @@ import sys
 REG = re.compile(r'\b([av])(\d+)\b|\b([av])\[(\d+):(\d+)\]')
 # instructions without a register destination: every operand is a source
 STORES = ('scratch_store', 'global_store', 'flat_store', 'buffer_store', 'ds_write', 'ds_store', 's_waitcnt', 's_nop')
-# (source file, mangled kernel name) of kernels without scratch memory: Float32 forward with bias / mask code; 16-bit forward
-# up to head dim 64 without weights or keep decisions, bias by rows or direct loads apart
-NO_SCRATCH = [(re.compile(r'attention_flash32'), re.compile(r'14flash32_kernelILi(64|128)ELi1ELb[01]ELb1E')),
+# (source file, mangled kernel name) of kernels without scratch memory: Float32 forward at head dims 65 to 128, or
+# with bias / mask code; 16-bit forward up to head dim 64 without weights or keep decisions, bias by rows or direct loads apart
+NO_SCRATCH = [(re.compile(r'attention_flash32'), re.compile(r'14flash32_kernelILi(64ELi1ELb[01]ELb1|128)E')),
               (re.compile(r'attention_flash16_b?f16_d64'), re.compile(r'14flash16_kernelILi1ELb[01]ELi[02347]ELb0EfLb0E'))]
 
 

@@ -696,7 +696,9 @@ __device__ inline void flash_softmax_tile(const FlashArgs &a, floatx16_t (&s)[QB
 
         // fdrop = dropout (src/attention.jl:126): after the softmax, so the row sum above is untouched;
         // before the value product and before the weights are written, which are post-dropout.
-        if constexpr (DROP && PHASE != PHASE_STATS) {
+        // (Float32: the test, true for every call that comes here, ends a scheduling region.  Without it the 128-wide causal
+        // kernel with the weights output has 512 registers and spills.)
+        if (DROP && PHASE != PHASE_STATS && (sizeof(elem_t) == 2 || p.drop_thresh != 0)) {
             const uint64_t row0 = (uint64_t)(p.Lkv * (qi + p.Lq * (h + p.H * b)) + j0);
             if ((p.Lkv & 3) == 0) {   // every run of four keys of a lane is one hash group
 #pragma unroll

@@ -64,17 +64,20 @@ def test_two_kernels_are_checked_apart(tmp_path):
 
 
 def test_scratch_of_kernels_that_have_none(tmp_path):
-    """A Float32 kernel with bias / mask code that spills is found (it took 588 bytes a lane once, for the code of a dropout
-    that its calls did not have); its neighbours without that code may."""
+    """A 128-wide Float32 kernel that spills is found, and a 64-wide one with bias / mask code (one took 588 bytes a lane once,
+    for the code of a dropout that its calls did not have; another 20 with the dropout that they had); the 64-wide ones without
+    that code may."""
     def described(name, scratch):
         return f"\t.amdhsa_kernel {name}\n\t\t.amdhsa_private_segment_fixed_size {scratch}\n\t.end_amdhsa_kernel\n"
-    kern = "_ZN12_GLOBAL__N_114flash32_kernelILi128ELi1ELb1ELb%dELb0ELb1EEEv9FlashArgs"
-    f = tmp_path / "attention_flash32-hip-amdgcn.s"
-    f.write_text(described(kern % 1, 588) + described(kern % 0, 28))
-    found = chk.check(str(f))
-    assert len(found) == 1 and kern % 1 in found[0] and "588" in found[0], found
-    f.write_text(described(kern % 1, 0))
-    assert chk.check(str(f)) == []
+    kern = "_ZN12_GLOBAL__N_114flash32_kernelILi%dELi1ELb1ELb%dELb0ELb1EEEv9FlashArgs"
+    for file in ("attention_flash32-hip-amdgcn.s", "attention_flash32_drop-hip-amdgcn.s"):
+        f = tmp_path / file
+        for head, extras in ((128, 1), (128, 0), (64, 1)):
+            f.write_text(described(kern % (head, extras), 588) + described(kern % (64, 0), 28))
+            found = chk.check(str(f))
+            assert len(found) == 1 and kern % (head, extras) in found[0] and "588" in found[0], found
+            f.write_text(described(kern % (head, extras), 0))
+            assert chk.check(str(f)) == []
     g = tmp_path / "attention_flash16_bf16_d64-hip-amdgcn.s"
     g.write_text(described("_ZN12_GLOBAL__N_114flash16_kernelILi1ELb0ELi0ELb0EfLb0EEEv9FlashArgs", 4)
                  + described("_ZN12_GLOBAL__N_114flash16_kernelILi1ELb0ELi7ELb0EfLb1EEEv9FlashArgs", 12))
