@@ -8,12 +8,14 @@
 // loads are in flight meanwhile.  SPLIT wavefronts of a workgroup take every SPLIT-th step of 16 k of one tile and add up
 // their sums through LDS, so that a small result still has many loads in flight; with SPLIT = 1 a wavefront is a workgroup.
 //
-// What bounds it: at k above about 100 the vector port (5.5 instructions of splitting and 2 of range checks per operand
-// element: 10 a matrix instruction for 2 x 2 blocks, 50 cycles where the matrix pipe alone takes 32); below, a launch's
+// What bounds it: at k above about 100 the vector instructions (splitting, range checks, addresses: 14 a matrix instruction for
+// 2 x 2 blocks, 56 cycles where the matrix pipe alone takes 32), which the two wavefronts of a SIMD overlap in part, and the
+// last round of workgroups.  Counters of 333 x 77 x 517, 96 slices, 1152 workgroups where the chip holds 512: vector
+// instructions 42 % of the SIMDs' cycles, matrix instructions 24 %, a CU has a wavefront 72 % of the time.  Below, a launch's
 // 4 us, the first step's memory round trip and the store of the result.  Against the LDS-staged kernels (one stage of 16 k
 // in flight, at least one 128 x 128 tile of four wavefronts): 320 x 16 x 816, 20 slices, 64.5 -> 8.0 us;
 // 100 x 100 x 100, 50 slices, 13.0 -> 5.6; 464 x 16 x 416, 28 slices, 34.8 -> 7.5; 333 x 517 x 16, 96 slices, 22.6 -> 17
-// (66 MB of results: 3.9 TB/s); 77 x 333 x 517, 96 slices, 59 -> 41 us.
+// (66 MB of results: 3.9 TB/s); 77 x 333 x 517, 96 slices, 59 to 69 -> 41 to 52 us by the operands' orientation.
 #include "common.h"
 
 namespace {
