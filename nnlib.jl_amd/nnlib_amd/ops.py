@@ -761,6 +761,8 @@ def batched_mul_pullback(A, B, dC):
     if A.ndim != 3 or B.ndim != 3 or dC.ndim != 3:
         raise DimensionMismatch("batched_mul_pullback expects 3-D arrays")
     nb = dC.dims[2]
+    if A.dims[2] not in (nb, 1) or B.dims[2] not in (nb, 1):
+        raise DimensionMismatch("batch size mismatch: A, B and dC must have one batch size, or A or B a single slice")
 
     def summed(X, make):
         if X.dims[2] != 1 or nb == 1:

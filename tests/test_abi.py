@@ -194,3 +194,15 @@ def test_promote_type_table():
             ("c64", "f32"): "c64", ("c64", "i64"): "c64", ("f16", "f32"): "f32", ("bf16", "f16"): "f32", ("f32", "f32"): "f32"}
     for (a, b), t in want.items():
         assert P(a, b) == t and P(b, a) == t, (a, b)
+
+
+def test_pullback_of_batched_mul_checks_the_batch_sizes():
+    """A shared operand's gradient walks the slices of the other arrays by dC's batch size: arrays with fewer are refused
+    before anything reads them."""
+    import torch
+    from nnlib_amd import DeviceArray, DimensionMismatch
+    from nnlib_amd.ops import batched_mul_pullback
+    arr = lambda *s: DeviceArray(torch.zeros(s[0] * s[1] * s[2]), s, "f32")
+    for a, b in (((4, 5, 1), (5, 6, 2)), ((4, 5, 2), (5, 6, 1)), ((4, 5, 2), (5, 6, 3))):
+        with pytest.raises(DimensionMismatch):
+            batched_mul_pullback(arr(*a), arr(*b), arr(4, 6, 3))
