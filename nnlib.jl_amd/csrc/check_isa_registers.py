@@ -10,7 +10,7 @@ flow-insensitive on purpose: it only asks, per kernel, that every VGPR / AGPR th
 a destination somewhere, which is cheap, has no false positives beyond the registers the hardware initialises (v0 - v2:
 work-item ids), and catches exactly that class of miscompile.
 
-It also holds the kernels of NO_SCRATCH to their registers: those whose 512 registers have spilled, or whose workgroups per
+It also holds the kernels of SCRATCH_MOST to their registers: those whose 512 registers have spilled, or whose workgroups per
 compute unit have dropped, when code behind a run-time test grew that their calls never reach.
 
 usage: check_isa_registers.py file.s [file.s ...]   (exit status 1 and one line per finding if any)
@@ -21,10 +21,12 @@ import sys
 REG = re.compile(r'\b([av])(\d+)\b|\b([av])\[(\d+):(\d+)\]')
 # instructions without a register destination: every operand is a source
 STORES = ('scratch_store', 'global_store', 'flat_store', 'buffer_store', 'ds_write', 'ds_store', 's_waitcnt', 's_nop')
-# (source file, mangled kernel name) of kernels without scratch memory: Float32 forward at head dims 65 to 128, or
-# with bias / mask code; 16-bit forward up to head dim 64 without weights or keep decisions, bias by rows or direct loads apart
-NO_SCRATCH = [(re.compile(r'attention_flash32'), re.compile(r'14flash32_kernelILi(64ELi1ELb[01]ELb1|128)E')),
-              (re.compile(r'attention_flash16_b?f16_d64'), re.compile(r'14flash16_kernelILi1ELb[01]ELi[02347]ELb0EfLb0E'))]
+# (source file, mangled kernel name, bytes of scratch memory a lane) of kernels that may have no more: Float32 forward at head
+# dims 65 to 128, or with bias / mask code; 16-bit forward up to head dim 64 without weights or keep decisions, bias by rows or
+# direct loads apart; the 16-bit gradient of short sequences
+SCRATCH_MOST = [(re.compile(r'attention_flash32'), re.compile(r'14flash32_kernelILi(64ELi1ELb[01]ELb1|128)E'), 0),
+                (re.compile(r'attention_flash16_b?f16_d64'), re.compile(r'14flash16_kernelILi1ELb[01]ELi[02347]ELb0EfLb0E'), 0),
+                (re.compile(r'attention_backward_pair16'), re.compile(r'15bwd_pair_kernelI'), 12)]
 
 
 def regs(text):
@@ -50,9 +52,10 @@ def check(path):
             continue
         if code.startswith('.amdhsa_kernel'):
             described = code.split()[1]
-        if code.startswith('.amdhsa_private_segment_fixed_size') and int(code.split()[1]) > 0:
-            if any(f.search(path) and k.search(described) for f, k in NO_SCRATCH):
-                findings.append(f"{path}: {described}: {code.split()[1]} bytes of scratch memory, none allowed")
+        if code.startswith('.amdhsa_private_segment_fixed_size'):
+            for f, k, most in SCRATCH_MOST:
+                if f.search(path) and k.search(described) and int(code.split()[1]) > most:
+                    findings.append(f"{path}: {described}: {code.split()[1]} bytes of scratch memory, {most} allowed")
         if code.startswith('.end_amdhsa_kernel') or code.startswith('.section'):
             continue
         if kernel is None or code.startswith('.'):

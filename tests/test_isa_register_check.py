@@ -82,3 +82,7 @@ def test_scratch_of_kernels_that_have_none(tmp_path):
     g.write_text(described("_ZN12_GLOBAL__N_114flash16_kernelILi1ELb0ELi0ELb0EfLb0EEEv9FlashArgs", 4)
                  + described("_ZN12_GLOBAL__N_114flash16_kernelILi1ELb0ELi7ELb0EfLb1EEEv9FlashArgs", 12))
     assert len(chk.check(str(g))) == 1
+    h = tmp_path / "attention_backward_pair16_bf16-hip-amdgcn.s"
+    for scratch, findings in ((12, 0), (152, 1)):   # as it was with bias entries loaded on both sides of the causal test
+        h.write_text(described("_ZN12_GLOBAL__N_115bwd_pair_kernelILb1ELi5ELi0ELi2ELi8EEEv9FlashArgs13AttnBwdParams", scratch))
+        assert len(chk.check(str(h))) == findings
