@@ -5,10 +5,16 @@
 // The work is a stream over K and V: every byte is read once and used once, so the kernel is
 // organised around HBM, not around the matrix cores.  A kv row (all heads) is E contiguous elements;
 // a wavefront owns a 1 KiB segment of the row (512 16-bit features: 4 heads at D = 128, 8 heads at D = 64; half as
-// many in Float32), each lane one 16-byte load (8 or 4 consecutive features), and walks a contiguous range of kv
-// rows.  The dot product over a head is finished with a butterfly over the lanes that share the head.
-// Each (segment, kv-split, batch) wavefront keeps an online-softmax state (m, l, o[8]) and writes it
-// to a workspace; a second small kernel merges the splits.
+// many in Float32), each lane one 16-byte load (8 or 4 consecutive features), and walks kv rows eight at a time.  The
+// dot product over a head is finished with a butterfly over the lanes that share the head.  A wavefront keeps an
+// online-softmax state (m, l, o[8]); the eight of a workgroup, which share a segment, merge theirs through LDS and write
+// one partial result to a workspace; a second small kernel merges those.
+//
+// What bounds it: large calls the K / V stream (8 segments x 16 x 32768 keys, 8.6 GB: 1380 us, 6.2 TB/s; 1434 with a
+// partial result per wavefront and four segments of a row in a workgroup), small ones the chain of one block's loads, the two
+// launches and the merge, since a call fills the chip with wavefronts of a single 8-row block where its keys allow it
+// (head dim 64, 8 heads, 2 x 5000 keys: 74 -> 13 us; 12 x 18 x 528: 45 -> 14; one sequence of 4096 keys, 32 heads of 128, with
+// the weights: 80 -> 22).
 //
 // Same arithmetic as the reference chain (src/attention.jl:112-127, fdrop = identity, no bias):
 //   s_j = sum_d k[d,j] * q[d] / sqrt(D),  a = softmax_j(s),  x[d] = sum_j a_j v[d,j].
@@ -24,6 +30,8 @@
 namespace {
 
 constexpr int ROWS = 8;        // kv rows in flight per lane and tensor
+constexpr int WAVES = 8;       // wavefronts per workgroup
+constexpr int MAX_SPLITS = 1024;
 // features per lane (one 16-byte load) and per wavefront
 template <typename T> constexpr int epl() { return 16 / (int)sizeof(typename T::type); }
 template <typename T> constexpr int seg_width() { return 64 * epl<T>(); }
@@ -32,8 +40,7 @@ struct DecodeArgs {
     AttnParams p;
     float c;           // log2(e) / sqrt(D)
     int32_t nsplit;
-    int32_t rows_per_split;
-    int32_t nseg;      // ceil(E / 512)
+    int32_t rows_per_wave;   // weights requested: contiguous keys of a wavefront, a multiple of ROWS
     float *scores;     // weights requested: [B][H][Lkv] raw dot products (-Inf where masked), else null
     float *final_ml;   // weights requested: [B][H][2] final maximum (raw units) and 1 / sum
 };
@@ -58,21 +65,24 @@ __device__ inline void unpack8(const u32x4_t &v, float *out, F32) {   // four fe
 // NQ: queries of one batch element that a wavefront carries through the stream (1, 2 or 4).  A handful of queries
 // against a long context (a few speculated tokens, a short chunk) is the same stream over K and V with NQ states: every
 // K / V row is read once for all of them, where the tiled kernel reads head-dim-wide pieces of it per head.
+//
+// The WAVES wavefronts of a workgroup share a segment and take different key rows, and their states are merged through
+// LDS before they leave, so a split costs one partial result per workgroup.
 template <typename T, int D, bool MASKED, bool SCORES, int NQ = 1>
-__global__ __launch_bounds__(256) void decode_split_kernel(DecodeArgs a) {
+__global__ __launch_bounds__(WAVES * 64, NQ <= 2 ? 4 : 2) void decode_split_kernel(DecodeArgs a) {
     const AttnParams &p = a.p;
     typedef typename T::type t;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr int EPL = epl<T>(), SEG = seg_width<T>(), LPH = D / EPL;   // features per lane and wavefront, lanes per head
     constexpr int NH = SEG / D;                        // heads per wavefront
-    __shared__ float sc_lds[SCORES ? 4 * NH * 64 : 1]; // scores on their way out: [wavefront][head][64 keys]
-    const int seg = blockIdx.x * 4 + wave;
+    __shared__ float sc_lds[SCORES ? WAVES * NH * 64 : 1]; // scores on their way out: [wavefront][head][64 keys]
+    __shared__ float o_lds[NQ * WAVES * SEG], ml_lds[NQ * WAVES * NH * 2];   // states of the wavefronts
+    const int seg = blockIdx.x;
     const int split = blockIdx.y;
     const int64_t ngroups = (p.Lq + NQ - 1) / NQ;      // groups of NQ queries per batch element
     const int64_t b = blockIdx.z / ngroups, q0 = (blockIdx.z % ngroups) * NQ;
     const int64_t f = (int64_t)seg * SEG + lane * EPL; // first feature of this lane
     const bool lane_ok = f < p.E;                      // E is a multiple of EPL (D is 64 or 128)
-    if (seg >= a.nseg) return;
 
     const t *kb = (const t *)p.k + p.E * p.Lkv * b + (lane_ok ? f : 0);
     const t *vb = (const t *)p.v + p.E * p.Lkv * b + (lane_ok ? f : 0);
@@ -83,17 +93,18 @@ __global__ __launch_bounds__(256) void decode_split_kernel(DecodeArgs a) {
         if (lane_ok) unpack8(*(const u32x4_t *)((const t *)p.q + p.E * (qi + p.Lq * b) + f), qf[n], T());
     }
 
-    // Without the score output the splits take the 8-row blocks of the key range in turn (block t belongs to split
-    // t mod nsplit) instead of one contiguous range each: the splits of a batch element run side by side, so at any
-    // moment the chip reads one moving window of consecutive rows rather than nsplit separate streams (a plain read
+    // Without the score output the wavefronts take the 8-row blocks of the key range in turn (block t belongs to
+    // wavefront t mod nwaves of the pair) instead of one contiguous range each: the splits of a batch element run side by side, so at any
+    // moment the chip reads one moving window of consecutive rows rather than nwaves separate streams (a plain read
     // of 8 GiB on this GPU: 6.97 TB/s with interleaved workgroups against 6.2-6.35 with a contiguous chunk per workgroup).
     // The online softmax does not depend on the order.  With scores the ranges stay contiguous: they leave in runs of
     // 64 consecutive keys.
     const bool interleave = !SCORES;
-    const int64_t j_begin = interleave ? (int64_t)split * ROWS : (int64_t)split * a.rows_per_split;
-    int64_t j_end = interleave ? p.Lkv : j_begin + a.rows_per_split;
+    const int64_t part = (int64_t)split * WAVES + wave, nwaves = (int64_t)a.nsplit * WAVES;
+    const int64_t j_begin = interleave ? part * ROWS : part * a.rows_per_wave;
+    int64_t j_end = interleave ? p.Lkv : j_begin + a.rows_per_wave;
     if (j_end > p.Lkv) j_end = p.Lkv;
-    const int64_t j_step = interleave ? (int64_t)a.nsplit * ROWS : ROWS;
+    const int64_t j_step = interleave ? nwaves * ROWS : ROWS;
 
     float m[NQ], l[NQ], o[NQ][EPL] = {};
 #pragma unroll
@@ -102,6 +113,7 @@ __global__ __launch_bounds__(256) void decode_split_kernel(DecodeArgs a) {
         l[n] = 0.0f;
     }
     const u32x4_t zero = {0, 0, 0, 0};
+    const float scale = p.drop_thresh != 0 ? p.drop_scale : 1.0f;
     // mask bytes of this lane's head: element (kv, 0, h, b)
     const uint8_t *mrow = MASKED ? p.mask + (lane_ok ? f / D : 0) * p.mask_strides[2] + b * p.mask_strides[3] : nullptr;
 
@@ -154,22 +166,22 @@ __global__ __launch_bounds__(256) void decode_split_kernel(DecodeArgs a) {
         // the row sum takes the weight as the softmax gives it, the value product takes it times the keep factor of
         // weight (key, query, head, batch) in the shared counter stream.  A chunk starts at a multiple of 8 keys, so it
         // is two hash groups of four; the hashes hide under the K / V stream.
-        float fac[NQ][ROWS];
+        // The decisions stay a bit each until the products: as factors they would take a register each.
+        uint32_t kept[NQ];
 #pragma unroll
-        for (int n = 0; n < NQ; n++)
-#pragma unroll
-            for (int r = 0; r < ROWS; r++) fac[n][r] = 1.0f;
+        for (int n = 0; n < NQ; n++) kept[n] = ~0u;
         if (p.drop_thresh != 0) {
             const int64_t hd = lane_ok ? f / D : 0;
 #pragma unroll
             for (int n = 0; n < NQ; n++) {
                 const int64_t qi = q0 + n < p.Lq ? q0 + n : p.Lq - 1;
                 const uint64_t i0 = (uint64_t)(j + p.Lkv * (qi + p.Lq * (hd + p.H * b)));
+                kept[n] = 0;
 #pragma unroll
                 for (int g = 0; g < ROWS / 4; g++) {
                     const uint64_t bits = mi_dropout_group_bits(p.drop_key, (i0 + 4 * g) >> 2);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) fac[n][4 * g + e] = mi_dropout_keep_in(bits, e, p.drop_thresh) ? p.drop_scale : 0.0f;
+                    for (int e = 0; e < 4; e++) kept[n] |= mi_dropout_keep_in(bits, e, p.drop_thresh) ? 1u << (4 * g + e) : 0u;
                 }
             }
         }
@@ -181,7 +193,7 @@ __global__ __launch_bounds__(256) void decode_split_kernel(DecodeArgs a) {
             for (int n = 0; n < NQ; n++) {
                 const float pr = mi_exp2((s[n][r] - mref[n]) * a.c);
                 l[n] += pr;
-                const float pd = pr * fac[n][r];
+                const float pd = pr * ((kept[n] >> r) & 1 ? scale : 0.0f);
 #pragma unroll
                 for (int e = 0; e < EPL; e++) o[n][e] = fmaf(pd, vf[e], o[n][e]);
             }
@@ -214,81 +226,126 @@ __global__ __launch_bounds__(256) void decode_split_kernel(DecodeArgs a) {
             }
         }
     }
-    if (!lane_ok) return;
-    // partial results: one slot per (batch element, query, split); the merge kernel sees B * Lq batch elements
-    float *ws = (float *)p.workspace;
-    const int64_t nbq = p.B * p.Lq;
+    // merge of the wavefronts' states; one that kept no key has m = -Inf and weight 0
 #pragma unroll
     for (int n = 0; n < NQ; n++) {
-        if (q0 + n >= p.Lq) break;
-        const int64_t slot = (b * p.Lq + q0 + n) * a.nsplit + split;
-        float *wo = ws + slot * p.E + f;
+        float *wo = o_lds + (n * WAVES + wave) * SEG + lane * EPL;
         *(floatx4_t *)wo = (floatx4_t){o[n][0], o[n][1], o[n][2], o[n][3]};
         if constexpr (EPL == 8) *(floatx4_t *)(wo + 4) = (floatx4_t){o[n][4], o[n][5], o[n][6], o[n][7]};
         if ((lane & (LPH - 1)) == 0) {
-            const int64_t h = f / D;
+            float *wml = ml_lds + ((n * WAVES + wave) * NH + lane / LPH) * 2;
+            wml[0] = m[n];
+            wml[1] = l[n];
+        }
+    }
+    __syncthreads();
+    // partial results: one slot per (batch element, query, split); the merge kernel sees B * Lq batch elements
+    float *ws = (float *)p.workspace;
+    const int64_t nbq = p.B * p.Lq;
+    for (int i = threadIdx.x; i < NQ * SEG; i += WAVES * 64) {
+        const int n = i / SEG, fl = i % SEG, hl = fl / D;
+        const int64_t fo = (int64_t)seg * SEG + fl;
+        if (fo >= p.E || q0 + n >= p.Lq) continue;
+        float mw[WAVES], mm = MI_NEG_INF;
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) {
+            mw[w] = ml_lds[((n * WAVES + w) * NH + hl) * 2];
+            mm = fmaxf(mm, mw[w]);
+        }
+        const float mr = mm == MI_NEG_INF ? 0.0f : mm;
+        float oo = 0.0f, ll = 0.0f;
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) {
+            const float wt = mi_exp2((mw[w] - mr) * a.c);
+            oo = fmaf(o_lds[(n * WAVES + w) * SEG + fl], wt, oo);
+            ll = fmaf(ml_lds[((n * WAVES + w) * NH + hl) * 2 + 1], wt, ll);
+        }
+        const int64_t slot = (b * p.Lq + q0 + n) * a.nsplit + split;
+        ws[slot * p.E + fo] = oo;
+        if (fl % D == 0) {
+            const int64_t h = fo / D;
             float *wm = ws + nbq * a.nsplit * p.E;
             float *wl = wm + nbq * a.nsplit * p.H;
-            wm[slot * p.H + h] = m[n];
-            wl[slot * p.H + h] = l[n];
+            wm[slot * p.H + h] = mm;
+            wl[slot * p.H + h] = ll;
         }
     }
 }
 
-// Merge of the splits with the usual log-sum-exp rule.  One workgroup per (256 features, batch): the
-// weights 2^(m_s - m) of every (head, split) pair are computed once into LDS, then each thread sums its
-// feature over the splits, eight independent loads at a time.
+// Merge of the splits with the usual log-sum-exp rule.  One workgroup per (64 features, batch), 64 features being (half of)
+// a head: the weights 2^(m_s - m) of the splits are computed once into LDS, then 16 groups of 16 threads each add up a
+// sixteenth of the splits, four features a thread and eight independent loads at a time.
 template <typename T>
 __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeArgs a) {
     const AttnParams &p = a.p;
-    __shared__ float wgt[4 * 1024];   // [heads of this workgroup <= 4][nsplit <= 1024]
-    __shared__ float inv_l[4];
+    __shared__ float wgt[MAX_SPLITS];
+    __shared__ float red[2][4];
+    __shared__ floatx4_t part[4][16];
     const int64_t b = blockIdx.y;
-    const int64_t f0 = (int64_t)blockIdx.x * 256, f = f0 + threadIdx.x;
+    const int64_t f0 = (int64_t)blockIdx.x * 64, h = f0 / p.D;
     const float *ws = (const float *)p.workspace;
-    const float *wm = ws + (int64_t)p.B * a.nsplit * p.E;
+    const float *wm = ws + (int64_t)p.B * a.nsplit * p.E + b * a.nsplit * p.H + h;
     const float *wl = wm + (int64_t)p.B * a.nsplit * p.H;
-    const int64_t h0 = f0 / p.D;
-    const int nh = (int)(256 / p.D);                 // 2 or 4 heads per workgroup
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (wave < nh && h0 + wave < p.H) {
-        // one wavefront per head: maximum over the splits, then the weights and the total sum
-        const int64_t h = h0 + wave;
-        float m = MI_NEG_INF;
-        for (int s = lane; s < a.nsplit; s += 64) m = fmaxf(m, wm[(b * a.nsplit + s) * p.H + h]);
-        m = mi_wave_max(m);
-        float l = 0.0f;
-        for (int s = lane; s < a.nsplit; s += 64) {
-            const int64_t slot = b * a.nsplit + s;
-            const float w = mi_exp2((wm[slot * p.H + h] - m) * a.c);
-            wgt[wave * 1024 + s] = w;
-            l = fmaf(wl[slot * p.H + h], w, l);
-        }
-        l = mi_wave_sum(l);
-        if (lane == 0) {
-            inv_l[wave] = 1.0f / l;
-            if (a.final_ml) {   // a head belongs to exactly one workgroup of this kernel (256 is a multiple of the head dim)
-                a.final_ml[(b * p.H + h) * 2] = m;
-                a.final_ml[(b * p.H + h) * 2 + 1] = 1.0f / l;
-            }
-        }
+    float ms[MAX_SPLITS / 256], ls[MAX_SPLITS / 256], m = MI_NEG_INF;
+#pragma unroll
+    for (int u = 0; u < MAX_SPLITS / 256; u++) {
+        const int s = u * 256 + threadIdx.x;
+        ms[u] = s < a.nsplit ? wm[(int64_t)s * p.H] : MI_NEG_INF;
+        ls[u] = s < a.nsplit ? wl[(int64_t)s * p.H] : 0.0f;
+        m = fmaxf(m, ms[u]);
     }
+    m = mi_wave_max(m);
+    if (lane == 0) red[0][wave] = m;
     __syncthreads();
-    if (f >= p.E) return;
-    const int hl = (int)(f / p.D - h0);
-    const float *src = ws + b * a.nsplit * p.E + f;
-    const float *w = wgt + hl * 1024;
-    float o = 0.0f;
-    int s = 0;
-    for (; s + 8 <= a.nsplit; s += 8) {
-        float x[8];
+    m = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
+    float l = 0.0f;
 #pragma unroll
-        for (int u = 0; u < 8; u++) x[u] = src[(int64_t)(s + u) * p.E];
-#pragma unroll
-        for (int u = 0; u < 8; u++) o = fmaf(x[u], w[s + u], o);
+    for (int u = 0; u < MAX_SPLITS / 256; u++) {
+        const int s = u * 256 + threadIdx.x;
+        if (s >= a.nsplit) break;
+        const float w = mi_exp2((ms[u] - m) * a.c);   // every key of the pair dropped: NaN, as the reference's softmax gives
+        wgt[s] = w;
+        l = fmaf(ls[u], w, l);
     }
-    for (; s < a.nsplit; s++) o = fmaf(src[(int64_t)s * p.E], w[s], o);
-    ((typename T::type *)p.out)[p.E * b + f] = T::from_f32(o * inv_l[hl]);
+    l = mi_wave_sum(l);
+    if (lane == 0) red[1][wave] = l;
+    __syncthreads();
+    const float inv = 1.0f / (red[1][0] + red[1][1] + red[1][2] + red[1][3]);
+    if (a.final_ml && threadIdx.x == 0 && f0 % p.D == 0) {
+        a.final_ml[(b * p.H + h) * 2] = m;
+        a.final_ml[(b * p.H + h) * 2 + 1] = inv;
+    }
+    const int fl = threadIdx.x & 15, g = threadIdx.x >> 4;
+    const float *src = ws + b * a.nsplit * p.E + f0 + fl * 4;
+    floatx4_t o = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s = g; s < a.nsplit; s += 16 * 8) {
+        floatx4_t x[8];
+        float w[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const bool ok = s + 16 * u < a.nsplit;
+            x[u] = ok ? *(const floatx4_t *)(src + (int64_t)(s + 16 * u) * p.E) : (floatx4_t){0.0f, 0.0f, 0.0f, 0.0f};
+            w[u] = ok ? wgt[s + 16 * u] : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[e] = fmaf(x[u][e], w[u], o[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        o[e] += __shfl_xor(o[e], 16, 64);
+        o[e] += __shfl_xor(o[e], 32, 64);
+    }
+    if (lane < 16) part[wave][lane] = o;
+    __syncthreads();
+    // one element a thread: the output may start at any element
+    if (threadIdx.x < 64) {
+        const int pf = threadIdx.x >> 2, e = threadIdx.x & 3;
+        const float sum = (part[0][pf][e] + part[1][pf][e]) + (part[2][pf][e] + part[3][pf][e]);
+        ((typename T::type *)p.out)[p.E * b + f0 + threadIdx.x] = T::from_f32(sum * inv);
+    }
 }
 
 // weights[kv, 0, h, b] = 2^((s - m) c) / l from the saved scores; a (head, batch) pair with every key masked has
@@ -308,16 +365,27 @@ __global__ __launch_bounds__(256) void decode_weights_kernel(DecodeArgs a, TW *w
 // queries per wavefront: 1, 2, or 4 (three queries run as four)
 int decode_nq(const AttnParams &p) { return p.Lq <= 1 ? 1 : p.Lq == 2 ? 2 : 4; }
 
+// Workgroups along the keys of one (segment, batch element, query group).  Two workgroups of eight wavefronts share a CU, so
+// 512 are one round of the chip.  Measured, us of GPU time, one segment unless said:
+//   - up to one round, down to one 8-row block per wavefront: a second round with little left in it costs more than it gives
+//     (head dim 128, 4 segments x 3 x 3300 keys: 26.6 with 512 workgroups, 30 with 624), more blocks per wavefront leave CUs idle
+//     (2 x 5000 keys: 13.1 with one block per wavefront, 14.5 with two, 19.8 with four; one wavefront per 250 keys, as it was: 74);
+//   - two to four queries: two blocks, since a workgroup's partial results are that many times larger (31041 keys, two queries:
+//     23.9 with one, 20.7 with two);
+//   - a single query with at least 32 blocks per wavefront: four rounds, whose ends are shorter (8 segments x 16 x 32768 keys:
+//     1407 with one round, 1389 with two, 1380 with four; Float32, 4 x 16 x 16384: 396, 403, 386), which costs two to four
+//     queries, with more to merge, up to a sixth (four queries, 8 segments x 8 x 8192 keys: 211, 222, 247).
+// With the weights requested the 256 keys per workgroup keep the partial results to what a call needed with one per split.
 int pick_nsplit(const AttnParams &p) {
-    // enough wavefronts to cover the chip several times over, at least 256 rows per split
     const int64_t SEG = p.dtype == MI_F32 ? seg_width<F32>() : seg_width<BF16>();
     const int64_t nseg = (p.E + SEG - 1) / SEG;
-    const int64_t groups = p.B * ((p.Lq + decode_nq(p) - 1) / decode_nq(p));   // (batch element, query group) pairs
-    int64_t want = 8192 / (nseg * groups > 0 ? nseg * groups : 1);   // (C5: 2048, 4096, 16384 ... 65536 wavefronts all measured slower)
-    int64_t maxs = (p.Lkv + 255) / 256;
+    const int64_t pairs = nseg * p.B * ((p.Lq + decode_nq(p) - 1) / decode_nq(p));   // (segment, batch element, query group)
+    int64_t want = pairs < 512 ? 512 / pairs : 1;
+    if (p.Lq == 1 && p.Lkv >= 32 * ROWS * WAVES * want) want = pairs < 2048 ? 2048 / pairs : 1;
+    const int64_t blocks = p.weights ? 4 : p.Lq == 1 ? 1 : 2;   // 8-row blocks per wavefront, at least
+    const int64_t maxs = (p.Lkv + ROWS * WAVES * blocks - 1) / (ROWS * WAVES * blocks);
     if (want > maxs) want = maxs;
-    if (want < 1) want = 1;
-    if (want > 1024) want = 1024;
+    if (want > MAX_SPLITS) want = MAX_SPLITS;
     return (int)want;
 }
 
@@ -347,38 +415,36 @@ int32_t launch_attention_decode(const AttnParams &p, hipStream_t st) {
     a.p = p;
     a.c = MI_LOG2E / sqrtf((float)p.D);
     a.nsplit = pick_nsplit(p);
-    a.rows_per_split = (int32_t)((p.Lkv + a.nsplit - 1) / a.nsplit);
-    a.nsplit = (int32_t)((p.Lkv + a.rows_per_split - 1) / a.rows_per_split);  // no empty split
+    const int64_t per_wave = (p.Lkv + (int64_t)a.nsplit * WAVES - 1) / ((int64_t)a.nsplit * WAVES);
+    a.rows_per_wave = (int32_t)((per_wave + ROWS - 1) / ROWS * ROWS);
     const int64_t SEG = p.dtype == MI_F32 ? seg_width<F32>() : seg_width<BF16>();
-    a.nseg = (int32_t)((p.E + SEG - 1) / SEG);
     if ((((uintptr_t)p.workspace) & 15) != 0)
         return mi_set_error(MI_EWORKSPACE, "decode workspace must be 16-byte aligned");
     a.scores = a.final_ml = nullptr;
     if (p.weights) {
-        // placed after the partial results, which are sized for pick_nsplit() splits (never fewer than a.nsplit)
-        a.scores = (float *)p.workspace + (size_t)pick_nsplit(p) * (size_t)p.B * (size_t)(p.E + 2 * p.H);
+        a.scores = (float *)p.workspace + (size_t)a.nsplit * (size_t)p.B * (size_t)(p.E + 2 * p.H);
         a.final_ml = a.scores + p.Lkv * p.H * p.B;
     }
     const int nq = decode_nq(p);
-    dim3 grid((unsigned)((a.nseg + 3) / 4), (unsigned)a.nsplit, (unsigned)(p.B * ((p.Lq + nq - 1) / nq)));
-    dim3 mgrid((unsigned)((p.E + 255) / 256), (unsigned)(p.B * p.Lq));
+    dim3 grid((unsigned)((p.E + SEG - 1) / SEG), (unsigned)a.nsplit, (unsigned)(p.B * ((p.Lq + nq - 1) / nq)));
+    dim3 mgrid((unsigned)(p.E / 64), (unsigned)(p.B * p.Lq));
     DecodeArgs am = a;      // the merge kernel takes every (batch element, query) pair for a batch element of its own:
     am.p.B = p.B * p.Lq;    // q and the output are (E, Lq, B) arrays, the partial results [B * Lq][split][...]
     am.p.Lq = 1;
 #define DECODE_LAUNCH(TT, DD)                                                                                        \
     {                                                                                                                \
         if (p.weights) {                                                                                             \
-            if (p.mask) hipLaunchKernelGGL((decode_split_kernel<TT, DD, true, true>), grid, dim3(256), 0, st, a);     \
-            else hipLaunchKernelGGL((decode_split_kernel<TT, DD, false, true>), grid, dim3(256), 0, st, a);           \
+            if (p.mask) hipLaunchKernelGGL((decode_split_kernel<TT, DD, true, true>), grid, dim3(WAVES * 64), 0, st, a);     \
+            else hipLaunchKernelGGL((decode_split_kernel<TT, DD, false, true>), grid, dim3(WAVES * 64), 0, st, a);           \
         } else if (nq == 1) {                                                                                        \
-            if (p.mask) hipLaunchKernelGGL((decode_split_kernel<TT, DD, true, false>), grid, dim3(256), 0, st, a);    \
-            else hipLaunchKernelGGL((decode_split_kernel<TT, DD, false, false>), grid, dim3(256), 0, st, a);          \
+            if (p.mask) hipLaunchKernelGGL((decode_split_kernel<TT, DD, true, false>), grid, dim3(WAVES * 64), 0, st, a);    \
+            else hipLaunchKernelGGL((decode_split_kernel<TT, DD, false, false>), grid, dim3(WAVES * 64), 0, st, a);          \
         } else if (nq == 2) {                                                                                        \
-            if (p.mask) hipLaunchKernelGGL((decode_split_kernel<TT, DD, true, false, 2>), grid, dim3(256), 0, st, a); \
-            else hipLaunchKernelGGL((decode_split_kernel<TT, DD, false, false, 2>), grid, dim3(256), 0, st, a);       \
+            if (p.mask) hipLaunchKernelGGL((decode_split_kernel<TT, DD, true, false, 2>), grid, dim3(WAVES * 64), 0, st, a); \
+            else hipLaunchKernelGGL((decode_split_kernel<TT, DD, false, false, 2>), grid, dim3(WAVES * 64), 0, st, a);       \
         } else {                                                                                                     \
-            if (p.mask) hipLaunchKernelGGL((decode_split_kernel<TT, DD, true, false, 4>), grid, dim3(256), 0, st, a); \
-            else hipLaunchKernelGGL((decode_split_kernel<TT, DD, false, false, 4>), grid, dim3(256), 0, st, a);       \
+            if (p.mask) hipLaunchKernelGGL((decode_split_kernel<TT, DD, true, false, 4>), grid, dim3(WAVES * 64), 0, st, a); \
+            else hipLaunchKernelGGL((decode_split_kernel<TT, DD, false, false, 4>), grid, dim3(WAVES * 64), 0, st, a);       \
         }                                                                                                            \
     }
     if (p.dtype == MI_BF16) {

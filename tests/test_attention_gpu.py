@@ -448,6 +448,43 @@ def test_decode_with_context_length_masks(nn, oracle, dtype, E, H, mask_shape):
             assert np.count_nonzero(a[okw & ~np.broadcast_to(mask.reshape(mask.shape + (1,) * (4 - mask.ndim)), a.shape)]) == 0
 
 
+@pytest.mark.parametrize("dtype,E,H,Lq,Lkv,B,masked", [
+    ("bf16", 1536, 12, 1, 512, 2, False),    # three segments, the fewest keys
+    ("bf16", 512, 8, 1, 513, 1, True),       # one key in the last block
+    ("f16", 768, 6, 2, 4100, 1, False),      # half a segment, two blocks per wavefront
+    ("bf16", 512, 4, 3, 1031, 3, True),      # three queries as four
+    ("f32", 320, 5, 1, 777, 2, True),
+    ("f16", 128, 1, 1, 70001, 1, False),     # one round of workgroups on a single pair
+    ("bf16", 64, 1, 1, 2051, 300, True),     # four rounds of workgroups
+])
+def test_decode_splits(nn, dtype, E, H, Lq, Lkv, B, masked):
+    """Every way the key range is cut, against the same call in Float64.  Bound: the rounding of the result to its
+    type (8, 11 and 24 bits), and 1e-5 for the Float32 sums."""
+    import torch
+
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(E + Lkv)
+    tt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[dtype]
+    q, k, v = (torch.randn(B, L, E, generator=gen, device="cuda").to(tt) for L in (Lq, Lkv, Lkv))
+    keep = torch.ones(B, Lkv, dtype=torch.bool, device="cuda")
+    if masked:
+        keep &= torch.rand(B, Lkv, generator=gen, device="cuda") < 0.7
+        keep[0, Lkv // 3:] = False               # wavefronts and workgroups that keep no key
+        keep[0, 0] = True
+    arr = [nn.DeviceArray.from_torch(t.reshape(-1), (E, t.shape[1], B), dtype) for t in (q, k, v)]
+    mask = nn.DeviceArray.from_torch(keep.to(torch.uint8).reshape(-1), (Lkv, 1, 1, B), "bool") if masked else None
+    y, _ = nn.dot_product_attention(*arr, mask=mask, nheads=H, return_weights=False)
+    assert nn.last_attention_kernel() == "decode"
+    D = E // H
+    qd, kd, vd = (t.double().reshape(B, -1, H, D).transpose(1, 2).contiguous() for t in (q, k, v))
+    s = qd @ kd.transpose(2, 3).contiguous() / np.sqrt(D)
+    s.masked_fill_(~keep[:, None, None, :], -np.inf)
+    ref = (torch.softmax(s, -1) @ vd).transpose(1, 2).reshape(B, Lq, E)
+    err = (y.storage.reshape(B, Lq, E).double() - ref).abs()
+    u = {"bf16": 2.0 ** -8, "f16": 2.0 ** -11, "f32": 2.0 ** -24}[dtype]
+    assert (err <= u * ref.abs() + 1e-5 * ref.abs().max()).all()
+
+
 def test_decode_matches_generic_on_device(nn):
     rng = np.random.default_rng(11)
     q = nn.DeviceArray.from_numpy(rng.standard_normal((512, 1, 2)).astype(np.float32), "bf16")
