@@ -193,6 +193,24 @@ def test_gradient_of_a_shared_bias_apart_from_dq(nn, oracle, dtype, D, H, Lq, Lk
          scale=0.4, saved=saved, expect="flash16")
 
 
+@pytest.mark.parametrize("dtype,D,H,Lq,Lkv,B,mask_kind,biased,dropout", [
+    ("bf16", 64, 9, 130, 260, 10, None, False, None),             # a query tile of 2, a key tile of 4
+    ("f16", 40, 9, 65, 385, 10, "lengths", False, None),          # features past the head dim, lengths and scattered masks
+    ("bf16", 64, 9, 300, 300, 16, "causal", False, None),
+    ("bf16", 8, 29, 1025, 1025, 2, "causal", False, None),        # more than eight key tiles
+    ("bf16", 64, 9, 70, 333, 10, "keys", False, (0.25, 4242)),    # keep words: rows off the hash groups
+    ("f16", 64, 9, 292, 292, 16, "causal", False, (0.25, 4242)),  # decisions redrawn
+    ("bf16", 64, 9, 100, 272, 10, "random", False, None),         # a dense mask as bits
+    ("bf16", 64, 9, 97, 270, 10, None, True, None),               # a bias from its copies
+])
+def test_both_key_gradients_in_one_pass(nn, oracle, dtype, D, H, Lq, Lkv, B, mask_kind, biased, dropout):
+    """Tiles of 64 features and more than 256 workgroups of 128 keys (with a causal mask 400, 512 beyond eight key tiles)."""
+    tiles = (Lkv + 127) // 128
+    assert Lkv > 256 and tiles * H * B > (256 if mask_kind != "causal" else 400 if tiles <= 8 else 512)
+    _run(nn, oracle, dtype, D * H, D * H, Lq, Lkv, (B,), H, bias_shape=(Lkv, Lq, H, 1) if biased else None, mask_kind=mask_kind,
+         seed=Lq + Lkv, scale=0.6, saved=True, dropout=dropout, expect="flash16")
+
+
 F32_CASES = [
     # D, H, Lq, Lkv, batch, mask_kind, saved statistics
     (64, 2, 200, 200, (2,), "causal", False),
