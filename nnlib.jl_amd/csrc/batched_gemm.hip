@@ -3,7 +3,8 @@
 // through the _batched_gemm! hook (src/batched/batchedmul.jl:298).  Column-major.
 //
 // The kernels of batched_gemm16.hip, batched_gemm32.hip and batched_gemm32_waves.hip take nearly every product; the one here
-// keeps 16-bit products of less than 64 x 64 elements or with leading dimensions below 16 bytes, and slices beyond 2 GiB.
+// keeps 16-bit products of few elements and terms (batched_gemm16_supports) or with leading dimensions below 16 bytes, and slices
+// beyond 2 GiB.
 //
 // Workgroup = 4 wavefronts, output tile 64 (m) x 64 (n), each wavefront one 32x32 block.
 // The MFMA is issued on the transposed problem (rows = n, columns = m) so that a lane's
@@ -12,7 +13,8 @@
 #include "common.h"
 
 // tiled 16-bit fast path (batched_gemm16.hip)
-bool batched_gemm16_supports(int32_t dtype, int transA, int transB, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb);
+bool batched_gemm16_supports(int32_t dtype, int transA, int transB, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
+                             int64_t batch);
 int32_t launch_batched_gemm16(int32_t dtype, int transA, int transB, int64_t m, int64_t n, int64_t k, float alpha, const void *A,
                               int64_t lda, int64_t sA, const void *B, int64_t ldb, int64_t sB, float beta, void *C, int64_t ldc,
                               int64_t sC, int64_t batch, hipStream_t st);
@@ -231,7 +233,7 @@ MI_API int32_t mi_batched_gemm(int32_t dtype, char transA, char transB, int64_t 
         return mi_set_error(MI_ESHAPE, "mi_batched_gemm: matrix too large for one launch (n tiles > 65535)");
     GemmArgs g = {A, B, C, m, n, k, lda, ldb, ldc, strideA, strideB, strideC, alpha, beta, ta, tb};
     hipStream_t st = (hipStream_t)s;
-    if (batched_gemm16_supports(dtype, ta, tb, m, n, k, lda, ldb))
+    if (batched_gemm16_supports(dtype, ta, tb, m, n, k, lda, ldb, batch))
         return launch_batched_gemm16(dtype, ta, tb, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, strideC, batch, st);
     if (batched_gemm32_supports(dtype, ta, tb, m, n, k, A, lda, strideA, B, ldb, strideB))
         return launch_batched_gemm32(ta, tb, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, strideC, batch, st);

@@ -531,9 +531,15 @@ int32_t launch_t(const Gemm16Args &g, int transA, int transB, int64_t nb, bool a
 }  // namespace
 
 // true when the tiled kernels take the product: slices that 32-bit byte offsets address and that hold a 16-byte piece
-bool batched_gemm16_supports(int32_t dtype, int transA, int transB, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb) {
+bool batched_gemm16_supports(int32_t dtype, int transA, int transB, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, int64_t batch) {
     if (dtype != MI_F16 && dtype != MI_BF16) return false;
-    if (k < 1 || m * n < 64 * 64) return false;   // tiny products: the small-tile kernel wastes less
+    if (k < 1) return false;
+    // Small results stay on the 64 x 64 kernel where its one memory round trip per 32 k is a short chain and its four to eight
+    // workgroups per CU (two of the tiled kernel, which fetches two stages of 64 k ahead) hold many slices.  GPU time, us, 64 x 64
+    // kernel / tiled, bf16: 64 x 48 x 832, 18 slices 47.9 / 11.4; 32 x 32 x 64, 256 slices 6.2 / 4.4, 4096 39 / 26;
+    // 16 x 16 x 256, 4096 slices 118 / 47; 8 x 200 x 64, 1024 slices 41 / 14.  The other way: 16 x 16 x 64, 4096 slices, 'T' 18.1 / 25.4;
+    // 56 x 56 x 32, 1024 slices 7.7 / 8.9; 17 x 33 x 128 of any alignment, 1024 slices 12.6 / 15.2; 17 x 33 x 32, 18 slices 4.7 / 5.7.
+    if (m * n < 64 * 64 && m <= 128 && n <= 128 && (batch <= 512 ? k <= 32 : m * n * k < 50 * 50 * 50)) return false;
     const int64_t extA = transA ? (m - 1) * lda + k : (k - 1) * lda + m, extB = transB ? (k - 1) * ldb + n : (n - 1) * ldb + k;
     if (extA * 2 >= 2147483647LL || extB * 2 >= 2147483647LL) return false;
     // leading dimensions of at least a piece: only the last k or row of a slice can hold a piece that ends past it

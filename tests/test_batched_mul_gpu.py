@@ -453,6 +453,14 @@ def test_operands_of_any_alignment(nn, dtype, ta, tb, m, n, k, batch):
     assert np.array_equal(got[:, :, m], before[1:].reshape(batch, n, m + 1)[:, :, m]) and after[0] == before[0]
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("m,n,k,batch", [(1, 1, 33, 2), (5, 7, 32, 3), (63, 65, 33, 2), (8, 129, 1, 2), (48, 64, 832, 2), (50, 50, 50, 513), (50, 49, 50, 513)])
+def test_few_results_of_16_bit_products(nn, dtype, ta, tb, m, n, k, batch):
+    """Results of less than 64 x 64 elements on both sides of the limits between the two 16-bit kernels (k, m * n * k, batch)."""
+    test_operands_of_any_alignment(nn, dtype, ta, tb, m, n, k, batch)
+
+
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("m,n,k,batch", [(131, 129, 77, 3), (67, 190, 5, 2), (511, 509, 131, 64)])
 def test_unaligned_float32_products_at_the_ends_of_the_range(nn, ta, tb, m, n, k, batch):
