@@ -170,6 +170,7 @@ struct CfgS {
     // chunk swizzle of the 16-bit kernel (conflict-free 16-byte operand reads and transposing reads)
     __device__ static inline int swz(int row) {
         if (D >= 128) return ((row & 3) << 2) | ((row >> 2) & 3);
+        if (D == 96) return (row >> 2) & 3;   // rows 12 chunks apart: four of them start 0, 12, 8 and 4 chunks into the 16 that the banks hold
         const int x = (row >> 1) & 7;
         return ((x & 1) << 2) | (x >> 1);
     }
@@ -284,6 +285,7 @@ __device__ inline void run_tiles32s(const FlashArgs &a, Frag32S<D, QB> &f, unsig
     const AttnParams &p = a.p;
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hh = lane >> 5;
     constexpr bool NEED_V = PHASE != PHASE_STATS;
+    constexpr bool AHEAD = D != 96;   // two workgroups per CU: the next tile's 48 registers do not fit beside the products, the other workgroup covers its latency
     const bool do_pv = NEED_V && p.out != nullptr;
     typedef __attribute__((address_space(3))) u32x2_t *lds8_t;
     typedef __attribute__((address_space(3))) const plane8 *lds_plane8_t;
@@ -335,7 +337,7 @@ __device__ inline void run_tiles32s(const FlashArgs &a, Frag32S<D, QB> &f, unsig
     for (int jt = jt0; jt < n_tiles; jt++) {
         const int64_t j0 = (int64_t)jt * BN;
         const bool more = jt + 1 < n_tiles;
-        if (more) load_tile(jt + 1);
+        if (more && AHEAD) load_tile(jt + 1);
 
         const bool active = !CAUSAL || j0 <= iw + 32 * QB - 1;
         if (active) {
@@ -348,6 +350,7 @@ __device__ inline void run_tiles32s(const FlashArgs &a, Frag32S<D, QB> &f, unsig
             if (do_pv) weights_times_values32s<D, QB>(f, Vs, s);
         }
         if (more) {
+            if (!AHEAD) load_tile(jt + 1);
             __syncthreads();   // every wavefront is done with the tile in LDS
             store_tile();
         }
@@ -362,8 +365,10 @@ struct FragSel<D, QB, true> { typedef Frag32S<D, QB> type; };
 
 template <int D, int QB, bool CAUSAL, bool EXTRAS, bool WEIGHTS, bool SPLIT>
 // Head dim 64 without bias / mask fits two workgroups per CU (256 registers, 70 KiB of LDS each; 56 KiB with the
-// bf16 planes, bias / mask or not).
-__global__ __launch_bounds__(256, (D == 64 && !EXTRAS) ? 2 : 1) void flash32_kernel(FlashArgs a) {
+// bf16 planes, bias / mask or not).  So do 96 features in planes (72 KiB, the next tile fetched behind the products): head dims
+// from 68 to 96 without bias / mask code, a quarter fewer matrix instructions than 128-wide tiles and two wavefronts per SIMD instead of
+// one (12 x 14 pairs of 585 x 585, head dim 96, weights returned: 551 -> 384 us; 16 x 13 of 576 x 576, head dim 80: 390 -> 233).
+__global__ __launch_bounds__(256, (D <= 96 && !EXTRAS) ? 2 : 1) void flash32_kernel(FlashArgs a) {
     constexpr int KS = Cfg<D>::KS, VS = Cfg<D>::VS;
     const AttnParams &p = a.p;
     extern __shared__ __attribute__((aligned(16))) unsigned char flash_smem[];
@@ -1415,6 +1420,12 @@ bool exact_instruction_wanted() {
 template <int D, int QB>
 int32_t launch_d(const FlashArgs &a, hipStream_t st, bool extras) {
     if (exact_instruction_wanted()) return launch_ds<D, QB, false>(a, st, extras);
+    if constexpr (D == 128)
+        if (!extras && a.p.D <= 96 && a.p.Dv <= 96) {
+            const bool w = a.p.weights != nullptr;
+            if (a.p.causal) return w ? launch_one<96, QB, true, false, true, true>(a, st) : launch_one<96, QB, true, false, false, true>(a, st);
+            return w ? launch_one<96, QB, false, false, true, true>(a, st) : launch_one<96, QB, false, false, false, true>(a, st);
+        }
     return launch_ds<D, QB, true>(a, st, extras);
 }
 
@@ -1495,7 +1506,7 @@ int32_t FLASH32_LAUNCH(const AttnParams &p, hipStream_t st) {
     }
     if (resident) return launch_resident<64>(a, st, extras);
     if (chunks) {
-        if (!narrow) return launch_resident_chunks<128, RES_CHUNKS>(a, st, extras);
+        if (!narrow) return p.D <= 96 && p.Dv <= 96 ? launch_resident_chunks<96, RES_CHUNKS>(a, st, extras) : launch_resident_chunks<128, RES_CHUNKS>(a, st, extras);
         return p.Lkv <= RES_CHUNKS * 128 ? launch_resident_chunks<64, RES_CHUNKS>(a, st, extras) : launch_resident_chunks<64, RES_CHUNKS_NARROW>(a, st, extras);
     }
     return narrow ? launch_d<64, 1>(a, st, extras) : launch_d<128, 1>(a, st, extras);

@@ -1077,3 +1077,14 @@ def test_a_short_key_range_with_a_bias_needs_no_workspace(nn):
     d.out = out.ptr
     nn._lib.check(lib.mi_attention_fwd(ctypes.byref(d), None))
     assert rel_err(out.to_numpy(), y.to_numpy()) <= 2 * 2.0 ** -11
+
+
+@pytest.mark.parametrize("weights", [False, True])
+@pytest.mark.parametrize("E,H,Lq,Lkv,B,kw", [
+    (68 * 2, 2, 130, 193, 2, {}), (96 * 12, 12, 129, 513, 6, {}), (80 * 2, 2, 257, 257, 2, dict(causal=True)),
+    (96 * 8, 8, 300, 300, 16, dict(causal=True)), (72 * 2, 2, 40, 70, 2, dict(mask_shape=(70, 40))),
+    (96 * 2, 2, 70, 520, 2, dict(mask_shape=(520, 1, 1, 2))), (96, 1, 70, 2500, 1, {}), (96 * 2, 2, 64, 600, 3, dict(Ev=80 * 2)),
+])
+def test_float32_tiles_of_96_features(nn, oracle, E, H, Lq, Lkv, B, kw, weights):
+    """Head dims 68 to 96: one and two passes, few and many workgroups, key pieces, context lengths."""
+    _check(nn, oracle, np.random.default_rng(E + Lkv), "f32", E, Lq, Lkv, B, H, expect="flash32", weights=weights, **kw)
