@@ -494,6 +494,7 @@ struct CfgS {
     // chunk swizzle of the 16-bit kernels (conflict-free 16-byte operand reads and transposing reads)
     __device__ static inline int swz(int row) {
         if (D >= 128) return ((row & 3) << 2) | ((row >> 2) & 3);
+        if (D == 96) return (row >> 2) & 3;   // rows 12 chunks apart: four of them start 0, 12, 8 and 4 chunks into the 16 that the banks hold
         const int x = (row >> 1) & 7;
         return ((x & 1) << 2) | (x >> 1);
     }
@@ -671,6 +672,7 @@ template <int D, bool CAUSAL, bool HAVE_STATS, int NW>
 __global__ __launch_bounds__(64 * NW, 1) void bwd32s_dq_kernel(FlashArgs a, AttnBwdParams bp) {
     typedef CfgS<D> C;
     constexpr int NDV = D / 32, NT = 64 * NW;
+    constexpr int KB_UNROLL = D == 128 && !CAUSAL ? 1 : 2;
     constexpr bool X_LDS = NW == 8;
     constexpr bool AHEAD = D == 64 && !X_LDS;
     constexpr int XPLANEB = 32 * NW * C::ROWB;
@@ -801,7 +803,7 @@ __global__ __launch_bounds__(64 * NW, 1) void bwd32s_dq_kernel(FlashArgs a, Attn
         if (more && AHEAD) ts.load(j0 + BN);
         if (!CAUSAL || j0 <= iw + 31) {
             const bool edge = (j0 + BN > kv_len) || (CAUSAL && j0 + BN - 1 > iw);
-#pragma unroll
+#pragma unroll KB_UNROLL
             for (int kb = 0; kb < 2; kb++) {
                 if (CAUSAL && j0 + 32 * kb > iw + 31) break;   // every key of this block is after every query of the wavefront
                 floatx16_t sb = first_product_s<D>(Ks, kb, qx, (floatx16_t){0}, r, hh);
@@ -849,13 +851,24 @@ __global__ __launch_bounds__(64 * NW, 1) void bwd32s_dq_kernel(FlashArgs a, Attn
     }
 }
 
-template <int D, bool CAUSAL, int WHICH>
-// Head dim 64 fits two workgroups per compute unit, each fetching its next tiles only once the products are done (no
-// staging registers live across them): the other workgroup covers the latency.  WHICH = BWD_DV | BWD_DK: both
-// gradients from one S and dP, one workgroup per compute unit (see launch_set_planes).
-__global__ __launch_bounds__(256, D == 64 && WHICH != 3 ? 2 : 1) void bwd32s_dkdv_kernel(FlashArgs a, AttnBwdParams bp) {
+// dK and dV.  WHICH = BWD_DV | BWD_DK: both from one S and dP (seven products for the gradient instead of eight).  OCC workgroups share a
+// compute unit, each fetching its next tiles only once the products are done (no staging registers live across them).  What a lane
+// holds (planes of its K and V rows, two accumulators, S, dP) and how it fits:
+//   - head dim 64, OCC = 1: one wavefront per SIMD, everything in registers (370);
+//   - head dim 64, OCC = 2: two wavefronts per SIMD from two workgroups, 256 registers and 72-140 bytes of scratch;
+//   - head dim 64, NW = 8 (256 keys a workgroup): the V planes live in LDS behind the tiles, 251 registers, no scratch;
+//   - up to 96 and 128: one wavefront per SIMD.  One 32-query block at a time (KB_UNROLL = 1): with both blocks of a tile in the
+//     scheduler's hands a lane of 128 features needed up to 1108 bytes of scratch, now 52 (causal none), and one kernel
+//     replaces the pair that formed S twice (12 x 6 pairs of 746 x 746: 462 -> 320 us; causal 8 x 8 of 1024 x 1024: 390 -> 250).
+//     96 features without the causal mask fit with both (437 us at 12 x 14 of 585 x 585, 452 one at a time; the 128-wide
+//     pair took 807).
+template <int D, bool CAUSAL, int WHICH, int NW = 4, int OCC = (D == 64 && WHICH != 3) ? 2 : 1>
+__global__ __launch_bounds__(64 * NW, OCC) void bwd32s_dkdv_kernel(FlashArgs a, AttnBwdParams bp) {
     typedef CfgS<D> C;
-    constexpr int NDV = D / 32;
+    constexpr int NDV = D / 32, NT = 64 * NW;
+    constexpr int KB_UNROLL = D == 128 || (D == 96 && CAUSAL) || OCC == 2 || NW == 8 ? 1 : 2;
+    constexpr bool X_LDS = NW == 8;
+    constexpr int XPLANEB = 32 * NW * C::ROWB;
     constexpr bool DO_DV = (WHICH & BWD_DV) != 0, DO_DK = (WHICH & BWD_DK) != 0;   // 3: both from one S and dP
     const AttnParams &p = a.p;
     extern __shared__ __attribute__((aligned(16))) unsigned char bwd_smem[];
@@ -864,7 +877,7 @@ __global__ __launch_bounds__(256, D == 64 && WHICH != 3 ? 2 : 1) void bwd32s_dkd
     const int64_t HB = p.H * p.B;
     const int64_t hb = blockIdx.x % HB, kt_idx = blockIdx.x / HB;   // with causal masks the early key tiles are the long ones
     const int64_t h = hb % p.H, b = hb / p.H;
-    const int64_t j0 = kt_idx * 128, jw = j0 + 32 * wave, kv = jw + r;
+    const int64_t j0 = kt_idx * (32 * NW), jw = j0 + 32 * wave, kv = jw + r;
     const bool kok = kv < p.Lkv;
     int64_t kv_len = p.Lkv;
     if (a.kv_len) {
@@ -888,9 +901,21 @@ __global__ __launch_bounds__(256, D == 64 && WHICH != 3 ? 2 : 1) void bwd32s_dkd
         return;
     }
 
-    plane8 kx[3][D / 16], vx[DO_DK ? 3 : 1][D / 16];
+    plane8 kx[3][D / 16], vx[DO_DK && !X_LDS ? 3 : 1][D / 16];
+    const unsigned xrow = Qs + 2 * C::TILEB + sizeof(float) * 2 * 3 * BN + (unsigned)(32 * wave + r) * C::ROWB;
+    const int xsw = C::swz(r);
     load_stationary_s<D>(kx, (const float *)p.k + off, kvalid, hh, (int)p.D);
-    if constexpr (DO_DK) load_stationary_s<D>(vx, (const float *)p.v + off, kvalid, hh, (int)p.D);
+    if constexpr (DO_DK && X_LDS) {
+        typedef __attribute__((address_space(3))) plane8 *lds_plane8_t;
+        plane8 tmp[3][D / 16];
+        load_stationary_s<D>(tmp, (const float *)p.v + off, kvalid, hh, (int)p.D);
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+#pragma unroll
+            for (int t = 0; t < D / 16; t++) *(lds_plane8_t)(uintptr_t)(xrow + q * XPLANEB + (((2 * t + hh) ^ xsw) << 4)) = tmp[q][t];
+    } else if constexpr (DO_DK) {
+        load_stationary_s<D>(vx, (const float *)p.v + off, kvalid, hh, (int)p.D);
+    }
     floatx16_t accv[DO_DV ? NDV : 1], acck[DO_DK ? NDV : 1];
 #pragma unroll
     for (int dvb = 0; dvb < (DO_DV ? NDV : 1); dvb++) accv[dvb] = (floatx16_t){0};
@@ -904,7 +929,7 @@ __global__ __launch_bounds__(256, D == 64 && WHICH != 3 ? 2 : 1) void bwd32s_dkd
     floatx4_t st_reg = {0, 0, 0, 0};
     const float cs = a.c;
 
-    PlaneStream<D> ts;
+    PlaneStream<D, NT> ts;
     ts.base1 = (const float *)p.q + p.E * (p.Lq * b) + p.D * h;
     ts.base2 = (const float *)bp.dout + p.E * (p.Lq * b) + p.D * h;
     ts.dh = (int)p.D;
@@ -928,12 +953,13 @@ __global__ __launch_bounds__(256, D == 64 && WHICH != 3 ? 2 : 1) void bwd32s_dkd
         if (!CAUSAL || i0 + BN - 1 >= jw) {
             const float *st = st_lds + buf * (3 * BN);
             const bool diag = CAUSAL && i0 < jw + 32;   // some (query, key) pair of this tile has key > query
-#pragma unroll
+#pragma unroll KB_UNROLL
             for (int kb = 0; kb < 2; kb++) {
                 floatx16_t s = first_product_s<D>(Qs, kb, kx, (floatx16_t){0}, r, hh);
                 SCHED_FENCE();
                 floatx16_t dp = (floatx16_t){0};
-                if constexpr (DO_DK) dp = first_product_s<D>(dOs, kb, vx, dp, r, hh);
+                if constexpr (DO_DK && X_LDS) dp = first_product_sl<D, XPLANEB>(dOs, kb, xrow, xsw, dp, r, hh);
+                else if constexpr (DO_DK) dp = first_product_s<D>(dOs, kb, vx, dp, r, hh);
                 SCHED_FENCE();
                 // accumulator register 4g+e of this lane: query i0 + 32kb + 8g + 4hh + e, key kv.  Rows past Lq carry
                 // statistics (0, 0, 0): their weights vanish; keys past the length only feed columns that store zeros
@@ -1321,23 +1347,33 @@ template <int D, bool CAUSAL>
 int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream_t st) {
     const AttnParams &p = a.p;
     constexpr size_t SMEM = CfgS<D>::SMEM;
-    // the dQ kernel on eight wavefronts (256 queries a workgroup) where those workgroups still fill the chip
+    // the dQ kernel on eight wavefronts (256 queries a workgroup) where the workgroups of four would need a second round of the chip
+    // (52 pairs of 1024 x 1024: 208 workgroups of eight 131 us, 416 of four 195); with a causal mask, whose lengths a second round evens
+    // out, where those of eight fill the chip (48 pairs of 1024 x 1024: 192 of eight 109 us, 384 of four 92)
     constexpr int NW_WIDE = D == 64 ? 8 : 4;
     constexpr size_t SMEM_WIDE = SMEM + 3 * 32 * NW_WIDE * CfgS<D>::ROWB;
     const int64_t wide_tiles = (p.Lq + 32 * NW_WIDE - 1) / (32 * NW_WIDE);
     // (not for sequences of at most 128 queries, where half of its wavefronts would have none: 4-6 % slower there)
-    const bool wide = NW_WIDE > 4 && bp.dq_nsplit <= 1 && wide_tiles * p.H * p.B >= 256 && p.Lq > 128;
+    const bool wide = NW_WIDE > 4 && bp.dq_nsplit <= 1 && p.Lq > 128 && wide_tiles * p.H * p.B >= (CAUSAL ? 256 : 129);
     auto k1 = bp.have_stats ? bwd32s_dq_kernel<D, CAUSAL, true, 4> : bwd32s_dq_kernel<D, CAUSAL, false, 4>;
     auto k1w = bp.have_stats ? bwd32s_dq_kernel<D, CAUSAL, true, NW_WIDE> : bwd32s_dq_kernel<D, CAUSAL, false, NW_WIDE>;
     auto k2 = bwd32s_dkdv_kernel<D, CAUSAL, BWD_DV>;
     auto k3 = bwd32s_dkdv_kernel<D, CAUSAL, BWD_DK>;
-    // Both from one S and dP (seven products for the gradient instead of eight) at one workgroup per compute unit: the
-    // two stationary rows and two accumulators of a lane do not fit 256 registers (428-512 bytes of scratch at two
-    // workgroups per unit).  Measured against the pair: C2-shaped gradient 0.437 -> 0.425 ms, the same without the causal
-    // mask 0.823 -> 0.712, 2048 x 2048 with 32 pairs 0.538 -> 0.440 (causal) and 0.777 -> 0.661, 4096 x 4096 with 8 pairs
-    // 0.94 -> 0.75.  128-wide tiles keep the pair (512 registers either way, 688-1108 bytes of scratch fused).
+    // Both gradients, head dim 64: the form that needs the fewest rounds of the chip, a round of 256 workgroups of eight wavefronts
+    // taking 1.5 times, one of 512 of four, two to a compute unit, 1.9 times as long as one of 256 of four (without a causal
+    // mask, us in this kernel: 128 pairs of 1024 x 1024 480 / 456 / 395 on one, two, eight; 52 pairs 227 / 197 / 167; 104 of
+    // 752 x 752 274 / 262 / 248; 264 of 120 x 120 43 / 34 / 50).  With a causal mask two workgroups to a unit even out the lengths of
+    // their loops (128 pairs of 1024 x 1024: 302 / 253 / 258; 128 of 648 x 648 164 / 109 / 112; whole steps, one / two: 80 of 1024 x
+    // 1024 373 / 344, 256 of 256 x 256 131 / 115), unless few are left for the second of a unit and the longest ones share one
+    // (48 pairs of 1024 x 1024 293 / 298).
     auto k23 = bwd32s_dkdv_kernel<D, CAUSAL, BWD_DV | BWD_DK>;
-    static const bool fused_dkdv = D == 64 && getenv("MI355ATTN_F32_DKDV_PAIR") == nullptr;   // the switch: for comparisons
+    auto k23two = bwd32s_dkdv_kernel<D, CAUSAL, BWD_DV | BWD_DK, 4, D == 64 ? 2 : 1>;
+    auto k23w = bwd32s_dkdv_kernel<D, CAUSAL, BWD_DV | BWD_DK, NW_WIDE>;
+    const int64_t key_tiles = (p.Lkv + 127) / 128 * p.H * p.B, wide_key_tiles = (p.Lkv + 32 * NW_WIDE - 1) / (32 * NW_WIDE) * p.H * p.B;
+    const auto rounds = [](int64_t tiles, int64_t slots) { return (double)((tiles + slots - 1) / slots); };
+    const bool two_dkdv = D == 64 && (CAUSAL ? key_tiles > (p.Lkv <= 512 ? 256 : 512) : 1.9 * rounds(key_tiles, 512) < rounds(key_tiles, 256));
+    const bool wide_dkdv = D == 64 && !CAUSAL && p.Lkv > 128 && 1.5 * rounds(wide_key_tiles, 256) <= (two_dkdv ? 1.9 * rounds(key_tiles, 512) : rounds(key_tiles, 256));
+    static const bool fused_dkdv = getenv("MI355ATTN_F32_DKDV_PAIR") == nullptr;   // the switch: for comparisons
     static bool attr_set = false;  // per instantiation; the attribute is idempotent, so a race is harmless
     if (!attr_set) {
         MI_HIP_CHECK(hipFuncSetAttribute((const void *)bwd32s_dq_kernel<D, CAUSAL, true, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMEM));
@@ -1349,6 +1385,8 @@ int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream
         MI_HIP_CHECK(hipFuncSetAttribute((const void *)k2, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMEM));
         MI_HIP_CHECK(hipFuncSetAttribute((const void *)k3, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMEM));
         MI_HIP_CHECK(hipFuncSetAttribute((const void *)k23, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMEM));
+        MI_HIP_CHECK(hipFuncSetAttribute((const void *)k23two, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMEM));
+        if (NW_WIDE > 4) MI_HIP_CHECK(hipFuncSetAttribute((const void *)k23w, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMEM_WIDE));
         attr_set = true;
     }
     // few 32-row blocks (at most two workgroups per compute unit) and the forward call's statistics: the workgroups per
@@ -1405,7 +1443,8 @@ int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream
         if constexpr (D == 64)
             if (bp.dv || bp.dk) hipLaunchKernelGGL((bwd32s_dkdv_small_kernel<D, CAUSAL, false>), dim3((unsigned)k_blocks), dim3(256), SmallBwd<D>::SMEM, st, a, bp);
     } else if (bp.dv && bp.dk && fused_dkdv) {
-        hipLaunchKernelGGL(k23, g2, dim3(256), SMEM, st, a, bp);
+        if (wide_dkdv) hipLaunchKernelGGL(k23w, dim3((unsigned)wide_key_tiles), dim3(64 * NW_WIDE), SMEM_WIDE, st, a, bp);
+        else hipLaunchKernelGGL(two_dkdv ? k23two : k23, g2, dim3(256), SMEM, st, a, bp);
     } else {
         if (bp.dv) hipLaunchKernelGGL(k2, g2, dim3(256), SMEM, st, a, bp);
         if (bp.dk) hipLaunchKernelGGL(k3, g2, dim3(256), SMEM, st, a, bp);
@@ -1417,7 +1456,11 @@ int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream
 template <int D, bool CAUSAL, int EXTRAS, bool DROP = false>
 int32_t launch_set(const FlashArgs &a, const AttnBwdParams &bp, hipStream_t st) {
     if constexpr (EXTRAS == EXTRAS_NONE && !DROP)
-        if (!bp.dbias && !exact_instruction_wanted()) return launch_set_planes<D, CAUSAL>(a, bp, st);
+        if (!bp.dbias && !exact_instruction_wanted()) {
+            if constexpr (D == 128)
+                if (bp.p.D <= 96) return launch_set_planes<96, CAUSAL>(a, bp, st);
+            return launch_set_planes<D, CAUSAL>(a, bp, st);
+        }
     const AttnParams &p = a.p;
     constexpr size_t SMEM = Cfg<D>::SMEM;
     constexpr size_t SMEM_Q = SMEM + (EXTRAS == EXTRAS_NONE ? 0 : 4 * FLASH_WSTAGE_BYTES);   // the dQ kernel's staging for the bias gradient

@@ -932,3 +932,16 @@ def test_shared_bias_gradient_in_tiles_of_128(nn, oracle, dtype, D, H, Lq, Lkv, 
     E = D * H
     for saved in (True, False):
         _run(nn, oracle, dtype, E, E, Lq, Lkv, batch, H, mask_kind=mask_kind, bias_shape=(Lkv, Lq, H), expect="flash16", saved=saved, seed=Lq + Lkv)
+
+
+@pytest.mark.parametrize("D,H,Lq,Lkv,B,mask_kind,saved", [
+    # tiles of 96 features (head dims 68 to 96) and both key gradients in one pass in tiles of 96 and 128
+    (68, 2, 130, 193, 2, None, True), (96, 2, 65, 127, 2, None, False), (80, 2, 257, 257, 1, "causal", True),
+    (96, 3, 100, 300, 4, "lengths", True), (128, 2, 129, 65, 2, None, False), (100, 2, 200, 200, 1, "causal", True),
+    # head dims up to 64: a workgroup of four wavefronts, two of them to a compute unit, one of eight
+    (64, 8, 40, 130, 12, None, True), (64, 12, 70, 120, 22, None, True), (64, 8, 66, 260, 12, None, True), (48, 8, 64, 385, 12, None, False),
+    (60, 8, 257, 257, 11, "causal", True), (64, 8, 130, 300, 12, "lengths", True),
+])
+def test_float32_key_gradients_in_one_pass(nn, oracle, D, H, Lq, Lkv, B, mask_kind, saved):
+    """The forms of the Float32 kernel that makes dK and dV from one S and dP, at the edges of their tiles and of the rule."""
+    _run(nn, oracle, "f32", D * H, D * H, Lq, Lkv, (B,), H, mask_kind=mask_kind, saved=saved, scale=0.4, seed=D + Lkv, expect="flash32")
