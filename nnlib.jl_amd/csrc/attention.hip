@@ -5,8 +5,12 @@
 
 // kv_len: null, or per (head, batch) context lengths (FlashArgs::kv_len)
 int32_t launch_flash16_bf16_d64(const AttnParams &, hipStream_t, const int32_t *kv_len = nullptr, bool lengths_variant = false);
+int32_t launch_flash16_bf16_d32(const AttnParams &, hipStream_t, const int32_t *kv_len = nullptr, bool lengths_variant = false);
+int32_t launch_flash16_bf16_d96(const AttnParams &, hipStream_t, const int32_t *kv_len = nullptr, bool lengths_variant = false);
 int32_t launch_flash16_bf16_d128(const AttnParams &, hipStream_t, const int32_t *kv_len = nullptr, bool lengths_variant = false);
 int32_t launch_flash16_f16_d64(const AttnParams &, hipStream_t, const int32_t *kv_len = nullptr, bool lengths_variant = false);
+int32_t launch_flash16_f16_d32(const AttnParams &, hipStream_t, const int32_t *kv_len = nullptr, bool lengths_variant = false);
+int32_t launch_flash16_f16_d96(const AttnParams &, hipStream_t, const int32_t *kv_len = nullptr, bool lengths_variant = false);
 int32_t launch_flash16_f16_d128(const AttnParams &, hipStream_t, const int32_t *kv_len = nullptr, bool lengths_variant = false);
 int32_t launch_flash16_bf16_d256(const AttnParams &, hipStream_t, const int32_t *kv_len = nullptr, bool lengths_variant = false);
 int32_t launch_flash16_f16_d256(const AttnParams &, hipStream_t, const int32_t *kv_len = nullptr, bool lengths_variant = false);
@@ -78,7 +82,7 @@ static bool takes_fast_path(const AttnParams &p);
 
 bool attention_flash16_supports(const AttnParams &p) {
     if (p.dtype != MI_F16 && p.dtype != MI_BF16) return false;
-    // head dims: multiples of 8 (16-byte chunks) up to the 256-wide tiles; the tile width (64, 128 or 256) is the
+    // head dims: multiples of 8 (16-byte chunks) up to the 256-wide tiles; the tile width (32, 64, 96, 128 or 256) is the
     // smallest that holds both, and what it has beyond them is zero-padded in flight
     if (p.D < 8 || p.Dv < 8 || p.D > 256 || p.Dv > 256 || (p.D & 7) || (p.Dv & 7)) return false;
     if (!aligned16(p.q) || !aligned16(p.k) || (p.out && (!aligned16(p.v) || !aligned16(p.out)))) return false;
@@ -179,11 +183,17 @@ int32_t launch_key_mask_lengths(const AttnParams &p, int32_t *lens, hipStream_t 
 
 static int32_t launch_general16(const AttnParams &p, hipStream_t st, const int32_t *kv_len, bool lv = false) {
     const int64_t dmax = p.D > p.Dv ? p.D : p.Dv;
-    if (p.dtype == MI_BF16)
-        return dmax <= 64    ? launch_flash16_bf16_d64(p, st, kv_len, lv)
-               : dmax <= 128 ? launch_flash16_bf16_d128(p, st, kv_len, lv)
-                             : launch_flash16_bf16_d256(p, st, kv_len, lv);
-    return dmax <= 64 ? launch_flash16_f16_d64(p, st, kv_len, lv) : dmax <= 128 ? launch_flash16_f16_d128(p, st, kv_len, lv) : launch_flash16_f16_d256(p, st, kv_len, lv);
+    auto kern = p.dtype == MI_BF16 ? (dmax <= 32    ? launch_flash16_bf16_d32
+                                      : dmax <= 64  ? launch_flash16_bf16_d64
+                                      : dmax <= 96  ? launch_flash16_bf16_d96
+                                      : dmax <= 128 ? launch_flash16_bf16_d128
+                                                    : launch_flash16_bf16_d256)
+                                   : (dmax <= 32    ? launch_flash16_f16_d32
+                                      : dmax <= 64  ? launch_flash16_f16_d64
+                                      : dmax <= 96  ? launch_flash16_f16_d96
+                                      : dmax <= 128 ? launch_flash16_f16_d128
+                                                    : launch_flash16_f16_d256);
+    return kern(p, st, kv_len, lv);
 }
 
 static int32_t launch_fast16(const AttnParams &p, hipStream_t st, const int32_t *kv_len, const AttnMaskWords *mw = nullptr) {

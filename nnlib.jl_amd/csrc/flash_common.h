@@ -160,8 +160,8 @@ __device__ inline i32x4_t flash_make_rsrc(const void *base, uint32_t bytes) {
 }
 
 // Streams [FLASH_BN][ROWB bytes] tiles of one row-major 16-bit array global -> LDS with 1 KiB DMA pieces: no staging
-// registers.  A piece (64 lanes x 16 bytes) covers 1024 / ROWB tile rows; lane l of piece i lands at chunk position
-// l % (ROWB / 16) of tile row i * (1024 / ROWB) + l / (ROWB / 16) and fetches the source chunk `position ^ swz(row)`,
+// registers.  Lane l of piece i (64 lanes x 16 bytes) lands at chunk 64 i + l of the tile, chunk position
+// (64 i + l) % (ROWB / 16) of tile row (64 i + l) / (ROWB / 16), and fetches the source chunk `position ^ swz(row)`,
 // which is how the consumers address the tile.  Each of the four wavefronts moves PIECES pieces per tile.
 // The buffer resource is rebuilt per tile with the tile's first row as its base (64-bit scalar arithmetic), so the
 // per-lane offsets are tile-local and arrays of any size work; rows past the end of the array lie outside the
@@ -169,7 +169,7 @@ __device__ inline i32x4_t flash_make_rsrc(const void *base, uint32_t bytes) {
 // beyond the 2 GiB - 1 the resource size is clamped to).
 template <int ROWB>
 struct FlashTileDma {
-    static constexpr int TILEB = FLASH_BN * ROWB, RPP = 1024 / ROWB, PIECES = TILEB / 1024 / 4;
+    static constexpr int TILEB = FLASH_BN * ROWB, PIECES = TILEB / 1024 / 4;
     const char *base;          // element (row 0, first feature of the head) of this batch element
     int64_t row_bytes, end;    // end: bytes from `base` to the end of the batch element's last row
     unsigned lds;              // LDS byte address of this wavefront's first piece in buffer 0
@@ -183,8 +183,9 @@ struct FlashTileDma {
         lds = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)tiles + wave * PIECES * 1024);   // wave-uniform: goes into M0
 #pragma unroll
         for (int i = 0; i < PIECES; i++) {
-            const int row = (wave * PIECES + i) * RPP + lane / (ROWB / 16);
-            const int chunk = (lane % (ROWB / 16)) ^ swz(row);
+            const int at = (wave * PIECES + i) * 64 + lane;   // chunk of the tile
+            const int row = at / (ROWB / 16);
+            const int chunk = (at % (ROWB / 16)) ^ swz(row);
             voff[i] = 8 * chunk < dh ? row * (int)row_bytes + chunk * 16 : (int)0x80000000;
         }
     }

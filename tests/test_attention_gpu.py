@@ -1088,3 +1088,15 @@ def test_a_short_key_range_with_a_bias_needs_no_workspace(nn):
 def test_float32_tiles_of_96_features(nn, oracle, E, H, Lq, Lkv, B, kw, weights):
     """Head dims 68 to 96: one and two passes, few and many workgroups, key pieces, context lengths."""
     _check(nn, oracle, np.random.default_rng(E + Lkv), "f32", E, Lq, Lkv, B, H, expect="flash32", weights=weights, **kw)
+
+
+@pytest.mark.parametrize("weights", [False, True])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("D", [8, 32, 72, 96])
+@pytest.mark.parametrize("Lq,Lkv,kw", [
+    (129, 193, {}), (257, 257, dict(causal=True)), (70, 130, dict(bias_shape=(130, 70, 2, 1))), (66, 131, dict(bias_shape=(131, 66), mask_shape=(131, 66))),
+    (65, 128, dict(mask_shape=(128, 65))), (40, 333, dict(mask_shape=(333, 1, 1, 3))), (30, 2500, {}),
+])
+def test_16_bit_tiles_of_32_and_96_features(nn, oracle, D, dtype, Lq, Lkv, kw, weights):
+    """Head dims up to 32 and from 72 to 96, every form of bias and mask input, key pieces."""
+    _check(nn, oracle, np.random.default_rng(D + Lkv), dtype, 2 * D, Lq, Lkv, 3, 2, expect="flash16", weights=weights, **kw)
