@@ -5,9 +5,13 @@
 #include "flash_common.h"
 #include "attention_pair_rule.h"
 
+int32_t launch_bwd_flash16_bf16_d32(const AttnBwdParams &, hipStream_t);
 int32_t launch_bwd_flash16_bf16_d64(const AttnBwdParams &, hipStream_t);
+int32_t launch_bwd_flash16_bf16_d96(const AttnBwdParams &, hipStream_t);
 int32_t launch_bwd_flash16_bf16_d128(const AttnBwdParams &, hipStream_t);
+int32_t launch_bwd_flash16_f16_d32(const AttnBwdParams &, hipStream_t);
 int32_t launch_bwd_flash16_f16_d64(const AttnBwdParams &, hipStream_t);
+int32_t launch_bwd_flash16_f16_d96(const AttnBwdParams &, hipStream_t);
 int32_t launch_bwd_flash16_f16_d128(const AttnBwdParams &, hipStream_t);
 int32_t launch_bwd_flash16_bf16_d256(const AttnBwdParams &, hipStream_t);
 int32_t launch_bwd_flash16_f16_d256(const AttnBwdParams &, hipStream_t);
@@ -368,9 +372,11 @@ int32_t launch_attention_bwd_flash16(const AttnBwdParams &bp_in, hipStream_t st)
             bp.dbias_only = 1;
         }
         if (p.dtype == MI_BF16)
-            rc = p.D <= 64 ? launch_bwd_flash16_bf16_d64(bp, st) : p.D <= 128 ? launch_bwd_flash16_bf16_d128(bp, st) : launch_bwd_flash16_bf16_d256(bp, st);
+            rc = p.D <= 32 ? launch_bwd_flash16_bf16_d32(bp, st)
+                 : p.D <= 64 ? launch_bwd_flash16_bf16_d64(bp, st) : p.D <= 96 ? launch_bwd_flash16_bf16_d96(bp, st) : p.D <= 128 ? launch_bwd_flash16_bf16_d128(bp, st) : launch_bwd_flash16_bf16_d256(bp, st);
         else
-            rc = p.D <= 64 ? launch_bwd_flash16_f16_d64(bp, st) : p.D <= 128 ? launch_bwd_flash16_f16_d128(bp, st) : launch_bwd_flash16_f16_d256(bp, st);
+            rc = p.D <= 32 ? launch_bwd_flash16_f16_d32(bp, st)
+                 : p.D <= 64 ? launch_bwd_flash16_f16_d64(bp, st) : p.D <= 96 ? launch_bwd_flash16_f16_d96(bp, st) : p.D <= 128 ? launch_bwd_flash16_f16_d128(bp, st) : launch_bwd_flash16_f16_d256(bp, st);
         if (rc != MI_OK) return rc;
     }
     if (bp.dq_nsplit <= 1) return MI_OK;

@@ -1,0 +1,5 @@
+// Instantiation of the MFMA attention backward for f16, head dims up to 96.
+#define BWD_T F16
+#define BWD_D 96
+#define BWD_ENTRY launch_bwd_flash16_f16_d96
+#include "attention_backward_flash16.inc"

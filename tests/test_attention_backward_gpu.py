@@ -945,3 +945,17 @@ def test_shared_bias_gradient_in_tiles_of_128(nn, oracle, dtype, D, H, Lq, Lkv, 
 def test_float32_key_gradients_in_one_pass(nn, oracle, D, H, Lq, Lkv, B, mask_kind, saved):
     """The forms of the Float32 kernel that makes dK and dV from one S and dP, at the edges of their tiles and of the rule."""
     _run(nn, oracle, "f32", D * H, D * H, Lq, Lkv, (B,), H, mask_kind=mask_kind, saved=saved, scale=0.4, seed=D + Lkv, expect="flash32")
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("D", [8, 32, 72, 96])
+@pytest.mark.parametrize("H,Lq,Lkv,B,mask_kind,bias,dropout", [
+    (2, 70, 300, 2, None, False, None), (2, 257, 257, 1, "causal", False, None), (2, 100, 272, 3, "random", False, None),
+    (2, 65, 333, 3, "lengths", False, (0.25, 4242)), (2, 66, 292, 2, None, False, (0.25, 4242)), (2, 97, 270, 3, None, True, None),
+    # more than 256 workgroups of 128 keys
+    (9, 70, 260, 10, None, False, None), (9, 300, 300, 16, "causal", False, None), (9, 97, 270, 10, None, True, None), (9, 70, 333, 10, "keys", False, (0.25, 4242)),
+])
+def test_16_bit_gradient_in_tiles_of_32_and_96_features(nn, oracle, D, dtype, H, Lq, Lkv, B, mask_kind, bias, dropout):
+    """Head dims up to 32 and from 72 to 96 on each kernel that makes dK and dV."""
+    _run(nn, oracle, dtype, D * H, D * H, Lq, Lkv, (B,), H, bias_shape=(Lkv, Lq, H, 1) if bias else None, mask_kind=mask_kind,
+         seed=D + Lkv, scale=0.6, saved=True, dropout=dropout, expect="flash16")
