@@ -69,9 +69,13 @@ inline int flash_pick_nsplit(const AttnParams &p, int bm) {
     const int64_t wgs = ((p.Lq + bm - 1) / bm) * p.H * p.B;
     if (wgs >= 512) return 1;
     if (p.Lkv < 2048) {
-        // Calls with a bias stay on the general kernel, where a workgroup that is alone on its CU takes 2.6 us per 64 keys: a
-        // few of them are worth the merge (5 us) from 768 keys on, at least 256 a piece (8 workgroups x 1511 keys: 64 -> 20 us)
-        if (p.dtype == MI_F32 || !p.bias || p.lean_workspace || wgs > 128 || p.Lkv < 768) return 1;
+        // The general kernel (all calls with a bias, and head dims that the pipelined kernel has no tiles for), where a workgroup that is
+        // alone on its CU takes 1 to 2.6 us per 64 keys: a few of them are worth the merge (5 us) from 768 keys on, at least 256
+        // a piece (us, one / several: 8 workgroups x 1511 keys with a bias 64 / 20, 18 x 1615 with a dense mask 54 / 18; without
+        // either, head dim 96, 18 x 1615 39 / 18, 64 x 1000, causal 28 / 21; 32, 128 x 1900 33 / 19).  Without a bias, more than 64
+        // workgroups from 1024 keys on (96, 128 x 800: 23.2 / 24.3; 32, 128 x 768, padded 18.9 / 19.8).
+        const bool pipelined = !p.bias && p.D == p.Dv && (p.D == 64 || p.D == 128);
+        if (p.dtype == MI_F32 || pipelined || p.lean_workspace || wgs > 128 || p.Lkv < (p.bias || wgs <= 64 ? 768 : 1024)) return 1;
         const int64_t n = 512 / wgs, most = p.Lkv / 256;
         return (int)(n < most ? n : most);
     }

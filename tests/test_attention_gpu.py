@@ -1100,3 +1100,12 @@ def test_float32_tiles_of_96_features(nn, oracle, E, H, Lq, Lkv, B, kw, weights)
 def test_16_bit_tiles_of_32_and_96_features(nn, oracle, D, dtype, Lq, Lkv, kw, weights):
     """Head dims up to 32 and from 72 to 96, every form of bias and mask input, key pieces."""
     _check(nn, oracle, np.random.default_rng(D + Lkv), dtype, 2 * D, Lq, Lkv, 3, 2, expect="flash16", weights=weights, **kw)
+
+
+@pytest.mark.parametrize("D,H,Lq,Lkv,B,kw", [
+    (32, 6, 112, 1615, 3, dict(mask_shape=(1615, 112))), (96, 2, 129, 768, 1, {}), (80, 8, 130, 1000, 5, dict(mask_shape=(1000, 1, 1, 5))),
+    (48, 8, 900, 900, 1, dict(causal=True)), (256, 2, 70, 1100, 2, {}), (96, 16, 128, 1023, 8, {}), (96, 16, 128, 1024, 8, {}),
+])
+def test_key_pieces_of_the_general_kernel_below_2048_keys(nn, oracle, D, H, Lq, Lkv, B, kw):
+    """Head dims without tiles of the pipelined kernel, no bias, both sides of the rule."""
+    _check(nn, oracle, np.random.default_rng(D + Lkv), "bf16", D * H, Lq, Lkv, B, H, expect="flash16", weights=False, **kw)
