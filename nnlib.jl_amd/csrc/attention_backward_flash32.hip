@@ -596,9 +596,10 @@ __device__ inline floatx16_t first_product_sl(unsigned tile, int kb, unsigned xr
 }
 
 // second_product on plane tiles: the B operand of k-step u is accumulator registers 8u .. 8u+7 of w (tile rows 0-3,
-// 8-11 | 4-7, 12-15 of the 16), split in registers; tile^T comes through the transposing read in that row order
-template <int D>
-__device__ inline void second_product_s(unsigned tile, int kb, const floatx16_t &w, floatx16_t (&out)[D / 32], int lane) {
+// 8-11 | 4-7, 12-15 of the 16), split in registers; tile^T comes through the transposing read in that row order.  N < D / 32:
+// the feature blocks from dvb0 on only
+template <int D, int N = D / 32>
+__device__ inline void second_product_s(unsigned tile, int kb, const floatx16_t &w, floatx16_t (&out)[N], int lane, int dvb0 = 0) {
     typedef CfgS<D> C;
     const int hh = lane >> 5;
     const int vrow = 4 * hh + ((lane & 15) >> 2);
@@ -619,12 +620,13 @@ __device__ inline void second_product_s(unsigned tile, int kb, const floatx16_t 
         for (int q = 0; q < 3; q++) wb[q] = __builtin_bit_cast(plane8, (u32x4_t){ww[q][0], ww[q][1], ww[q][2], ww[q][3]});
         const unsigned src = vt + (unsigned)(32 * kb + 16 * u) * C::ROWB;
 #pragma unroll
-        for (int dvb = 0; dvb < D / 32; dvb++) {
+        for (int dvb = 0; dvb < N; dvb++) {
+            if (N < D / 32 && dvb0 + dvb >= D / 32) break;
             plane8 ta[3];
 #pragma unroll
             for (int q = 0; q < 3; q++) {
-                const plane4 lo = tr(src + q * C::PLANEB + (((4 * dvb + vchunk) ^ sw_lo) << 4));
-                const plane4 hi = tr(src + q * C::PLANEB + 8 * C::ROWB + (((4 * dvb + vchunk) ^ sw_hi) << 4));
+                const plane4 lo = tr(src + q * C::PLANEB + (((4 * (dvb0 + dvb) + vchunk) ^ sw_lo) << 4));
+                const plane4 hi = tr(src + q * C::PLANEB + 8 * C::ROWB + (((4 * (dvb0 + dvb) + vchunk) ^ sw_hi) << 4));
                 ta[q] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
             }
             out[dvb] = mfma_split(ta, wb, out[dvb]);
@@ -1333,6 +1335,247 @@ __global__ __launch_bounds__(256, 1) void bwd32s_dkdv_small_kernel(FlashArgs a, 
     if (bp.dk) SB::reduce_store(xout + 4 * 64 * (D / 2), acck, (float *)bp.dk + off, kok, (int)p.D, a.cn, false);
 }
 
+// The same for tiles of 96 and 128 features, whose planes leave no room for 128-row chunks and stationary rows in LDS: the four
+// wavefronts of a workgroup of 32 rows take the two 32-row blocks of every 64-row tile in pairs.  One of a pair holds the
+// planes of Q (K) in registers and makes S and P, the other those of dO (V) and makes dP; they meet through LDS (4 KiB a block), and
+// then each makes half the features of dQ, or one dV and the other dK.  What bounds it is the chain of one tile: its split, the two
+// products and three barriers (training steps, workgroups of 128 rows / these: head dim 128, 8 pairs of 424 x 424, causal 203 / 121 us, 24 of
+// 120 x 120 83 / 52; 96, 36 of 218 x 218, causal 110 / 70).
+template <int D>
+struct PairBwd {
+    typedef CfgS<D> C;
+    static constexpr unsigned OFF_ST = 2 * C::TILEB;                    // statistics of a query tile: [3][64] floats
+    static constexpr unsigned OFF_X = OFF_ST + 3 * BN * sizeof(float);  // blocks that change hands: [4 wavefronts][4][64 lanes] x 16 bytes
+    static constexpr size_t SMEM = OFF_X + 4 * 4 * 64 * 16;
+    static_assert(4 * 64 * (D / 2) * sizeof(float) <= 2 * C::TILEB, "the partial gradients of four wavefronts fit the tiles");
+
+    __device__ static void give(unsigned char *smem, int slot, int lane, const floatx16_t &y) {
+        floatx4_t *x = (floatx4_t *)(smem + OFF_X) + slot * 256 + lane;
+#pragma unroll
+        for (int g = 0; g < 4; g++) x[64 * g] = (floatx4_t){y[4 * g], y[4 * g + 1], y[4 * g + 2], y[4 * g + 3]};
+    }
+    __device__ static void times(const unsigned char *smem, int slot, int lane, floatx16_t &y) {
+        const floatx4_t *x = (const floatx4_t *)(smem + OFF_X) + slot * 256 + lane;
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const floatx4_t v = x[64 * g];
+#pragma unroll
+            for (int e = 0; e < 4; e++) y[4 * g + e] *= v[e];
+        }
+    }
+    // the N feature blocks (from dvb0 on) of the two wavefronts of a role added up, every second block stored by each
+    template <int N>
+    __device__ static void reduce_store(float *xout, const floatx16_t (&acc)[N], float *grad_row, bool ok, int dh, float scale, int dvb0) {
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, hh = lane >> 5;
+        __syncthreads();   // the tiles are read by nobody any more
+        float *mine = xout + wave * N * 1024;
+#pragma unroll
+        for (int i = 0; i < N; i++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) mine[(16 * i + v) * 64 + lane] = acc[i][v];
+        __syncthreads();
+        if (!ok) return;
+        const float *other = xout + (wave ^ 1) * N * 1024;
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            if ((i & 1) != (wave & 1)) continue;
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const int d0 = 32 * (dvb0 + i) + 8 * g + 4 * hh;
+                floatx4_t o4;
+#pragma unroll
+                for (int e = 0; e < 4; e++) o4[e] = (acc[i][4 * g + e] + other[(16 * i + 4 * g + e) * 64 + lane]) * scale;
+                if (d0 < dh) *(floatx4_t *)(grad_row + d0) = o4;
+            }
+        }
+    }
+};
+
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__(256, 1) void bwd32s_dq_halves_kernel(FlashArgs a, AttnBwdParams bp) {
+    typedef CfgS<D> C;
+    typedef PairBwd<D> PB;
+    constexpr int OWN = (D / 32 + 1) / 2;   // feature blocks of dQ that a wavefront makes
+    const AttnParams &p = a.p;
+    extern __shared__ __attribute__((aligned(16))) unsigned char bwd_smem[];
+    const unsigned Ks = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)bwd_smem, Vs = Ks + C::TILEB;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 31, hh = lane >> 5;
+    const int role = wave >> 1, kb = wave & 1;   // role 0: S and P, 1: dP - delta
+    const int64_t HB = p.H * p.B;
+    const int64_t n_qblocks = (p.Lq + 31) / 32;
+    const int64_t hb = blockIdx.x % HB, qblk = n_qblocks - 1 - blockIdx.x / HB;
+    const int64_t h = hb % p.H, b = hb / p.H;
+    const int64_t iw = qblk * 32, qi = iw + r;
+    const bool qok = qi < p.Lq;
+    const int64_t off = p.E * (qi + p.Lq * b) + p.D * h;   // E == Ev for these kernels
+
+    PlaneStream<D> ts;
+    ts.base1 = (const float *)p.k + p.E * (p.Lkv * b) + p.D * h;
+    ts.base2 = (const float *)p.v + p.E * (p.Lkv * b) + p.D * h;
+    ts.dh = (int)p.D;
+    ts.stride = p.E;
+    ts.nrows = p.Lkv;
+    ts.s1 = Ks;
+    ts.s2 = Vs;
+    int64_t kv_end = p.Lkv;
+    if (CAUSAL && iw + 32 < kv_end) kv_end = iw + 32;
+    const int n_tiles = (int)((kv_end + BN - 1) / BN);
+    if (bp.dq && n_tiles > 0) ts.load(0);
+    plane8 x[3][D / 16];
+    load_stationary_s<D>(x, (const float *)(role ? bp.dout : p.q) + off, qok, hh, (int)p.D);
+
+    // delta = rowsum(O * dO) of the lane's query, saved for the dK / dV kernel
+    float delta = 0.0f;
+    {
+        floatx4_t o4[D / 8], d4[D / 8];
+#pragma unroll
+        for (int c = 0; c < D / 8; c++) {
+            const bool ok = qok && 8 * c + 4 * hh < p.D;
+            o4[c] = ldg16f((const float *)p.out + off + 8 * c + 4 * hh, ok);
+            d4[c] = ldg16f((const float *)bp.dout + off + 8 * c + 4 * hh, ok);
+        }
+#pragma unroll
+        for (int c = 0; c < D / 8; c++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) delta = fmaf(o4[c][j], d4[c][j], delta);
+        delta += mi_swap32(delta);
+    }
+    const int64_t pad = lq_pad(p.Lq), plane = p.B * p.H * pad, at = (b * p.H + h) * pad + qi;
+    const float m2 = bp.stats[at], linv = bp.stats[plane + at];
+    if (wave == 0 && hh == 0) bp.stats[2 * plane + at] = qok ? delta : 0.0f;
+    if (wave == 1 && qblk == n_qblocks - 1)   // rows no query block covers: a finite delta, their weights are zeros
+        for (int64_t q2 = iw + 32 + lane; q2 < pad; q2 += 64) bp.stats[2 * plane + (b * p.H + h) * pad + q2] = 0.0f;
+    if (!bp.dq) return;
+
+    floatx16_t dq[OWN];
+#pragma unroll
+    for (int i = 0; i < OWN; i++) dq[i] = (floatx16_t){0};
+    const float cs = a.c;
+    for (int jt = 0; jt < n_tiles; jt++) {
+        if (jt > 0) __syncthreads();   // every wavefront is done with tile jt - 1
+        ts.store();
+        __syncthreads();               // tile jt in LDS
+        if (jt + 1 < n_tiles) ts.load((int64_t)(jt + 1) * BN);
+        const int64_t j0 = (int64_t)jt * BN + 32 * kb;   // the wavefront's key block
+        const bool on = j0 < p.Lkv && (!CAUSAL || j0 <= iw + 31);
+        floatx16_t y;
+        if (on) {
+            y = first_product_s<D>(role ? Vs : Ks, kb, x, (floatx16_t){0}, r, hh);
+            if (role == 0) {
+                // keys of the block this lane's query keeps, counted from the lane's first key of a group of four
+                int64_t lim64 = p.Lkv - j0;
+                if (CAUSAL && qi - j0 + 1 < lim64) lim64 = qi - j0 + 1;
+                const int lim = (lim64 > 32 ? 32 : (lim64 < 0 ? 0 : (int)lim64)) - 4 * hh;
+#pragma unroll
+                for (int v = 0; v < 16; v++) y[v] = 8 * (v / 4) + (v % 4) < lim ? mi_exp2(fmaf(y[v], cs, -m2)) * linv : 0.0f;
+            } else {
+#pragma unroll
+                for (int v = 0; v < 16; v++) y[v] -= delta;
+            }
+            PB::give(bwd_smem, wave, lane, y);
+        }
+        __syncthreads();               // P and dP - delta of both blocks in LDS
+        if (on) {
+            PB::times(bwd_smem, wave ^ 2, lane, y);   // dS
+            second_product_s<D, OWN>(Ks, kb, y, dq, lane, role * OWN);
+        }
+    }
+    const int dvb0 = role * OWN;
+    PB::template reduce_store<OWN>((float *)bwd_smem, dq, (float *)bp.dq + off, qok, (int)p.D, a.cn, dvb0);
+}
+
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__(256, 1) void bwd32s_dkdv_halves_kernel(FlashArgs a, AttnBwdParams bp) {
+    typedef CfgS<D> C;
+    typedef PairBwd<D> PB;
+    constexpr int NDV = D / 32;
+    const AttnParams &p = a.p;
+    extern __shared__ __attribute__((aligned(16))) unsigned char bwd_smem[];
+    const unsigned Qs = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)bwd_smem, dOs = Qs + C::TILEB;
+    float *st_lds = (float *)(bwd_smem + PB::OFF_ST);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 31, hh = lane >> 5;
+    const int role = wave >> 1, kb = wave & 1;   // role 0: S, P and dV, 1: dP and dK
+    const int64_t HB = p.H * p.B;
+    const int64_t hb = blockIdx.x % HB, kblk = blockIdx.x / HB;   // with causal masks the early key blocks are the long ones
+    const int64_t h = hb % p.H, b = hb / p.H;
+    const int64_t jw = kblk * 32, kv = jw + r;
+    const bool kok = kv < p.Lkv;
+    const int64_t off = p.E * (kv + p.Lkv * b) + p.D * h;
+
+    const int64_t pad = lq_pad(p.Lq), plane = p.B * p.H * pad;
+    // the statistics of a query tile travel with it through LDS: 48 threads x 4 floats (maximum, 1 / row sum, delta)
+    const float *st_src = bp.stats + (b * p.H + h) * pad + (int64_t)(tid >> 4) * plane + 4 * (tid & 15);
+    floatx4_t st_reg = {0, 0, 0, 0};
+    PlaneStream<D> ts;
+    ts.base1 = (const float *)p.q + p.E * (p.Lq * b) + p.D * h;
+    ts.base2 = (const float *)bp.dout + p.E * (p.Lq * b) + p.D * h;
+    ts.dh = (int)p.D;
+    ts.stride = p.E;
+    ts.nrows = p.Lq;
+    ts.s1 = Qs;
+    ts.s2 = dOs;
+    const int n_qt = (int)((p.Lq + BN - 1) / BN);
+    const int it0 = CAUSAL ? (int)(jw / BN) : 0;   // query tiles before the first key of the workgroup see none of its keys
+    if (it0 < n_qt) {
+        ts.load((int64_t)it0 * BN);
+        if (tid < 48) st_reg = *(const floatx4_t *)(st_src + (int64_t)it0 * BN);
+    }
+    plane8 x[3][D / 16];
+    load_stationary_s<D>(x, (const float *)(role ? p.v : p.k) + off, kok, hh, (int)p.D);
+    floatx16_t acc[NDV];
+#pragma unroll
+    for (int dvb = 0; dvb < NDV; dvb++) acc[dvb] = (floatx16_t){0};
+    const float cs = a.c;
+    for (int it = it0; it < n_qt; it++) {
+        if (it > it0) __syncthreads();   // every wavefront is done with tile it - 1
+        ts.store();
+        if (tid < 48) *(floatx4_t *)(st_lds + 4 * tid) = st_reg;
+        __syncthreads();                 // tile it in LDS
+        if (it + 1 < n_qt) {
+            ts.load((int64_t)(it + 1) * BN);
+            if (tid < 48) st_reg = *(const floatx4_t *)(st_src + (int64_t)(it + 1) * BN);
+        }
+        const int64_t i0 = (int64_t)it * BN + 32 * kb;   // the wavefront's query block
+        const bool on = i0 < p.Lq && (!CAUSAL || i0 + 31 >= jw);
+        const float *st = st_lds + 32 * kb + 4 * hh;
+        floatx16_t y;
+        if (on) {
+            y = first_product_s<D>(role ? dOs : Qs, kb, x, (floatx16_t){0}, r, hh);
+            // accumulator register 4g+e of this lane: query i0 + 8g + 4hh + e, key kv.  Rows past Lq carry statistics
+            // (0, 0, 0): their weights vanish; keys past the last one only feed columns that are not stored
+            if (role == 0) {
+                const bool diag = CAUSAL && i0 < jw + 32;   // some (query, key) pair of this block has key > query
+                const int rel = (int)(jw - i0) + r - 4 * hh;
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const floatx4_t m4 = *(const floatx4_t *)(st + 8 * g), linv4 = *(const floatx4_t *)(st + BN + 8 * g);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const float pw = mi_exp2(fmaf(y[4 * g + e], cs, -m4[e])) * linv4[e];
+                        y[4 * g + e] = diag && rel - 8 * g - e > 0 ? 0.0f : pw;
+                    }
+                }
+                PB::give(bwd_smem, kb, lane, y);
+            }
+        }
+        __syncthreads();                 // P of both blocks in LDS
+        if (on) {
+            if (role == 1) {
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const floatx4_t delta4 = *(const floatx4_t *)(st + 2 * BN + 8 * g);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) y[4 * g + e] -= delta4[e];
+                }
+                PB::times(bwd_smem, kb, lane, y);   // dS
+            }
+            second_product_s<D>(role ? Qs : dOs, kb, y, acc, lane);
+        }
+    }
+    float *grad = (float *)(role ? bp.dk : bp.dv);
+    PB::template reduce_store<NDV>((float *)bwd_smem, acc, grad + off, kok && grad, (int)p.D, role ? a.cn : 1.0f, 0);
+}
+
 // Products on the 16-bit matrix cores through three bf16 planes unless the caller's environment asks for the
 // Float32 matrix instruction (MI355ATTN_F32_MFMA=1), as in the forward kernel.
 bool exact_instruction_wanted() {
@@ -1424,6 +1667,22 @@ int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream
             }
         }
     }
+    if constexpr (D > 64) {
+        const bool can = !a.kv_len && !no_small;
+        // A compute unit holds one workgroup (116 KiB of LDS at 128 features), which takes half as long as one of 128 rows: one
+        // round of the chip, and two where a causal mask leaves the workgroups of 128 rows with unequal loops (whole steps, us, 128
+        // rows / 32: head dim 128, 8 x 4 pairs of 256 x 256 130 / 80, causal 131 / 80; 8 x 6 151 / 146; 8 x 8 155 / 149, causal 157 /
+        // 123; 8 x 12 159 / 204; 96, 8 x 8 of 256 x 256 122 / 124, 8 x 4 of 512 x 512, causal 196 / 145; 80, 6 x 31 of 40 x 40,
+        // causal 58 / 66).
+        small_q = can && bp.have_stats && bp.dq_nsplit <= 1 && q_blocks <= (CAUSAL && p.Lq > 128 ? 512 : 256);
+        small_k = can && k_blocks <= (CAUSAL && p.Lkv > 128 ? 512 : 256);
+        static bool halves_attr_set = false;
+        if ((small_q || small_k) && !halves_attr_set) {
+            MI_HIP_CHECK(hipFuncSetAttribute((const void *)bwd32s_dq_halves_kernel<D, CAUSAL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)PairBwd<D>::SMEM));
+            MI_HIP_CHECK(hipFuncSetAttribute((const void *)bwd32s_dkdv_halves_kernel<D, CAUSAL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)PairBwd<D>::SMEM));
+            halves_attr_set = true;
+        }
+    }
     FlashArgs a1 = a;
     if (bp.dq_nsplit > 1) {   // the dQ kernel's key range in pieces (the dK / dV kernels keep a.nsplit = 1)
         a1.nsplit = bp.dq_nsplit;
@@ -1431,6 +1690,7 @@ int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream
     }
     if (small_q) {
         if constexpr (D == 64) hipLaunchKernelGGL((bwd32s_dq_small_kernel<D, CAUSAL, false>), dim3((unsigned)q_blocks), dim3(256), SmallBwd<D>::SMEM, st, a, bp);
+        else hipLaunchKernelGGL((bwd32s_dq_halves_kernel<D, CAUSAL>), dim3((unsigned)q_blocks), dim3(256), PairBwd<D>::SMEM, st, a, bp);
     } else if (wide) {
         a1.n_qtiles = (int32_t)wide_tiles;
         hipLaunchKernelGGL(k1w, dim3((unsigned)(wide_tiles * p.H * p.B)), dim3(64 * NW_WIDE), SMEM_WIDE, st, a1, bp);
@@ -1440,8 +1700,11 @@ int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream
     MI_LAUNCH_CHECK();
     const dim3 g2((unsigned)(((p.Lkv + 127) / 128) * p.H * p.B));
     if (small_k) {
-        if constexpr (D == 64)
+        if constexpr (D == 64) {
             if (bp.dv || bp.dk) hipLaunchKernelGGL((bwd32s_dkdv_small_kernel<D, CAUSAL, false>), dim3((unsigned)k_blocks), dim3(256), SmallBwd<D>::SMEM, st, a, bp);
+        } else if (bp.dv || bp.dk) {
+            hipLaunchKernelGGL((bwd32s_dkdv_halves_kernel<D, CAUSAL>), dim3((unsigned)k_blocks), dim3(256), PairBwd<D>::SMEM, st, a, bp);
+        }
     } else if (bp.dv && bp.dk && fused_dkdv) {
         if (wide_dkdv) hipLaunchKernelGGL(k23w, dim3((unsigned)wide_key_tiles), dim3(64 * NW_WIDE), SMEM_WIDE, st, a, bp);
         else hipLaunchKernelGGL(two_dkdv ? k23two : k23, g2, dim3(256), SMEM, st, a, bp);
