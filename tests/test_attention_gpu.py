@@ -1109,3 +1109,12 @@ def test_16_bit_tiles_of_32_and_96_features(nn, oracle, D, dtype, Lq, Lkv, kw, w
 def test_key_pieces_of_the_general_kernel_below_2048_keys(nn, oracle, D, H, Lq, Lkv, B, kw):
     """Head dims without tiles of the pipelined kernel, no bias, both sides of the rule."""
     _check(nn, oracle, np.random.default_rng(D + Lkv), "bf16", D * H, Lq, Lkv, B, H, expect="flash16", weights=False, **kw)
+
+
+@pytest.mark.parametrize("Lq,Lkv,kw", [
+    (300, 128, dict(bias_shape=(128, 300, 8, 1))), (257, 131, dict(bias_shape=(131, 257, 8, 1))), (130, 192, dict(bias_shape=(192, 130, 8, 6), mask_shape=(192, 130))),
+    (129, 133, dict(bias_shape=(133, 129, 8, 6), mask_shape=(133, 129))), (150, 150, dict(bias_shape=(150, 150, 8, 1), causal=True)),
+])
+def test_two_workgroups_with_bias_tiles_of_96_features(nn, oracle, Lq, Lkv, kw):
+    """LDS sized by the arrays that the call has: bias alone, bias and mask, staged tiles and rows of any alignment."""
+    _check(nn, oracle, np.random.default_rng(Lkv), "bf16", 96 * 8, Lq, Lkv, 6, 8, expect="flash16", weights=False, **kw)
