@@ -1335,7 +1335,7 @@ __global__ __launch_bounds__(256, 1) void bwd32s_dkdv_small_kernel(FlashArgs a, 
     if (bp.dk) SB::reduce_store(xout + 4 * 64 * (D / 2), acck, (float *)bp.dk + off, kok, (int)p.D, a.cn, false);
 }
 
-// The same for tiles of 96 and 128 features, whose planes leave no room for 128-row chunks and stationary rows in LDS: the four
+// The same for more workgroups and for tiles of 96 and 128 features, whose planes leave no room for 128-row chunks and stationary rows in LDS: the four
 // wavefronts of a workgroup of 32 rows take the two 32-row blocks of every 64-row tile in pairs.  One of a pair holds the
 // planes of Q (K) in registers and makes S and P, the other those of dO (V) and makes dP; they meet through LDS (4 KiB a block), and
 // then each makes half the features of dQ, or one dV and the other dK.  What bounds it is the chain of one tile: its split, the two
@@ -1667,6 +1667,7 @@ int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream
             }
         }
     }
+    bool halves_q = false, halves_k = false;
     if constexpr (D > 64) {
         const bool can = !a.kv_len && !no_small;
         // A compute unit holds one workgroup (116 KiB of LDS at 128 features), which takes half as long as one of 128 rows: one
@@ -1676,8 +1677,18 @@ int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream
         // causal 58 / 66).
         small_q = can && bp.have_stats && bp.dq_nsplit <= 1 && q_blocks <= (CAUSAL && p.Lq > 128 ? 512 : 256);
         small_k = can && k_blocks <= (CAUSAL && p.Lkv > 128 ? 512 : 256);
+        halves_q = small_q;
+        halves_k = small_k;
+    } else {
+        // head dims up to 64: two of those workgroups fit a compute unit (65 KiB), one of the kernels above (147 KiB), so they are faster
+        // where those need a second round (12 x 5 pairs of 160 x 160 72.8 / 52.1 us, causal 60.2 / 47.0; 8 x 4 of 512 x 512 128 / 103; 8 x
+        // 30 of 64 x 64, causal 48.9 / 33.9) and slower in the first (8 x 2 of 512 x 512 71.5 / 77.5; 4 x 2 of 1000 x 1000 127 / 139)
+        halves_q = small_q && q_blocks > 256 && p.Lq > 32;
+        halves_k = small_k && k_blocks > 256 && p.Lkv > 32;
+    }
+    if (halves_q || halves_k) {
         static bool halves_attr_set = false;
-        if ((small_q || small_k) && !halves_attr_set) {
+        if (!halves_attr_set) {
             MI_HIP_CHECK(hipFuncSetAttribute((const void *)bwd32s_dq_halves_kernel<D, CAUSAL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)PairBwd<D>::SMEM));
             MI_HIP_CHECK(hipFuncSetAttribute((const void *)bwd32s_dkdv_halves_kernel<D, CAUSAL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)PairBwd<D>::SMEM));
             halves_attr_set = true;
@@ -1688,9 +1699,10 @@ int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream
         a1.nsplit = bp.dq_nsplit;
         a1.tiles_per_split = (int32_t)(((p.Lkv + BN - 1) / BN + bp.dq_nsplit - 1) / bp.dq_nsplit);
     }
-    if (small_q) {
+    if (halves_q) {
+        hipLaunchKernelGGL((bwd32s_dq_halves_kernel<D, CAUSAL>), dim3((unsigned)q_blocks), dim3(256), PairBwd<D>::SMEM, st, a, bp);
+    } else if (small_q) {
         if constexpr (D == 64) hipLaunchKernelGGL((bwd32s_dq_small_kernel<D, CAUSAL, false>), dim3((unsigned)q_blocks), dim3(256), SmallBwd<D>::SMEM, st, a, bp);
-        else hipLaunchKernelGGL((bwd32s_dq_halves_kernel<D, CAUSAL>), dim3((unsigned)q_blocks), dim3(256), PairBwd<D>::SMEM, st, a, bp);
     } else if (wide) {
         a1.n_qtiles = (int32_t)wide_tiles;
         hipLaunchKernelGGL(k1w, dim3((unsigned)(wide_tiles * p.H * p.B)), dim3(64 * NW_WIDE), SMEM_WIDE, st, a1, bp);
@@ -1699,12 +1711,11 @@ int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream
     }
     MI_LAUNCH_CHECK();
     const dim3 g2((unsigned)(((p.Lkv + 127) / 128) * p.H * p.B));
-    if (small_k) {
-        if constexpr (D == 64) {
+    if (halves_k) {
+        if (bp.dv || bp.dk) hipLaunchKernelGGL((bwd32s_dkdv_halves_kernel<D, CAUSAL>), dim3((unsigned)k_blocks), dim3(256), PairBwd<D>::SMEM, st, a, bp);
+    } else if (small_k) {
+        if constexpr (D == 64)
             if (bp.dv || bp.dk) hipLaunchKernelGGL((bwd32s_dkdv_small_kernel<D, CAUSAL, false>), dim3((unsigned)k_blocks), dim3(256), SmallBwd<D>::SMEM, st, a, bp);
-        } else if (bp.dv || bp.dk) {
-            hipLaunchKernelGGL((bwd32s_dkdv_halves_kernel<D, CAUSAL>), dim3((unsigned)k_blocks), dim3(256), PairBwd<D>::SMEM, st, a, bp);
-        }
     } else if (bp.dv && bp.dk && fused_dkdv) {
         if (wide_dkdv) hipLaunchKernelGGL(k23w, dim3((unsigned)wide_key_tiles), dim3(64 * NW_WIDE), SMEM_WIDE, st, a, bp);
         else hipLaunchKernelGGL(two_dkdv ? k23two : k23, g2, dim3(256), SMEM, st, a, bp);

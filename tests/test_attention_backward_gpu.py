@@ -964,7 +964,10 @@ def test_16_bit_gradient_in_tiles_of_32_and_96_features(nn, oracle, D, dtype, H,
 @pytest.mark.parametrize("D,H,Lq,Lkv,B,mask_kind", [
     (68, 2, 1, 64, 2, None), (96, 2, 33, 65, 1, None), (128, 3, 97, 31, 2, None), (100, 2, 200, 129, 1, None), (96, 1, 130, 400, 2, None),
     (72, 2, 63, 63, 2, "causal"), (128, 2, 129, 129, 2, "causal"), (96, 8, 257, 257, 5, "causal"), (128, 8, 32, 64, 33, None),
+    # head dims up to 64, 257 to 512 blocks: both gradients, one of them
+    (64, 8, 161, 190, 7, None), (36, 8, 130, 130, 8, "causal"), (64, 16, 64, 96, 17, None), (48, 16, 33, 65, 9, None),
 ])
-def test_float32_gradient_of_few_rows_at_wide_heads(nn, oracle, D, H, Lq, Lkv, B, mask_kind):
-    """Head dims 68 to 128, at most 256 blocks of 32 rows (512 with a causal mask): pairs of wavefronts that share a block."""
+def test_float32_gradient_by_pairs_of_wavefronts(nn, oracle, D, H, Lq, Lkv, B, mask_kind):
+    """Head dims 68 to 128, at most 256 blocks of 32 rows (512 with a causal mask), up to 64, more than 256 and at most 512: pairs of
+    wavefronts that share a block."""
     _run(nn, oracle, "f32", D * H, D * H, Lq, Lkv, (B,), H, mask_kind=mask_kind, saved=True, scale=0.4, seed=D + Lkv, expect="flash32")
