@@ -187,9 +187,11 @@ struct FlashTileDma {
         lds = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)tiles + wave * PIECES * 1024);   // wave-uniform: goes into M0
 #pragma unroll
         for (int i = 0; i < PIECES; i++) {
+            constexpr int CPR = ROWB / 16;   // chunks per row
             const int at = (wave * PIECES + i) * 64 + lane;   // chunk of the tile
-            const int row = at / (ROWB / 16);
-            const int chunk = (at % (ROWB / 16)) ^ swz(row);
+            // (whole rows in a piece written out: the compiler makes branches of the general form)
+            const int row = 64 % CPR == 0 ? (wave * PIECES + i) * (64 / CPR) + lane / CPR : at / CPR;
+            const int chunk = (64 % CPR == 0 ? lane % CPR : at % CPR) ^ swz(row);
             voff[i] = 8 * chunk < dh ? row * (int)row_bytes + chunk * 16 : (int)0x80000000;
         }
     }
