@@ -481,9 +481,9 @@ static int32_t attention_forward(const mi_attn_desc *d, mi_stream s, bool static
     size_t ws = 0;
     int32_t kernel = choose(d, p, &ws);
     const size_t have = static_workspace ? (size_t)MI_ATTN_STATIC_WORKSPACE_BYTES : (d->workspace ? d->workspace_bytes : (size_t)0);
-    if (ws > have && kernel == MI_ATTN_KERNEL_FLASH16 && (p.mask || p.bias)) {
-        // a dense mask too large to pack into the workspace at hand: the general kernel reads it as it is; a short key range
-        // with a bias is not split
+    if (ws > have && kernel == MI_ATTN_KERNEL_FLASH16) {
+        // a dense mask too large to pack into the workspace at hand: the general kernel reads it as it is; a key range below 2048
+        // is not split
         p.lean_workspace = true;
         kernel = choose(d, p, &ws);
     }

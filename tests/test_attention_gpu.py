@@ -1118,3 +1118,17 @@ def test_key_pieces_of_the_general_kernel_below_2048_keys(nn, oracle, D, H, Lq, 
 def test_two_workgroups_with_bias_tiles_of_96_features(nn, oracle, Lq, Lkv, kw):
     """LDS sized by the arrays that the call has: bias alone, bias and mask, staged tiles and rows of any alignment."""
     _check(nn, oracle, np.random.default_rng(Lkv), "bf16", 96 * 8, Lq, Lkv, 6, 8, expect="flash16", weights=False, **kw)
+
+
+def test_a_short_key_range_without_a_bias_needs_no_workspace(nn):
+    """The same for a head dim that only the general kernel has tiles for, no bias and no mask."""
+    rng = np.random.default_rng(4)
+    q, k, v = (nn.DeviceArray.from_numpy(round_to(rng.standard_normal((192, n, 1)), "f16"), "f16") for n in (50, 1001, 1001))
+    y, _ = nn.dot_product_attention(q, k, v, nheads=2, return_weights=False)
+    assert nn.ops.last_attention_workspace() > 0
+    lib, d = nn._lib.load(), nn._lib.mi_attn_desc()
+    out = nn.DeviceArray.empty((192, 50, 1), "f16")
+    nn.ops._fill_desc(d, q, k, v, None, None, 2, 1, 192, 192, 50, 1001, 0)
+    d.out = out.ptr
+    nn._lib.check(lib.mi_attention_fwd(ctypes.byref(d), None))
+    assert rel_err(out.to_numpy(), y.to_numpy()) <= 2 * 2.0 ** -11
