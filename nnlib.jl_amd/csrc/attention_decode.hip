@@ -154,8 +154,8 @@ __global__ __launch_bounds__(WAVES * 64, NQ <= 2 ? 4 : 2) void decode_split_kern
         float mref[NQ];
 #pragma unroll
         for (int n = 0; n < NQ; n++) {
-            const float mnew = fmaxf(m[n], mx[n]);            // finite without a mask: at least one row of the chunk is valid
-            mref[n] = (MASKED && mnew == MI_NEG_INF) ? 0.0f : mnew;   // nothing kept so far: every term below is 0
+            const float mnew = fmaxf(m[n], mx[n]);
+            mref[n] = mnew == MI_NEG_INF ? 0.0f : mnew;   // no score above -Inf so far (dropped keys, infinite features of k): every term below is 0
             const float resc = mi_exp2((m[n] - mref[n]) * a.c);
             m[n] = mnew;
             l[n] *= resc;

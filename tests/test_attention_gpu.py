@@ -485,6 +485,41 @@ def test_decode_splits(nn, dtype, E, H, Lq, Lkv, B, masked):
     assert (err <= u * ref.abs() + 1e-5 * ref.abs().max()).all()
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("Lq,weights", [(1, False), (1, True), (2, False), (4, False)])
+@pytest.mark.parametrize("Lkv", [512, 4096, 32768])
+def test_decode_with_blocks_of_minus_infinity(nn, dtype, Lq, weights, Lkv):
+    """Runs of eight keys, the block that a wavefront takes at a time, whose scores are all -Inf (a feature of k is) in a call
+    without a mask: the first block, one in the middle, the last 96 keys and, in one head, every key.  Against the same call in
+    Float64, which gives such keys no weight.  Bounds: test_decode_splits; a weight is at most 1, rounded to its type."""
+    import torch
+
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(Lkv + Lq)
+    tt = {"bf16": torch.bfloat16, "f32": torch.float32}[dtype]
+    H, D, B = 4, 64, 2
+    q, k, v = (torch.randn(B, L, H, D, generator=gen, device="cuda") for L in (Lq, Lkv, Lkv))
+    q[..., 0] = q[..., 0].abs() + 0.5
+    for j in (0, Lkv // 2, Lkv - 96):
+        k[:, j:j + (96 if j == Lkv - 96 else 8), :, 0] = -np.inf
+    k[1, :, 3, 0] = -np.inf
+    q, k, v = (t.to(tt).reshape(B, -1, H * D) for t in (q, k, v))
+    arr = [nn.DeviceArray.from_torch(t.reshape(-1), (H * D, t.shape[1], B), dtype) for t in (q, k, v)]
+    y, a = nn.dot_product_attention(*arr, nheads=H, return_weights=weights, weights_dtype="f32" if weights else None)
+    assert nn.last_attention_kernel() == "decode"
+    qd, kd, vd = (t.double().reshape(B, -1, H, D).transpose(1, 2).contiguous() for t in (q, k, v))
+    al = torch.softmax(qd @ kd.transpose(2, 3).contiguous() / np.sqrt(D), -1)
+    ref = (al @ vd).transpose(1, 2)
+    got = y.storage.reshape(B, Lq, H, D).double()
+    assert torch.isnan(ref[1, :, 3]).all() and torch.isnan(got).equal(torch.isnan(ref))
+    ok = ~torch.isnan(ref)
+    u = {"bf16": 2.0 ** -8, "f32": 2.0 ** -24}[dtype]
+    assert ((got - ref).abs()[ok] <= u * ref.abs()[ok] + 1e-5 * ref[ok].abs().max()).all()
+    if weights:
+        aw = a.storage.reshape(B, H, Lq, Lkv).double()
+        assert torch.isnan(aw).equal(torch.isnan(al)) and (aw - al).abs()[~torch.isnan(al)].max() <= 1e-5
+
+
 def test_decode_matches_generic_on_device(nn):
     rng = np.random.default_rng(11)
     q = nn.DeviceArray.from_numpy(rng.standard_normal((512, 1, 2)).astype(np.float32), "bf16")
