@@ -481,7 +481,10 @@ static int32_t attention_forward(const mi_attn_desc *d, mi_stream s, bool static
     size_t ws = 0;
     int32_t kernel = choose(d, p, &ws);
     const size_t have = static_workspace ? (size_t)MI_ATTN_STATIC_WORKSPACE_BYTES : (d->workspace ? d->workspace_bytes : (size_t)0);
-    if (ws > have && kernel == MI_ATTN_KERNEL_FLASH16) {
+    // partial results of key pieces start at a multiple of 16 bytes (context lengths and mask words, at one of 4)
+    const bool misplaced = kernel == MI_ATTN_KERNEL_FLASH16 && !static_workspace && ws > 0 && (((uintptr_t)d->workspace) & 15) != 0 &&
+                           !takes_length_path(p) && !takes_mask_words_path(p);
+    if (misplaced || (ws > have && kernel == MI_ATTN_KERNEL_FLASH16)) {
         // a dense mask too large to pack into the workspace at hand: the general kernel reads it as it is; a key range below 2048
         // is not split
         p.lean_workspace = true;

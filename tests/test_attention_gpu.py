@@ -1167,3 +1167,30 @@ def test_a_short_key_range_without_a_bias_needs_no_workspace(nn):
     d.out = out.ptr
     nn._lib.check(lib.mi_attention_fwd(ctypes.byref(d), None))
     assert rel_err(out.to_numpy(), y.to_numpy()) <= 2 * 2.0 ** -11
+
+
+@pytest.mark.parametrize("Lkv,kw", [(1001, {}), (1900, dict(mask=True)), (1000, dict(bias=True)), (2100, {})])
+def test_workspace_that_key_pieces_cannot_start_in(nn, Lkv, kw):
+    """A workspace that is not 16-byte aligned: a key range below 2048 runs in one piece, as with none, and does not write there; a
+    longer one is refused.  Two orders of the Float32 sums, rounded to f16: a unit in the last place apart."""
+    import torch
+
+    rng = np.random.default_rng(Lkv)
+    q, k, v = (nn.DeviceArray.from_numpy(round_to(rng.standard_normal((192, n, 1)), "f16"), "f16") for n in (50, Lkv, Lkv))
+    mask = nn.DeviceArray.from_numpy(rng.random((Lkv, 50)) < 0.8, "bool") if kw.get("mask") else None
+    bias = nn.DeviceArray.from_numpy(round_to(rng.standard_normal((Lkv, 50, 2, 1)), "f16"), "f16") if kw.get("bias") else None
+    y, _ = nn.dot_product_attention(q, k, v, bias, mask=mask, nheads=2, return_weights=False)
+    need = nn.ops.last_attention_workspace()
+    assert nn.last_attention_kernel() == "flash16" and need > 0
+    lib, d = nn._lib.load(), nn._lib.mi_attn_desc()
+    out = nn.DeviceArray.empty((192, 50, 1), "f16")
+    nn.ops._fill_desc(d, q, k, v, bias, mask, 2, 1, 192, 192, 50, Lkv, 0)
+    room = torch.full((need + 16,), 0xA5, dtype=torch.uint8, device="cuda")
+    d.out, d.workspace, d.workspace_bytes = out.ptr, room.data_ptr() + 4, need
+    rc = lib.mi_attention_fwd(ctypes.byref(d), None)
+    if Lkv >= 2048:
+        assert rc == nn._lib.MI_EWORKSPACE
+        return
+    nn._lib.check(rc)
+    assert rel_err(out.to_numpy(), y.to_numpy()) <= 2 * 2.0 ** -11
+    assert (room == 0xA5).all()
