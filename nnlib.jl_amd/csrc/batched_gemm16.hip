@@ -539,7 +539,18 @@ bool batched_gemm16_supports(int32_t dtype, int transA, int transB, int64_t m, i
     // kernel / tiled, bf16: 64 x 48 x 832, 18 slices 47.9 / 11.4; 32 x 32 x 64, 256 slices 6.2 / 4.4, 4096 39 / 26;
     // 16 x 16 x 256, 4096 slices 118 / 47; 8 x 200 x 64, 1024 slices 41 / 14.  The other way: 16 x 16 x 64, 4096 slices, 'T' 18.1 / 25.4;
     // 56 x 56 x 32, 1024 slices 7.7 / 8.9; 17 x 33 x 128 of any alignment, 1024 slices 12.6 / 15.2; 17 x 33 x 32, 18 slices 4.7 / 5.7.
-    if (m * n < 64 * 64 && m <= 128 && n <= 128 && (batch <= 512 ? k <= 32 : m * n * k < 50 * 50 * 50)) return false;
+    if (m * n < 64 * 64) {
+        const bool wide = m > 128 || n > 128;
+        if (k <= 32) {
+            // one step of k on either kernel: the tiled one only where its tiles stand for two of 64 x 64 each, most of the step is there
+            // and there are rounds of them (8 x 200 x 32, 1024 slices 22.3 / 14.0; but 30 x 136, three of 64 for two of 128, 17.6 / 21.6;
+            // 200 x 8 x 20 15.7 / 18.9; 255 x 16 x 24, 600 slices 13.2 / 15.0, 18 slices 4.2 / 5.7; 8 x 130 x 16, 'T' 'T' 13.0 / 18.5)
+            const int64_t of64 = ((m + 63) / 64) * ((n + 63) / 64), of128 = ((m + 127) / 128) * ((n + 127) / 128);
+            if (!wide || k < 24 || batch < 1024 || of64 < 2 * of128) return false;
+        } else if (!wide && batch > 512 && m * n * k < 50 * 50 * 50) {
+            return false;
+        }
+    }
     const int64_t extA = transA ? (m - 1) * lda + k : (k - 1) * lda + m, extB = transB ? (k - 1) * ldb + n : (n - 1) * ldb + k;
     if (extA * 2 >= 2147483647LL || extB * 2 >= 2147483647LL) return false;
     // leading dimensions of at least a piece: only the last k or row of a slice can hold a piece that ends past it

@@ -455,9 +455,11 @@ def test_operands_of_any_alignment(nn, dtype, ta, tb, m, n, k, batch):
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
-@pytest.mark.parametrize("m,n,k,batch", [(1, 1, 33, 2), (5, 7, 32, 3), (63, 65, 33, 2), (8, 129, 1, 2), (48, 64, 832, 2), (50, 50, 50, 513), (50, 49, 50, 513)])
+@pytest.mark.parametrize("m,n,k,batch", [(1, 1, 33, 2), (5, 7, 32, 3), (63, 65, 33, 2), (8, 129, 1, 2), (48, 64, 832, 2), (50, 50, 50, 513), (50, 49, 50, 513),
+                                       (8, 200, 33, 2), (9, 200, 24, 1023), (9, 200, 24, 1024), (255, 8, 23, 1024), (130, 8, 32, 1024), (64, 63, 32, 1024)])
 def test_few_results_of_16_bit_products(nn, dtype, ta, tb, m, n, k, batch):
-    """Results of less than 64 x 64 elements on both sides of the limits between the two 16-bit kernels (k, m * n * k, batch)."""
+    """Results of less than 64 x 64 elements on both sides of the limits between the two 16-bit kernels (k, m * n * k, batch, and for
+    results wider than 128 the tiles of either kernel)."""
     test_operands_of_any_alignment(nn, dtype, ta, tb, m, n, k, batch)
 
 
