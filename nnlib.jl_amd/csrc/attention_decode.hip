@@ -365,25 +365,51 @@ __global__ __launch_bounds__(256) void decode_weights_kernel(DecodeArgs a, TW *w
 // queries per wavefront: 1, 2, or 4 (three queries run as four)
 int decode_nq(const AttnParams &p) { return p.Lq <= 1 ? 1 : p.Lq == 2 ? 2 : 4; }
 
-// Workgroups along the keys of one (segment, batch element, query group).  Two workgroups of eight wavefronts share a CU, so
-// 512 are one round of the chip.  Measured, us of GPU time, one segment unless said:
-//   - up to one round, down to one 8-row block per wavefront: a second round with little left in it costs more than it gives
+// Share of the chip at work when every (segment, batch element, query group) has n workgroups: compute units in the last of the
+// rounds of 256 workgroups, wavefronts in the last 8-row blocks.
+double share_at_work(int64_t pairs, int64_t blocks, int64_t n) {
+    const int64_t rounds = (pairs * n + 255) / 256, per_wave = (blocks + WAVES * n - 1) / (WAVES * n);
+    return (double)(pairs * n) / (double)(256 * rounds) * (double)blocks / (double)(WAVES * n * per_wave);
+}
+
+// Workgroups along the keys of one (segment, batch element, query group).  A CU holds two workgroups of eight wavefronts with one
+// or two queries and one with four (203-207 registers).  Measured, us of GPU time, one segment unless said:
+//   - up to 512, down to one 8-row block per wavefront: another round with little left in it costs more than it gives
 //     (head dim 128, 4 segments x 3 x 3300 keys: 26.6 with 512 workgroups, 30 with 624), more blocks per wavefront leave CUs idle
 //     (2 x 5000 keys: 13.1 with one block per wavefront, 14.5 with two, 19.8 with four; one wavefront per 250 keys, as it was: 74);
 //   - two to four queries: two blocks, since a workgroup's partial results are that many times larger (31041 keys, two queries:
-//     23.9 with one, 20.7 with two);
-//   - a single query with at least 32 blocks per wavefront: four rounds, whose ends are shorter (8 segments x 16 x 32768 keys:
+//     23.9 with one, 20.7 with two), and from 16 blocks on one workgroup per CU (two queries, 8 segments x 8 x 8192 keys
+//     192 with 256 workgroups, 211 with 512; Float32, 8 x 16 x 16384 704, 817; four queries, 16-bit 199, 205; 718, 718);
+//   - a single query with at least 32 blocks per wavefront: four rounds of 512, whose ends are shorter (8 segments x 16 x 32768 keys:
 //     1407 with one round, 1389 with two, 1380 with four; Float32, 4 x 16 x 16384: 396, 403, 386), which costs two to four
-//     queries, with more to merge, up to a sixth (four queries, 8 segments x 8 x 8192 keys: 211, 222, 247).
+//     queries, with more to merge, up to a sixth (four queries, 8 segments x 8 x 8192 keys: 211, 222, 247);
+//   - more pairs than CUs: the fewest that keep 0.88 of the chip at work, or the best of 16.  With one workgroup per pair a few CUs have two
+//     of them and the others wait (2 segments x 140 pairs, a single query, keys: 600 80.7 with one / 66.7 with ten, 1000 133 / 104 with
+//     eight, 2000 258 / 202; two queries 1000 147 / 114, 2 x 130 x 4096 539 / 413 with eight; 2 x 270 x 600, a single query 136 / 124 with five).
+//     At most 8192 partial rows of a segment: 16 MiB of workspace.
 // With the weights requested the 256 keys per workgroup keep the partial results to what a call needed with one per split.
 int pick_nsplit(const AttnParams &p) {
     const int64_t SEG = p.dtype == MI_F32 ? seg_width<F32>() : seg_width<BF16>();
     const int64_t nseg = (p.E + SEG - 1) / SEG;
     const int64_t pairs = nseg * p.B * ((p.Lq + decode_nq(p) - 1) / decode_nq(p));   // (segment, batch element, query group)
-    int64_t want = pairs < 512 ? 512 / pairs : 1;
-    if (p.Lq == 1 && p.Lkv >= 32 * ROWS * WAVES * want) want = pairs < 2048 ? 2048 / pairs : 1;
     const int64_t blocks = p.weights ? 4 : p.Lq == 1 ? 1 : 2;   // 8-row blocks per wavefront, at least
     const int64_t maxs = (p.Lkv + ROWS * WAVES * blocks - 1) / (ROWS * WAVES * blocks);
+    int64_t want = pairs < 512 ? 512 / pairs : 1;
+    if (p.Lq == 1 && p.Lkv >= 32 * ROWS * WAVES * want) {
+        want = pairs < 2048 ? 2048 / pairs : 1;
+    } else if (pairs > 256) {
+        const int64_t all = (p.Lkv + ROWS - 1) / ROWS;
+        double best = 0.0;
+        for (int64_t n = 1; n <= 16 && n <= maxs && (n == 1 || n * pairs * decode_nq(p) <= 8192) && best < 0.88; n++) {
+            const double share = share_at_work(pairs, all, n);
+            if (share > best) {
+                best = share;
+                want = n;
+            }
+        }
+    } else if (p.Lq > 1 && p.Lkv >= 16 * ROWS * WAVES * want) {
+        want = 256 / pairs;
+    }
     if (want > maxs) want = maxs;
     if (want > MAX_SPLITS) want = MAX_SPLITS;
     return (int)want;

@@ -456,6 +456,10 @@ def test_decode_with_context_length_masks(nn, oracle, dtype, E, H, mask_shape):
     ("f32", 320, 5, 1, 777, 2, True),
     ("f16", 128, 1, 1, 70001, 1, False),     # one round of workgroups on a single pair
     ("bf16", 64, 1, 1, 2051, 300, True),     # four rounds of workgroups
+    # more than 256 pairs of a segment and a batch element (or group of queries): ten, eight, eight and six workgroups each
+    ("bf16", 1024, 16, 1, 600, 140, False), ("f32", 128, 2, 1, 1003, 280, True), ("f16", 64, 1, 2, 2000, 270, False),
+    ("bf16", 64, 1, 4, 1031, 270, True),
+    ("f16", 512, 4, 2, 2049, 64, False),     # two queries, long ranges: one workgroup per CU
 ])
 def test_decode_splits(nn, dtype, E, H, Lq, Lkv, B, masked):
     """Every way the key range is cut, against the same call in Float64.  Bound: the rounding of the result to its
