@@ -1590,14 +1590,16 @@ template <int D, bool CAUSAL>
 int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream_t st) {
     const AttnParams &p = a.p;
     constexpr size_t SMEM = CfgS<D>::SMEM;
-    // the dQ kernel on eight wavefronts (256 queries a workgroup) where the workgroups of four would need a second round of the chip
-    // (52 pairs of 1024 x 1024: 208 workgroups of eight 131 us, 416 of four 195); with a causal mask, whose lengths a second round evens
-    // out, where those of eight fill the chip (48 pairs of 1024 x 1024: 192 of eight 109 us, 384 of four 92)
+    // the dQ kernel on eight wavefronts (256 queries a workgroup) where those workgroups fill the chip, and without a causal mask, whose
+    // lengths a second round evens out, where the workgroups of four would need a second round (52 pairs of 1024 x 1024: 208 workgroups
+    // of eight 131 us, 416 of four 195; 48 causal ones: 192 of eight 109, 384 of four 92).  Where four make one round they are the
+    // shorter ones (whole steps, eight / four: 65 pairs of 300 x 300 112 / 105, 33 of 896 x 896 250 / 240).
     constexpr int NW_WIDE = D == 64 ? 8 : 4;
     constexpr size_t SMEM_WIDE = SMEM + 3 * 32 * NW_WIDE * CfgS<D>::ROWB;
     const int64_t wide_tiles = (p.Lq + 32 * NW_WIDE - 1) / (32 * NW_WIDE);
     // (not for sequences of at most 128 queries, where half of its wavefronts would have none: 4-6 % slower there)
-    const bool wide = NW_WIDE > 4 && bp.dq_nsplit <= 1 && p.Lq > 128 && wide_tiles * p.H * p.B >= (CAUSAL ? 256 : 129);
+    const bool wide = NW_WIDE > 4 && bp.dq_nsplit <= 1 && p.Lq > 128 &&
+                      (wide_tiles * p.H * p.B >= 256 || (!CAUSAL && (p.Lq + 127) / 128 * p.H * p.B > 256));
     auto k1 = bp.have_stats ? bwd32s_dq_kernel<D, CAUSAL, true, 4> : bwd32s_dq_kernel<D, CAUSAL, false, 4>;
     auto k1w = bp.have_stats ? bwd32s_dq_kernel<D, CAUSAL, true, NW_WIDE> : bwd32s_dq_kernel<D, CAUSAL, false, NW_WIDE>;
     auto k2 = bwd32s_dkdv_kernel<D, CAUSAL, BWD_DV>;
