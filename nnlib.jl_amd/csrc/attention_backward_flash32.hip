@@ -1609,14 +1609,14 @@ int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream
     // mask, us in this kernel: 128 pairs of 1024 x 1024 480 / 456 / 395 on one, two, eight; 52 pairs 227 / 197 / 167; 104 of
     // 752 x 752 274 / 262 / 248; 264 of 120 x 120 43 / 34 / 50).  With a causal mask two workgroups to a unit even out the lengths of
     // their loops (128 pairs of 1024 x 1024: 302 / 253 / 258; 128 of 648 x 648 164 / 109 / 112; whole steps, one / two: 80 of 1024 x
-    // 1024 373 / 344, 256 of 256 x 256 131 / 115), unless few are left for the second of a unit and the longest ones share one
-    // (48 pairs of 1024 x 1024 293 / 298).
+    // 1024 373 / 344, 256 of 256 x 256 131 / 115, 140 of 300 x 300 159 / 151), unless few are left for the second of a unit and the longest
+    // ones share one (48 pairs of 1024 x 1024 293 / 298, 96 of 400 x 400 148 / 153).
     auto k23 = bwd32s_dkdv_kernel<D, CAUSAL, BWD_DV | BWD_DK>;
     auto k23two = bwd32s_dkdv_kernel<D, CAUSAL, BWD_DV | BWD_DK, 4, D == 64 ? 2 : 1>;
     auto k23w = bwd32s_dkdv_kernel<D, CAUSAL, BWD_DV | BWD_DK, NW_WIDE>;
     const int64_t key_tiles = (p.Lkv + 127) / 128 * p.H * p.B, wide_key_tiles = (p.Lkv + 32 * NW_WIDE - 1) / (32 * NW_WIDE) * p.H * p.B;
     const auto rounds = [](int64_t tiles, int64_t slots) { return (double)((tiles + slots - 1) / slots); };
-    const bool two_dkdv = D == 64 && (CAUSAL ? key_tiles > (p.Lkv <= 512 ? 256 : 512) : 1.9 * rounds(key_tiles, 512) < rounds(key_tiles, 256));
+    const bool two_dkdv = D == 64 && (CAUSAL ? key_tiles > (p.Lkv <= 256 ? 256 : p.Lkv <= 512 ? 384 : 512) : 1.9 * rounds(key_tiles, 512) < rounds(key_tiles, 256));
     const bool wide_dkdv = D == 64 && !CAUSAL && p.Lkv > 128 && 1.5 * rounds(wide_key_tiles, 256) <= (two_dkdv ? 1.9 * rounds(key_tiles, 512) : rounds(key_tiles, 256));
     static const bool fused_dkdv = getenv("MI355ATTN_F32_DKDV_PAIR") == nullptr;   // the switch: for comparisons
     static bool attr_set = false;  // per instantiation; the attribute is idempotent, so a race is harmless
