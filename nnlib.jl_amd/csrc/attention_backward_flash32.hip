@@ -1613,11 +1613,12 @@ int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream
     // ones share one (48 pairs of 1024 x 1024 293 / 298, 96 of 400 x 400 148 / 153).
     auto k23 = bwd32s_dkdv_kernel<D, CAUSAL, BWD_DV | BWD_DK>;
     auto k23two = bwd32s_dkdv_kernel<D, CAUSAL, BWD_DV | BWD_DK, 4, D == 64 ? 2 : 1>;
-    auto k23w = bwd32s_dkdv_kernel<D, CAUSAL, BWD_DV | BWD_DK, NW_WIDE>;
-    const int64_t key_tiles = (p.Lkv + 127) / 128 * p.H * p.B, wide_key_tiles = (p.Lkv + 32 * NW_WIDE - 1) / (32 * NW_WIDE) * p.H * p.B;
+    constexpr int NW_WIDE_K = CAUSAL ? 4 : NW_WIDE;   // (without a causal mask only)
+    auto k23w = bwd32s_dkdv_kernel<D, CAUSAL, BWD_DV | BWD_DK, NW_WIDE_K>;
+    const int64_t key_tiles = (p.Lkv + 127) / 128 * p.H * p.B, wide_key_tiles = (p.Lkv + 32 * NW_WIDE_K - 1) / (32 * NW_WIDE_K) * p.H * p.B;
     const auto rounds = [](int64_t tiles, int64_t slots) { return (double)((tiles + slots - 1) / slots); };
     const bool two_dkdv = D == 64 && (CAUSAL ? key_tiles > (p.Lkv <= 256 ? 256 : p.Lkv <= 512 ? 384 : 512) : 1.9 * rounds(key_tiles, 512) < rounds(key_tiles, 256));
-    const bool wide_dkdv = D == 64 && !CAUSAL && p.Lkv > 128 && 1.5 * rounds(wide_key_tiles, 256) <= (two_dkdv ? 1.9 * rounds(key_tiles, 512) : rounds(key_tiles, 256));
+    const bool wide_dkdv = NW_WIDE_K > 4 && p.Lkv > 128 && 1.5 * rounds(wide_key_tiles, 256) <= (two_dkdv ? 1.9 * rounds(key_tiles, 512) : rounds(key_tiles, 256));
     static const bool fused_dkdv = getenv("MI355ATTN_F32_DKDV_PAIR") == nullptr;   // the switch: for comparisons
     static bool attr_set = false;  // per instantiation; the attribute is idempotent, so a race is harmless
     if (!attr_set) {
@@ -1631,7 +1632,7 @@ int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream
         MI_HIP_CHECK(hipFuncSetAttribute((const void *)k3, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMEM));
         MI_HIP_CHECK(hipFuncSetAttribute((const void *)k23, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMEM));
         MI_HIP_CHECK(hipFuncSetAttribute((const void *)k23two, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMEM));
-        if (NW_WIDE > 4) MI_HIP_CHECK(hipFuncSetAttribute((const void *)k23w, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMEM_WIDE));
+        if (NW_WIDE_K > 4) MI_HIP_CHECK(hipFuncSetAttribute((const void *)k23w, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMEM_WIDE));
         attr_set = true;
     }
     // few 32-row blocks (at most two workgroups per compute unit) and the forward call's statistics: the workgroups per
@@ -1719,7 +1720,7 @@ int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream
         if constexpr (D == 64)
             if (bp.dv || bp.dk) hipLaunchKernelGGL((bwd32s_dkdv_small_kernel<D, CAUSAL, false>), dim3((unsigned)k_blocks), dim3(256), SmallBwd<D>::SMEM, st, a, bp);
     } else if (bp.dv && bp.dk && fused_dkdv) {
-        if (wide_dkdv) hipLaunchKernelGGL(k23w, dim3((unsigned)wide_key_tiles), dim3(64 * NW_WIDE), SMEM_WIDE, st, a, bp);
+        if (wide_dkdv) hipLaunchKernelGGL(k23w, dim3((unsigned)wide_key_tiles), dim3(64 * NW_WIDE_K), SMEM_WIDE, st, a, bp);
         else hipLaunchKernelGGL(two_dkdv ? k23two : k23, g2, dim3(256), SMEM, st, a, bp);
     } else {
         if (bp.dv) hipLaunchKernelGGL(k2, g2, dim3(256), SMEM, st, a, bp);
