@@ -609,8 +609,9 @@ np.savez(sys.argv[2], dq=g[0].to_numpy(), dk=g[1].to_numpy(), dv=g[2].to_numpy()
 
 
 @pytest.mark.parametrize("E,H,Lq,Lkv,causal,saved", [(256, 4, 300, 300, False, True), (256, 4, 257, 257, True, False),
-                                                     (256, 2, 200, 330, False, False), (96, 1, 130, 130, True, True)],
-                         ids=["D64-saved", "D64-causal", "D128-cross", "D96-causal-saved"])
+                                                     (256, 2, 200, 330, False, False), (96, 1, 130, 130, True, True),
+                                                     (2048, 16, 200, 330, False, True), (3072, 32, 260, 260, True, True)],
+                         ids=["D64-saved", "D64-causal", "D128-cross", "D96-causal-saved", "D128-one-pass", "D96-one-pass-causal"])
 def test_float32_gradient_through_bf16_planes_keeps_float32_accuracy(nn, oracle, tmp_path, E, H, Lq, Lkv, causal, saved):
     """Float32 gradient calls without bias / mask arrays run their products as six bf16 matrix instructions per Float32
     one (three planes per operand).  Against float64 on the same inputs every gradient must be as close as the Float32
@@ -934,16 +935,31 @@ def test_shared_bias_gradient_in_tiles_of_128(nn, oracle, dtype, D, H, Lq, Lkv, 
         _run(nn, oracle, dtype, E, E, Lq, Lkv, batch, H, mask_kind=mask_kind, bias_shape=(Lkv, Lq, H), expect="flash16", saved=saved, seed=Lq + Lkv)
 
 
+def _shared_by_pairs(D, L, H, B, mask_kind):
+    """Whether calls with so many rows of 32 go to the Float32 gradient kernel whose wavefronts share a block in pairs (dK and dV: any
+    statistics; dQ: the forward call's)."""
+    blocks = (L + 31) // 32 * H * B
+    if mask_kind == "lengths":
+        return False
+    if D > 64:
+        return blocks <= (512 if mask_kind == "causal" and L > 128 else 256)
+    return 256 < blocks <= 512 and L > 32
+
+
 @pytest.mark.parametrize("D,H,Lq,Lkv,B,mask_kind,saved", [
-    # tiles of 96 features (head dims 68 to 96) and both key gradients in one pass in tiles of 96 and 128
-    (68, 2, 130, 193, 2, None, True), (96, 2, 65, 127, 2, None, False), (80, 2, 257, 257, 1, "causal", True),
-    (96, 3, 100, 300, 4, "lengths", True), (128, 2, 129, 65, 2, None, False), (100, 2, 200, 200, 1, "causal", True),
+    # tiles of 96 and 128 features: several query tiles, ragged ends, more blocks of 32 keys than the pairs of wavefronts take
+    (96, 3, 100, 300, 4, "lengths", True), (80, 8, 200, 257, 4, None, False), (96, 8, 257, 257, 8, "causal", True),
+    (68, 8, 257, 257, 8, "causal", False), (128, 8, 130, 193, 5, None, True), (100, 8, 200, 200, 5, None, False),
+    (128, 8, 257, 257, 8, "causal", True), (128, 8, 32, 64, 33, None, True),
     # head dims up to 64: a workgroup of four wavefronts, two of them to a compute unit, one of eight
-    (64, 8, 40, 130, 12, None, True), (64, 12, 70, 120, 22, None, True), (64, 8, 66, 260, 12, None, True), (48, 8, 64, 385, 12, None, False),
-    (60, 8, 257, 257, 11, "causal", True), (64, 8, 130, 300, 12, "lengths", True),
+    (64, 12, 70, 120, 22, None, True), (64, 8, 66, 260, 12, None, True), (48, 8, 64, 385, 12, None, False),
+    (60, 8, 257, 257, 11, "causal", True), (64, 8, 130, 300, 12, "lengths", True), (64, 16, 64, 96, 17, None, True),
+    # with a causal mask from 385 workgroups of 128 keys on two to a compute unit
+    (64, 8, 257, 257, 16, "causal", True), (64, 8, 260, 260, 17, "causal", False),
 ])
 def test_float32_key_gradients_in_one_pass(nn, oracle, D, H, Lq, Lkv, B, mask_kind, saved):
     """The forms of the Float32 kernel that makes dK and dV from one S and dP, at the edges of their tiles and of the rule."""
+    assert not _shared_by_pairs(D, Lkv, H, B, mask_kind)
     _run(nn, oracle, "f32", D * H, D * H, Lq, Lkv, (B,), H, mask_kind=mask_kind, saved=saved, scale=0.4, seed=D + Lkv, expect="flash32")
 
 
@@ -961,13 +977,18 @@ def test_16_bit_gradient_in_tiles_of_32_and_96_features(nn, oracle, D, dtype, H,
          seed=D + Lkv, scale=0.6, saved=True, dropout=dropout, expect="flash16")
 
 
-@pytest.mark.parametrize("D,H,Lq,Lkv,B,mask_kind", [
-    (68, 2, 1, 64, 2, None), (96, 2, 33, 65, 1, None), (128, 3, 97, 31, 2, None), (100, 2, 200, 129, 1, None), (96, 1, 130, 400, 2, None),
-    (72, 2, 63, 63, 2, "causal"), (128, 2, 129, 129, 2, "causal"), (96, 8, 257, 257, 5, "causal"), (128, 8, 32, 64, 33, None),
+@pytest.mark.parametrize("D,H,Lq,Lkv,B,mask_kind,saved", [
+    (68, 2, 1, 64, 2, None, True), (96, 2, 33, 65, 1, None, True), (128, 3, 97, 31, 2, None, True), (100, 2, 200, 129, 1, None, True),
+    (96, 1, 130, 400, 2, None, True), (72, 2, 63, 63, 2, "causal", True), (128, 2, 129, 129, 2, "causal", True),
+    (96, 8, 257, 257, 5, "causal", True), (68, 2, 130, 193, 2, None, True), (96, 2, 65, 127, 2, None, False),
+    (80, 2, 257, 257, 1, "causal", True), (128, 2, 129, 65, 2, None, False), (100, 2, 200, 200, 1, "causal", True),
     # head dims up to 64, 257 to 512 blocks: both gradients, one of them
-    (64, 8, 161, 190, 7, None), (36, 8, 130, 130, 8, "causal"), (64, 16, 64, 96, 17, None), (48, 16, 33, 65, 9, None),
+    (64, 8, 161, 190, 7, None, True), (36, 8, 130, 130, 8, "causal", True), (48, 16, 33, 65, 9, None, True),
+    (64, 8, 128, 400, 10, None, True), (64, 8, 400, 128, 10, None, True), (64, 8, 40, 130, 12, None, True),
 ])
-def test_float32_gradient_by_pairs_of_wavefronts(nn, oracle, D, H, Lq, Lkv, B, mask_kind):
+def test_float32_gradient_by_pairs_of_wavefronts(nn, oracle, D, H, Lq, Lkv, B, mask_kind, saved):
     """Head dims 68 to 128, at most 256 blocks of 32 rows (512 with a causal mask), up to 64, more than 256 and at most 512: pairs of
     wavefronts that share a block."""
-    _run(nn, oracle, "f32", D * H, D * H, Lq, Lkv, (B,), H, mask_kind=mask_kind, saved=True, scale=0.4, seed=D + Lkv, expect="flash32")
+    q_pairs, k_pairs = saved and _shared_by_pairs(D, Lq, H, B, mask_kind), _shared_by_pairs(D, Lkv, H, B, mask_kind)
+    assert q_pairs or k_pairs
+    _run(nn, oracle, "f32", D * H, D * H, Lq, Lkv, (B,), H, mask_kind=mask_kind, saved=saved, scale=0.4, seed=D + Lkv, expect="flash32")
