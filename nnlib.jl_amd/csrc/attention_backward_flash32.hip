@@ -1673,7 +1673,7 @@ int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream
     bool halves_q = false, halves_k = false;
     if constexpr (D > 64) {
         const bool can = !a.kv_len && !no_small;
-        // A compute unit holds one workgroup (116 KiB of LDS at 128 features), which takes half as long as one of 128 rows: one
+        // A compute unit holds one workgroup (113 KiB of LDS at 128 features), which takes half as long as one of 128 rows: one
         // round of the chip, and two where a causal mask leaves the workgroups of 128 rows with unequal loops (whole steps, us, 128
         // rows / 32: head dim 128, 8 x 4 pairs of 256 x 256 130 / 80, causal 131 / 80; 8 x 6 151 / 146; 8 x 8 155 / 149, causal 157 /
         // 123; 8 x 12 159 / 204; 96, 8 x 8 of 256 x 256 122 / 124, 8 x 4 of 512 x 512, causal 196 / 145; 80, 6 x 31 of 40 x 40,
@@ -1685,9 +1685,17 @@ int32_t launch_set_planes(const FlashArgs &a, const AttnBwdParams &bp, hipStream
     } else {
         // head dims up to 64: two of those workgroups fit a compute unit (65 KiB), one of the kernels above (147 KiB), so they are faster
         // where those need a second round (12 x 5 pairs of 160 x 160 72.8 / 52.1 us, causal 60.2 / 47.0; 8 x 4 of 512 x 512 128 / 103; 8 x
-        // 30 of 64 x 64, causal 48.9 / 33.9) and slower in the first (8 x 2 of 512 x 512 71.5 / 77.5; 4 x 2 of 1000 x 1000 127 / 139)
-        halves_q = small_q && q_blocks > 256 && p.Lq > 32;
-        halves_k = small_k && k_blocks > 256 && p.Lkv > 32;
+        // 30 of 64 x 64, causal 48.9 / 33.9) and slower in the first (8 x 2 of 512 x 512 71.5 / 77.5; 4 x 2 of 1000 x 1000 127 / 139).
+        // With a causal mask the second round is made of the shortest blocks: of sequences of n blocks it ends with the first while
+        // there are at most about 512 n / (n + constant) of them, and a workgroup of these kernels takes a tenth longer (whole steps,
+        // above / these: 512 x 512, 18 pairs 76 / 82, 22 90 / 88, 30 104 / 92; 768 x 768, 12 101 / 113, 18 130 / 124; 1024 x 1024, 12 133 /
+        // 147, 14 158 / 156; 1400 x 1400, 8 200 / 220, 11 222 / 222; 2048 x 2048, 6 287 / 312, 8 302 / 310; head dims 8 and 32 alike).
+        const auto second_round = [](int64_t blocks, int64_t rows) {
+            const int64_t n = (rows + 31) / 32;
+            return blocks > 256 && n > 1 && (!CAUSAL || blocks * (n + 11) > 600 * n);
+        };
+        halves_q = small_q && second_round(q_blocks, p.Lq);
+        halves_k = small_k && second_round(k_blocks, p.Lkv);
     }
     if (halves_q || halves_k) {
         static bool halves_attr_set = false;

@@ -943,7 +943,8 @@ def _shared_by_pairs(D, L, H, B, mask_kind):
         return False
     if D > 64:
         return blocks <= (512 if mask_kind == "causal" and L > 128 else 256)
-    return 256 < blocks <= 512 and L > 32
+    n = (L + 31) // 32
+    return 256 < blocks <= 512 and n > 1 and (mask_kind != "causal" or blocks * (n + 11) > 600 * n)
 
 
 @pytest.mark.parametrize("D,H,Lq,Lkv,B,mask_kind,saved", [
@@ -961,6 +962,14 @@ def test_float32_key_gradients_in_one_pass(nn, oracle, D, H, Lq, Lkv, B, mask_ki
     """The forms of the Float32 kernel that makes dK and dV from one S and dP, at the edges of their tiles and of the rule."""
     assert not _shared_by_pairs(D, Lkv, H, B, mask_kind)
     _run(nn, oracle, "f32", D * H, D * H, Lq, Lkv, (B,), H, mask_kind=mask_kind, saved=saved, scale=0.4, seed=D + Lkv, expect="flash32")
+
+
+@pytest.mark.parametrize("D,H,L,B", [(64, 4, 320, 7), (40, 4, 500, 5), (64, 4, 513, 4)])
+def test_float32_causal_gradient_of_few_long_sequences(nn, oracle, D, H, L, B):
+    """Head dims up to 64, 257 to 512 blocks of 32 rows whose second round of the chip is over with the first: the workgroups of 32 rows
+    that share a compute unit with no other."""
+    assert 256 < (L + 31) // 32 * H * B <= 512 and not _shared_by_pairs(D, L, H, B, "causal")
+    _run(nn, oracle, "f32", D * H, D * H, L, L, (B,), H, mask_kind="causal", saved=True, scale=0.4, seed=D + L, expect="flash32")
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
@@ -985,6 +994,7 @@ def test_16_bit_gradient_in_tiles_of_32_and_96_features(nn, oracle, D, dtype, H,
     # head dims up to 64, 257 to 512 blocks: both gradients, one of them
     (64, 8, 161, 190, 7, None, True), (36, 8, 130, 130, 8, "causal", True), (48, 16, 33, 65, 9, None, True),
     (64, 8, 128, 400, 10, None, True), (64, 8, 400, 128, 10, None, True), (64, 8, 40, 130, 12, None, True),
+    (64, 6, 320, 320, 5, "causal", True), (40, 4, 500, 500, 6, "causal", True),
 ])
 def test_float32_gradient_by_pairs_of_wavefronts(nn, oracle, D, H, Lq, Lkv, B, mask_kind, saved):
     """Head dims 68 to 128, at most 256 blocks of 32 rows (512 with a causal mask), up to 64, more than 256 and at most 512: pairs of
