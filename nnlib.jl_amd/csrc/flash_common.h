@@ -64,20 +64,36 @@ __device__ inline void flash_zero_stats_padding(const AttnParams &p, int64_t b, 
 // Split-kv bookkeeping shared by the planner (workspace size) and the launchers.
 // Partials live in the caller's workspace: o as [split][B][Lq][Ev] floats, then (m, l) as
 // [split][B][H][Lq][2] floats, m in log2 units.
+inline bool flash_is_query_independent_mask(const AttnParams &p);
 inline int flash_pick_nsplit(const AttnParams &p, int bm) {
     if (p.weights || !p.out || p.stats) return 1;           // weights need the global maximum up front; saved statistics are per whole row
     const int64_t wgs = ((p.Lq + bm - 1) / bm) * p.H * p.B;
     if (wgs >= 512) return 1;
     if (p.Lkv < 2048) {
-        // The general kernel (all calls with a bias, and head dims that the pipelined kernel has no tiles for), where a workgroup that is
-        // alone on its CU takes 1 to 2.6 us per 64 keys: a few of them are worth the merge (5 us) from 768 keys on, at least 256
-        // a piece (us, one / several: 8 workgroups x 1511 keys with a bias 64 / 20, 18 x 1615 with a dense mask 54 / 18; without
-        // either, head dim 96, 18 x 1615 39 / 18, 64 x 1000, causal 28 / 21; 32, 128 x 1900 33 / 19).  Without a bias, more than 64
-        // workgroups from 1024 keys on (96, 128 x 800: 23.2 / 24.3; 32, 128 x 768, padded 18.9 / 19.8).
+        // The general kernel (all calls with a bias, and head dims that the pipelined kernel has no tiles for): a few workgroups are worth
+        // the merge (5 us) from 768 keys on, at least 256 a piece (8 workgroups x 1511 keys with a bias, which take 2.6 us per 64 keys: 64 us in
+        // one, 20 in several).
         const bool pipelined = !p.bias && p.D == p.Dv && (p.D == 64 || p.D == 128);
-        if (p.dtype == MI_F32 || pipelined || p.lean_workspace || wgs > 128 || p.Lkv < (p.bias || wgs <= 64 ? 768 : 1024)) return 1;
-        const int64_t n = 512 / wgs, most = p.Lkv / 256;
-        return (int)(n < most ? n : most);
+        if (p.dtype == MI_F32 || pipelined || p.lean_workspace || wgs > 128 || p.Lkv < 768) return 1;
+        const int64_t most = p.Lkv / 256;
+        const int64_t n = 512 / wgs < most ? 512 / wgs : most;
+        if (p.bias) return (int)n;
+        if (wgs > 64 && p.Lkv < 1024) return 1;   // pieces of 256 keys are few (us, one / several, head dim 96, dense mask, 100 x 768 24.8 / 28.8)
+        // Without a bias a workgroup alone on its CU takes 0.7 to 2 us per 64 keys, and the pieces cost their tiles, a second round of the
+        // chip at 256 features, and a merge that grows with the partial results of `parts` workgroups.  A padding mask that pieces read
+        // entry by entry would else give context lengths: a call in one piece then stops at the longest.  The constants (us) are fitted to
+        // 1440 calls at head dims 32 to 192: 42 of them are 1 to 22 % slower in the pieces they get, 24 up to 11 % in the one (us, one /
+        // several, head dim 96: 24 workgroups x 1100 keys 27 / 17, 64 x 1100 27 / 23, 100 x 1100 28 / 30, 64 x 768 20 / 21, 128 x 2040 45 / 40,
+        // padded 50 / 51; 32: 24 x 768 12 / 15, 24 x 1300 19 / 15, 100 x 1300 19 / 26, padded 23 / 33, 128 x 1100 with a dense mask 34 / 31).
+        const int64_t dmax = p.D > p.Dv ? p.D : p.Dv, tile = dmax <= 32 ? 32 : dmax <= 64 ? 64 : dmax <= 96 ? 96 : dmax <= 128 ? 128 : 256;
+        const int64_t tiles = (p.Lkv + 63) / 64, per_piece = (tiles + n - 1) / n, parts = wgs * n;
+        const int64_t rounds = tile == 256 ? (parts + 255) / 256 : 1;
+        const bool padded = flash_is_query_independent_mask(p);
+        const double us_per_tile = 0.48 + 0.008 * tile + (tile == 256 ? 1.1 : 0.0) + (p.mask && !padded ? 0.8 : 0.0) + (p.drop_thresh ? 0.63 : 0.0);
+        const double saved = us_per_tile * ((padded ? 0.9 : 1.0) * tiles - per_piece * rounds);
+        const double base = 7.2 - 0.0375 * tile;
+        const double merge = (base > 4.0 ? base : 4.0) + (0.0225 + 0.0002 * tile) * (parts > 64 ? parts - 64 : 0) + (padded ? 1.9 : 0.0);
+        return saved > merge ? (int)n : 1;
     }
     // aim at one resident round: two workgroups per CU on 256 CUs (measured best on the f16 cross-attention case)
     int64_t n = (512 + wgs - 1) / wgs;

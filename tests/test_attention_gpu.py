@@ -1141,13 +1141,19 @@ def test_16_bit_tiles_of_32_and_96_features(nn, oracle, D, dtype, Lq, Lkv, kw, w
     _check(nn, oracle, np.random.default_rng(D + Lkv), dtype, 2 * D, Lq, Lkv, 3, 2, expect="flash16", weights=weights, **kw)
 
 
-@pytest.mark.parametrize("D,H,Lq,Lkv,B,kw", [
-    (32, 6, 112, 1615, 3, dict(mask_shape=(1615, 112))), (96, 2, 129, 768, 1, {}), (80, 8, 130, 1000, 5, dict(mask_shape=(1000, 1, 1, 5))),
-    (48, 8, 900, 900, 1, dict(causal=True)), (256, 2, 70, 1100, 2, {}), (96, 16, 128, 1023, 8, {}), (96, 16, 128, 1024, 8, {}),
+@pytest.mark.parametrize("D,H,Lq,Lkv,B,kw,pieces", [
+    (32, 6, 112, 1615, 3, dict(mask_shape=(1615, 112)), 6), (96, 2, 129, 768, 1, {}, 3), (80, 8, 130, 1000, 5, dict(mask_shape=(1000, 1, 1, 5)), 1),
+    (48, 8, 900, 900, 1, dict(causal=True), 3), (256, 2, 70, 1100, 2, {}, 4), (96, 16, 128, 1023, 8, {}, 1), (96, 16, 128, 1024, 8, {}, 1),
+    # the merge grows with the workgroups, a padding mask in pieces is read entry by entry
+    (96, 8, 40, 1100, 8, {}, 4), (96, 10, 40, 1100, 10, {}, 1), (32, 8, 40, 768, 3, {}, 1), (32, 8, 40, 1300, 3, {}, 5),
+    (96, 8, 40, 1100, 3, dict(mask_shape=(1100, 1, 1, 3)), 4), (32, 8, 40, 1100, 6, dict(mask_shape=(1100, 1, 1, 6)), 1),
+    (32, 16, 40, 1100, 8, dict(mask_shape=(1100, 40)), 4), (200, 8, 40, 1100, 8, {}, 4), (200, 8, 40, 800, 16, {}, 1),
 ])
-def test_key_pieces_of_the_general_kernel_below_2048_keys(nn, oracle, D, H, Lq, Lkv, B, kw):
+def test_key_pieces_of_the_general_kernel_below_2048_keys(nn, oracle, D, H, Lq, Lkv, B, kw, pieces):
     """Head dims without tiles of the pipelined kernel, no bias, both sides of the rule."""
     _check(nn, oracle, np.random.default_rng(D + Lkv), "bf16", D * H, Lq, Lkv, B, H, expect="flash16", weights=False, **kw)
+    lengths = (4 * H * B + 15) // 16 * 16 if len(kw.get("mask_shape", ())) == 4 else 0
+    assert nn.ops.last_attention_workspace() == (4 * pieces * B * Lq * (D + 2) * H if pieces > 1 else lengths)
 
 
 @pytest.mark.parametrize("Lq,Lkv,kw", [
