@@ -380,13 +380,17 @@ double share_at_work(int64_t pairs, int64_t blocks, int64_t n) {
 //   - two to four queries: two blocks, since a workgroup's partial results are that many times larger (31041 keys, two queries:
 //     23.9 with one, 20.7 with two), and from 16 blocks on one workgroup per CU (two queries, 8 segments x 8 x 8192 keys
 //     192 with 256 workgroups, 211 with 512; Float32, 8 x 16 x 16384 704, 817; four queries, 16-bit 199, 205; 718, 718);
-//   - a single query with at least 32 blocks per wavefront: four rounds of 512, whose ends are shorter (8 segments x 16 x 32768 keys:
-//     1407 with one round, 1389 with two, 1380 with four; Float32, 4 x 16 x 16384: 396, 403, 386), which costs two to four
-//     queries, with more to merge, up to a sixth (four queries, 8 segments x 8 x 8192 keys: 211, 222, 247);
-//   - more pairs than CUs: the fewest that keep 0.88 of the chip at work, or the best of 16.  With one workgroup per pair a few CUs have two
-//     of them and the others wait (2 segments x 140 pairs, a single query, keys: 600 80.7 with one / 66.7 with ten, 1000 133 / 104 with
-//     eight, 2000 258 / 202; two queries 1000 147 / 114, 2 x 130 x 4096 539 / 413 with eight; 2 x 270 x 600, a single query 136 / 124 with five).
-//     At most 8192 partial rows of a segment: 16 MiB of workspace.
+//   - a single query, 12 blocks and more for each wavefront of 256 workgroups: four blocks per wavefront, at most 8192 workgroups.  Where
+//     the batch elements are powers of two apart, few long wavefronts run in step on the same channels (head dim 64, 16-bit, 4 segments x
+//     8 x 16384 keys 219 with 512 workgroups, 197 with 2048, 188 with one result per wavefront as it was; 4 x 16 x 8192 220, 185, 185; Float32, head
+//     dim 128, 8 x 16 x 16384 765, 708 with 8192, 722); elsewhere it costs up to 2 % (15 x 5 x 20000 109, 111).  With the weights requested
+//     four rounds of 512 (8 segments x 16 x 32768 keys 1524, as it was 1597), which cost two to four queries, with more to merge, up to a
+//     sixth (four queries, 8 segments x 8 x 8192 keys: 211, 222, 247);
+//   - more pairs than CUs, or two to four queries and a number of them that fills no round: the fewest that keep 0.88 (0.8) of the
+//     chip at work, or the best of 16.  With one
+//     workgroup per pair a few CUs have two of them and the others wait (2 segments x 140 pairs, a single query, keys: 600 80.7 with one / 66.7
+//     with ten, two queries 1000 147 / 114; 2 x 130 x 4096 539 / 413 with eight; 2 x 270 x 600, a single query 136 / 124 with five), or some
+//     have none (three queries, Float32, 2 x 88 x 8192 645 with one / 520 with four).  At most 8192 partial rows of a segment: 16 MiB of workspace.
 // With the weights requested the 256 keys per workgroup keep the partial results to what a call needed with one per split.
 int pick_nsplit(const AttnParams &p) {
     const int64_t SEG = p.dtype == MI_F32 ? seg_width<F32>() : seg_width<BF16>();
@@ -394,21 +398,25 @@ int pick_nsplit(const AttnParams &p) {
     const int64_t pairs = nseg * p.B * ((p.Lq + decode_nq(p) - 1) / decode_nq(p));   // (segment, batch element, query group)
     const int64_t blocks = p.weights ? 4 : p.Lq == 1 ? 1 : 2;   // 8-row blocks per wavefront, at least
     const int64_t maxs = (p.Lkv + ROWS * WAVES * blocks - 1) / (ROWS * WAVES * blocks);
+    const int64_t all = (p.Lkv + ROWS - 1) / ROWS;
     int64_t want = pairs < 512 ? 512 / pairs : 1;
-    if (p.Lq == 1 && p.Lkv >= 32 * ROWS * WAVES * want) {
+    const bool long_range = p.Lkv >= (p.Lq == 1 ? 32 : 16) * ROWS * WAVES * want;
+    if (p.Lq == 1 && p.weights && long_range) {
         want = pairs < 2048 ? 2048 / pairs : 1;
-    } else if (pairs > 256) {
-        const int64_t all = (p.Lkv + ROWS - 1) / ROWS;
+    } else if (p.Lq == 1 && !p.weights && p.Lkv >= 1024 && pairs * all >= 12 * WAVES * 256) {
+        want = (all + WAVES * 4 - 1) / (WAVES * 4);
+        if (want * pairs > 8192) want = pairs < 8192 ? 8192 / pairs : 1;
+    } else if (pairs > 256 || (p.Lq > 1 && long_range)) {
+        const int64_t first = pairs > 256 ? 1 : 256 / pairs;
+        const double enough = pairs > 256 ? 0.88 : 0.8;
         double best = 0.0;
-        for (int64_t n = 1; n <= 16 && n <= maxs && (n == 1 || n * pairs * decode_nq(p) <= 8192) && best < 0.88; n++) {
+        for (int64_t n = first; n <= maxs && (n == first || (n <= 16 && n * pairs * decode_nq(p) <= 8192)) && best < enough; n++) {
             const double share = share_at_work(pairs, all, n);
             if (share > best) {
                 best = share;
                 want = n;
             }
         }
-    } else if (p.Lq > 1 && p.Lkv >= 16 * ROWS * WAVES * want) {
-        want = 256 / pairs;
     }
     if (want > maxs) want = maxs;
     if (want > MAX_SPLITS) want = MAX_SPLITS;

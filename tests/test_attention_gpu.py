@@ -455,7 +455,9 @@ def test_decode_with_context_length_masks(nn, oracle, dtype, E, H, mask_shape):
     ("bf16", 512, 4, 3, 1031, 3, True),      # three queries as four
     ("f32", 320, 5, 1, 777, 2, True),
     ("f16", 128, 1, 1, 70001, 1, False),     # one round of workgroups on a single pair
-    ("bf16", 64, 1, 1, 2051, 300, True),     # four rounds of workgroups
+    ("bf16", 64, 1, 1, 2051, 300, True),     # four blocks per wavefront
+    ("bf16", 64, 1, 1, 7001, 300, False),    # at most 8192 workgroups
+    ("f32", 64, 1, 3, 3100, 144, True),      # three queries: one workgroup per pair would leave CUs idle
     # more than 256 pairs of a segment and a batch element (or group of queries): ten, eight, eight and six workgroups each
     ("bf16", 1024, 16, 1, 600, 140, False), ("f32", 128, 2, 1, 1003, 280, True), ("f16", 64, 1, 2, 2000, 270, False),
     ("bf16", 64, 1, 4, 1031, 270, True),
