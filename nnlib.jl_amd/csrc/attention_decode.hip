@@ -373,7 +373,7 @@ double share_at_work(int64_t pairs, int64_t blocks, int64_t n) {
 }
 
 // Workgroups along the keys of one (segment, batch element, query group).  A CU holds two workgroups of eight wavefronts with one
-// or two queries and one with four (203-207 registers).  Measured, us of GPU time, one segment unless said:
+// or two queries and one with four (171-207 registers).  Measured, us of GPU time, one segment unless said:
 //   - up to 512, down to one 8-row block per wavefront: another round with little left in it costs more than it gives
 //     (head dim 128, 4 segments x 3 x 3300 keys: 26.6 with 512 workgroups, 30 with 624), more blocks per wavefront leave CUs idle
 //     (2 x 5000 keys: 13.1 with one block per wavefront, 14.5 with two, 19.8 with four; one wavefront per 250 keys, as it was: 74);
