@@ -1417,11 +1417,25 @@ bool exact_instruction_wanted() {
     return wanted;
 }
 
+// Head dims 68 to 96 without bias / mask code: tiles of 96 features.  They gain by two workgroups per CU; one that has its CU to itself
+// misses the next tile's loads ahead of the products, with dropout also 132 bytes of scratch.  Tiles of 128 therefore take (us, 128 /
+// 96, head dim 80): with dropout calls that one round of the chip holds (1500 x 1500, 120 workgroups 165 / 190; 600 x 600, 250 76 / 85;
+// from 257 on 96: 300 x 1200, 300 0.64 times), with a causal mask, whose long workgroups end alone, up to 400, or 520 with the weights
+// (from 4 query tiles on: 1000 x 1000, 296 1.13 and 1.14 times, 400 1.04 and 1.12, 520 0.86 and 0.97; 300 x 300, 300 0.80); without, calls
+// of one round whose keys few query tiles share (256 pairs of 17 x 2000 203 / 246, of 17 x 1000 level; 12 of 1419 x 1419 144 / 126).
+bool takes_tiles_of_96(const FlashArgs &a) {
+    const AttnParams &p = a.p;
+    const int64_t wgs = (int64_t)a.n_qtiles * p.H * p.B * a.nsplit;
+    if (!p.drop_thresh) return wgs > 256 || a.n_qtiles > 2 || p.causal || p.weights;
+    if (p.causal) return a.nsplit > 1 || a.n_qtiles < 4 || (p.weights ? wgs > 520 : wgs <= 128 || wgs > 400);
+    return wgs > 256 || p.weights;
+}
+
 template <int D, int QB>
 int32_t launch_d(const FlashArgs &a, hipStream_t st, bool extras) {
     if (exact_instruction_wanted()) return launch_ds<D, QB, false>(a, st, extras);
     if constexpr (D == 128)
-        if (!extras && a.p.D <= 96 && a.p.Dv <= 96) {
+        if (!extras && a.p.D <= 96 && a.p.Dv <= 96 && takes_tiles_of_96(a)) {
             const bool w = a.p.weights != nullptr;
             if (a.p.causal) return w ? launch_one<96, QB, true, false, true, true>(a, st) : launch_one<96, QB, true, false, false, true>(a, st);
             return w ? launch_one<96, QB, false, false, true, true>(a, st) : launch_one<96, QB, false, false, false, true>(a, st);

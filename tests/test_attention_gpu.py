@@ -1125,9 +1125,11 @@ def test_a_short_key_range_with_a_bias_needs_no_workspace(nn):
     (68 * 2, 2, 130, 193, 2, {}), (96 * 12, 12, 129, 513, 6, {}), (80 * 2, 2, 257, 257, 2, dict(causal=True)),
     (96 * 8, 8, 300, 300, 16, dict(causal=True)), (72 * 2, 2, 40, 70, 2, dict(mask_shape=(70, 40))),
     (96 * 2, 2, 70, 520, 2, dict(mask_shape=(520, 1, 1, 2))), (96, 1, 70, 2500, 1, {}), (96 * 2, 2, 64, 600, 3, dict(Ev=80 * 2)),
+    (80 * 8, 8, 40, 600, 33, {}), (80 * 2, 2, 300, 600, 2, {}), (96 * 8, 8, 40, 530, 33, dict(mask_shape=(530, 1, 1, 33))),
 ])
 def test_float32_tiles_of_96_features(nn, oracle, E, H, Lq, Lkv, B, kw, weights):
-    """Head dims 68 to 96: one and two passes, few and many workgroups, key pieces, context lengths."""
+    """Head dims 68 to 96: one and two passes, few workgroups (in tiles of 128 features where few query tiles share the keys) and many,
+    key pieces, context lengths."""
     _check(nn, oracle, np.random.default_rng(E + Lkv), "f32", E, Lq, Lkv, B, H, expect="flash32", weights=weights, **kw)
 
 

@@ -40,6 +40,10 @@ CASES = [
     ("f32", 128, 100, 100, 1, 2, True, False, "flash32"),
     ("f32", 128, 150, 100, 2, 2, False, True, "flash32"),       # at most 128 keys with the weights returned: the resident kernel
     ("f32", 96, 128, 128, 1, 2, True, True, "flash32"),
+    ("f32", 160, 60, 600, 2, 2, False, False, "flash32"),       # head dims 68 to 96: one round of the chip, in tiles of 128 features
+    ("f32", 640, 40, 530, 33, 8, False, False, "flash32"),      # more than a round, of 96
+    ("f32", 192, 520, 520, 13, 2, True, False, "flash32"),      # causal: 130 workgroups, of 128
+    ("f32", 144, 520, 520, 2, 2, True, True, "flash32"),
     ("bf16", 128, 70, 200, 2, 2, False, False, "flash16"),
     ("bf16", 256, 130, 130, 2, 2, True, True, "flash16"),
     ("f16", 128, 64, 4096, 1, 2, False, False, "flash16"),      # few query tiles, long keys: split-kv + merge
