@@ -205,10 +205,10 @@ def test_gradient_of_a_shared_bias_apart_from_dq(nn, oracle, dtype, D, H, Lq, Lk
 ])
 def test_both_key_gradients_in_one_pass(nn, oracle, dtype, D, H, Lq, Lkv, B, mask_kind, biased, dropout):
     """Tiles of 64 features and more than 256 workgroups of 128 keys (with a causal mask 400, 512 beyond eight key tiles); with a padding
-    mask, more than 215 of sequences of three quarters of the keys."""
+    mask, more than 217 of sequences of three quarters of the keys."""
     tiles = (Lkv + 127) // 128
     assert Lkv > 256 and tiles * H * B > (256 if mask_kind != "causal" else 400 if tiles <= 8 else 512)
-    assert mask_kind not in ("lengths", "keys") or D <= 32 or H * B * (3 * Lkv + 256) > 215 * 4 * 128
+    assert mask_kind not in ("lengths", "keys") or D <= 32 or H * B * (3 * Lkv + 256) > 217 * 4 * 128
     _run(nn, oracle, dtype, D * H, D * H, Lq, Lkv, (B,), H, bias_shape=(Lkv, Lq, H, 1) if biased else None, mask_kind=mask_kind,
          seed=Lq + Lkv, scale=0.6, saved=True, dropout=dropout, expect="flash16")
 
@@ -218,7 +218,7 @@ def test_both_key_gradients_in_one_pass(nn, oracle, dtype, D, H, Lq, Lkv, B, mas
 ])
 def test_key_gradients_of_few_padded_sequences(nn, oracle, dtype, D, H, Lq, Lkv, B, mask_kind, dropout):
     """Little more than 256 workgroups of 128 keys, of which padding leaves one round: the fused kernel and the pair."""
-    assert (Lkv + 127) // 128 * H * B > 256 and H * B * (3 * Lkv + 256) <= 215 * 4 * 128
+    assert (Lkv + 127) // 128 * H * B > 256 and H * B * (3 * Lkv + 256) <= 217 * 4 * 128
     _run(nn, oracle, dtype, D * H, D * H, Lq, Lkv, (B,), H, mask_kind=mask_kind, seed=Lq + Lkv, scale=0.6, saved=True, dropout=dropout,
          expect="flash16")
 
