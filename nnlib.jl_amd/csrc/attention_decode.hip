@@ -365,6 +365,11 @@ __global__ __launch_bounds__(256) void decode_weights_kernel(DecodeArgs a, TW *w
 // queries per wavefront: 1, 2, or 4 (three queries run as four)
 int decode_nq(const AttnParams &p) { return p.Lq <= 1 ? 1 : p.Lq == 2 ? 2 : 4; }
 
+// Bytes of the partial results of ns splits, then (weights requested) the raw scores and the final statistics
+size_t workspace_of(const AttnParams &p, size_t ns) {
+    return sizeof(float) * (ns * (size_t)(p.B * p.Lq) * (size_t)(p.E + 2 * p.H) + (p.weights ? (size_t)(p.Lkv * p.H * p.B + 2 * p.H * p.B) : 0));
+}
+
 // Share of the chip at work when every (segment, batch element, query group) has n workgroups: compute units in the last of the
 // rounds of 256 workgroups, wavefronts in the last 8-row blocks.
 double share_at_work(int64_t pairs, int64_t blocks, int64_t n) {
@@ -411,6 +416,8 @@ int pick_nsplit(const AttnParams &p) {
         const double enough = pairs > 256 ? 0.88 : 0.8;
         double best = 0.0;
         for (int64_t n = first; n <= maxs && (n == first || (n <= 16 && n * pairs * decode_nq(p) <= 8192)) && best < enough; n++) {
+            // scores that the built-in workspace holds beside one workgroup's results stay in it
+            if (n > first && p.weights && workspace_of(p, (size_t)n) > MI_ATTN_STATIC_WORKSPACE_BYTES && workspace_of(p, (size_t)first) <= MI_ATTN_STATIC_WORKSPACE_BYTES) break;
             const double share = share_at_work(pairs, all, n);
             if (share > best) {
                 best = share;
@@ -439,9 +446,7 @@ bool attention_decode_supports(const AttnParams &p) {
 }
 
 size_t attention_decode_workspace(const AttnParams &p) {
-    const size_t ns = (size_t)pick_nsplit(p);
-    // partial results of the splits, then (weights requested) the raw scores and the final statistics
-    return sizeof(float) * (ns * (size_t)(p.B * p.Lq) * (size_t)(p.E + 2 * p.H) + (p.weights ? (size_t)(p.Lkv * p.H * p.B + 2 * p.H * p.B) : 0));
+    return workspace_of(p, (size_t)pick_nsplit(p));
 }
 
 int32_t launch_attention_decode(const AttnParams &p, hipStream_t st) {

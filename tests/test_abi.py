@@ -76,6 +76,16 @@ def test_plan_validation_status_codes(L):
         L.check(L.MI_ESHAPE, L.DimensionMismatch)
 
 
+@pytest.mark.parametrize("D,H,Lkv,B", [(128, 12, 1282, 448), (128, 64, 902, 115), (128, 32, 1185, 197)])
+def test_single_query_calls_with_weights_keep_the_builtin_workspace(L, D, H, Lkv, B):
+    """More pairs than compute units, and scores that leave room for one partial result per pair: no more of them than the built-in
+    workspace holds."""
+    rc, kern, ws = _plan(L, _desc(L, dtype=L.MI_BF16, weights_dtype=L.MI_BF16, E=D * H, Ev=D * H, H=H, Lq=1, Lkv=Lkv, B=B, weights=0x1000))
+    one = 4 * (B * (D + 2) * H + (Lkv + 2) * H * B)
+    assert rc == L.MI_OK and kern == L.KERNEL_DECODE and one <= L.MI_ATTN_STATIC_WORKSPACE_BYTES
+    assert one <= ws <= L.MI_ATTN_STATIC_WORKSPACE_BYTES
+
+
 def test_plan_kernel_selection(L):
     K = L.KERNEL_NAMES
     big = dict(E=4096, Ev=4096, H=32, Lq=4096, Lkv=4096, B=2)
